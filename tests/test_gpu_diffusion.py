@@ -84,3 +84,43 @@ def test_diffusion_vs_oracle(torch_dev, oracle, mech, workload, order, molar, ga
     assert np.allclose(src, want, rtol=1e-12, atol=1e-12 * np.abs(dc_o).max())
     assert np.array_equal(src[..., nsp + 1], src0[..., nsp + 1])
     print("   max |diff_corr| species %.3e, T %.3e" % (np.abs(dc_o[..., :nsp]).max(), np.abs(dc_o[..., nsp]).max()))
+
+
+@pytest.mark.parametrize("mech,nx,ny,nz,molar", [("h2", 1, 1, 1, True), ("gri30", 16, 16, 2, True),
+                                                 ("dme39", 257, 1, 3, False), ("h2", 33, 32, 5, True)])
+def test_second_order_workgroup_edges(torch_dev, oracle, mech, nx, ny, nz, molar):
+    """One cell, exactly one workgroup, one cell over, and over a strip of
+    workgroups; the row and column past the block are walls that hold NaN
+    species and diffusivities, which no flux may read.  Bound: as above, the
+    sums differ in their order only."""
+    torch = torch_dev
+    from tiger_nga_amd.finitechem import FiniteChem
+    sh = (nx + 2, ny + 2, nz + 2)
+    _, Y, T, rho, P, dt = inputs.states(mech, n=int(np.prod(sh)), seed=23)
+    nsp = Y.shape[1]
+    g = Grid.block(nx, ny, nz, nsp + 1, 1, nsp + 1, nover=1)
+    SC_ = np.zeros(sh + (nsp + 1,), order="F")
+    for k in range(nsp):
+        SC_[..., k] = Y[:, k].reshape(sh, order="F")
+    SC_[..., nsp] = T.reshape(sh, order="F")
+    RHO_ = np.asfortranarray(rho.reshape(sh, order="F"))
+    rng = np.random.default_rng(6)
+    DIFF_ = np.asfortranarray(10.0 ** rng.uniform(-5.0, -4.0, SC_.shape))
+    x, y = (np.cumsum(np.concatenate([[0.0], 1e-4 * (1.0 + 0.3 * rng.random(n))])) for n in sh[:2])
+    m = metric.cartesian(g, x, y, 1.1e-4, 2)
+    mask = np.zeros(g.mask_shape, dtype=np.int32, order="F")
+    mask[-1, :] = mask[:, -1] = 1
+    dc_o, gp_o = oracle.diffusion(mech, g, m, dt, RHO_, SC_, DIFF_, mask=mask, molar=molar)
+    for a in (SC_[..., :nsp], DIFF_):
+        a[-1] = a[:, -1] = np.nan
+    fc = FiniteChem(mech, 1e-6, 1e-12)
+    md = {k: (v if k in ("st1", "st2") else _dev(torch, np.asfortranarray(v))) for k, v in m.items()}
+    dc, gp = (_dev(torch, np.zeros(sh + (n,), order="F")) for n in (nsp + 1, 3))
+    fc.diffusion(dt, g, md, _dev(torch, RHO_), _dev(torch, SC_), _dev(torch, DIFF_), mask=_dev(torch, mask),
+                 diff_corr=dc, diff_gp=gp, molar=molar)
+    torch.cuda.synchronize()
+    fc.close()
+    for got, want in ((dc.cpu().numpy(), dc_o), (gp.cpu().numpy(), gp_o)):
+        for k in range(want.shape[-1]):
+            scale = max(np.abs(want[..., k]).max(), 1e-300)
+            assert np.abs(got[..., k] - want[..., k]).max() <= 1e-12 * scale + 1e-300, k

@@ -286,247 +286,309 @@ __global__ __launch_bounds__(256) void diff_main_kernel(DiffParams p) {
 }
 
 // ---- second order (st1 = 0, st2 = 1) ----------------------------------------
-// The same sums as the kernels above, in the same order, with what does not
-// depend on the species hoisted out of the species loop: the operator
-// coefficients, the molar factors w / W_gp and sum grad * W_gp (the molar
-// term's w (Y / W_gp) becomes (w / W_gp) Y: no division per species), the
-// correction velocity at each face; per species only Y and D at the cell and its six
-// neighbours are loaded (each once), instead of once per face and stencil
-// point.
+// Two passes over the species fields: diff_sums2_kernel (W_gp, cp_mix and the
+// correction velocities, whose species sums the second pass needs complete)
+// and diff_main2_kernel (the per-cell terms).  Both are bound by the rate at
+// which the L1 serves the loads of Y and D (0.6 accesses per clock and CU,
+// VALU busy a quarter of the time): each species costs a cell 8 (14) of them
+// and about 35 (105) FP64 instructions, so
+//   * everything that does not depend on the species is formed before the
+//     species loop (operator coefficients, w / W_gp, sum grad * W_gp, the
+//     correction velocity, and the products of the divergence and enthalpy
+//     weights), and the loop loads the next species while it computes one;
+//   * the cp coefficients are read from LDS, where the lanes of a wave differ
+//     only in the temperature range;
+//   * workgroups that share stencil planes run on the same XCD at the same
+//     time (Brick below), so that the y and z neighbours are L2 hits.
+// GRI-3.0 128^3, molar term on: 2.37 -> 1.36 ms a call (separate W_gp / cp pass
+// 0.25 ms and face sums 0.44 ms -> 0.53 ms; main 1.79 -> 0.83 ms).
 
-// correction velocities at the face cells (diff_face_kernel, st1 = 0, st2 = 1:
-// a face interpolates its cell and the one before it in each direction)
+// Order of the workgroups: 256 consecutive cells of a plane each, kStrip of
+// them side by side, then the next plane.  The hardware deals workgroups to
+// the 8 XCDs in turn, so XCD e (blockIdx % 8) takes the e-th contiguous piece
+// of that order: its resident workgroups cover a brick of kStrip chunks by
+// some 16 planes, whose halo is a third of its volume (GRI-3.0 128^3: 1394 us in
+// the order of the planes, 1415 / 1376 / 1376 / 1436 us with strips of 2 / 4 / 8 /
+// 16).
+constexpr int kXcd = 8, kStrip = 4;
+struct Brick {
+  int plane, nz, per_xcd;  // cells of a plane, planes, workgroups per XCD
+};
+
+__device__ __forceinline__ bool brick_cell(const Brick& b, int& q, int& z) {
+  const unsigned seq = (blockIdx.x % kXcd) * (unsigned)b.per_xcd + blockIdx.x / kXcd;
+  const unsigned per_strip = (unsigned)b.nz * kStrip;
+  const unsigned strip = seq / per_strip, r = seq - strip * per_strip;
+  z = (int)(r / kStrip);
+  q = (int)((strip * kStrip + r % kStrip) * 256 + threadIdx.x);
+  return q < b.plane;
+}
+
+// a[byte offset]: a wave-uniform base and a 32-bit lane offset (the launcher
+// checks that a plane has less than 2^32 bytes)
+__device__ __forceinline__ double ldo(const double* a, unsigned off) {
+  return *(const double*)((const char*)a + off);
+}
+
+// cp rows of the species in LDS, [species][T > tmid][6]
 template <int NEQ>
-__global__ __launch_bounds__(256) void diff_face2_kernel(DiffParams p) {
+__device__ __forceinline__ void stage_cp(double* cps, const char* tab) {
+  constexpr TabLayout L = tab_layout<NEQ>();
+  for (int t = threadIdx.x; t < (NEQ - 1) * 12; t += 256) {
+    const int k = t / 12, hi = (t / 6) % 2, c = t % 6;
+    cps[t] = *(const double*)(tab + L.th + (hi ? 0 : 13 * kRow) + (7 + c) * kRow + k * 8);
+  }
+  __syncthreads();
+}
+
+__device__ __forceinline__ double cp_lds(const double* c, double T) {
+  return c[0] * (c[1] + T * (c[2] + T * (c[3] + T * (c[4] + T * c[5]))));
+}
+
+// W_gp and cp_mix of the interior and one cell around it, correction
+// velocities at the face cells (diff_cell_kernel and diff_face_kernel; a face
+// interpolates its cell and the one before it).  The molar term
+// sum_k a_k (w0 Y0_k / W0 + w1 Y1_k / W1) is summed as (w0 / W0) sum a_k Y0_k +
+// (w1 / W1) sum a_k Y1_k, so that W_gp of the four cells can be summed in the
+// same pass instead of being read back.
+template <int NEQ, bool MOLAR>
+__global__ __launch_bounds__(256) void diff_sums2_kernel(DiffParams p, Brick bk) {
   constexpr int N = NEQ - 1;
+  constexpr TabLayout L = tab_layout<NEQ>();
+  __shared__ __attribute__((aligned(16))) double cps[N * 12];
+  stage_cp<NEQ>(cps, p.mech.tab);
   const DiffGeom& g = p.gm;
   const tgr_metric_dev& m = p.m;
-  const int fi0 = g.imin_, fni = g.imax_ + 1 - fi0 + 1;
-  const int fj0 = g.jmin_, fnj = g.jmax_ + 1 - fj0 + 1;
-  const int fk0 = g.kmin_, fnk = g.kmax_ + 1 - fk0 + 1;
-  const int64_t n = (int64_t)fni * fnj * fnk;
-  const int64_t sy = g.nxo, sz = (int64_t)g.nxo * g.nyo;
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
-    const int i = fi0 + (int)(q % fni), j = fj0 + (int)((q / fni) % fnj), k = fk0 + (int)(q / ((int64_t)fni * fnj));
-    const int64_t o = c3(g, i, j, k);
-    double vx = 0.0, vy = 0.0, vz = 0.0;
-    if (!wall(g, p.mask, i, j)) {
-      // coefficients of the two stencil points (s = -1, 0) per direction
-      double w[3][2], gg[3][2], wi[3][2], gw[3];
-      const int64_t nb[3] = {o - 1, o - sy, o - sz};
+  int q, z;
+  if (!brick_cell(bk, q, z)) return;
+  const int fni = g.imax_ + 1 - g.imin_ + 1, fnj = g.jmax_ + 1 - g.jmin_ + 1;  // face range
+  const int i = g.imin_ - 1 + q % (fni + 1), j = g.jmin_ - 1 + q / (fni + 1), k = g.kmin_ - 1 + z;
+  const int64_t o = c3(g, i, j, k);
+  const bool face = i >= g.imin_ && j >= g.jmin_ && k >= g.kmin_;
+  if (wall(g, p.mask, i, j)) {
+    p.wg[o] = 1.0;
+    p.cpm[o] = 0.0;
+    if (face) p.cvel[o] = p.cvel[g.plane + o] = p.cvel[2 * g.plane + o] = 0.0;
+    return;
+  }
+  const double T = p.sc[(int64_t)g.isc_T0 * g.plane + o];
+  // offsets of the cell and of the ones before it (the cell itself outside the face range)
+  const unsigned oc = (unsigned)o * 8u;
+  unsigned on[3] = {oc, oc, oc};
+  double w[3][2] = {}, gg[3][2] = {};
+  bool wn[3] = {false, false, false};
+  if (face) {
+    on[0] = oc - 8u;
+    on[1] = oc - (unsigned)g.nxo * 8u;
+    on[2] = oc - (unsigned)g.nxo * (unsigned)g.nyo * 8u;
+    wn[0] = wall(g, p.mask, i - 1, j);
+    wn[1] = wall(g, p.mask, i, j - 1);
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int s = t - 1;
-        w[0][t] = op(m.interp_sc_x, i, fi0, fni, j, g.jmino_, g.nyo, s, -1);
-        w[1][t] = op(m.interp_sc_y, i, g.imino_, g.nxo, j, fj0, fnj, s, -1);
-        w[2][t] = op(m.interp_sc_z, i, g.imino_, g.nxo, j, fj0, fnj, s, -1);
-        gg[0][t] = op(m.grad_x, i, fi0, fni, j, fj0, fnj, s, -1);
-        gg[1][t] = op(m.grad_y, i, fi0, fni, j, fj0, fnj, s, -1);
-        gg[2][t] = op(m.grad_z, i, fi0, fni, j, fj0, fnj, s, -1);
-      }
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        gw[d] = 0.0;
-        if (p.molar) {
-          const double w0 = p.wg[nb[d]], w1 = p.wg[o];
-          gw[d] += gg[d][0] * w0;
-          gw[d] += gg[d][1] * w1;
-          wi[d][0] = 1.0 / w0;
-          wi[d][1] = 1.0 / w1;
-        }
-      }
-      double acc[3] = {0.0, 0.0, 0.0};
-#pragma unroll 2
-      for (int sp = 0; sp < N; ++sp) {
-        const double* Y = p.sc + (int64_t)(g.isc_sc0 + sp) * g.plane;
-        const double* D = p.diff + (int64_t)(g.isc_sc0 + sp) * g.plane;
-        const double yc = Y[o], dc = D[o];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          const double y0 = Y[nb[d]], d0 = D[nb[d]];
-          double a = 0, b = 0, ii = 0;
-          a += w[d][0] * d0;
-          b += gg[d][0] * y0;
-          a += w[d][1] * dc;
-          b += gg[d][1] * yc;
-          acc[d] += a * b;
-          if (p.molar) {
-            ii += w[d][0] * (y0 * wi[d][0]);
-            ii += w[d][1] * (yc * wi[d][1]);
-            acc[d] += a * ii * gw[d];
-          }
-        }
-      }
-      vx = acc[0];
-      vy = acc[1];
-      vz = acc[2];
+    for (int t = 0; t < 2; ++t) {
+      w[0][t] = op(m.interp_sc_x, i, g.imin_, fni, j, g.jmino_, g.nyo, t - 1, -1);
+      w[1][t] = op(m.interp_sc_y, i, g.imino_, g.nxo, j, g.jmin_, fnj, t - 1, -1);
+      w[2][t] = op(m.interp_sc_z, i, g.imino_, g.nxo, j, g.jmin_, fnj, t - 1, -1);
+      gg[0][t] = op(m.grad_x, i, g.imin_, fni, j, g.jmin_, fnj, t - 1, -1);
+      gg[1][t] = op(m.grad_y, i, g.imin_, fni, j, g.jmin_, fnj, t - 1, -1);
+      gg[2][t] = op(m.grad_z, i, g.imin_, fni, j, g.jmin_, fnj, t - 1, -1);
     }
-    p.cvel[o] = vx;
-    p.cvel[g.plane + o] = vy;
-    p.cvel[2 * g.plane + o] = vz;
+  }
+  const double* __restrict__ Y = p.sc + (int64_t)g.isc_sc0 * g.plane;
+  const double* __restrict__ D = p.diff + (int64_t)g.isc_sc0 * g.plane;
+  const TGR_CONST double* iw = (const TGR_CONST double*)(p.mech.tab + L.iw);  // 1 / W_k
+  const double* cr = cps + (T > p.mech.tmid ? 6 : 0);
+  double yc = ldo(Y, oc), dc = ldo(D, oc), yn[3], dn[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) yn[d] = ldo(Y, on[d]), dn[d] = ldo(D, on[d]);
+  double fick[3] = {}, m0[3] = {}, m1[3] = {}, s1 = 0.0, s2 = 0.0, t1[3] = {}, t2[3] = {}, cp = 0.0;
+#pragma unroll 1
+  for (int sp = 0; sp < N; ++sp) {
+    const int64_t step = sp + 1 < N ? g.plane : 0;
+    Y += step;
+    D += step;
+    const double yc2 = ldo(Y, oc), dc2 = ldo(D, oc);
+    double yn2[3], dn2[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) yn2[d] = ldo(Y, on[d]), dn2[d] = ldo(D, on[d]);
+    const double r = iw[sp];
+    const double y = fmin(fmax(yc, 0.0), 1.0);
+    s1 += y;
+    s2 = fma(y, r, s2);
+    cp += yc * cp_lds(cr + sp * 12, T);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const double a = w[d][0] * dn[d] + w[d][1] * dc;
+      fick[d] += a * (gg[d][0] * yn[d] + gg[d][1] * yc);
+      if constexpr (MOLAR) {
+        m0[d] = fma(a, yn[d], m0[d]);
+        m1[d] = fma(a, yc, m1[d]);
+        const double yt = fmin(fmax(yn[d], 0.0), 1.0);
+        t1[d] += yt;
+        t2[d] = fma(yt, r, t2[d]);
+      }
+    }
+    yc = yc2;
+    dc = dc2;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) yn[d] = yn2[d], dn[d] = dn2[d];
+  }
+  const double wc = s1 / s2;
+  p.wg[o] = wc;
+  p.cpm[o] = p.cv ? cp - 8314.34 / wc : cp;
+  if (!face) return;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    double v = fick[d];
+    if constexpr (MOLAR) {
+      const double wb = wn[d] ? 1.0 : t1[d] / t2[d];
+      v += (w[d][0] / wb * m0[d] + w[d][1] / wc * m1[d]) * (gg[d][0] * wb + gg[d][1] * wc);
+    }
+    p.cvel[d * g.plane + o] = v;
   }
 }
 
-// the per-cell terms (diff_main_kernel, st1 = 0, st2 = 1: faces at the cell
-// and the next one in each direction, each interpolating two cells).  The
-// species loop reads the operator coefficients through restrict pointers, so
-// that the compiler keeps the loop-invariant ones in registers as far as they
-// fit; per species it loads Y and D at the cell and its six neighbours once.
-template <int NEQ>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void diff_main2_kernel(DiffParams p) {
-  constexpr TabLayout L = tab_layout<NEQ>();
+// The per-cell terms (diff_main_kernel: faces at the cell and the next one in
+// each direction, each interpolating two cells).  Per face and species, with
+// the weights below, a = w0 D0 + w1 D1, the Fickian flux f = a (g0 Y0 + g1 Y1) and
+// the correction c = v (w0 Y0 + w1 Y1) + a (u0 Y0 + u1 Y1); the species term sums
+// dv c, the enthalpy flux cp_k sum e (c + f), the dump dv c and dv f.
+struct FaceW {
+  double w0, w1, g0, g1;  // interpolation and gradient weights
+  double v, u0, u1;       // -correction velocity; molar term: w / W_gp times sum grad * W_gp
+  double dv, e;           // divergence weight; interp_m weight times the cell's T gradient
+};
+
+// Y and D at a cell and its neighbours: the cell, then -, + in x, y, z
+struct Stencil {
+  double y[7], d[7];
+};
+
+__device__ __forceinline__ void load_stencil(Stencil& s, const double* Y, const double* D, unsigned oc, unsigned oxp,
+                                             unsigned oyp, int64_t sy, int64_t sz) {
+  s.y[0] = ldo(Y, oc), s.d[0] = ldo(D, oc);
+  s.y[1] = ldo(Y - 1, oc), s.d[1] = ldo(D - 1, oc);
+  s.y[2] = ldo(Y, oxp), s.d[2] = ldo(D, oxp);
+  s.y[3] = ldo(Y - sy, oc), s.d[3] = ldo(D - sy, oc);
+  s.y[4] = ldo(Y, oyp), s.d[4] = ldo(D, oyp);
+  s.y[5] = ldo(Y - sz, oc), s.d[5] = ldo(D - sz, oc);
+  s.y[6] = ldo(Y + sz, oc), s.d[6] = ldo(D + sz, oc);
+}
+
+template <int NEQ, bool MOLAR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void diff_main2_kernel(DiffParams p, Brick bk) {
   constexpr int N = NEQ - 1;
+  __shared__ __attribute__((aligned(16))) double cps[N * 12];
+  stage_cp<NEQ>(cps, p.mech.tab);
   const DiffGeom& g = p.gm;
-  const int nx = g.imax_ - g.imin_ + 1, ny = g.jmax_ - g.jmin_ + 1, nz = g.kmax_ - g.kmin_ + 1;
-  const int fi0 = g.imin_, fni = nx + 1, fj0 = g.jmin_, fnj = ny + 1;
-  const int64_t n = (int64_t)nx * ny * nz;
+  int q, z;
+  if (!brick_cell(bk, q, z)) return;
+  const int nx = g.imax_ - g.imin_ + 1, ny = g.jmax_ - g.jmin_ + 1;
+  const int fni = nx + 1, fnj = ny + 1;
+  const int i = g.imin_ + q % nx, j = g.jmin_ + q / nx, k = g.kmin_ + z;
+  if (wall(g, p.mask, i, j)) return;
+  const int64_t o = c3(g, i, j, k);
   const int64_t sy = g.nxo, sz = (int64_t)g.nxo * g.nyo;
-  const double* __restrict__ isx = p.m.interp_sc_x;
-  const double* __restrict__ isy = p.m.interp_sc_y;
-  const double* __restrict__ isz = p.m.interp_sc_z;
-  const double* __restrict__ grx = p.m.grad_x;
-  const double* __restrict__ gry = p.m.grad_y;
-  const double* __restrict__ grz = p.m.grad_z;
-  const double* __restrict__ dvu = p.m.div_u;
-  const double* __restrict__ dvv = p.m.div_v;
-  const double* __restrict__ dvw = p.m.div_w;
-  const double* __restrict__ imx = p.m.interp_u_xm;
-  const double* __restrict__ imy = p.m.interp_v_ym;
-  const double* __restrict__ imz = p.m.interp_w_zm;
-  const double* __restrict__ sc = p.sc;
-  const double* __restrict__ df = p.diff;
-  const double* __restrict__ wgp = p.wg;
-  const double* __restrict__ cpm = p.cpm;
-  const double* __restrict__ cvel = p.cvel;
-  const char* __restrict__ tab = p.mech.tab;
+  const int64_t step[3] = {1, sy, sz};
+  const double* Tf = p.sc + (int64_t)g.isc_T0 * g.plane;
+  const double T = Tf[o];
+  // cell gradients of T and cp_mix (stp = 1)
+  double tg[3] = {}, cg[3] = {};
+#pragma unroll
+  for (int s = -1; s <= 1; ++s)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const double* gm = d == 0 ? p.m.grad_xm : (d == 1 ? p.m.grad_ym : p.m.grad_zm);
+      const double c = op(gm, i, g.imin_, nx, j, g.jmin_, ny, s, -1);
+      tg[d] += c * Tf[o + s * step[d]];
+      cg[d] += c * p.cpm[o + s * step[d]];
+    }
+  // wall faces carry no flux (the z faces of a non-wall cell are never walls):
+  // weights 0 and the cell itself as the neighbour, whose values are finite
+  const bool live[3] = {!wall(g, p.mask, i + 1, j), !wall(g, p.mask, i, j + 1), true};
+  FaceW fw[3][2];
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      // the face cell is (i, j, k) + f along d; its two points are (-1, 0) for f = 0 and (0, +1) for f = 1
+      FaceW& F = fw[d][f];
+      F = FaceW{};
+      if (f && !live[d]) continue;
+      const int fi = d == 0 ? i + f : i, fj = d == 1 ? j + f : j;
+      const int64_t fo = o + f * step[d];
+      if (d == 0) {
+        F.w0 = op(p.m.interp_sc_x, fi, g.imin_, fni, fj, g.jmino_, g.nyo, -1, -1);
+        F.w1 = op(p.m.interp_sc_x, fi, g.imin_, fni, fj, g.jmino_, g.nyo, 0, -1);
+      } else {
+        const double* ws = d == 1 ? p.m.interp_sc_y : p.m.interp_sc_z;
+        F.w0 = op(ws, fi, g.imino_, g.nxo, fj, g.jmin_, fnj, -1, -1);
+        F.w1 = op(ws, fi, g.imino_, g.nxo, fj, g.jmin_, fnj, 0, -1);
+      }
+      const double* gs = d == 0 ? p.m.grad_x : (d == 1 ? p.m.grad_y : p.m.grad_z);
+      F.g0 = op(gs, fi, g.imin_, fni, fj, g.jmin_, fnj, -1, -1);
+      F.g1 = op(gs, fi, g.imin_, fni, fj, g.jmin_, fnj, 0, -1);
+      F.v = -p.cvel[d * g.plane + fo];
+      if constexpr (MOLAR) {
+        const double wa = p.wg[fo - step[d]], wb = p.wg[fo];
+        const double gw = F.g0 * wa + F.g1 * wb;
+        F.u0 = F.w0 / wa * gw;
+        F.u1 = F.w1 / wb * gw;
+      }
+      const double* dv = d == 0 ? p.m.div_u : (d == 1 ? p.m.div_v : p.m.div_w);
+      const double* im = d == 0 ? p.m.interp_u_xm : (d == 1 ? p.m.interp_v_ym : p.m.interp_w_zm);
+      F.dv = op(dv, i, g.imin_, nx, j, g.jmin_, ny, f, 0);
+      F.e = op(im, i, g.imin_, nx, j, g.jmin_, ny, f, 0) * tg[d];
+    }
+  const unsigned oc = (unsigned)o * 8u;
+  const unsigned oxp = live[0] ? oc + 8u : oc, oyp = live[1] ? oc + (unsigned)sy * 8u : oc;
+  const double* __restrict__ Y = p.sc + (int64_t)g.isc_sc0 * g.plane;
+  const double* __restrict__ D = p.diff + (int64_t)g.isc_sc0 * g.plane;
+  const double* cr = cps + (T > p.mech.tmid ? 6 : 0);
   double* __restrict__ corr = p.corr;
   double* __restrict__ src = p.src;
   double* __restrict__ dgp = p.dgp;
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
-    const int i = g.imin_ + (int)(q % nx), j = g.jmin_ + (int)((q / nx) % ny), k = g.kmin_ + (int)(q / ((int64_t)nx * ny));
-    const int64_t o = c3(g, i, j, k);
-    if (wall(g, p.mask, i, j)) continue;
-    const double* Tf = sc + (int64_t)g.isc_T0 * g.plane;
-    const double T = Tf[o];
-    // cell gradients of T and cp_mix (stp = 1)
-    double tx = 0, ty = 0, tz = 0, cx = 0, cy = 0, cz = 0;
-#pragma unroll
-    for (int s = -1; s <= 1; ++s) {
-      const double gxm = op(p.m.grad_xm, i, g.imin_, nx, j, g.jmin_, ny, s, -1);
-      const double gym = op(p.m.grad_ym, i, g.imin_, nx, j, g.jmin_, ny, s, -1);
-      const double gzm = op(p.m.grad_zm, i, g.imin_, nx, j, g.jmin_, ny, s, -1);
-      tx += gxm * Tf[o + s];
-      ty += gym * Tf[o + s * sy];
-      tz += gzm * Tf[o + s * sz];
-      cx += gxm * cpm[o + s];
-      cy += gym * cpm[o + s * sy];
-      cz += gzm * cpm[o + s * sz];
-    }
-    const int64_t step[3] = {1, sy, sz};
-    // wall faces carry no flux (the z faces of a non-wall cell are never walls)
-    const bool live[3][2] = {{true, !wall(g, p.mask, i + 1, j)}, {true, !wall(g, p.mask, i, j + 1)}, {true, true}};
-    // per face (d, f) what does not depend on the species: the interpolation
-    // and gradient weights of its two points, the correction velocity and,
-    // for the molar term, w_m / W_gp,m and sum_m grad_m W_gp,m (the
-    // reference's SC / W_gp then reads (w_m / W_gp,m) Y_m: no division in the
-    // species loop)
-    double fw0[3][2], fw1[3][2], fg0[3][2], fg1[3][2], fcv[3][2], fu0[3][2], fu1[3][2], fgw[3][2];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-#pragma unroll
-      for (int f = 0; f < 2; ++f) {
-        // the face cell is (i, j, k) + f along d; its two points are
-        // (-1, 0) for f = 0 and (0, +1) for f = 1
-        const int fi = d == 0 ? i + f : i, fj = d == 1 ? j + f : j;
-        const int64_t fo = o + f * step[d];
-        double w0, w1;
-        if (d == 0) {
-          w0 = op(isx, fi, fi0, fni, fj, g.jmino_, g.nyo, -1, -1);
-          w1 = op(isx, fi, fi0, fni, fj, g.jmino_, g.nyo, 0, -1);
-        } else {
-          const double* ws = d == 1 ? isy : isz;
-          w0 = op(ws, fi, g.imino_, g.nxo, fj, fj0, fnj, -1, -1);
-          w1 = op(ws, fi, g.imino_, g.nxo, fj, fj0, fnj, 0, -1);
-        }
-        const double* gs = d == 0 ? grx : (d == 1 ? gry : grz);
-        const double g0 = op(gs, fi, fi0, fni, fj, fj0, fnj, -1, -1);
-        const double g1 = op(gs, fi, fi0, fni, fj, fj0, fnj, 0, -1);
-        fw0[d][f] = w0;
-        fw1[d][f] = w1;
-        fg0[d][f] = g0;
-        fg1[d][f] = g1;
-        fcv[d][f] = -cvel[(int64_t)d * g.plane + fo];
-        if (p.molar) {
-          const double wa = wgp[fo - step[d]], wb = wgp[fo];
-          fu0[d][f] = w0 / wa;
-          fu1[d][f] = w1 / wb;
-          fgw[d][f] = g0 * wa + g1 * wb;
-        } else {
-          fu0[d][f] = fu1[d][f] = fgw[d][f] = 0.0;
-        }
-      }
-    }
-    double eT = 0.0;  // temperature term before the cp-gradient part and / cp
+  double eT = 0.0;  // temperature term before the cp-gradient part and / cp
+  Stencil s;
+  load_stencil(s, Y, D, oc, oxp, oyp, sy, sz);
 #pragma unroll 1
-    for (int sp = 0; sp < N; ++sp) {
-      const double* Y = sc + (int64_t)(g.isc_sc0 + sp) * g.plane;
-      const double* D = df + (int64_t)(g.isc_sc0 + sp) * g.plane;
-      const double yc = Y[o], dc = D[o];
-      double dcor = 0.0, dfick = 0.0, fm[3] = {0.0, 0.0, 0.0};
-      double fc[3][2], ff[3][2];
+  for (int sp = 0; sp < N; ++sp) {
+    const int64_t next = sp + 1 < N ? g.plane : 0;
+    Y += next;
+    D += next;
+    Stencil s2;
+    load_stencil(s2, Y, D, oc, oxp, oyp, sy, sz);
+    double dcor = 0.0, dfick = 0.0, en = 0.0;
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        const double ym = Y[o - step[d]], yp = Y[o + step[d]], dm = D[o - step[d]], dp = D[o + step[d]];
-#pragma unroll
-        for (int f = 0; f < 2; ++f) {
-          const double y0 = f ? yc : ym, y1 = f ? yp : yc;
-          const double d0 = f ? dc : dm, d1 = f ? dp : dc;
-          const double w0 = fw0[d][f], w1 = fw1[d][f], g0 = fg0[d][f], g1 = fg1[d][f];
-          double syf = 0, a = 0, b = 0;
-          syf += w0 * y0;
-          a += w0 * d0;
-          b += g0 * y0;
-          syf += w1 * y1;
-          a += w1 * d1;
-          b += g1 * y1;
-          double c = fcv[d][f] * syf;
-          if (p.molar) c += a * (fu0[d][f] * y0 + fu1[d][f] * y1) * fgw[d][f];
-          fc[d][f] = live[d][f] ? c : 0.0;
-          ff[d][f] = live[d][f] ? a * b : 0.0;
-        }
+        const FaceW& F = fw[d][f];
+        const double y0 = f ? s.y[0] : s.y[2 * d + 1], y1 = f ? s.y[2 * d + 2] : s.y[0];
+        const double d0 = f ? s.d[0] : s.d[2 * d + 1], d1 = f ? s.d[2 * d + 2] : s.d[0];
+        const double a = F.w0 * d0 + F.w1 * d1;
+        double c = F.v * (F.w0 * y0 + F.w1 * y1);
+        if constexpr (MOLAR) c += a * (F.u0 * y0 + F.u1 * y1);
+        const double fick = a * (F.g0 * y0 + F.g1 * y1);
+        dcor += F.dv * c;
+        dfick += F.dv * fick;
+        en += F.e * (c + fick);
       }
-#pragma unroll
-      for (int f = 0; f < 2; ++f) {
-        const double du = op(dvu, i, g.imin_, nx, j, g.jmin_, ny, f, 0);
-        const double dv = op(dvv, i, g.imin_, nx, j, g.jmin_, ny, f, 0);
-        const double dw = op(dvw, i, g.imin_, nx, j, g.jmin_, ny, f, 0);
-        dcor += du * fc[0][f] + dv * fc[1][f] + dw * fc[2][f];
-        dfick += du * ff[0][f] + dv * ff[1][f] + dw * ff[2][f];
-        fm[0] += op(imx, i, g.imin_, nx, j, g.jmin_, ny, f, 0) * (fc[0][f] + ff[0][f]);
-        fm[1] += op(imy, i, g.imin_, nx, j, g.jmin_, ny, f, 0) * (fc[1][f] + ff[1][f]);
-        fm[2] += op(imz, i, g.imin_, nx, j, g.jmin_, ny, f, 0) * (fc[2][f] + ff[2][f]);
-      }
-      double cpk;
-      cp_species(tab, L, p.mech.tmid, T, sp, cpk);
-      eT = eT + cpk * fm[0] * tx;
-      eT = eT + cpk * fm[1] * ty;
-      eT = eT + cpk * fm[2] * tz;
-      if (corr) corr[(int64_t)sp * g.plane + o] = dcor * p.dt;
-      if (src) src[(int64_t)(g.isc_sc0 + sp) * g.plane + o] += dcor * p.dt;
-      if (dgp) {
-        const int slot = sp == p.i_h2o ? 0 : (sp == p.i_co ? 1 : (sp == p.i_co2 ? 2 : -1));
-        if (slot >= 0) dgp[(int64_t)slot * g.plane + o] = dfick + dcor;
-      }
+    eT += cp_lds(cr + sp * 12, T) * en;
+    if (corr) corr[(int64_t)sp * g.plane + o] = dcor * p.dt;
+    if (src) src[(int64_t)(g.isc_sc0 + sp) * g.plane + o] += dcor * p.dt;
+    if (dgp) {
+      const int slot = sp == p.i_h2o ? 0 : (sp == p.i_co ? 1 : (sp == p.i_co2 ? 2 : -1));
+      if (slot >= 0) dgp[(int64_t)slot * g.plane + o] = dfick + dcor;
     }
-    if (p.gasrad) eT += gas_radiation(p, T, o);
-    const double dT = df[(int64_t)g.isc_T0 * g.plane + o];
-    eT = eT + dT * cx * tx;
-    eT = eT + dT * cy * ty;
-    eT = eT + dT * cz * tz;
-    eT = eT / cpm[o] * p.dt;
-    if (corr) corr[(int64_t)N * g.plane + o] = eT;
-    if (src) src[(int64_t)g.isc_T0 * g.plane + o] += eT;
+    s = s2;
   }
+  if (p.gasrad) eT += gas_radiation(p, T, o);
+  const double dT = p.diff[(int64_t)g.isc_T0 * g.plane + o];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) eT = eT + dT * cg[d] * tg[d];
+  eT = eT / p.cpm[o] * p.dt;
+  if (corr) corr[(int64_t)N * g.plane + o] = eT;
+  if (src) src[(int64_t)g.isc_T0 * g.plane + o] += eT;
 }
 
 }  // namespace tgr
@@ -542,14 +604,25 @@ extern "C" int tgr_launch_diffusion(const DiffParams* p, int neq, hipStream_t s)
   const int64_t nint = (int64_t)(g.imax_ - g.imin_ + 1) * (g.jmax_ - g.jmin_ + 1) * (g.kmax_ - g.kmin_ + 1);
   auto blocks = [](int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 256, 65535); };
   // second order (the reference's default stencil) has its own pair of
-  // kernels; other orders take the general ones
-  const bool o2 = st1 == 0 && st2 == 1;
+  // kernels, which address a plane by 32-bit byte offsets; other orders and
+  // larger planes take the general ones
+  const bool o2 = st1 == 0 && st2 == 1 && g.plane < ((int64_t)1 << 29);
+  auto brick = [](int64_t ni, int64_t nj, int64_t nk) {
+    const int64_t pl = ni * nj, chunks = (pl + 255) / 256, strips = (chunks + kStrip - 1) / kStrip;
+    return Brick{(int)pl, (int)nk, (int)((strips * kStrip * nk + kXcd - 1) / kXcd)};
+  };
+  const int nx = g.imax_ - g.imin_ + 1, ny = g.jmax_ - g.jmin_ + 1, nz = g.kmax_ - g.kmin_ + 1;
+  const Brick bs = brick(nx + 2, ny + 2, nz + 2), bm = brick(nx, ny, nz);
+#define TGR_DIFF_LAUNCH2(NEQ_, MOLAR_)                                                                        \
+  hipLaunchKernelGGL((diff_sums2_kernel<NEQ_, MOLAR_>), dim3(bs.per_xcd * kXcd), dim3(256), 0, s, *p, bs);   \
+  hipLaunchKernelGGL((diff_main2_kernel<NEQ_, MOLAR_>), dim3(bm.per_xcd * kXcd), dim3(256), 0, s, *p, bm);
 #define TGR_DIFF_LAUNCH(NEQ_)                                                                  \
-  hipLaunchKernelGGL(diff_cell_kernel<NEQ_>, dim3(blocks(ncell)), dim3(256), 0, s, *p);       \
-  if (o2) {                                                                                     \
-    hipLaunchKernelGGL(diff_face2_kernel<NEQ_>, dim3(blocks(nface)), dim3(256), 0, s, *p);    \
-    hipLaunchKernelGGL(diff_main2_kernel<NEQ_>, dim3(blocks(nint)), dim3(256), 0, s, *p);     \
+  if (o2 && p->molar) {                                                                         \
+    TGR_DIFF_LAUNCH2(NEQ_, true)                                                                \
+  } else if (o2) {                                                                              \
+    TGR_DIFF_LAUNCH2(NEQ_, false)                                                               \
   } else {                                                                                      \
+    hipLaunchKernelGGL(diff_cell_kernel<NEQ_>, dim3(blocks(ncell)), dim3(256), 0, s, *p);     \
     hipLaunchKernelGGL(diff_face_kernel<NEQ_>, dim3(blocks(nface)), dim3(256), 0, s, *p);     \
     hipLaunchKernelGGL(diff_main_kernel<NEQ_>, dim3(blocks(nint)), dim3(256), 0, s, *p);      \
   }
@@ -561,5 +634,6 @@ extern "C" int tgr_launch_diffusion(const DiffParams* p, int neq, hipStream_t s)
     default: return -1;
   }
 #undef TGR_DIFF_LAUNCH
+#undef TGR_DIFF_LAUNCH2
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }

@@ -38,8 +38,11 @@ constexpr double UROUND = 2.2204460492503131e-16;
 enum { NF_FIRST = 0, NF_PREV_CONV = 1, NF_PREV_ERR = 2, NF_OK = 3, NF_CONV_FAIL = 4, NF_TRY_AGAIN = 5 };
 enum { CF_NONE = 0, CF_BAD_J = 1, CF_OTHER = 2 };
 
-// x^y for x >= 0 through the project's exp/log (step-size ratios only)
-__device__ __forceinline__ double rpow(double x, double y) { return fexp(y * flog(x)); }
+// x^y for x >= 0 through the project's 2^x / log2 (step-size ratios only)
+__device__ __forceinline__ double rpow(double x, double y) {
+  const double v = fexp2(y * flog2(x));
+  return x == 0.0 || x == INFINITY ? ((x == 0.0) == (y > 0.0) ? 0.0 : INFINITY) : v;
+}
 
 template <class T, int N>
 __device__ __forceinline__ T pick(const T (&a)[N], int i) {

@@ -49,6 +49,11 @@ constexpr double kTroeN1 = (double)1.27f;
 constexpr double kTroeC0 = (double)0.4f;
 constexpr double kTroeC1 = (double)0.67f;
 constexpr double kTroeD = (double)0.14f;
+// temperature unit of the rate constants: |log2(T / 512)| stays below 2.3 from
+// 105 to 2500 K, where log2 T is just above 8, so b log2(T / unit) carries a
+// quarter of the rounding of b log2 T (and less than b ln T)
+constexpr double kTUnit = 512.0;
+constexpr double kLog10Of2 = 0.30102999566398119521;
 constexpr double kInvLn10 = 0.43429448190325182765;
 
 // Compile-time shape of each compiled mechanism, keyed by neq = nsp + 1.  The
@@ -76,13 +81,15 @@ struct MechT<46> {  // ethyred (EthyRedF, the mechanism combustion/Makefile:3 li
 
 // Byte layout of the table block for a mechanism shape (rows of 64 lanes:
 // a double row is 512 bytes, an int row 256).
-//   RX  per 64-reaction round: double rows A_f b_f e_f A_b b_b e_b, int rows
+//   RX  per 64-reaction round: double rows A_f b_f e_f A_b b_b e_b (A for T in
+//       units of kTUnit, here and in FO), int rows
 //       I0 = r0 | r1 << 8 | r2 << 16 | m << 24 (reactant slots, third-body slot)
 //       I1 = p0 | p1 << 8 | p2 << 16 | falloff << 24 | rev << 25
-//   FO  (round-0 lanes < nfo) double rows A0_f b0_f e0_f A0_b b0_b e0_b c0 c1 c2
-//       g0 g1 g2 and an int row kinds | mfo << 8: Fc = sum_i c_i exp(-g_i T) or,
-//       where bit i of kinds is set, c_i exp(-g_i / T); mfo: slot of the
-//       third-body sum of GETLINDRATECOEFF (kZero: none, conc = P/RT)
+//   FO  fall-off reaction r in lane r (forward) and lane 32 + r (backward):
+//       double rows A0 b0 e0 c0 c1 c2 g0 g1 g2 and an int row kinds | mfo << 8 |
+//       on << 16: Fc = sum_i c_i 2^(-g_i T) or, where bit i of kinds is set,
+//       c_i 2^(-g_i / T); mfo: slot of the third-body sum of GETLINDRATECOEFF
+//       (kZero: none, conc = P/RT); on: the lane has a rate
 //   TH  [2][13] double rows (range, coefficient), species in lanes
 //   W, IW  double rows: molar mass and its reciprocal
 //   EV, EK  [maxe] double / int rows: third-body corrections (eff - 1, slot)
@@ -95,7 +102,7 @@ struct TabLayout {
   size_t rx, fo, th, w, iw, ev, ek, gn, gr, sf, sn, bytes;
   __host__ __device__ constexpr TabLayout(int nsp_, int nrxn_, int nfo_, int nthird_, int gmax_, int maxe_)
       : nsp(nsp_), nrxn(nrxn_), rounds((nrxn_ + 63) / 64), nfo(nfo_), nthird(nthird_), gmax(gmax_), maxe(maxe_),
-        rx(0), fo(rx + (size_t)((nrxn_ + 63) / 64) * kRxRound), th(fo + 12 * kRow + kIRow), w(th + 26 * kRow),
+        rx(0), fo(rx + (size_t)((nrxn_ + 63) / 64) * kRxRound), th(fo + 9 * kRow + kIRow), w(th + 26 * kRow),
         iw(w + kRow), ev(iw + kRow), ek(ev + (size_t)maxe_ * kRow), gn(ek + (size_t)maxe_ * kIRow),
         gr(gn + (size_t)gmax_ * kRow), sf(gr + (size_t)gmax_ * kIRow), sn(sf + kIRow), bytes(sn + kIRow) {}
 };
@@ -211,8 +218,9 @@ __device__ __forceinline__ void stage_tables(TGR_LDS char* dst, const char* src,
 }
 #endif
 
+// A T^b exp(e / (R T)) from A kTUnit^b: lt = log2(T / kTUnit), irt = log2(e) / (R T)
 __device__ __forceinline__ double arrhenius(double A, double b, double e, double lt, double irt) {
-  return A * fexp(fma(b, lt, e * irt));
+  return A * fexp2(fma(b, lt, e * irt));
 }
 
 // NASA-7 enthalpy / heat capacity of the species in this lane
@@ -233,26 +241,28 @@ __device__ __forceinline__ void thermo_lane(tchar* tab, double tmid, double T, i
 
 // Troe fall-off rate (GETLINDRATECOEFF, HYDROGENF.f90:280-316, ITROE = 1):
 // k = k_inf * F * Pr / (1 + Pr), Pr = k0 * conc / max(k_inf, 1e-60),
-// log10 F = log10 Fc / (1 + ((log10 Pr + c) / (n - d (log10 Pr + c)))^2).
-__device__ __forceinline__ double troe(double kinf, double k0, double conc, double lnfc, double ntmp, double cco) {
+// log10 F = log10 Fc / (1 + (l / d)^2), l = log10 Pr + c, d = n - 0.14 l, the
+// quotient taken as d^2 / (d^2 + l^2); l2fc = log2 Fc.
+__device__ __forceinline__ double troe(double kinf, double k0, double conc, double l2fc, double ntmp, double cco) {
   const double pr = k0 * conc / fmax(kinf, 1.0e-60);
-  const double lg = fma(flog(pr), kInvLn10, cco);
-  const double x = lg / fma(-kTroeD, lg, ntmp);
-  const double F = fexp(lnfc / fma(x, x, 1.0));
-  return kinf * F * pr / (1.0 + pr);
+  const double l = fma(flog2(pr), kLog10Of2, cco);
+  const double d = fma(-kTroeD, l, ntmp);
+  const double d2 = d * d;
+  const double F = fexp2(l2fc * (d2 / fma(l, l, d2)));
+  return kinf * F * (pr / (1.0 + pr));  // the quotient does not wait for F
 }
 
 // Temperature-dependent factors of one right-hand side, kept for others at
 // the same temperature (the species columns of a difference-quotient
 // Jacobian taken at fixed T): rate constants of every reaction lane (the
 // high-pressure limits on fall-off lanes), the low-pressure limits and
-// ln Fcent of the fall-off lanes, and each species' h and cp.  Every lane
-// reads back only what it wrote.
+// log2 Fcent of the fall-off lanes (forward, and backward from lane 32), and
+// each species' h and cp.  Every lane reads back only what it wrote.
 template <int NEQ>
 struct RateCache {
   double kf[((MechT<NEQ>::nrxn + 63) / 64) * 64];
   double kb[((MechT<NEQ>::nrxn + 63) / 64) * 64];
-  double k0f[kWave], k0b[kWave], lnfc[kWave];
+  double k0[kWave], l2fc[kWave];
   double h[kWave], cp[kWave];
 };
 
@@ -266,10 +276,11 @@ __device__ __forceinline__ double prodrates_wave(tchar* tab, TGR_LDS RhsLds<NEQ>
                                                  double T, double P, TGR_LDS RateCache<NEQ>* rc = nullptr) {
   using MT = MechT<NEQ>;
   constexpr TabLayout L = tab_layout<NEQ>();
+  static_assert(MT::nfo <= 32, "fall-off reactions take a forward lane and a backward lane");
   const int lane = lane_id();
-  const double lt = MODE == 2 ? 0.0 : flog(T);
+  const double lt = MODE == 2 ? 0.0 : flog2(T * (1.0 / kTUnit));
   const double rt = kRgasF4 * T;
-  const double irt = 1.0 / rt;
+  const double irt = MODE == 2 ? 0.0 : kLog2e / rt;
   S.C[lane] = lane == kOne ? 1.0 : Ck;
   wave_sync();
   // third-body sums: M_j = ctot + sum_e (eff_je - 1) C_e (padding: weight 0 on slot kOne)
@@ -299,43 +310,45 @@ __device__ __forceinline__ double prodrates_wave(tchar* tab, TGR_LDS RhsLds<NEQ>
         rc->kb[rd * 64 + lane] = kb;
       }
     }
-    if (rd == 0 && ((i1 >> 24) & 1)) {
-      tchar* fo = tab + L.fo + lane * 8;
-      const int fi = ld<int>(tab, L.fo + 12 * kRow + lane * 4);
-      const double mv = S.M[(fi >> 8) & 255];
-      const double conc = mv > 0.0 ? mv : P / rt;
-      if constexpr (MODE == 2) {
-        const double lnfc = rc->lnfc[lane];
-        const double lfc = lnfc * kInvLn10;
-        const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
-        const double cco = fma(-kTroeC1, lfc, -kTroeC0);
-        kf = troe(kf, rc->k0f[lane], conc, lnfc, ntmp, cco);
-        if ((i1 >> 25) & 1) kb = troe(kb, rc->k0b[lane], conc, lnfc, ntmp, cco);
-      } else {
-        const double invT = 1.0 / T;
-        double fc = 0.0;
+    if (rd == 0) {
+      // both directions of a fall-off reaction at once: the backward one in
+      // lane 32 + r, which takes k_inf from lane r through LDS
+      S.part[lane] = kb;
+      wave_sync();
+      const int fi = ld<int>(tab, L.fo + 9 * kRow + lane * 4);
+      if ((fi >> 16) & 1) {
+        tchar* fo = tab + L.fo + lane * 8;
+        const double kinf = lane < 32 ? kf : S.part[lane - 32];
+        const double mv = S.M[(fi >> 8) & 255];
+        const double conc = mv > 0.0 ? mv : P / rt;
+        double l2fc, k0;
+        if constexpr (MODE == 2) {
+          l2fc = rc->l2fc[lane];
+          k0 = rc->k0[lane];
+        } else {
+          const double invT = 1.0 / T;
+          double fc = 0.0;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          const double x = -(ld<double>(fo, (9 + i) * kRow) * (((fi >> i) & 1) ? invT : T));
-          fc = fma(ld<double>(fo, (6 + i) * kRow), fexp(x), fc);
+          for (int i = 0; i < 3; ++i) {
+            const double x = -(ld<double>(fo, (6 + i) * kRow) * (((fi >> i) & 1) ? invT : T));
+            fc = fma(ld<double>(fo, (3 + i) * kRow), fexp2(x), fc);
+          }
+          l2fc = flog2(fc);
+          k0 = arrhenius(ld<double>(fo, 0), ld<double>(fo, kRow), ld<double>(fo, 2 * kRow), lt, irt);
+          if constexpr (MODE == 1) {
+            rc->l2fc[lane] = l2fc;
+            rc->k0[lane] = k0;
+          }
         }
-        const double lnfc = flog(fc);
-        const double lfc = lnfc * kInvLn10;
+        const double lfc = l2fc * kLog10Of2;
         const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
         const double cco = fma(-kTroeC1, lfc, -kTroeC0);
-        const double k0f = arrhenius(ld<double>(fo, 0), ld<double>(fo, kRow), ld<double>(fo, 2 * kRow), lt, irt);
-        if constexpr (MODE == 1) {
-          rc->lnfc[lane] = lnfc;
-          rc->k0f[lane] = k0f;
-        }
-        kf = troe(kf, k0f, conc, lnfc, ntmp, cco);
-        if ((i1 >> 25) & 1) {
-          const double k0b =
-              arrhenius(ld<double>(fo, 3 * kRow), ld<double>(fo, 4 * kRow), ld<double>(fo, 5 * kRow), lt, irt);
-          if constexpr (MODE == 1) rc->k0b[lane] = k0b;
-          kb = troe(kb, k0b, conc, lnfc, ntmp, cco);
-        }
+        const double k = troe(kinf, k0, conc, l2fc, ntmp, cco);
+        if (lane < 32) kf = k;
+        else S.part[lane] = k;
       }
+      wave_sync();
+      if (((i1 >> 24) & 3) == 3) kb = S.part[lane + 32];  // reversible fall-off lane
     }
     const double wf = kf * S.C[i0 & 255] * S.C[(i0 >> 8) & 255] * S.C[(i0 >> 16) & 255];
     const double wb = kb * S.C[i1 & 255] * S.C[(i1 >> 8) & 255] * S.C[(i1 >> 16) & 255];
@@ -448,24 +461,24 @@ __device__ __forceinline__ void thermo_lane_d(tchar* tab, double tmid, double T,
 // k_inf, k_0, Fc (and conc = P/RT when dlconc = -1/T), dk_dconc at fixed T.
 // dl*: logarithmic derivatives d ln(.)/dT.
 __device__ __forceinline__ double troe_d(double kinf, double dlkinf, double k0, double dlk0, double conc,
-                                         double dlconc, double lnfc, double dlfc, double ntmp, double cco,
+                                         double dlconc, double l2fc, double dlfc, double ntmp, double cco,
                                          double& dk_dT, double& dk_dconc) {
   const double kin = fmax(kinf, 1.0e-60);
   const double pr = k0 * conc / kin;
-  const double lg = fma(flog(pr), kInvLn10, cco);
-  const double D = fma(-kTroeD, lg, ntmp);
-  const double x = lg / D;
-  const double x2 = fma(x, x, 1.0);
-  const double F = fexp(lnfc / x2);
-  const double k = kinf * F * pr / (1.0 + pr);  // as troe(), bit for bit
-  const double ix2 = 1.0 / x2;
+  const double l = fma(flog2(pr), kLog10Of2, cco);
+  const double D = fma(-kTroeD, l, ntmp);
+  const double D2 = D * D;
+  const double ix2 = D2 / fma(l, l, D2);  // 1 / (1 + x^2)
+  const double F = fexp2(l2fc * ix2);
+  const double k = kinf * F * (pr / (1.0 + pr));  // as troe(), bit for bit
+  const double x = l / D;
   const double ipr1 = 1.0 / (1.0 + pr);
   const double dlpr = dlk0 + dlconc - (kinf > 1.0e-60 ? dlkinf : 0.0);
   const double dL = (dlpr - kTroeC1 * dlfc) * kInvLn10;
   const double dn = -kTroeN1 * dlfc * kInvLn10;
-  const double iD2 = 1.0 / (D * D);
-  const double dx = (ntmp * dL - lg * dn) * iD2;
-  const double c2x = lnfc * 2.0 * x * ix2 * ix2;
+  const double iD2 = 1.0 / D2;
+  const double dx = (ntmp * dL - l * dn) * iD2;
+  const double c2x = l2fc * (2.0 * kLn2) * x * ix2 * ix2;
   dk_dT = k * (dlkinf + dlfc * ix2 - c2x * dx + dlpr * ipr1);
   const double dlFp = -c2x * ntmp * kInvLn10 * iD2;
   dk_dconc = kinf * F * (dlFp * ipr1 + ipr1 * ipr1) * (k0 / kin);
@@ -490,9 +503,10 @@ __device__ __forceinline__ double prodrates_jac_base(tchar* tab, TGR_LDS RhsLds<
   using MT = MechT<NEQ>;
   constexpr TabLayout L = tab_layout<NEQ>();
   const int lane = lane_id();
-  const double lt = flog(T);
+  const double lt = flog2(T * (1.0 / kTUnit));
   const double rt = kRgasF4 * T;
-  const double irt = 1.0 / rt;
+  const double irt2 = kLog2e / rt;  // of the rate constants
+  const double irt = 1.0 / rt;      // of their logarithmic derivatives
   const double invT = 1.0 / T;
   S.C[lane] = lane == kOne ? 1.0 : Ck;
   wave_sync();
@@ -512,15 +526,16 @@ __device__ __forceinline__ double prodrates_jac_base(tchar* tab, TGR_LDS RhsLds<
     const int i0 = ld<int>(rxi, 0), i1 = ld<int>(rxi, kIRow);
     const double bf = ld<double>(rx, kRow), ef = ld<double>(rx, 2 * kRow);
     const double bb = ld<double>(rx, 4 * kRow), eb = ld<double>(rx, 5 * kRow);
-    double kf = arrhenius(ld<double>(rx, 0), bf, ef, lt, irt);
-    double kb = arrhenius(ld<double>(rx, 3 * kRow), bb, eb, lt, irt);
+    double kf = arrhenius(ld<double>(rx, 0), bf, ef, lt, irt2);
+    double kb = arrhenius(ld<double>(rx, 3 * kRow), bb, eb, lt, irt2);
     // d ln k / dT of the Arrhenius forms: (b - e/(R T)) / T
     double dkf = kf * (fma(-ef, irt, bf) * invT), dkb = kb * (fma(-eb, irt, bb) * invT);
     double dkfc = 0.0, dkbc = 0.0;
     int md = (i0 >> 24) & 255;
     if (rd == 0 && ((i1 >> 24) & 1)) {
       tchar* fo = tab + L.fo + lane * 8;
-      const int fi = ld<int>(tab, L.fo + 12 * kRow + lane * 4);
+      tchar* fob = fo + 32 * 8;  // the backward direction's rows
+      const int fi = ld<int>(tab, L.fo + 9 * kRow + lane * 4);
       const double mv = S.M[(fi >> 8) & 255];
       const bool usem = mv > 0.0;
       const double conc = usem ? mv : P / rt;
@@ -529,25 +544,25 @@ __device__ __forceinline__ double prodrates_jac_base(tchar* tab, TGR_LDS RhsLds<
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
         const bool inv = (fi >> i) & 1;
-        const double gi = ld<double>(fo, (9 + i) * kRow);
-        const double x = -(gi * (inv ? invT : T));
-        const double ci = ld<double>(fo, (6 + i) * kRow), ex = fexp(x);
+        const double g2 = ld<double>(fo, (6 + i) * kRow);
+        const double x = -(g2 * (inv ? invT : T)), gi = g2 * kLn2;
+        const double ci = ld<double>(fo, (3 + i) * kRow), ex = fexp2(x);
         fc = fma(ci, ex, fc);
         dfc = fma(ci * ex, inv ? gi * invT * invT : -gi, dfc);
       }
-      const double lnfc = flog(fc);
-      const double lfc = lnfc * kInvLn10;
+      const double l2fc = flog2(fc);
+      const double lfc = l2fc * kLog10Of2;
       const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
       const double cco = fma(-kTroeC1, lfc, -kTroeC0);
       const double dlfc = dfc / fc;
       const double bf0 = ld<double>(fo, kRow), ef0 = ld<double>(fo, 2 * kRow);
-      const double k0f = arrhenius(ld<double>(fo, 0), bf0, ef0, lt, irt);
+      const double k0f = arrhenius(ld<double>(fo, 0), bf0, ef0, lt, irt2);
       const double dlinf = fma(-ef, irt, bf) * invT;
-      kf = troe_d(kf, dlinf, k0f, fma(-ef0, irt, bf0) * invT, conc, dlconc, lnfc, dlfc, ntmp, cco, dkf, dkfc);
+      kf = troe_d(kf, dlinf, k0f, fma(-ef0, irt, bf0) * invT, conc, dlconc, l2fc, dlfc, ntmp, cco, dkf, dkfc);
       if ((i1 >> 25) & 1) {
-        const double bb0 = ld<double>(fo, 4 * kRow), eb0 = ld<double>(fo, 5 * kRow);
-        const double k0b = arrhenius(ld<double>(fo, 3 * kRow), bb0, eb0, lt, irt);
-        kb = troe_d(kb, fma(-eb, irt, bb) * invT, k0b, fma(-eb0, irt, bb0) * invT, conc, dlconc, lnfc, dlfc, ntmp,
+        const double bb0 = ld<double>(fob, kRow), eb0 = ld<double>(fob, 2 * kRow);
+        const double k0b = arrhenius(ld<double>(fob, 0), bb0, eb0, lt, irt2);
+        kb = troe_d(kb, fma(-eb, irt, bb) * invT, k0b, fma(-eb0, irt, bb0) * invT, conc, dlconc, l2fc, dlfc, ntmp,
                     cco, dkb, dkbc);
       }
       md = usem ? ((fi >> 8) & 255) : kZero;

@@ -1,19 +1,30 @@
-// FP64 exp and log for the chemistry kernels, with a fixed, documented
+// FP64 2^x and log2 for the chemistry kernels, with a fixed, documented
 // operation count (used by the FLOP accounting of the roofline).
 //
-// exp: Cody-Waite argument reduction (W. J. Cody, W. Waite, "Software Manual
-//   for the Elementary Functions", 1980): x = k ln2 + r, k = rint(x/ln2),
-//   ln2 split into a 32-bit head and a tail so that k*ln2_hi is exact for
-//   |k| <= 1100; e^r on |r| <= ln2/2 by its degree-13 Taylor polynomial in
-//   Horner form (truncation < 5e-18 relative); result = 2^k * p by ldexp.
-//   Inputs below -746 give 0 (through ldexp underflow), above 710 give +inf,
-//   NaN propagates.  Ops: 1 mul, 1 rint, 15 fma, 1 ldexp, 1 cvt (plus the
-//   clamp: min, max and a NaN select).
-// log: x = 2^e m with m in [sqrt(1/2), sqrt(2)) (frexp); with f = m - 1 and
-//   s = f/(2 + f), ln m = 2 atanh(s) = 2s(1 + z/3 + z^2/5 + ...), z = s^2,
-//   |s| <= 0.1716, truncated after z^10 (< 1e-18 relative); ln x =
-//   e ln2_hi + (2s P(z) + e ln2_lo).  x = 0 gives -inf, x < 0 NaN, +inf +inf.
-//   Ops: 2 frexp, 1 cmp/select pair, 2 add, 1 div, 1 mul, 13 fma.
+// Rate constants are evaluated in base 2, k = A 2^(b log2 T + e log2(e) / (R T)):
+// the reduction of the exponent to an integer and a fraction is then exact
+// without the two-part product with ln 2 that base e needs: 15 instructions
+// instead of 24, of which the right-hand side of GRI-3.0 has 13 per lane.  With
+// both directions of a fall-off reaction in one pass (prodrates_wave) its wave
+// evaluation went from 1,165 to 801 VALU instructions, and the guided step of
+// 491,520 GRI-3.0 cells, which VALU issue bounds, from 347 to 306 ms.  Against
+// 64-bit evaluation in another order the rates are as far off as before
+// (3e-16 to 3e-15 of their norm).
+//
+// fexp2: k = rint(x), r = x - k (exact), 2^r on |r| <= 1/2 by a degree-11
+//   polynomial 1 + r q(r), q interpolating (2^r - 1) / r at the Chebyshev points
+//   (relative error 2e-17, mostly the rounding of the ln 2 coefficient),
+//   result 2^k p by ldexp.
+//   Finite x under- and overflow to 0 and +inf as they should, NaN propagates,
+//   +-inf gives NaN (the exponents here are sums of finite terms; a rate at
+//   T = 0 is undefined in any case).  Ops: 1 rint, 1 sub, 11 fma, 1 ldexp.
+// flog2: x = 2^e m with m in [sqrt(1/2), sqrt(2)) (frexp); with f = m - 1 and
+//   s = f/(1 + m), log2 m = (2 / ln 2) atanh(s) = s P(s^2), |s| <= 0.1716, P the
+//   degree-7 interpolant at the Chebyshev points of [0, 0.0295] (relative
+//   error 2e-18).  Arguments that are not positive and finite give NaN: they
+//   have no rate constant, and Pr = 0 has none either (its log10 Pr = -inf makes
+//   the Troe blending -inf / +inf).  Ops: 2 frexp, 1 ldexp, 2 add, 1 div, 1 mul,
+//   8 fma.
 #pragma once
 #include "wave_target.h"
 
@@ -21,64 +32,59 @@ namespace tgr {
 
 // Operation counts in the FLOP convention of the roofline (add, sub, mul,
 // div, rint, ldexp, frexp = 1 flop; fma = 2 flops; compares and selects = 0).
-constexpr double kFlopsExp = 1 + 1 + 15 * 2 + 1;       // 33
-constexpr double kFlopsLog = 2 + 2 + 1 + 1 + 13 * 2;   // 32
+constexpr double kFlopsExp = 1 + 1 + 11 * 2 + 1;           // 25
+constexpr double kFlopsLog = 2 + 1 + 2 + 1 + 1 + 8 * 2;    // 23
 
-__host__ __device__ __forceinline__ double fexp(double x) {
-  const double kLog2e = 1.4426950408889634074;
-  const double kLn2Hi = 6.93147180369123816490e-01;  // 32 significant bits
-  const double kLn2Lo = 1.90821492927058770002e-10;
-  // clamp (maxnum/minnum: a NaN becomes -746 here and is restored at the end)
-  const double xc = fmin(fmax(x, -746.0), 710.0);
-  const double k = rint(xc * kLog2e);
-  double r = fma(-k, kLn2Hi, xc);
-  r = fma(-k, kLn2Lo, r);
-  double p = 1.6059043836821614599e-10;      // 1/13!
-  p = fma(p, r, 2.0876756987868098979e-09);  // 1/12!
-  p = fma(p, r, 2.5052108385441718775e-08);  // 1/11!
-  p = fma(p, r, 2.7557319223985890653e-07);  // 1/10!
-  p = fma(p, r, 2.7557319223985892511e-06);  // 1/9!
-  p = fma(p, r, 2.4801587301587301566e-05);  // 1/8!
-  p = fma(p, r, 1.9841269841269841253e-04);  // 1/7!
-  p = fma(p, r, 1.3888888888888888889e-03);  // 1/6!
-  p = fma(p, r, 8.3333333333333333333e-03);  // 1/5!
-  p = fma(p, r, 4.1666666666666666667e-02);  // 1/4!
-  p = fma(p, r, 1.6666666666666666667e-01);  // 1/3!
-  p = fma(p, r, 0.5);
-  p = fma(p, r, 1.0);
-  p = fma(p, r, 1.0);
-  const double v = ldexp(p, (int)k);
-  return x == x ? v : x;
+constexpr double kLog2e = 1.4426950408889634074;
+constexpr double kLn2 = 0.69314718055994530942;
+
+// nearest integer of k as the hardware converts it: out of range saturates
+__host__ __device__ __forceinline__ int sat_int(double k) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  int i;
+  asm("v_cvt_i32_f64 %0, %1" : "=v"(i) : "v"(k));
+  return i;
+#else
+  return k >= 2147483647.0 ? 2147483647 : (k <= -2147483648.0 ? -2147483647 - 1 : (k == k ? (int)k : 0));
+#endif
 }
 
-__host__ __device__ __forceinline__ double flog(double x) {
-  const double kLn2Hi = 6.93147180369123816490e-01;
-  const double kLn2Lo = 1.90821492927058770002e-10;
+__host__ __device__ __forceinline__ double fexp2(double x) {
+  const double k = rint(x);
+  const double r = x - k;
+  double p = 4.4549605981865186e-10;
+  p = fma(p, r, 7.072585949269223e-09);
+  p = fma(p, r, 1.0178062445845774e-07);
+  p = fma(p, r, 1.321544258792169e-06);
+  p = fma(p, r, 1.525273382983612e-05);
+  p = fma(p, r, 0.0001540353044173605);
+  p = fma(p, r, 0.0013333558146416936);
+  p = fma(p, r, 0.009618129107606888);
+  p = fma(p, r, 0.0555041086648216);
+  p = fma(p, r, 0.24022650695910097);
+  p = fma(p, r, 0.6931471805599453);
+  p = fma(p, r, 1.0);
+  return ldexp(p, sat_int(k));
+}
+
+__host__ __device__ __forceinline__ double flog2(double x) {
   int e;
   double m = frexp(x, &e);  // m in [0.5, 1)
-  const bool lo = m < 0.70710678118654752440;
-  m = lo ? m + m : m;
-  e = lo ? e - 1 : e;
-  const double f = m - 1.0;
-  const double s = f / (2.0 + f);
+  const int lo = m < 0.70710678118654752440 ? 1 : 0;
+  m = ldexp(m, lo);
+  e -= lo;
+  const double s = (m - 1.0) / (m + 1.0);
   const double z = s * s;
-  double p = 1.0 / 21.0;
-  p = fma(p, z, 1.0 / 19.0);
-  p = fma(p, z, 1.0 / 17.0);
-  p = fma(p, z, 1.0 / 15.0);
-  p = fma(p, z, 1.0 / 13.0);
-  p = fma(p, z, 1.0 / 11.0);
-  p = fma(p, z, 1.0 / 9.0);
-  p = fma(p, z, 1.0 / 7.0);
-  p = fma(p, z, 1.0 / 5.0);
-  p = fma(p, z, 1.0 / 3.0);
-  p = fma(p, z, 1.0);
-  const double de = (double)e;
-  const double t = fma(s + s, p, de * kLn2Lo);
-  double y = fma(de, kLn2Hi, t);
-  // special values: frexp leaves 0, inf and NaN unchanged
-  if (!(x > 0.0) || x == INFINITY) y = (x == 0.0) ? -INFINITY : (x == INFINITY ? INFINITY : NAN);
-  return y;
+  double p = 0.2136589569431927;
+  p = fma(p, z, 0.2209130842311768);
+  p = fma(p, z, 0.262334352504183);
+  p = fma(p, z, 0.32059853491395984);
+  p = fma(p, z, 0.4121985858409005);
+  p = fma(p, z, 0.5770780163455203);
+  p = fma(p, z, 0.9617966939259898);
+  p = fma(p, z, 2.8853900817779268);
+  const double y = fma(s, p, (double)e);
+  return x > 0.0 && x < INFINITY ? y : NAN;
 }
 
 }  // namespace tgr

@@ -8,174 +8,51 @@ namespace tgr {
 
 template <>
 struct LaneRhs<40> {
-  // s: [rho*Y (39), rho*T] of this lane's state; f: the right-hand side
-  static __device__ __forceinline__ void eval(const double (&s)[40], double P, double (&f)[40]) {
-    double rho = s[0];
-    rho += s[1];
-    rho += s[2];
-    rho += s[3];
-    rho += s[4];
-    rho += s[5];
-    rho += s[6];
-    rho += s[7];
-    rho += s[8];
-    rho += s[9];
-    rho += s[10];
-    rho += s[11];
-    rho += s[12];
-    rho += s[13];
-    rho += s[14];
-    rho += s[15];
-    rho += s[16];
-    rho += s[17];
-    rho += s[18];
-    rho += s[19];
-    rho += s[20];
-    rho += s[21];
-    rho += s[22];
-    rho += s[23];
-    rho += s[24];
-    rho += s[25];
-    rho += s[26];
-    rho += s[27];
-    rho += s[28];
-    rho += s[29];
-    rho += s[30];
-    rho += s[31];
-    rho += s[32];
-    rho += s[33];
-    rho += s[34];
-    rho += s[35];
-    rho += s[36];
-    rho += s[37];
-    rho += s[38];
-    const double T = s[39] / rho;
-    const double irho = 1.0 / rho;
-    const double C0 = s[0] * 0x1.245cd2eb40a46p-5;
-    const double C1 = s[1] * 0x1.fbefbe72dfd0bp-1;
-    const double C2 = s[2] * 0x1.0000000000000p-5;
-    const double C3 = s[3] * 0x1.0000000000000p-4;
-    const double C4 = s[4] * 0x1.e1a7dc7865ca7p-5;
-    const double C5 = s[5] * 0x1.fbefbe72dfd0bp-2;
-    const double C6 = s[6] * 0x1.c6b4f7f1539dfp-5;
-    const double C7 = s[7] * 0x1.f05d519a5a4afp-6;
-    const double C8 = s[8] * 0x1.e1a7dc7865ca7p-6;
-    const double C9 = s[9] * 0x1.24778b96770f5p-5;
-    const double C10 = s[10] * 0x1.74476f46bcafbp-6;
-    const double C11 = s[11] * 0x1.1a4ebab921f45p-5;
-    const double C12 = s[12] * 0x1.1072f8c06c358p-4;
-    const double C13 = s[13] * 0x1.fea8d69a8976dp-5;
-    const double C14 = s[14] * 0x1.10d4897263b9dp-5;
-    const double C15 = s[15] * 0x1.07f7f2b66042cp-5;
-    const double C16 = s[16] * 0x1.1072f8c06c358p-5;
-    const double C17 = s[17] * 0x1.07f7f2b66042cp-5;
-    const double C18 = s[18] * 0x1.19e6472ab1c54p-5;
-    const double C19 = s[19] * 0x1.24077255ac595p-4;
-    const double C20 = s[20] * 0x1.24077255ac595p-4;
-    const double C21 = s[21] * 0x1.24077255ac595p-5;
-    const double C22 = s[22] * 0x1.73ec922c64208p-6;
-    const double C23 = s[23] * 0x1.3aa42a8f7dbc3p-5;
-    const double C24 = s[24] * 0x1.2ee9ec61a82a7p-5;
-    const double C25 = s[25] * 0x1.63a5ee375c49ep-6;
-    const double C26 = s[26] * 0x1.6b9aa47c82749p-6;
-    const double C27 = s[27] * 0x1.0c5383d6ca193p-6;
-    const double C28 = s[28] * 0x1.10d4897263b9dp-6;
-    const double C29 = s[29] * 0x1.157cec54345d8p-6;
-    const double C30 = s[30] * 0x1.a93a23d4ccfb1p-7;
-    const double C31 = s[31] * 0x1.07f7f2b66042cp-6;
-    const double C32 = s[32] * 0x1.a93a23d4ccfb1p-7;
-    const double C33 = s[33] * 0x1.2c755e4980b9ap-7;
-    const double C34 = s[34] * 0x1.63f903191dee4p-7;
-    const double C35 = s[35] * 0x1.b4a6878cdb28cp-7;
-    const double C36 = s[36] * 0x1.b4a6878cdb28cp-7;
-    const double C37 = s[37] * 0x1.5c57ffe4ff8dcp-6;
-    const double C38 = s[38] * 0x1.63f903191dee4p-6;
-    const bool hi = T > 0x1.f400000000000p+9;
-    double cpm = 0.0;
-    if (hi) {
-      cpm = fma(s[0] * irho, 0x1.28ba9057d1783p+8 * (0x1.769c23b7952d2p+1 + T * (0x1.8610723573f79p-10 + T * (-0x1.3132c2a042109p-21 + T * (0x1.bc12905f47c3dp-34 + T * -0x1.e6a15668d1fd9p-48)))), cpm);
-      cpm = fma(s[1] * irho, 0x1.01c2d34acaff7p+13 * (0x1.4000000000000p+1 + T * (0.0 + T * (0.0 + T * (0.0 + T * 0.0)))), cpm);
-      cpm = fma(s[2] * irho, 0x1.03d2b851eb852p+8 * (0x1.d94a3c64345d0p+1 + T * (0x1.41a93860283abp-11 + T * (-0x1.0e559221b1d58p-23 + T * (0x1.384f8c6a8c0c9p-36 + T * -0x1.478e1a3741480p-50)))), cpm);
-      cpm = fma(s[3] * irho, 0x1.03d2b851eb852p+9 * (0x1.456238da3c212p+1 + T * (-0x1.ce39030add37ep-16 + T * (-0x1.aa722cde846c4p-29 + T * (0x1.4040bc0d8605ep-38 + T * -0x1.f79a23c6c03bdp-52)))), cpm);
-      cpm = fma(s[4] * irho, 0x1.e8d949731098dp+8 * (0x1.6eaf6f6ecdbe1p+1 + T * (0x1.14f4d0c23ad0ap-10 + T * (-0x1.163020518c34ep-22 + T * (0x1.0c7922a4a2d04p-35 + T * -0x1.7fe9359e80e81p-50)))), cpm);
-      cpm = fma(s[5] * irho, 0x1.01c2d350092cdp+12 * (0x1.7ee6f2e8c0486p+1 + T * (0x1.6f090d9fefacdp-11 + T * (-0x1.e3f135bb38dc3p-25 + T * (-0x1.44cea998664c2p-37 + T * 0x1.c8327bfb6303ap-50)))), cpm);
-      cpm = fma(s[6] * irho, 0x1.cd7f5ff609dd0p+8 * (0x1.5608e15011905p+1 + T * (0x1.90982cf6c7e1cp-9 + T * (-0x1.d4b3c7a091cb6p-21 + T * (0x1.081a10711c1a4p-33 + T * -0x1.cc908a9d50493p-48)))), cpm);
-      cpm = fma(s[7] * irho, 0x1.f7c6fae7924afp+7 * (0x1.0119fbbf289f6p+2 + T * (0x1.2593e46a1f9dfp-9 + T * (-0x1.5431502070c84p-21 + T * (0x1.f675fa32f618cp-34 + T * -0x1.84c80e71ea191p-47)))), cpm);
-      cpm = fma(s[8] * irho, 0x1.e8d94983d7907p+7 * (0x1.24aec4a4095f2p+2 + T * (0x1.1c2c4a4f9e3cbp-8 + T * (-0x1.8bdbdb3ee32aap-20 + T * (0x1.0243c5162bd81p-32 + T * -0x1.01e7632962eb8p-46)))), cpm);
-      cpm = fma(s[9] * irho, 0x1.28d5af07bfe7ep+8 * (0x1.8335c182ecaefp+1 + T * (0x1.7a31384b0ee0ep-10 + T * (-0x1.2e4d82c084790p-21 + T * (0x1.bffa067a23237p-34 + T * -0x1.f1fc9016ead82p-48)))), cpm);
-      cpm = fma(s[10] * irho, 0x1.79d6b356da017p+7 * (0x1.1d0828c36da88p+2 + T * (0x1.9b9696515d0c4p-9 + T * (-0x1.572bbc2739f1ap-20 + T * (0x1.07390665390c5p-32 + T * -0x1.2caa8fbeb8df6p-46)))), cpm);
-      cpm = fma(s[11] * irho, 0x1.1e860685553efp+8 * (0x1.c754a7f8012e0p+1 + T * (0x1.b682cd3e25996p-9 + T * (-0x1.665ce9ec232b2p-20 + T * (0x1.0fa472a0a4455p-32 + T * -0x1.34bd6d4c2e4e2p-46)))), cpm);
-      cpm = fma(s[12] * irho, 0x1.148494a2b9d3dp+9 * (0x1.7d330e4a459e7p+1 + T * (0x1.7bf7d0ba1fd49p-8 + T * (-0x1.09286973eb98fp-19 + T * (0x1.51e0ab53b03a6p-32 + T * -0x1.42c57f31cb480p-46)))), cpm);
-      cpm = fma(s[13] * irho, 0x1.03249374bc6a8p+9 * (0x1.aef87ad080b67p+0 + T * (0x1.4f7431802ab2bp-7 + T * (-0x1.040e35941a681p-18 + T * (0x1.750a9e764526bp-31 + T * -0x1.95a1dd4aaed6dp-45)))), cpm);
-      cpm = fma(s[14] * irho, 0x1.14e7994e1a3f4p+8 * (-0x1.29b956f9360c5p-1 + T * (0x1.d4fb29078981ep-7 + T * (-0x1.02da607522242p-17 + T * (0x1.98ffbf1c3e520p-30 + T * 0.0)))), cpm);
-      cpm = fma(s[15] * irho, 0x1.0be922424a277p+8 * (0x1.e2a9930be0dedp+1 + T * (0x1.01eee717c07fdp-7 + T * (-0x1.6488a8c446c70p-19 + T * (0x1.b1b1dcc557332p-32 + T * -0x1.7c93377953d3bp-46)))), cpm);
-      cpm = fma(s[16] * irho, 0x1.148494a2b9d3dp+8 * (0x1.34dc2b0ea1837p+2 + T * (0x1.c585f11b35bb8p-7 + T * (-0x1.31d51d0b8ec61p-18 + T * (0x1.71b57f19a838bp-31 + T * -0x1.4417f1a209b9ep-45)))), cpm);
-      cpm = fma(s[17] * irho, 0x1.0be922424a277p+8 * (0x1.df9ac1b7c5d49p+1 + T * (0x1.2279c187d63ffp-7 + T * (-0x1.1dc11f954f259p-18 + T * (0x1.154c454622351p-30 + T * -0x1.a998e1c3ec971p-44)))), cpm);
-      cpm = fma(s[18] * irho, 0x1.1e1c0389f83bep+8 * (0x1.126ca61b881bcp+2 + T * (0x1.976f0de602e4fp-7 + T * (-0x1.28366dd505844p-18 + T * (0x1.846ccefec2441p-31 + T * -0x1.7a9e6cab2d327p-45)))), cpm);
-      cpm = fma(s[19] * irho, 0x1.2863e90ff9724p+9 * (0x1.6fe28bbb5f921p+1 + T * (0x1.df4030068403dp-9 + T * (-0x1.7a3607a17a275p-20 + T * (0x1.1e1208519dbd9p-32 + T * -0x1.522e0f41fe4e3p-46)))), cpm);
-      cpm = fma(s[20] * irho, 0x1.2863e90ff9724p+9 * (0x1.256183d389aa6p+1 + T * (0x1.3120cfb16b35fp-8 + T * (-0x1.0e0906cfb21aep-19 + T * (0x1.cb7e14e4de1f4p-32 + T * -0x1.31fd42b26d354p-45)))), cpm);
-      cpm = fma(s[21] * irho, 0x1.2863e90ff9724p+8 * (0x1.049f4a5d9c3d6p+1 + T * (0x1.dfe6a5720731ep-7 + T * (-0x1.c25a4ed3d3908p-18 + T * (0x1.94aeec0be93f2p-30 + T * -0x1.1b109c49479cdp-43)))), cpm);
-      cpm = fma(s[22] * irho, 0x1.797a7aa68f4b6p+7 * (0x1.59dcf38b7d772p+2 + T * (0x1.80242581cd52bp-7 + T * (-0x1.1b9f84391e21fp-18 + T * (0x1.77e1ab96723c6p-31 + T * -0x1.7128a8eac22f7p-45)))), cpm);
-      cpm = fma(s[23] * irho, 0x1.3f5713ad5bee4p+8 * (0x1.0971c7ee6bae0p+2 + T * (0x1.86b42b3f9ab1ep-8 + T * (-0x1.3e7de3eb387edp-19 + T * (0x1.00f66a3bafde2p-31 + T * -0x1.455f2b475f023p-45)))), cpm);
-      cpm = fma(s[24] * irho, 0x1.33700096feb4ap+8 * (0x1.8224031487768p+1 + T * (0x1.52803e497ede9p-7 + T * (-0x1.3a1fef6b5677dp-18 + T * (0x1.17b98c3c9686ep-30 + T * -0x1.847bd21d4a0a4p-44)))), cpm);
-      cpm = fma(s[25] * irho, 0x1.68f59ea57214fp+7 * (0x1.a960a7be2821ep-1 + T * (0x1.b9037309df683p-6 + T * (-0x1.d1fc866c5ac12p-17 + T * (0x1.dd9eff9b15bf0p-29 + T * -0x1.80ba465eec50fp-42)))), cpm);
-      cpm = fma(s[26] * irho, 0x1.7108bfc2224eep+7 * (0x1.715ca8219cb2dp+1 + T * (0x1.4945d1eddf464p-6 + T * (-0x1.29706021400c0p-17 + T * (0x1.8b2885f927e26p-30 + T * 0.0)))), cpm);
-      cpm = fma(s[27] * irho, 0x1.10555c74751cep+7 * (0x1.f4d63f1162d3ep+0 + T * (0x1.afeec33e440d9p-6 + T * (-0x1.a7afef5c5cbc2p-17 + T * (0x1.2f294619f38b8p-29 + T * 0.0)))), cpm);
-      cpm = fma(s[28] * irho, 0x1.14e7993d5347ap+7 * (0x1.9fa9e5ed044fcp+0 + T * (0x1.9c2271983e67dp-6 + T * (-0x1.a5e2869b51b8cp-17 + T * (0x1.3498f77908422p-29 + T * 0.0)))), cpm);
-      cpm = fma(s[29] * irho, 0x1.19a1cb039ef0fp+7 * (0x1.a416232243f7ap+2 + T * (0x1.15c8f688c5d25p-6 + T * (-0x1.3894f4cfc2708p-17 + T * (0x1.e85dafb029bb6p-30 + T * 0.0)))), cpm);
-      cpm = fma(s[30] * irho, 0x1.af93d5347a5b1p+6 * (0x1.b1d47e7cb2ae1p+2 + T * (0x1.6357a14abfa13p-6 + T * (-0x1.41d2138ffbd5ap-17 + T * (0x1.aeeaddfd9036dp-30 + T * 0.0)))), cpm);
-      cpm = fma(s[31] * irho, 0x1.0be92231832fdp+7 * (0x1.e79f2823e084ep+0 + T * (0x1.d1c4ec8c3865bp-6 + T * (-0x1.bf7f44eeb209bp-17 + T * (0x1.3c57cc99adf86p-29 + T * 0.0)))), cpm);
-      cpm = fma(s[32] * irho, 0x1.af93d5347a5b1p+6 * (0x1.35bfd1e23569cp+3 + T * (0x1.34bf03e4d09f7p-6 + T * (-0x1.23a2b6ebe421cp-17 + T * (0x1.938755aa34d79p-30 + T * 0.0)))), cpm);
-      cpm = fma(s[33] * irho, 0x1.30f20e8add3e3p+6 * (0x1.ae80987683eaep+3 + T * (0x1.506bfc3c20f99p-6 + T * (-0x1.39a086249982bp-17 + T * (0x1.ad90fcb7dc7bap-30 + T * 0.0)))), cpm);
-      cpm = fma(s[34] * irho, 0x1.6949f13561e1ap+6 * (0x1.29e2cc07d5e25p+3 + T * (0x1.5f9bc8034a9e7p-6 + T * (-0x1.6528655d0532cp-17 + T * (0x1.0389665afce1bp-29 + T * 0.0)))), cpm);
-      cpm = fma(s[35] * irho, 0x1.bb2be596c82e0p+6 * (0x1.52aaa9a1cf732p+1 + T * (0x1.a5d278d079bf3p-6 + T * (-0x1.ca7bbf737701dp-17 + T * (0x1.5e4443e746d41p-29 + T * 0.0)))), cpm);
-      cpm = fma(s[36] * irho, 0x1.bb2be596c82e0p+6 * (0x1.9afc1ac324d85p+1 + T * (0x1.7e2b97bbfc789p-6 + T * (-0x1.93f65f3c91806p-17 + T * (0x1.2e9f6c132879dp-29 + T * 0.0)))), cpm);
-      cpm = fma(s[37] * irho, 0x1.618bc31df761dp+7 * (0x1.bad19f9a649abp+0 + T * (0x1.0894798c4274fp-6 + T * (-0x1.044771a062409p-17 + T * (0x1.78d3d656b5c5dp-30 + T * 0.0)))), cpm);
-      cpm = fma(s[38] * irho, 0x1.6949f127f5e85p+7 * (0x1.5be9b13415057p+1 + T * (0x1.938e119a140f7p-7 + T * (-0x1.94a69161b7cb6p-18 + T * (0x1.23bf509827fa9p-30 + T * 0.0)))), cpm);
-    } else {
-      cpm = fma(s[0] * irho, 0x1.28ba9057d1783p+8 * (0x1.a63b0c4588a05p+1 + T * (0x1.712962facc0e9p-10 + T * (-0x1.09f7a2b098bd4p-18 + T * (0x1.83ae94da0fe59p-28 + T * -0x1.58152f3dbcf65p-39)))), cpm);
-      cpm = fma(s[1] * irho, 0x1.01c2d34acaff7p+13 * (0x1.4000000000000p+1 + T * (0.0 + T * (0.0 + T * (0.0 + T * 0.0)))), cpm);
-      cpm = fma(s[2] * irho, 0x1.03d2b851eb852p+8 * (0x1.9b417ca2120e2p+1 + T * (0x1.27904dfc9e5cep-10 + T * (-0x1.3507ec57048a6p-21 + T * (0x1.6927dfded5549p-30 + T * -0x1.eda02e4e9106fp-41)))), cpm);
-      cpm = fma(s[3] * irho, 0x1.03d2b851eb852p+9 * (0x1.792495e17e34cp+1 + T * (-0x1.ad6f7594e8c10p-10 + T * (0x1.44f206ae86a97p-19 + T * (-0x1.b8960c8cd58ecp-30 + T * 0x1.b60dad5a2c8b3p-42)))), cpm);
-      cpm = fma(s[4] * irho, 0x1.e8d949731098dp+8 * (0x1.080501d23d242p+2 + T * (-0x1.a6c41f4a374cap-9 + T * (0x1.b6101eb7dedbep-18 + T * (-0x1.8e78ee8164a9cp-28 + T * 0x1.2240d8be85bd5p-39)))), cpm);
-      cpm = fma(s[5] * irho, 0x1.01c2d350092cdp+12 * (0x1.a628ed5f138bdp+1 + T * (0x1.b08222e154b9ep-11 + T * (-0x1.b52cbef7ef399p-21 + T * (-0x1.a0bbe70f69bcfp-34 + T * 0x1.d18b923980a1ep-42)))), cpm);
-      cpm = fma(s[6] * irho, 0x1.cd7f5ff609dd0p+8 * (0x1.b18409e55c0fdp+1 + T * (0x1.c7790c169fe5dp-9 + T * (-0x1.aa74d89269c73p-18 + T * (0x1.dee092cb7ea3cp-28 + T * -0x1.60c559aac818ep-39)))), cpm);
-      cpm = fma(s[7] * irho, 0x1.f7c6fae7924afp+7 * (0x1.1350a899bcaa1p+2 + T * (-0x1.373d054674594p-8 + T * (0x1.62fa28e3a8ea6p-16 + T * (-0x1.a110b0905e0fcp-26 + T * 0x1.46f1288fc5c1cp-37)))), cpm);
-      cpm = fma(s[8] * irho, 0x1.e8d94983d7907p+7 * (0x1.b1c2b0ea18373p+1 + T * (0x1.ae8552d47d093p-8 + T * (-0x1.3ee773fac0950p-23 + T * (-0x1.3de20a2d8a14dp-28 + T * 0x1.5bd5b656f46cdp-39)))), cpm);
-      cpm = fma(s[9] * irho, 0x1.28d5af07bfe7ep+8 * (0x1.a19806f262889p+1 + T * (0x1.8c58a4980b8b3p-10 + T * (-0x1.04800b08e2c9bp-18 + T * (0x1.7f9698eb1c752p-28 + T * -0x1.5c5181d89285ep-39)))), cpm);
-      cpm = fma(s[10] * irho, 0x1.79d6b356da017p+7 * (0x1.234af4f0d844dp+1 + T * (0x1.45205f5fd0b9ep-7 + T * (-0x1.5d4592f5a845bp-17 + T * (0x1.d7e00903b44b7p-28 + T * -0x1.29fb0d256cd4cp-39)))), cpm);
-      cpm = fma(s[11] * irho, 0x1.1e860685553efp+8 * (0x1.72fc7a398201dp+1 + T * (0x1.96446da0caeeep-8 + T * (-0x1.42e5a98191c27p-17 + T * (0x1.76760551ca70ep-27 + T * -0x1.41edcd30beeb1p-38)))), cpm);
-      cpm = fma(s[12] * irho, 0x1.148494a2b9d3dp+9 * (0x1.d41e76e38c2bfp+1 + T * (0x1.16bcc8dd4edc2p-9 + T * (0x1.6e4e659e7b1a3p-18 + T * (-0x1.c6cada0b83d8bp-28 + T * 0x1.5b0478af296dap-39)))), cpm);
-      cpm = fma(s[13] * irho, 0x1.03249374bc6a8p+9 * (0x1.8eb734b51372ap-1 + T * (0x1.1e568242bae5ap-6 + T * (-0x1.d2fa819a83265p-16 + T * (0x1.05f7c9c3f6e46p-25 + T * -0x1.aea1e766ae70ep-37)))), cpm);
-      cpm = fma(s[14] * irho, 0x1.14e7994e1a3f4p+8 * (0x1.591f1645bca2bp+1 + T * (0x1.42d6f412ede0ap-8 + T * (0x1.bcabddd64bccbp-21 + T * (-0x1.2e935feb740d0p-31 + T * -0x1.bdf8fddb1e1b3p-42)))), cpm);
-      cpm = fma(s[15] * irho, 0x1.0be922424a277p+8 * (0x1.0d9817b95a294p+1 + T * (0x1.d8f25f83733c9p-8 + T * (0x1.664240277b618p-18 + T * (-0x1.fafcbebd8fc7ap-28 + T * 0x1.241dc474f011fp-39)))), cpm);
-      cpm = fma(s[16] * irho, 0x1.148494a2b9d3dp+8 * (0x1.7668f4b61fe22p+0 + T * (0x1.fbbab674c6a67p-7 + T * (0x1.83ec5aa4cd9a5p-18 + T * (-0x1.b03012a1e9c75p-27 + T * 0x1.42bad76692a1bp-38)))), cpm);
-      cpm = fma(s[17] * irho, 0x1.0be922424a277p+8 * (0x1.61e03e841f33fp+1 + T * (0x1.876a6f2bff2ecp-7 + T * (-0x1.ef1c02ca6da7ap-18 + T * (0x1.0a0bd49f52b27p-29 + T * 0.0)))), cpm);
-      cpm = fma(s[18] * irho, 0x1.1e1c0389f83bep+8 * (0x1.13932d6ece13fp+2 + T * (-0x1.122932b551339p-8 + T * (0x1.a0f98cacccd65p-15 + T * (-0x1.014b347d2de42p-24 + T * 0x1.95791def45bc0p-36)))), cpm);
-      cpm = fma(s[19] * irho, 0x1.2863e90ff9724p+9 * (0x1.e19f746480de1p+1 + T * (0x1.fbf7d158743a2p-11 + T * (0x1.771ffa66e83e0p-19 + T * (-0x1.08a1f3bb46844p-28 + T * 0x1.daf7390cac908p-40)))), cpm);
-      cpm = fma(s[20] * irho, 0x1.2863e90ff9724p+9 * (0x1.0cb5ee035346ap+2 + T * (-0x1.36326518bab75p-9 + T * (0x1.14409b5702698p-17 + T * (-0x1.cb9b5a07323d1p-28 + T * 0x1.1179431daea17p-39)))), cpm);
-      cpm = fma(s[21] * irho, 0x1.2863e90ff9724p+8 * (0x1.fac71d356ff96p+1 + T * (-0x1.f0244a6c1abf8p-8 + T * (0x1.defb3b4522b25p-15 + T * (-0x1.2908fcd07cb16p-24 + T * 0x1.dac91dbd28c88p-36)))), cpm);
-      cpm = fma(s[22] * irho, 0x1.797a7aa68f4b6p+7 * (0x1.2eaf76e6106abp+2 + T * (-0x1.a28ce427d2efep-9 + T * (0x1.8ec0772eb57cep-15 + T * (-0x1.ed90d262d7aa3p-25 + T * 0x1.81d0f2a50dc3bp-36)))), cpm);
-      cpm = fma(s[23] * irho, 0x1.3f5713ad5bee4p+8 * (0x1.9e0b72c73f3bap-1 + T * (0x1.7ec17f28e481ap-6 + T * (-0x1.29f09105c533cp-15 + T * (0x1.e14c5845a203fp-26 + T * -0x1.2b17c43e837e8p-37)))), cpm);
-      cpm = fma(s[24] * irho, 0x1.33700096feb4ap+8 * (0x1.9b3219c31fa4ep+1 + T * (0x1.8d17f1df63fcdp-10 + T * (0x1.b2e198409699cp-16 + T * (-0x1.3339cad4b897fp-25 + T * 0x1.02dedc9720552p-36)))), cpm);
-      cpm = fma(s[25] * irho, 0x1.68f59ea57214fp+7 * (0x1.15498ca66c0ffp+1 + T * (0x1.5d97e24e2d237p-6 + T * (-0x1.acff45bbb4ce8p-18 + T * (-0x1.018f4704e51a1p-33 + T * 0.0)))), cpm);
-      cpm = fma(s[26] * irho, 0x1.7108bfc2224eep+7 * (0x1.74e62ad7441f1p+1 + T * (0x1.4d3151fd3ae33p-6 + T * (-0x1.4206a99644805p-17 + T * (0x1.1d280428550a3p-29 + T * -0x1.81d4b92e2b024p-43)))), cpm);
-      cpm = fma(s[27] * irho, 0x1.10555c74751cep+7 * (0x1.a1236b2999ac6p+1 + T * (0x1.6bf6efabb70d0p-6 + T * (-0x1.053d7af963800p-17 + T * (-0x1.0983bf6c7b32ap-32 + T * 0x1.fccf7c342220dp-42)))), cpm);
-      cpm = fma(s[28] * irho, 0x1.14e7993d5347ap+7 * (0x1.8b509ebe71954p+1 + T * (0x1.4dd7288f4e0dcp-6 + T * (-0x1.cb8bccb7708ecp-18 + T * (-0x1.905318e65fa7ep-31 + T * 0x1.3c73807617e5ap-41)))), cpm);
-      cpm = fma(s[29] * irho, 0x1.19a1cb039ef0fp+7 * (0x1.f8932e301419fp+1 + T * (0x1.8ed7fda31b87fp-6 + T * (-0x1.15d2c05f70557p-16 + T * (0x1.3b1ac1221623bp-28 + T * -0x1.75919a0a7a109p-42)))), cpm);
-      cpm = fma(s[30] * irho, 0x1.af93d5347a5b1p+6 * (0x1.1aeafbb6f016bp+1 + T * (0x1.2e2f3583b7b37p-5 + T * (-0x1.da0f43874b909p-16 + T * (0x1.8da5a743c3ff8p-27 + T * -0x1.156fbca566d5ep-39)))), cpm);
-      cpm = fma(s[31] * irho, 0x1.0be92231832fdp+7 * (0x1.944a57bd00511p+1 + T * (0x1.904da5c0bd76ap-6 + T * (-0x1.22e96d05b2a72p-17 + T * (-0x1.04f1d14f0a606p-34 + T * 0x1.eb57bcad2a681p-42)))), cpm);
-      cpm = fma(s[32] * irho, 0x1.af93d5347a5b1p+6 * (0x1.43b4ccbb5a08bp+1 + T * (0x1.5b72262f8c012p-5 + T * (-0x1.393c692a25e41p-15 + T * (0x1.1e48c0f339dd7p-26 + T * -0x1.a134f58b4c605p-39)))), cpm);
-      cpm = fma(s[33] * irho, 0x1.30f20e8add3e3p+6 * (0x1.ff146e7701135p+0 + T * (0x1.ddc767e8598bbp-5 + T * (-0x1.d01ba1f45fe82p-15 + T * (0x1.be59e2473ce95p-26 + T * -0x1.4fc21504096eap-38)))), cpm);
-      cpm = fma(s[34] * irho, 0x1.6949f13561e1ap+6 * (0x1.bd5b92377a95ap+1 + T * (0x1.4a193dd18d4a0p-5 + T * (-0x1.14ea6e782db5ap-15 + T * (0x1.cda868a48a234p-27 + T * -0x1.33a7850078c3cp-39)))), cpm);
-      cpm = fma(s[35] * irho, 0x1.bb2be596c82e0p+6 * (0x1.4c9a25905d5adp+2 + T * (0x1.043e3563c7cd2p-6 + T * (0x1.7b9c7c4eeb122p-22 + T * (-0x1.a380b7b5a0d5cp-28 + T * 0x1.11f64e1eafecap-39)))), cpm);
-      cpm = fma(s[36] * irho, 0x1.bb2be596c82e0p+6 * (0x1.853c57a9e00dcp+2 + T * (0x1.a5f2ba8881b83p-7 + T * (0x1.125dfa29a9147p-19 + T * (-0x1.a34b96bfa03c3p-28 + T * 0x1.fa265e4f865bap-40)))), cpm);
-      cpm = fma(s[37] * irho, 0x1.618bc31df761dp+7 * (0x1.07283f191a834p+2 + T * (0x1.ee0b28e595de3p-8 + T * (0x1.fa7422129ff3ep-19 + T * (-0x1.72393312daf39p-28 + T * 0x1.99df4e016bdccp-40)))), cpm);
-      cpm = fma(s[38] * irho, 0x1.6949f127f5e85p+7 * (0x1.6f7bbd0fc0676p+0 + T * (0x1.0ba76a4703902p-6 + T * (-0x1.648a6dfc430a3p-17 + T * (0x1.c87ae70772a4cp-29 + T * -0x1.c4cf5e9412c52p-42)))), cpm);
-    }
-    const double lt = flog(T);
+  // production rates cd (kmol/m3/s) from the concentrations, temperature and pressure of this lane's state
+  static __device__ __forceinline__ void rates(const double (&C)[39], double T, double P, double (&cd)[39]) {
+    const double C0 = C[0];
+    const double C1 = C[1];
+    const double C2 = C[2];
+    const double C3 = C[3];
+    const double C4 = C[4];
+    const double C5 = C[5];
+    const double C6 = C[6];
+    const double C7 = C[7];
+    const double C8 = C[8];
+    const double C9 = C[9];
+    const double C10 = C[10];
+    const double C11 = C[11];
+    const double C12 = C[12];
+    const double C13 = C[13];
+    const double C14 = C[14];
+    const double C15 = C[15];
+    const double C16 = C[16];
+    const double C17 = C[17];
+    const double C18 = C[18];
+    const double C19 = C[19];
+    const double C20 = C[20];
+    const double C21 = C[21];
+    const double C22 = C[22];
+    const double C23 = C[23];
+    const double C24 = C[24];
+    const double C25 = C[25];
+    const double C26 = C[26];
+    const double C27 = C[27];
+    const double C28 = C[28];
+    const double C29 = C[29];
+    const double C30 = C[30];
+    const double C31 = C[31];
+    const double C32 = C[32];
+    const double C33 = C[33];
+    const double C34 = C[34];
+    const double C35 = C[35];
+    const double C36 = C[36];
+    const double C37 = C[37];
+    const double C38 = C[38];
+    const double lt = flog2(T * (1.0 / kTUnit));
     const double rt = kRgasF4 * T;
-    const double irt = 1.0 / rt;
+    const double irt = kLog2e / rt;
+    const double invT = 1.0 / T;
     const double p_rt = P / rt;
     double ctot = C0;
     ctot += C1;
@@ -276,8 +153,8 @@ struct LaneRhs<40> {
     double cd37 = 0.0;
     double cd38 = 0.0;
     {  // R1 (elementary)
-    const double kf = 0x1.9cecd66700000p+41 * fexp(fma(-0x1.9fbe760000000p-2, lt, -0x1.08ee440000000p+26 * irt));
-    const double kb = 0x1.a4648c5d1999ap+32 * fexp(fma(0x1.da70fa0000000p-6, lt, 0x1.0f45b20000000p+20 * irt));
+    const double kf = 0x1.066ba563b9219p+38 * fexp2(fma(-0x1.08ee440000000p+26, irt, -0x1.9fbe760000000p-2 * lt));
+    const double kb = 0x1.f7a09124abc93p+32 * fexp2(fma(0x1.0f45b20000000p+20, irt, 0x1.da70fa0000000p-6 * lt));
     const double q = kf * C1 * C2 - kb * C4 * C3;
     cd1 -= q;
     cd2 -= q;
@@ -285,8 +162,8 @@ struct LaneRhs<40> {
     cd4 += q;
     }
     {  // R2 (elementary)
-    const double kf = 0x1.9666666666666p+5 * fexp(fma(0x1.55c2900000000p+1, lt, -0x1.9190c80000000p+24 * irt));
-    const double kb = 0x1.dcbbd77d66187p+4 * fexp(fma(0x1.5146b20000000p+1, lt, -0x1.3994fe0000000p+24 * irt));
+    const double kf = 0x1.9ef084bc2d181p+29 * fexp2(fma(-0x1.9190c80000000p+24, irt, 0x1.55c2900000000p+1 * lt));
+    const double kb = 0x1.8733aee92c286p+28 * fexp2(fma(-0x1.3994fe0000000p+24, irt, 0x1.5146b20000000p+1 * lt));
     const double q = kf * C3 * C5 - kb * C4 * C1;
     cd1 += q;
     cd3 -= q;
@@ -294,8 +171,8 @@ struct LaneRhs<40> {
     cd5 -= q;
     }
     {  // R3 (elementary)
-    const double kf = 0x1.a5e0000000000p+17 * fexp(fma(0x1.828f5c0000000p+0, lt, -0x1.b5f5300000000p+23 * irt));
-    const double kb = 0x1.0ec8e7c60aa65p+21 * fexp(fma(0x1.6a97e20000000p+0, lt, -0x1.25f53a0000000p+26 * irt));
+    const double kf = 0x1.3d8351cc599e2p+31 * fexp2(fma(-0x1.b5f5300000000p+23, irt, 0x1.828f5c0000000p+0 * lt));
+    const double kb = 0x1.c697225f0efccp+33 * fexp2(fma(-0x1.25f53a0000000p+26, irt, 0x1.6a97e20000000p+0 * lt));
     const double q = kf * C5 * C4 - kb * C1 * C6;
     cd1 += q;
     cd4 -= q;
@@ -303,16 +180,16 @@ struct LaneRhs<40> {
     cd6 += q;
     }
     {  // R4 (elementary)
-    const double kf = 0x1.7340000000000p+11 * fexp(fma(0x1.028f5c0000000p+1, lt, -0x1.abbfe80000000p+25 * irt));
-    const double kb = 0x1.533fab486dad0p+7 * fexp(fma(0x1.0a0f3c0000000p+1, lt, 0x1.7aac960000000p+23 * irt));
+    const double kf = 0x1.a495458aad9ebp+29 * fexp2(fma(-0x1.abbfe80000000p+25, irt, 0x1.028f5c0000000p+1 * lt));
+    const double kb = 0x1.14f48735c229bp+26 * fexp2(fma(0x1.7aac960000000p+23, irt, 0x1.0a0f3c0000000p+1 * lt));
     const double q = kf * C3 * C6 - kb * C4 * C4;
     cd3 -= q;
     cd4 = fma(0x1.0000000000000p+1, q, cd4);
     cd6 -= q;
     }
     {  // R10 (elementary)
-    const double kf = 0x1.eeb7f30000000p+33 * fexp(fma(0.0, lt, -0x1.a449c00000000p+21 * irt));
-    const double kb = 0x1.457c1e1933333p+31 * fexp(fma(0x1.7263520000000p-2, lt, -0x1.ba397a0000000p+27 * irt));
+    const double kf = 0x1.eeb7f30000000p+33 * fexp2(fma(-0x1.a449c00000000p+21, irt, 0.0 * lt));
+    const double kb = 0x1.8482abbc12ac8p+34 * fexp2(fma(-0x1.ba397a0000000p+27, irt, 0x1.7263520000000p-2 * lt));
     const double q = kf * C7 * C1 - kb * C2 * C5;
     cd1 -= q;
     cd2 += q;
@@ -320,16 +197,16 @@ struct LaneRhs<40> {
     cd7 -= q;
     }
     {  // R11 (elementary)
-    const double kf = 0x1.07b69ad800000p+36 * fexp(fma(0.0, lt, -0x1.2d45000000000p+20 * irt));
-    const double kb = 0x1.9e6b84b333333p+23 * fexp(fma(0x1.85f4800000000p-1, lt, -0x1.246db80000000p+27 * irt));
+    const double kf = 0x1.07b69ad800000p+36 * fexp2(fma(-0x1.2d45000000000p+20, irt, 0.0 * lt));
+    const double kb = 0x1.76b5a48463bb2p+30 * fexp2(fma(-0x1.246db80000000p+27, irt, 0x1.85f4800000000p-1 * lt));
     const double q = kf * C7 * C1 - kb * C4 * C4;
     cd1 -= q;
     cd4 = fma(0x1.0000000000000p+1, q, cd4);
     cd7 -= q;
     }
     {  // R12 (elementary)
-    const double kf = 0x1.e449a94000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.75c3c10666666p+31 * fexp(fma(0x1.4e835e0000000p-2, lt, -0x1.a8a8da0000000p+27 * irt));
+    const double kf = 0x1.e449a94000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.668d9e7d59f18p+34 * fexp2(fma(-0x1.a8a8da0000000p+27, irt, 0x1.4e835e0000000p-2 * lt));
     const double q = kf * C7 * C3 - kb * C4 * C2;
     cd2 += q;
     cd3 -= q;
@@ -337,8 +214,8 @@ struct LaneRhs<40> {
     cd7 -= q;
     }
     {  // R13 (elementary)
-    const double kf = 0x1.aea4c04000000p+34 * fexp(fma(0.0, lt, 0x1.fb91800000000p+20 * irt));
-    const double kb = 0x1.6bb6fdab20000p+35 * fexp(fma(0x1.12845a0000000p-2, lt, -0x1.13a63e0000000p+28 * irt));
+    const double kf = 0x1.aea4c04000000p+34 * fexp2(fma(0x1.fb91800000000p+20, irt, 0.0 * lt));
+    const double kb = 0x1.e42f0b88714bep+37 * fexp2(fma(-0x1.13a63e0000000p+28, irt, 0x1.12845a0000000p-2 * lt));
     const double q = kf * C7 * C4 - kb * C2 * C6;
     cd2 += q;
     cd4 -= q;
@@ -346,24 +223,24 @@ struct LaneRhs<40> {
     cd7 -= q;
     }
     {  // R14 (elementary)
-    const double kf = 0x1.8727cda000000p+38 * fexp(fma(0.0, lt, -0x1.7e7c040000000p+25 * irt));
-    const double kb = 0x1.ce90f36622000p+45 * fexp(fma(-0x1.8e9d940000000p-2, lt, -0x1.94c1840000000p+27 * irt));
+    const double kf = 0x1.8727cda000000p+38 * fexp2(fma(-0x1.7e7c040000000p+25, irt, 0.0 * lt));
+    const double kb = 0x1.464d0856bb04dp+42 * fexp2(fma(-0x1.94c1840000000p+27, irt, -0x1.8e9d940000000p-2 * lt));
     const double q = kf * C7 * C7 - kb * C2 * C8;
     cd2 += q;
     cd7 = fma(-0x1.0000000000000p+1, q, cd7);
     cd8 += q;
     }
     {  // R15 (elementary)
-    const double kf = 0x1.efe9200000000p+26 * fexp(fma(0.0, lt, 0x1.a013a00000000p+22 * irt));
-    const double kb = 0x1.253911a940000p+34 * fexp(fma(-0x1.8e9d940000000p-2, lt, -0x1.2821e60000000p+27 * irt));
+    const double kf = 0x1.efe9200000000p+26 * fexp2(fma(0x1.a013a00000000p+22, irt, 0.0 * lt));
+    const double kb = 0x1.9daff9687ba13p+30 * fexp2(fma(-0x1.2821e60000000p+27, irt, -0x1.8e9d940000000p-2 * lt));
     const double q = kf * C7 * C7 - kb * C2 * C8;
     cd2 += q;
     cd7 = fma(-0x1.0000000000000p+1, q, cd7);
     cd8 += q;
     }
     {  // R17 (elementary)
-    const double kf = 0x1.671e344000000p+34 * fexp(fma(0.0, lt, -0x1.fae5a00000000p+23 * irt));
-    const double kb = 0x1.930e1762d83c7p+15 * fexp(fma(0x1.6b42ee0000000p+0, lt, -0x1.1bf1520000000p+28 * irt));
+    const double kf = 0x1.671e344000000p+34 * fexp2(fma(-0x1.fae5a00000000p+23, irt, 0.0 * lt));
+    const double kb = 0x1.57e02b89f45ccp+28 * fexp2(fma(-0x1.1bf1520000000p+28, irt, 0x1.6b42ee0000000p+0 * lt));
     const double q = kf * C8 * C1 - kb * C4 * C6;
     cd1 -= q;
     cd4 += q;
@@ -371,8 +248,8 @@ struct LaneRhs<40> {
     cd8 -= q;
     }
     {  // R18 (elementary)
-    const double kf = 0x1.671e344000000p+35 * fexp(fma(0.0, lt, -0x1.fb8d980000000p+24 * irt));
-    const double kb = 0x1.8f972f345a1cbp+25 * fexp(fma(0x1.8080740000000p-1, lt, -0x1.7bef080000000p+26 * irt));
+    const double kf = 0x1.671e344000000p+35 * fexp2(fma(-0x1.fb8d980000000p+24, irt, 0.0 * lt));
+    const double kb = 0x1.5213294fb0299p+32 * fexp2(fma(-0x1.7bef080000000p+26, irt, 0x1.8080740000000p-1 * lt));
     const double q = kf * C8 * C1 - kb * C5 * C7;
     cd1 -= q;
     cd5 += q;
@@ -380,8 +257,8 @@ struct LaneRhs<40> {
     cd8 -= q;
     }
     {  // R19 (elementary)
-    const double kf = 0x1.2a70000000000p+13 * fexp(fma(0x1.0000000000000p+1, lt, -0x1.fae5a00000000p+23 * irt));
-    const double kb = 0x1.858a9bf2d5c42p+2 * fexp(fma(0x1.5ba4400000000p+1, lt, -0x1.2669640000000p+26 * irt));
+    const double kf = 0x1.2a70000000000p+31 * fexp2(fma(-0x1.fae5a00000000p+23, irt, 0x1.0000000000000p+1 * lt));
+    const double kb = 0x1.08e0b77663642p+27 * fexp2(fma(-0x1.2669640000000p+26, irt, 0x1.5ba4400000000p+1 * lt));
     const double q = kf * C8 * C3 - kb * C7 * C4;
     cd3 -= q;
     cd4 += q;
@@ -389,8 +266,8 @@ struct LaneRhs<40> {
     cd8 -= q;
     }
     {  // R20 (elementary)
-    const double kf = 0x1.dcd6500000000p+29 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.548e5adeb851fp+23 * fexp(fma(0x1.5090f80000000p-1, lt, -0x1.ec42360000000p+26 * irt));
+    const double kf = 0x1.dcd6500000000p+29 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.4156cfde42d8bp+29 * fexp2(fma(-0x1.ec42360000000p+26, irt, 0x1.5090f80000000p-1 * lt));
     const double q = kf * C8 * C4 - kb * C6 * C7;
     cd4 -= q;
     cd6 += q;
@@ -398,8 +275,8 @@ struct LaneRhs<40> {
     cd8 -= q;
     }
     {  // R21 (elementary)
-    const double kf = 0x1.0e15635000000p+39 * fexp(fma(0.0, lt, -0x1.3111a80000000p+25 * irt));
-    const double kb = 0x1.81c942f04cccdp+32 * fexp(fma(0x1.5090f80000000p-1, lt, -0x1.4265840000000p+27 * irt));
+    const double kf = 0x1.0e15635000000p+39 * fexp2(fma(-0x1.3111a80000000p+25, irt, 0.0 * lt));
+    const double kb = 0x1.6c045779c7b98p+38 * fexp2(fma(-0x1.4265840000000p+27, irt, 0x1.5090f80000000p-1 * lt));
     const double q = kf * C8 * C4 - kb * C6 * C7;
     cd4 -= q;
     cd6 += q;
@@ -407,8 +284,8 @@ struct LaneRhs<40> {
     cd8 -= q;
     }
     {  // R23 (elementary)
-    const double kf = 0x1.2d99790000000p+31 * fexp(fma(0.0, lt, -0x1.7ca9b50000000p+27 * irt));
-    const double kb = 0x1.994d75fb94800p+44 * fexp(fma(-0x1.b040180000000p-1, lt, -0x1.c30f7f0000000p+27 * irt));
+    const double kf = 0x1.2d99790000000p+31 * fexp2(fma(-0x1.7ca9b50000000p+27, irt, 0.0 * lt));
+    const double kb = 0x1.0e62a3fc5ebf5p+37 * fexp2(fma(-0x1.c30f7f0000000p+27, irt, -0x1.b040180000000p-1 * lt));
     const double q = kf * C9 * C2 - kb * C3 * C10;
     cd2 -= q;
     cd3 += q;
@@ -416,8 +293,8 @@ struct LaneRhs<40> {
     cd10 += q;
     }
     {  // R24 (elementary)
-    const double kf = 0x1.c086634000000p+34 * fexp(fma(0.0, lt, -0x1.6f18900000000p+26 * irt));
-    const double kb = 0x1.d5c7e0bb06000p+44 * fexp(fma(-0x1.08fe6a0000000p-1, lt, -0x1.534d760000000p+28 * irt));
+    const double kf = 0x1.c086634000000p+34 * fexp2(fma(-0x1.6f18900000000p+26, irt, 0.0 * lt));
+    const double kb = 0x1.29b501f6ba9f1p+40 * fexp2(fma(-0x1.534d760000000p+28, irt, -0x1.08fe6a0000000p-1 * lt));
     const double q = kf * C9 * C7 - kb * C4 * C10;
     cd4 += q;
     cd7 -= q;
@@ -425,8 +302,8 @@ struct LaneRhs<40> {
     cd10 += q;
     }
     {  // R25 (elementary)
-    const double kf = 0x1.bdccccccccccdp+7 * fexp(fma(0x1.e3d70a0000000p+0, lt, 0x1.27e6000000000p+22 * irt));
-    const double kb = 0x1.2920255b9999ap+30 * fexp(fma(0x1.38bb2c0000000p-1, lt, -0x1.87788e0000000p+26 * irt));
+    const double kf = 0x1.c0e6972b4185ap+24 * fexp2(fma(0x1.27e6000000000p+22, irt, 0x1.e3d70a0000000p+0 * lt));
+    const double kb = 0x1.a364639359a4cp+35 * fexp2(fma(-0x1.87788e0000000p+26, irt, 0x1.38bb2c0000000p-1 * lt));
     const double q = kf * C9 * C4 - kb * C1 * C10;
     cd1 += q;
     cd4 -= q;
@@ -434,8 +311,8 @@ struct LaneRhs<40> {
     cd10 += q;
     }
     {  // R27 (elementary)
-    const double kf = 0x1.c3cd9f0000000p+32 * fexp(fma(0.0, lt, -0x1.a2b3800000000p+20 * irt));
-    const double kb = 0x1.01000f139999ap+31 * fexp(fma(0x1.c1a5880000000p-3, lt, -0x1.0f30360000000p+27 * irt));
+    const double kf = 0x1.c3cd9f0000000p+32 * fexp2(fma(-0x1.a2b3800000000p+20, irt, 0.0 * lt));
+    const double kb = 0x1.f98400ab895bcp+32 * fexp2(fma(-0x1.0f30360000000p+27, irt, 0x1.c1a5880000000p-3 * lt));
     const double q = kf * C11 * C2 - kb * C7 * C9;
     cd2 -= q;
     cd7 += q;
@@ -443,8 +320,8 @@ struct LaneRhs<40> {
     cd11 -= q;
     }
     {  // R28 (elementary)
-    const double kf = 0x1.0d56a73000000p+36 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.9331edb466666p+31 * fexp(fma(0x1.299b2c0000000p-1, lt, -0x1.5fc9920000000p+28 * irt));
+    const double kf = 0x1.0d56a73000000p+36 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.d95397ba5473dp+36 * fexp2(fma(-0x1.5fc9920000000p+28, irt, 0x1.299b2c0000000p-1 * lt));
     const double q = kf * C11 * C1 - kb * C5 * C9;
     cd1 -= q;
     cd5 += q;
@@ -452,8 +329,8 @@ struct LaneRhs<40> {
     cd11 -= q;
     }
     {  // R29 (elementary)
-    const double kf = 0x1.c203db8000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.8b205a231eb85p+29 * fexp(fma(0x1.17ab100000000p-1, lt, -0x1.5a49d60000000p+28 * irt));
+    const double kf = 0x1.c203db8000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.74c9d4619d3cap+34 * fexp2(fma(-0x1.5a49d60000000p+28, irt, 0x1.17ab100000000p-1 * lt));
     const double q = kf * C11 * C3 - kb * C4 * C9;
     cd3 -= q;
     cd4 += q;
@@ -461,8 +338,8 @@ struct LaneRhs<40> {
     cd11 -= q;
     }
     {  // R30 (elementary)
-    const double kf = 0x1.c203db8000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.b0660acc00000p+33 * fexp(fma(0x1.f357600000000p-2, lt, -0x1.9b9736b000000p+28 * irt));
+    const double kf = 0x1.c203db8000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.1b0f27eb41fe2p+38 * fexp2(fma(-0x1.9b9736b000000p+28, irt, 0x1.f357600000000p-2 * lt));
     const double q = kf * C11 * C4 - kb * C6 * C9;
     cd4 -= q;
     cd6 += q;
@@ -470,8 +347,8 @@ struct LaneRhs<40> {
     cd11 -= q;
     }
     {  // R31 (elementary)
-    const double kf = 0x1.bf08eb0000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.059b8949640e0p+52 * fexp(fma(-0x1.7747d80000000p-1, lt, -0x1.c0c7900000000p+28 * irt));
+    const double kf = 0x1.bf08eb0000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.59f9ff371c5f5p+45 * fexp2(fma(-0x1.c0c7900000000p+28, irt, -0x1.7747d80000000p-1 * lt));
     const double q = kf * C11 * C3 - kb * C1 * C10;
     cd1 += q;
     cd3 -= q;
@@ -479,8 +356,8 @@ struct LaneRhs<40> {
     cd11 -= q;
     }
     {  // R32 (elementary)
-    const double kf = 0x1.bf08eb0000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.8091bae6ccccdp+32 * fexp(fma(-0x1.23f2900000000p-2, lt, -0x1.749c2e0000000p+27 * irt));
+    const double kf = 0x1.bf08eb0000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.03c80e71dff43p+30 * fexp2(fma(-0x1.749c2e0000000p+27, irt, -0x1.23f2900000000p-2 * lt));
     const double q = kf * C11 * C7 - kb * C1 * C4 * C10;
     cd1 += q;
     cd4 += q;
@@ -489,16 +366,16 @@ struct LaneRhs<40> {
     cd11 -= q;
     }
     {  // R33 (elementary)
-    const double kf = 0x1.65a0bc0000000p+31 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.b7b766db50f41p+14 * fexp(fma(0x1.a0a04e0000000p-1, lt, -0x1.2290560000000p+28 * irt));
+    const double kf = 0x1.65a0bc0000000p+31 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.131fad708d3f5p+22 * fexp2(fma(-0x1.2290560000000p+28, irt, 0x1.a0a04e0000000p-1 * lt));
     const double q = kf * C11 * C11 - kb * C9 * C9 * C5;
     cd5 += q;
     cd9 = fma(0x1.0000000000000p+1, q, cd9);
     cd11 = fma(-0x1.0000000000000p+1, q, cd11);
     }
     {  // R34 (elementary)
-    const double kf = 0x1.8ae17a4000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.888c4f8178000p+38 * fexp(fma(0x1.2a11aa0000000p-2, lt, -0x1.675b5c0000000p+28 * irt));
+    const double kf = 0x1.8ae17a4000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.2d98882ccc5efp+41 * fexp2(fma(-0x1.675b5c0000000p+28, irt, 0x1.2a11aa0000000p-2 * lt));
     const double q = kf * C11 * C12 - kb * C13 * C9;
     cd9 += q;
     cd11 -= q;
@@ -506,16 +383,16 @@ struct LaneRhs<40> {
     cd13 += q;
     }
     {  // R35 (elementary)
-    const double kf = 0x1.bf08eb0000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.ca18315f54000p+39 * fexp(fma(0x1.ca5bda0000000p-4, lt, -0x1.2bd16a0000000p+28 * irt));
+    const double kf = 0x1.bf08eb0000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.cc5db1ef97340p+40 * fexp2(fma(-0x1.2bd16a0000000p+28, irt, 0x1.ca5bda0000000p-4 * lt));
     const double q = kf * C11 * C11 - kb * C9 * C14;
     cd9 += q;
     cd11 = fma(-0x1.0000000000000p+1, q, cd11);
     cd14 += q;
     }
     {  // R38 (elementary)
-    const double kf = 0x1.c070000000000p+15 * fexp(fma(0x1.e666660000000p+0, lt, -0x1.5ef3c00000000p+23 * irt));
-    const double kb = 0x1.478c4a8f3cc0cp+6 * fexp(fma(0x1.2f47300000000p+1, lt, -0x1.f77e280000000p+25 * irt));
+    const double kf = 0x1.e09f93403f5d2p+32 * fexp2(fma(-0x1.5ef3c00000000p+23, irt, 0x1.e666660000000p+0 * lt));
+    const double kb = 0x1.9a1771db5774dp+27 * fexp2(fma(-0x1.f77e280000000p+25, irt, 0x1.2f47300000000p+1 * lt));
     const double q = kf * C14 * C1 - kb * C5 * C11;
     cd1 -= q;
     cd5 += q;
@@ -523,8 +400,8 @@ struct LaneRhs<40> {
     cd14 -= q;
     }
     {  // R39 (elementary)
-    const double kf = 0x1.0db6054000000p+34 * fexp(fma(0.0, lt, -0x1.8947b00000000p+23 * irt));
-    const double kb = 0x1.ce3190483126fp+23 * fexp(fma(0x1.bcbf2c0000000p-2, lt, -0x1.d615400000000p+25 * irt));
+    const double kf = 0x1.0db6054000000p+34 * fexp2(fma(-0x1.8947b00000000p+23, irt, 0.0 * lt));
+    const double kb = 0x1.b1e99f0731613p+27 * fexp2(fma(-0x1.d615400000000p+25, irt, 0x1.bcbf2c0000000p-2 * lt));
     const double q = kf * C14 * C3 - kb * C4 * C11;
     cd3 -= q;
     cd4 += q;
@@ -532,8 +409,8 @@ struct LaneRhs<40> {
     cd14 -= q;
     }
     {  // R40 (elementary)
-    const double kf = 0x1.a2b3800000000p+21 * fexp(fma(0x1.2e147a0000000p+0, lt, 0x1.c88b000000000p+20 * irt));
-    const double kb = 0x1.8898ff2f33ca3p+15 * fexp(fma(0x1.8e44520000000p+0, lt, -0x1.b7f5040000000p+26 * irt));
+    const double kf = 0x1.41bee09672314p+32 * fexp2(fma(0x1.c88b000000000p+20, irt, 0x1.2e147a0000000p+0 * lt));
+    const double kb = 0x1.89066bb61c1ebp+29 * fexp2(fma(-0x1.b7f5040000000p+26, irt, 0x1.8e44520000000p+0 * lt));
     const double q = kf * C14 * C4 - kb * C6 * C11;
     cd4 -= q;
     cd6 += q;
@@ -541,8 +418,8 @@ struct LaneRhs<40> {
     cd14 -= q;
     }
     {  // R41 (elementary)
-    const double kf = 0x1.3380000000000p+10 * fexp(fma(0x1.8000000000000p+1, lt, -0x1.9efa600000000p+27 * irt));
-    const double kb = 0x1.5562cba25debfp+3 * fexp(fma(0x1.8dc77a0000000p+1, lt, -0x1.4d09680000000p+25 * irt));
+    const double kf = 0x1.3380000000000p+37 * fexp2(fma(-0x1.9efa600000000p+27, irt, 0x1.8000000000000p+1 * lt));
+    const double kb = 0x1.4e180e3701c3bp+31 * fexp2(fma(-0x1.4d09680000000p+25, irt, 0x1.8dc77a0000000p+1 * lt));
     const double q = kf * C14 * C2 - kb * C7 * C11;
     cd2 -= q;
     cd7 += q;
@@ -550,8 +427,8 @@ struct LaneRhs<40> {
     cd14 -= q;
     }
     {  // R42 (elementary)
-    const double kf = 0x1.48ccccccccccdp+5 * fexp(fma(0x1.4000000000000p+1, lt, -0x1.45eb8c0000000p+25 * irt));
-    const double kb = 0x1.afacc53eb8f86p+5 * fexp(fma(0x1.1bf3e00000000p+1, lt, -0x1.d72b020000000p+24 * irt));
+    const double kf = 0x1.d0fe50ba50401p+27 * fexp2(fma(-0x1.45eb8c0000000p+25, irt, 0x1.4000000000000p+1 * lt));
+    const double kb = 0x1.a5737523cf108p+25 * fexp2(fma(-0x1.d72b020000000p+24, irt, 0x1.1bf3e00000000p+1 * lt));
     const double q = kf * C14 * C7 - kb * C8 * C11;
     cd7 -= q;
     cd8 += q;
@@ -559,8 +436,8 @@ struct LaneRhs<40> {
     cd14 -= q;
     }
     {  // R43 (elementary)
-    const double kf = 0x1.f3ba607d8040fp-29 * fexp(fma(0x1.5ae1480000000p+2, lt, -0x1.fdc4000000000p+21 * irt));
-    const double kb = 0x1.e4c84e0553513p-30 * fexp(fma(0x1.6658f80000000p+2, lt, -0x1.fc2bc60000000p+25 * irt));
+    const double kf = 0x1.ad0ca6f45a157p+20 * fexp2(fma(-0x1.fdc4000000000p+21, irt, 0x1.5ae1480000000p+2 * lt));
+    const double kb = 0x1.3e34a543cdb1dp+21 * fexp2(fma(-0x1.fc2bc60000000p+25, irt, 0x1.6658f80000000p+2 * lt));
     const double q = kf * C14 * C12 - kb * C13 * C11;
     cd11 += q;
     cd12 -= q;
@@ -568,8 +445,8 @@ struct LaneRhs<40> {
     cd14 -= q;
     }
     {  // R44 (elementary)
-    const double kf = 0x1.3a0abeb000000p+36 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.8948ed0a1c000p+43 * fexp(fma(-0x1.3794ea0000000p-2, lt, -0x1.1a7de40000000p+28 * irt));
+    const double kf = 0x1.3a0abeb000000p+36 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.d76fc32055919p+40 * fexp2(fma(-0x1.1a7de40000000p+28, irt, -0x1.3794ea0000000p-2 * lt));
     const double q = kf * C12 * C3 - kb * C1 * C14;
     cd1 += q;
     cd3 -= q;
@@ -577,8 +454,8 @@ struct LaneRhs<40> {
     cd14 += q;
     }
     {  // R45 (elementary)
-    const double kf = 0x1.c4793ec698000p+50 * fexp(fma(-0x1.91eb860000000p+0, lt, -0x1.d287a40000000p+26 * irt));
-    const double kb = 0x1.3a528b132883ap+58 * fexp(fma(-0x1.06eac80000000p+1, lt, -0x1.c51f6c0000000p+22 * irt));
+    const double kf = 0x1.9d7c071f9a764p+36 * fexp2(fma(-0x1.d287a40000000p+26, irt, -0x1.91eb860000000p+0 * lt));
+    const double kb = 0x1.c0bde8218b7acp+39 * fexp2(fma(-0x1.c51f6c0000000p+22, irt, -0x1.06eac80000000p+1 * lt));
     const double q = kf * C12 * C2 - kb * C3 * C15;
     cd2 -= q;
     cd3 += q;
@@ -586,8 +463,8 @@ struct LaneRhs<40> {
     cd15 += q;
     }
     {  // R46 (elementary)
-    const double kf = 0x1.64ac980000000p+28 * fexp(fma(0.0, lt, -0x1.d354b80000000p+25 * irt));
-    const double kb = 0x1.c6c0a65c28f5cp+26 * fexp(fma(0x1.0ba0e80000000p-3, lt, -0x1.119da40000000p+28 * irt));
+    const double kf = 0x1.64ac980000000p+28 * fexp2(fma(-0x1.d354b80000000p+25, irt, 0.0 * lt));
+    const double kb = 0x1.00e557774649ep+28 * fexp2(fma(-0x1.119da40000000p+28, irt, 0x1.0ba0e80000000p-3 * lt));
     const double q = kf * C12 * C2 - kb * C4 * C14;
     cd2 -= q;
     cd4 += q;
@@ -595,8 +472,8 @@ struct LaneRhs<40> {
     cd14 += q;
     }
     {  // R47 (elementary)
-    const double kf = 0x1.6fbca00000000p+24 * fexp(fma(0x1.851eb80000000p-1, lt, 0x1.28e0000000000p+23 * irt));
-    const double kb = 0x1.8a50cd55c28f6p+28 * fexp(fma(0x1.348c0c0000000p-1, lt, -0x1.7600080000000p+26 * irt));
+    const double kf = 0x1.492236ed14120p+31 * fexp2(fma(0x1.28e0000000000p+23, irt, 0x1.851eb80000000p-1 * lt));
+    const double kb = 0x1.0874d3ed7b6fbp+34 * fexp2(fma(-0x1.7600080000000p+26, irt, 0x1.348c0c0000000p-1 * lt));
     const double q = kf * C12 * C7 - kb * C4 * C15;
     cd4 += q;
     cd7 -= q;
@@ -604,8 +481,8 @@ struct LaneRhs<40> {
     cd15 += q;
     }
     {  // R50 (elementary)
-    const double kf = 0x1.ab58000000000p+15 * fexp(fma(0x1.f851ec0000000p+0, lt, -0x1.65d76c0000000p+25 * irt));
-    const double kb = 0x1.41c38b03a9adcp+7 * fexp(fma(0x1.214d940000000p+1, lt, -0x1.29491e0000000p+25 * irt));
+    const double kf = 0x1.62679312c4f10p+33 * fexp2(fma(-0x1.65d76c0000000p+25, irt, 0x1.f851ec0000000p+0 * lt));
+    const double kb = 0x1.97bb7694f5acep+27 * fexp2(fma(-0x1.29491e0000000p+25, irt, 0x1.214d940000000p+1 * lt));
     const double q = kf * C13 * C1 - kb * C5 * C12;
     cd1 -= q;
     cd5 += q;
@@ -613,8 +490,8 @@ struct LaneRhs<40> {
     cd13 -= q;
     }
     {  // R51 (elementary)
-    const double kf = 0x1.77825f0000000p+31 * fexp(fma(0x1.0000000000000p-1, lt, -0x1.4877e40000000p+25 * irt));
-    const double kb = 0x1.4baad85638866p+22 * fexp(fma(0x1.82a25e0000000p-1, lt, -0x1.bfd7640000000p+24 * irt));
+    const double kf = 0x1.09866ff179a9fp+36 * fexp2(fma(-0x1.4877e40000000p+25, irt, 0x1.0000000000000p-1 * lt));
+    const double kb = 0x1.1ffea389f7dadp+29 * fexp2(fma(-0x1.bfd7640000000p+24, irt, 0x1.82a25e0000000p-1 * lt));
     const double q = kf * C13 * C3 - kb * C4 * C12;
     cd3 -= q;
     cd4 += q;
@@ -622,8 +499,8 @@ struct LaneRhs<40> {
     cd13 -= q;
     }
     {  // R52 (elementary)
-    const double kf = 0x1.6580000000000p+12 * fexp(fma(0x1.f5c2900000000p+0, lt, -0x1.50f9a00000000p+23 * irt));
-    const double kb = 0x1.598be1dfd96efp+7 * fexp(fma(0x1.140a280000000p+1, lt, -0x1.f61d440000000p+25 * irt));
+    const double kf = 0x1.168d28c7e5cabp+30 * fexp2(fma(-0x1.50f9a00000000p+23, irt, 0x1.f5c2900000000p+0 * lt));
+    const double kb = 0x1.cad12a5122b1cp+26 * fexp2(fma(-0x1.f61d440000000p+25, irt, 0x1.140a280000000p+1 * lt));
     const double q = kf * C13 * C4 - kb * C6 * C12;
     cd4 -= q;
     cd6 += q;
@@ -631,8 +508,8 @@ struct LaneRhs<40> {
     cd13 -= q;
     }
     {  // R53 (elementary)
-    const double kf = 0x1.78b38c0000000p+31 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.4929815c90000p+37 * fexp(fma(0x1.24fadc0000000p-4, lt, -0x1.c2cbe72000000p+27 * irt));
+    const double kf = 0x1.78b38c0000000p+31 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.0123cb9a1cd5bp+38 * fexp2(fma(-0x1.c2cbe72000000p+27, irt, 0x1.24fadc0000000p-4 * lt));
     const double q = kf * C12 * C7 - kb * C2 * C13;
     cd2 += q;
     cd7 -= q;
@@ -640,8 +517,8 @@ struct LaneRhs<40> {
     cd13 += q;
     }
     {  // R54 (elementary)
-    const double kf = 0x1.593ae80000000p+27 * fexp(fma(0.0, lt, -0x1.288cfe0000000p+26 * irt));
-    const double kb = 0x1.d3380e1fd70a4p+28 * fexp(fma(-0x1.d7dc380000000p-2, lt, -0x1.a746b80000000p+21 * irt));
+    const double kf = 0x1.593ae80000000p+27 * fexp2(fma(-0x1.288cfe0000000p+26, irt, 0.0 * lt));
+    const double kb = 0x1.a5e58ddf05750p+24 * fexp2(fma(-0x1.a746b80000000p+21, irt, -0x1.d7dc380000000p-2 * lt));
     const double q = kf * C13 * C7 - kb * C8 * C12;
     cd7 -= q;
     cd8 += q;
@@ -649,8 +526,8 @@ struct LaneRhs<40> {
     cd13 -= q;
     }
     {  // R56 (elementary)
-    const double kf = 0x1.65a0bc0000000p+32 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.aeb9dc4000000p+27 * fexp(fma(0x1.5638860000000p-1, lt, -0x1.2c42580000000p+28 * irt));
+    const double kf = 0x1.65a0bc0000000p+32 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.b368a3585505fp+33 * fexp2(fma(-0x1.2c42580000000p+28, irt, 0x1.5638860000000p-1 * lt));
     const double q = kf * C17 * C1 - kb * C5 * C14;
     cd1 -= q;
     cd5 += q;
@@ -658,8 +535,8 @@ struct LaneRhs<40> {
     cd17 -= q;
     }
     {  // R57 (elementary)
-    const double kf = 0x1.66ee853800000p+36 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.94ef1b71a9fbep+23 * fexp(fma(0x1.e012e00000000p-1, lt, -0x1.8896f60000000p+23 * irt));
+    const double kf = 0x1.66ee853800000p+36 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.127041585f3dep+32 * fexp2(fma(-0x1.8896f60000000p+23, irt, 0x1.e012e00000000p-1 * lt));
     const double q = kf * C17 * C1 - kb * C4 * C12;
     cd1 -= q;
     cd4 += q;
@@ -667,8 +544,8 @@ struct LaneRhs<40> {
     cd17 -= q;
     }
     {  // R58 (elementary)
-    const double kf = 0x1.38eca48000000p+35 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.ba1c6d5ef5c29p+29 * fexp(fma(0x1.44486a0000000p-1, lt, -0x1.26c29c0000000p+28 * irt));
+    const double kf = 0x1.38eca48000000p+35 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.672d38be57531p+35 * fexp2(fma(-0x1.26c29c0000000p+28, irt, 0x1.44486a0000000p-1 * lt));
     const double q = kf * C17 * C3 - kb * C4 * C14;
     cd3 -= q;
     cd4 += q;
@@ -676,8 +553,8 @@ struct LaneRhs<40> {
     cd17 -= q;
     }
     {  // R59 (elementary)
-    const double kf = 0x1.65a0bc0000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.14774561d999ap+33 * fexp(fma(0x1.26490a0000000p-1, lt, -0x1.680ffe0000000p+28 * irt));
+    const double kf = 0x1.65a0bc0000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.37af2e85ea31bp+38 * fexp2(fma(-0x1.680ffe0000000p+28, irt, 0x1.26490a0000000p-1 * lt));
     const double q = kf * C17 * C4 - kb * C6 * C14;
     cd4 -= q;
     cd6 += q;
@@ -685,8 +562,8 @@ struct LaneRhs<40> {
     cd17 -= q;
     }
     {  // R60 (elementary)
-    const double kf = 0x1.c0e5c15000000p+37 * fexp(fma(0.0, lt, -0x1.404c180000000p+24 * irt));
-    const double kb = 0x1.9ae11fff00000p+35 * fexp(fma(0x1.3a0d780000000p-2, lt, -0x1.99cbc00000000p+26 * irt));
+    const double kf = 0x1.c0e5c15000000p+37 * fexp2(fma(-0x1.404c180000000p+24, irt, 0.0 * lt));
+    const double kb = 0x1.5bf71730024bep+38 * fexp2(fma(-0x1.99cbc00000000p+26, irt, 0x1.3a0d780000000p-2 * lt));
     const double q = kf * C17 * C2 - kb * C7 * C14;
     cd2 -= q;
     cd7 += q;
@@ -694,8 +571,8 @@ struct LaneRhs<40> {
     cd17 -= q;
     }
     {  // R61 (elementary)
-    const double kf = 0x1.5f93037c00000p+40 * fexp(fma(-0x1.0000000000000p+0, lt, 0.0 * irt));
-    const double kb = 0x1.41cc775538000p+38 * fexp(fma(-0x1.62f9440000000p-1, lt, -0x1.49b8ba0000000p+26 * irt));
+    const double kf = 0x1.5f93037c00000p+31 * fexp2(fma(0.0, irt, -0x1.0000000000000p+0 * lt));
+    const double kb = 0x1.10864cd959e36p+32 * fexp2(fma(-0x1.49b8ba0000000p+26, irt, -0x1.62f9440000000p-1 * lt));
     const double q = kf * C17 * C2 - kb * C7 * C14;
     cd2 -= q;
     cd7 += q;
@@ -703,8 +580,8 @@ struct LaneRhs<40> {
     cd17 -= q;
     }
     {  // R62 (elementary)
-    const double kf = 0x1.65a0bc0000000p+33 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.831991b520000p+38 * fexp(fma(-0x1.523fee0000000p-4, lt, -0x1.d9fee00000000p+27 * irt));
+    const double kf = 0x1.65a0bc0000000p+33 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.ce824c40b73e7p+37 * fexp2(fma(-0x1.d9fee00000000p+27, irt, -0x1.523fee0000000p-4 * lt));
     const double q = kf * C17 * C7 - kb * C8 * C14;
     cd7 -= q;
     cd8 += q;
@@ -712,16 +589,16 @@ struct LaneRhs<40> {
     cd17 -= q;
     }
     {  // R63 (elementary)
-    const double kf = 0x1.bf08eb0000000p+33 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.708f5553b0000p+38 * fexp(fma(0x1.97a3560000000p-3, lt, -0x1.f09462e000000p+27 * irt));
+    const double kf = 0x1.bf08eb0000000p+33 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.3ef0319c66305p+40 * fexp2(fma(-0x1.f09462e000000p+27, irt, 0x1.97a3560000000p-3 * lt));
     const double q = kf * C17 * C11 - kb * C14 * C14;
     cd11 -= q;
     cd14 = fma(0x1.0000000000000p+1, q, cd14);
     cd17 -= q;
     }
     {  // R65 (elementary)
-    const double kf = 0x1.dcd6500000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.5d6a4efd75e20p+18 * fexp(fma(0x1.d6872c0000000p-1, lt, -0x1.5214a40000000p+25 * irt));
+    const double kf = 0x1.dcd6500000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.a59eb0dafa7f8p+26 * fexp2(fma(-0x1.5214a40000000p+25, irt, 0x1.d6872c0000000p-1 * lt));
     const double q = kf * C15 * C1 - kb * C4 * C12;
     cd1 -= q;
     cd4 += q;
@@ -729,8 +606,8 @@ struct LaneRhs<40> {
     cd15 -= q;
     }
     {  // R66 (elementary)
-    const double kf = 0x1.65a0bc0000000p+32 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.48301ff22d0e5p+23 * fexp(fma(0x1.3abc940000000p-1, lt, -0x1.44c0780000000p+28 * irt));
+    const double kf = 0x1.65a0bc0000000p+32 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.dab20b0aa9b31p+28 * fexp2(fma(-0x1.44c0780000000p+28, irt, 0x1.3abc940000000p-1 * lt));
     const double q = kf * C15 * C3 - kb * C4 * C14;
     cd3 -= q;
     cd4 += q;
@@ -738,8 +615,8 @@ struct LaneRhs<40> {
     cd15 -= q;
     }
     {  // R67 (elementary)
-    const double kf = 0x1.0c388d0000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.0d5c0470ccccdp+29 * fexp(fma(0x1.1cbd340000000p-1, lt, -0x1.860dda0000000p+28 * irt));
+    const double kf = 0x1.0c388d0000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.0e5400e0088cdp+34 * fexp2(fma(-0x1.860dda0000000p+28, irt, 0x1.1cbd340000000p-1 * lt));
     const double q = kf * C15 * C4 - kb * C6 * C14;
     cd4 -= q;
     cd6 += q;
@@ -747,8 +624,8 @@ struct LaneRhs<40> {
     cd15 -= q;
     }
     {  // R68 (elementary)
-    const double kf = 0x1.508166a800000p+36 * fexp(fma(0.0, lt, -0x1.7e6a700000000p+25 * irt));
-    const double kb = 0x1.901e599533333p+30 * fexp(fma(0x1.26f60e0000000p-2, lt, -0x1.4072b2e000000p+27 * irt));
+    const double kf = 0x1.508166a800000p+36 * fexp2(fma(-0x1.7e6a700000000p+25, irt, 0.0 * lt));
+    const double kb = 0x1.2da58a5a20cd7p+33 * fexp2(fma(-0x1.4072b2e000000p+27, irt, 0x1.26f60e0000000p-2 * lt));
     const double q = kf * C15 * C2 - kb * C7 * C14;
     cd2 -= q;
     cd7 += q;
@@ -756,8 +633,8 @@ struct LaneRhs<40> {
     cd15 -= q;
     }
     {  // R69 (elementary)
-    const double kf = 0x1.4fb1800000000p+24 * fexp(fma(0.0, lt, -0x1.be69400000000p+22 * irt));
-    const double kb = 0x1.8f2725b37c99bp+18 * fexp(fma(0x1.26f60e0000000p-2, lt, -0x1.dd96c1c000000p+26 * irt));
+    const double kf = 0x1.4fb1800000000p+24 * fexp2(fma(-0x1.be69400000000p+22, irt, 0.0 * lt));
+    const double kb = 0x1.2ceb2d10fd3efp+21 * fexp2(fma(-0x1.dd96c1c000000p+26, irt, 0x1.26f60e0000000p-2 * lt));
     const double q = kf * C15 * C2 - kb * C7 * C14;
     cd2 -= q;
     cd7 += q;
@@ -765,8 +642,8 @@ struct LaneRhs<40> {
     cd15 -= q;
     }
     {  // R70 (elementary)
-    const double kf = 0x1.1e1a300000000p+28 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.924afcc651eb8p+29 * fexp(fma(-0x1.9e9e1c0000000p-4, lt, -0x1.0afd4c0000000p+28 * irt));
+    const double kf = 0x1.1e1a300000000p+28 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.abe26c8e87deap+28 * fexp2(fma(-0x1.0afd4c0000000p+28, irt, -0x1.9e9e1c0000000p-4 * lt));
     const double q = kf * C15 * C7 - kb * C8 * C14;
     cd7 -= q;
     cd8 += q;
@@ -774,8 +651,8 @@ struct LaneRhs<40> {
     cd15 -= q;
     }
     {  // R71 (elementary)
-    const double kf = 0x1.dcd6500000000p+33 * fexp(fma(0.0, lt, -0x1.78abbc0000000p+25 * irt));
-    const double kb = 0x1.d1c5358b10000p+39 * fexp(fma(-0x1.70d77c0000000p-2, lt, -0x1.7fab900000000p+27 * irt));
+    const double kf = 0x1.dcd6500000000p+33 * fexp2(fma(-0x1.78abbc0000000p+25, irt, 0.0 * lt));
+    const double kb = 0x1.89e78a47d325fp+36 * fexp2(fma(-0x1.7fab900000000p+27, irt, -0x1.70d77c0000000p-2 * lt));
     const double q = kf * C15 * C9 - kb * C10 * C12;
     cd9 -= q;
     cd10 += q;
@@ -783,32 +660,32 @@ struct LaneRhs<40> {
     cd15 -= q;
     }
     {  // R72 (elementary)
-    const double kf = 0x1.296d5b8000000p+32 * fexp(fma(0x1.99999a0000000p-4, lt, -0x1.525d180000000p+25 * irt));
-    const double kb = 0x1.466016bc3af00p+49 * fexp(fma(-0x1.110ffa0000000p+0, lt, -0x1.afab2c0000000p+22 * irt));
+    const double kf = 0x1.1582662f0c6b0p+33 * fexp2(fma(-0x1.525d180000000p+25, irt, 0x1.99999a0000000p-4 * lt));
+    const double kb = 0x1.aeb3152d40710p+39 * fexp2(fma(-0x1.afab2c0000000p+22, irt, -0x1.110ffa0000000p+0 * lt));
     const double q = kf * C12 * C12 - kb * C18 * C1;
     cd1 += q;
     cd12 = fma(-0x1.0000000000000p+1, q, cd12);
     cd18 += q;
     }
     {  // R73 (elementary)
-    const double kf = 0x1.3380000000000p+11 * fexp(fma(0x1.0000000000000p+1, lt, -0x1.07fe080000000p+25 * irt));
-    const double kb = 0x1.770908eb610c9p+11 * fexp(fma(0x1.c773c00000000p+0, lt, -0x1.b929040000000p+25 * irt));
+    const double kf = 0x1.3380000000000p+29 * fexp2(fma(-0x1.07fe080000000p+25, irt, 0x1.0000000000000p+1 * lt));
+    const double kb = 0x1.7a2a3f6677c87p+27 * fexp2(fma(-0x1.b929040000000p+25, irt, 0x1.c773c00000000p+0 * lt));
     const double q = kf * C13 * C19 - kb * C12 * C12;
     cd12 = fma(0x1.0000000000000p+1, q, cd12);
     cd13 -= q;
     cd19 -= q;
     }
     {  // R74 (elementary)
-    const double kf = 0x1.dcd6500000000p+33 * fexp(fma(0.0, lt, 0x1.2323400000000p+21 * irt));
-    const double kb = 0x1.a803ae4e00000p+33 * fexp(fma(-0x1.21f8a00000000p-2, lt, -0x1.bb922e0000000p+25 * irt));
+    const double kf = 0x1.dcd6500000000p+33 * fexp2(fma(0x1.2323400000000p+21, irt, 0.0 * lt));
+    const double kb = 0x1.21e5859ac215bp+31 * fexp2(fma(-0x1.bb922e0000000p+25, irt, -0x1.21f8a00000000p-2 * lt));
     const double q = kf * C13 * C20 - kb * C12 * C12;
     cd12 = fma(0x1.0000000000000p+1, q, cd12);
     cd13 -= q;
     cd20 -= q;
     }
     {  // R75 (elementary)
-    const double kf = 0x1.b580000000000p+15 * fexp(fma(0x1.99999a0000000p+0, lt, -0x1.5a06080000000p+24 * irt));
-    const double kb = 0x1.5ab8d43dda562p+10 * fexp(fma(0x1.023b7a0000000p+1, lt, -0x1.9db6e20000000p+25 * irt));
+    const double kf = 0x1.20a47438ebc8ep+30 * fexp2(fma(-0x1.5a06080000000p+24, irt, 0x1.99999a0000000p+0 * lt));
+    const double kb = 0x1.8292a1c2e682cp+28 * fexp2(fma(-0x1.9db6e20000000p+25, irt, 0x1.023b7a0000000p+1 * lt));
     const double q = kf * C12 * C4 - kb * C6 * C19;
     cd4 -= q;
     cd6 += q;
@@ -816,8 +693,8 @@ struct LaneRhs<40> {
     cd19 += q;
     }
     {  // R76 (elementary)
-    const double kf = 0x1.74ad942000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.95178cc228f5cp+29 * fexp(fma(0x1.eb3e580000000p-2, lt, 0x1.5f2c3e0000000p+22 * irt));
+    const double kf = 0x1.74ad942000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.f8d67394608f6p+33 * fexp2(fma(0x1.5f2c3e0000000p+22, irt, 0x1.eb3e580000000p-2 * lt));
     const double q = kf * C12 * C4 - kb * C6 * C20;
     cd4 -= q;
     cd6 += q;
@@ -825,8 +702,8 @@ struct LaneRhs<40> {
     cd20 += q;
     }
     {  // R77 (elementary)
-    const double kf = 0x1.2a05f20000000p+35 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.40dd1d80acac8p+58 * fexp(fma(-0x1.3b2ca60000000p+0, lt, -0x1.0700392000000p+28 * irt));
+    const double kf = 0x1.2a05f20000000p+35 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.2f7b5d62acb31p+47 * fexp2(fma(-0x1.0700392000000p+28, irt, -0x1.3b2ca60000000p+0 * lt));
     const double q = kf * C12 * C19 - kb * C1 * C21;
     cd1 += q;
     cd12 -= q;
@@ -834,8 +711,8 @@ struct LaneRhs<40> {
     cd21 += q;
     }
     {  // R78 (elementary)
-    const double kf = 0x1.65a0bc0000000p+33 * fexp(fma(0.0, lt, 0x1.2323400000000p+21 * irt));
-    const double kb = 0x1.18ba4e0c9fd34p+56 * fexp(fma(-0x1.4b1ee20000000p+0, lt, -0x1.284d1f6000000p+28 * irt));
+    const double kf = 0x1.65a0bc0000000p+33 * fexp2(fma(0x1.2323400000000p+21, irt, 0.0 * lt));
+    const double kb = 0x1.680dbb28d9926p+44 * fexp2(fma(-0x1.284d1f6000000p+28, irt, -0x1.4b1ee20000000p+0 * lt));
     const double q = kf * C12 * C20 - kb * C1 * C21;
     cd1 += q;
     cd12 -= q;
@@ -843,8 +720,8 @@ struct LaneRhs<40> {
     cd21 += q;
     }
     {  // R79 (elementary)
-    const double kf = 0x1.dcd6500000000p+33 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.7bce50d3dd624p+12 * fexp(fma(0x1.66132c0000000p+0, lt, -0x1.262f1e0000000p+25 * irt));
+    const double kf = 0x1.dcd6500000000p+33 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.1d91541007b92p+25 * fexp2(fma(-0x1.262f1e0000000p+25, irt, 0x1.66132c0000000p+0 * lt));
     const double q = kf * C15 * C1 - kb * C6 * C20;
     cd1 -= q;
     cd6 += q;
@@ -852,8 +729,8 @@ struct LaneRhs<40> {
     cd20 += q;
     }
     {  // R80 (elementary)
-    const double kf = 0x1.c138000000000p+16 * fexp(fma(0x1.e666660000000p+0, lt, -0x1.e0be500000000p+24 * irt));
-    const double kb = 0x1.8db5106e9e548p+4 * fexp(fma(0x1.383f3e0000000p+1, lt, -0x1.489e160000000p+25 * irt));
+    const double kf = 0x1.e175ee0b49494p+33 * fexp2(fma(-0x1.e0be500000000p+24, irt, 0x1.e666660000000p+0 * lt));
+    const double kb = 0x1.81757924ed2c0p+26 * fexp2(fma(-0x1.489e160000000p+25, irt, 0x1.383f3e0000000p+1 * lt));
     const double q = kf * C16 * C1 - kb * C5 * C18;
     cd1 -= q;
     cd5 += q;
@@ -861,8 +738,8 @@ struct LaneRhs<40> {
     cd18 += q;
     }
     {  // R81 (elementary)
-    const double kf = 0x1.5ec8000000000p+16 * fexp(fma(0x1.eb851e0000000p+0, lt, -0x1.6b44180000000p+24 * irt));
-    const double kb = 0x1.6c4de3b7054b8p+3 * fexp(fma(0x1.3652be0000000p+1, lt, -0x1.c3c62a0000000p+24 * irt));
+    const double kf = 0x1.a9eaabe2b355ep+33 * fexp2(fma(-0x1.6b44180000000p+24, irt, 0x1.eb851e0000000p+0 * lt));
+    const double kb = 0x1.417bc64dee4edp+25 * fexp2(fma(-0x1.c3c62a0000000p+24, irt, 0x1.3652be0000000p+1 * lt));
     const double q = kf * C16 * C3 - kb * C4 * C18;
     cd3 -= q;
     cd4 += q;
@@ -870,8 +747,8 @@ struct LaneRhs<40> {
     cd18 += q;
     }
     {  // R82 (elementary)
-    const double kf = 0x1.ba80000000000p+11 * fexp(fma(0x1.0f5c280000000p+1, lt, -0x1.bc56000000000p+21 * irt));
-    const double kb = 0x1.f6e8b45731ab8p+2 * fexp(fma(0x1.486c760000000p+1, lt, -0x1.2938bc0000000p+26 * irt));
+    const double kf = 0x1.d3baeb0bee559p+30 * fexp2(fma(-0x1.bc56000000000p+21, irt, 0x1.0f5c280000000p+1 * lt));
+    const double kb = 0x1.0c10d6f4804a7p+26 * fexp2(fma(-0x1.2938bc0000000p+26, irt, 0x1.486c760000000p+1 * lt));
     const double q = kf * C16 * C4 - kb * C6 * C18;
     cd4 -= q;
     cd6 += q;
@@ -879,8 +756,8 @@ struct LaneRhs<40> {
     cd18 += q;
     }
     {  // R83 (elementary)
-    const double kf = 0x1.2a05f20000000p+35 * fexp(fma(0.0, lt, -0x1.96334e0000000p+27 * irt));
-    const double kb = 0x1.91092e876c8b4p+25 * fexp(fma(0x1.6bfa0a0000000p-3, lt, 0x1.d952920000000p+21 * irt));
+    const double kf = 0x1.2a05f20000000p+35 * fexp2(fma(-0x1.96334e0000000p+27, irt, 0.0 * lt));
+    const double kb = 0x1.2fd313e3a5cfep+27 * fexp2(fma(0x1.d952920000000p+21, irt, 0x1.6bfa0a0000000p-3 * lt));
     const double q = kf * C16 * C2 - kb * C7 * C18;
     cd2 -= q;
     cd7 += q;
@@ -888,8 +765,8 @@ struct LaneRhs<40> {
     cd18 += q;
     }
     {  // R84 (elementary)
-    const double kf = 0x1.1861580000000p+28 * fexp(fma(0.0, lt, -0x1.dce7e40000000p+25 * irt));
-    const double kb = 0x1.be2cbdf45a1cbp+25 * fexp(fma(-0x1.b141200000000p-3, lt, -0x1.d87c780000000p+22 * irt));
+    const double kf = 0x1.1861580000000p+28 * fexp2(fma(-0x1.dce7e40000000p+25, irt, 0.0 * lt));
+    const double kb = 0x1.dce40be43f732p+23 * fexp2(fma(-0x1.d87c780000000p+22, irt, -0x1.b141200000000p-3 * lt));
     const double q = kf * C16 * C7 - kb * C8 * C18;
     cd7 -= q;
     cd8 += q;
@@ -897,8 +774,8 @@ struct LaneRhs<40> {
     cd18 += q;
     }
     {  // R85 (elementary)
-    const double kf = 0x1.7fc0000000000p+12 * fexp(fma(0x1.bd70a40000000p+0, lt, -0x1.4d947c0000000p+25 * irt));
-    const double kb = 0x1.c339df474dc76p+8 * fexp(fma(0x1.fd3f7c0000000p+0, lt, -0x1.e261b80000000p+25 * irt));
+    const double kf = 0x1.2f2da9c097388p+28 * fexp2(fma(-0x1.4d947c0000000p+25, irt, 0x1.bd70a40000000p+0 * lt));
+    const double kb = 0x1.a5f54906c0298p+26 * fexp2(fma(-0x1.e261b80000000p+25, irt, 0x1.fd3f7c0000000p+0 * lt));
     const double q = kf * C16 * C12 - kb * C13 * C18;
     cd12 -= q;
     cd13 += q;
@@ -906,8 +783,8 @@ struct LaneRhs<40> {
     cd18 += q;
     }
     {  // R87 (elementary)
-    const double kf = 0x1.dcd6500000000p+30 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.20d38a230a3d7p+28 * fexp(fma(0x1.c949a60000000p-2, lt, -0x1.0cd6060000000p+28 * irt));
+    const double kf = 0x1.dcd6500000000p+30 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.24ae811027c75p+32 * fexp2(fma(-0x1.0cd6060000000p+28, irt, 0x1.c949a60000000p-2 * lt));
     const double q = kf * C18 * C1 - kb * C5 * C21;
     cd1 -= q;
     cd5 += q;
@@ -915,8 +792,8 @@ struct LaneRhs<40> {
     cd21 += q;
     }
     {  // R88 (elementary)
-    const double kf = 0x1.ebbd028000000p+36 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.18997920f5c29p+27 * fexp(fma(0x1.b989380000000p-1, lt, -0x1.3e0ada0000000p+28 * irt));
+    const double kf = 0x1.ebbd028000000p+36 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.dba553645762dp+34 * fexp2(fma(-0x1.3e0ada0000000p+28, irt, 0x1.b989380000000p-1 * lt));
     const double q = kf * C18 * C3 - kb * C14 * C12;
     cd3 -= q;
     cd12 += q;
@@ -924,8 +801,8 @@ struct LaneRhs<40> {
     cd18 -= q;
     }
     {  // R89 (elementary)
-    const double kf = 0x1.312d000000000p+24 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.18f5b5a2d0e56p+24 * fexp(fma(0x1.5b994e0000000p-4, lt, -0x1.980ee20000000p+25 * irt));
+    const double kf = 0x1.312d000000000p+24 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.dd0bf981d990dp+24 * fexp2(fma(-0x1.980ee20000000p+25, irt, 0x1.5b994e0000000p-4 * lt));
     const double q = kf * C18 * C2 - kb * C7 * C21;
     cd2 -= q;
     cd7 += q;
@@ -933,16 +810,16 @@ struct LaneRhs<40> {
     cd21 += q;
     }
     {  // R90 (elementary)
-    const double kf = 0x1.4dc9380000000p+30 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.c8bac6189c000p+39 * fexp(fma(-0x1.7c5a8e0000000p-4, lt, -0x1.01ce280000000p+28 * irt));
+    const double kf = 0x1.4dc9380000000p+30 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.ffceca7e999c2p+38 * fexp2(fma(-0x1.01ce280000000p+28, irt, -0x1.7c5a8e0000000p-4 * lt));
     const double q = kf * C18 * C18 - kb * C16 * C21;
     cd16 += q;
     cd18 = fma(-0x1.0000000000000p+1, q, cd18);
     cd21 += q;
     }
     {  // R91 (elementary)
-    const double kf = 0x1.bf08eb0000000p+36 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.79f08d093f000p+44 * fexp(fma(0x1.56af3a0000000p-5, lt, -0x1.54c1b3e000000p+28 * irt));
+    const double kf = 0x1.bf08eb0000000p+36 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.eaa1b3c686b97p+44 * fexp2(fma(-0x1.54c1b3e000000p+28, irt, 0x1.56af3a0000000p-5 * lt));
     const double q = kf * C18 * C11 - kb * C9 * C16;
     cd9 += q;
     cd11 -= q;
@@ -950,8 +827,8 @@ struct LaneRhs<40> {
     cd18 -= q;
     }
     {  // R92 (elementary)
-    const double kf = 0x1.2ac4ae2000000p+36 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.70afce461dc00p+46 * fexp(fma(-0x1.12ce240000000p-1, lt, -0x1.2ea5ee0000000p+28 * irt));
+    const double kf = 0x1.2ac4ae2000000p+36 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.9ea2084ec80a6p+41 * fexp2(fma(-0x1.2ea5ee0000000p+28, irt, -0x1.12ce240000000p-1 * lt));
     const double q = kf * C18 * C3 - kb * C1 * C22;
     cd1 += q;
     cd3 -= q;
@@ -959,8 +836,8 @@ struct LaneRhs<40> {
     cd22 += q;
     }
     {  // R96 (elementary)
-    const double kf = 0x1.4b40000000000p+10 * fexp(fma(0x1.43d70a0000000p+1, lt, -0x1.86b7700000000p+25 * irt));
-    const double kb = 0x1.20988bdbb7949p-1 * fexp(fma(0x1.81d8d80000000p+1, lt, -0x1.0f58c80000000p+24 * irt));
+    const double kf = 0x1.1a6f6d08e9166p+33 * fexp2(fma(-0x1.86b7700000000p+25, irt, 0x1.43d70a0000000p+1 * lt));
+    const double kb = 0x1.3bc7c1478b392p+26 * fexp2(fma(-0x1.0f58c80000000p+24, irt, 0x1.81d8d80000000p+1 * lt));
     const double q = kf * C21 * C1 - kb * C5 * C24;
     cd1 -= q;
     cd5 += q;
@@ -968,8 +845,8 @@ struct LaneRhs<40> {
     cd24 += q;
     }
     {  // R97 (elementary)
-    const double kf = 0x1.c200000000000p+10 * fexp(fma(0x1.0000000000000p+1, lt, -0x1.3f36c00000000p+23 * irt));
-    const double kb = 0x1.f749ebc6fe7acp+2 * fexp(fma(0x1.3206100000000p+1, lt, -0x1.2f2fcc0000000p+25 * irt));
+    const double kf = 0x1.c200000000000p+28 * fexp2(fma(-0x1.3f36c00000000p+23, irt, 0x1.0000000000000p+1 * lt));
+    const double kb = 0x1.682b6be39e3c1p+24 * fexp2(fma(-0x1.2f2fcc0000000p+25, irt, 0x1.3206100000000p+1 * lt));
     const double q = kf * C21 * C4 - kb * C6 * C24;
     cd4 -= q;
     cd6 += q;
@@ -977,8 +854,8 @@ struct LaneRhs<40> {
     cd24 += q;
     }
     {  // R98 (elementary)
-    const double kf = 0x1.c600000000000p+7 * fexp(fma(0x1.0000000000000p+1, lt, -0x1.25ada40000000p+25 * irt));
-    const double kb = 0x1.06a9eed33a82cp+5 * fexp(fma(0x1.18dd300000000p+1, lt, -0x1.8cc3940000000p+23 * irt));
+    const double kf = 0x1.c600000000000p+25 * fexp2(fma(-0x1.25ada40000000p+25, irt, 0x1.0000000000000p+1 * lt));
+    const double kb = 0x1.b935fbd4d2f85p+24 * fexp2(fma(-0x1.8cc3940000000p+23, irt, 0x1.18dd300000000p+1 * lt));
     const double q = kf * C21 * C12 - kb * C13 * C24;
     cd12 -= q;
     cd13 += q;
@@ -986,8 +863,8 @@ struct LaneRhs<40> {
     cd24 += q;
     }
     {  // R99 (elementary)
-    const double kf = 0x1.2c00000000000p+14 * fexp(fma(0x1.d47ae20000000p+0, lt, -0x1.c138000000000p+19 * irt));
-    const double kb = 0x1.9cde058e9d2ccp-3 * fexp(fma(0x1.5b8a5c0000000p+1, lt, -0x1.98365e0000000p+26 * irt));
+    const double kf = 0x1.9f886f8572949p+30 * fexp2(fma(-0x1.c138000000000p+19, irt, 0x1.d47ae20000000p+0 * lt));
+    const double kb = 0x1.175bbecdf455cp+22 * fexp2(fma(-0x1.98365e0000000p+26, irt, 0x1.5b8a5c0000000p+1 * lt));
     const double q = kf * C21 * C3 - kb * C11 * C12;
     cd3 -= q;
     cd11 += q;
@@ -995,8 +872,8 @@ struct LaneRhs<40> {
     cd21 -= q;
     }
     {  // R100 (elementary)
-    const double kf = 0x1.2a05f20000000p+32 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.983d7432c0000p+35 * fexp(fma(0x1.552af00000000p-4, lt, -0x1.4cd46c0000000p+28 * irt));
+    const double kf = 0x1.2a05f20000000p+32 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.5733763b04ec7p+36 * fexp2(fma(-0x1.4cd46c0000000p+28, irt, 0x1.552af00000000p-4 * lt));
     const double q = kf * C24 * C4 - kb * C6 * C23;
     cd4 -= q;
     cd6 += q;
@@ -1004,8 +881,8 @@ struct LaneRhs<40> {
     cd24 -= q;
     }
     {  // R101 (elementary)
-    const double kf = 0x1.d7e0000000000p+13 * fexp(fma(0x1.e8f5c20000000p+0, lt, -0x1.dd8a000000000p+23 * irt));
-    const double kb = 0x1.e2432de951a5bp+1 * fexp(fma(0x1.2e00d20000000p+1, lt, 0x1.674ce20000000p+24 * irt));
+    const double kf = 0x1.0d261d3514bccp+31 * fexp2(fma(-0x1.dd8a000000000p+23, irt, 0x1.e8f5c20000000p+0 * lt));
+    const double kb = 0x1.1bb5d86546227p+23 * fexp2(fma(0x1.674ce20000000p+24, irt, 0x1.2e00d20000000p+1 * lt));
     const double q = kf * C21 * C3 - kb * C24 * C4;
     cd3 -= q;
     cd4 += q;
@@ -1013,8 +890,8 @@ struct LaneRhs<40> {
     cd24 += q;
     }
     {  // R102 (elementary)
-    const double kf = 0x1.3a0abeb000000p+35 * fexp(fma(0.0, lt, -0x1.cbaace0000000p+27 * irt));
-    const double kb = 0x1.9fdcb4ff5c28fp+26 * fexp(fma(0x1.f6af8a0000000p-4, lt, 0x1.3e02460000000p+24 * irt));
+    const double kf = 0x1.3a0abeb000000p+35 * fexp2(fma(-0x1.cbaace0000000p+27, irt, 0.0 * lt));
+    const double kb = 0x1.bf1cea8c9db36p+27 * fexp2(fma(0x1.3e02460000000p+24, irt, 0x1.f6af8a0000000p-4 * lt));
     const double q = kf * C21 * C2 - kb * C7 * C24;
     cd2 -= q;
     cd7 += q;
@@ -1022,8 +899,8 @@ struct LaneRhs<40> {
     cd24 += q;
     }
     {  // R103 (elementary)
-    const double kf = 0x1.671e344000000p+36 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.7f34b63e60000p+36 * fexp(fma(0x1.6a53760000000p-3, lt, -0x1.1106c60000000p+28 * irt));
+    const double kf = 0x1.671e344000000p+36 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.20dc480edbd02p+38 * fexp2(fma(-0x1.1106c60000000p+28, irt, 0x1.6a53760000000p-3 * lt));
     const double q = kf * C24 * C1 - kb * C5 * C23;
     cd1 -= q;
     cd5 += q;
@@ -1031,8 +908,8 @@ struct LaneRhs<40> {
     cd24 -= q;
     }
     {  // R104 (elementary)
-    const double kf = 0x1.7143400000000p+23 * fexp(fma(0.0, lt, 0x1.3071800000000p+21 * irt));
-    const double kb = 0x1.d79b1e4c08312p+24 * fexp(fma(0x1.10f1b20000000p-2, lt, -0x1.730d9c0000000p+26 * irt));
+    const double kf = 0x1.7143400000000p+23 * fexp2(fma(0x1.3071800000000p+21, irt, 0.0 * lt));
+    const double kb = 0x1.36e963d0eade6p+27 * fexp2(fma(-0x1.730d9c0000000p+26, irt, 0x1.10f1b20000000p-2 * lt));
     const double q = kf * C24 * C8 - kb * C7 * C21;
     cd7 += q;
     cd8 -= q;
@@ -1040,8 +917,8 @@ struct LaneRhs<40> {
     cd24 -= q;
     }
     {  // R105 (elementary)
-    const double kf = 0x1.73eed80000000p+28 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.078ddcb000000p+37 * fexp(fma(-0x1.cfebd00000000p-4, lt, -0x1.1898900000000p+28 * irt));
+    const double kf = 0x1.73eed80000000p+28 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.040a9a5430a76p+36 * fexp2(fma(-0x1.1898900000000p+28, irt, -0x1.cfebd00000000p-4 * lt));
     const double q = kf * C24 * C12 - kb * C13 * C23;
     cd12 -= q;
     cd13 += q;
@@ -1049,16 +926,16 @@ struct LaneRhs<40> {
     cd24 -= q;
     }
     {  // R106 (elementary)
-    const double kf = 0x1.c9c3800000000p+29 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.1854e67cca000p+41 * fexp(fma(-0x1.3ae5bc0000000p-2, lt, -0x1.30e8280000000p+28 * irt));
+    const double kf = 0x1.c9c3800000000p+29 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.49516ce405132p+38 * fexp2(fma(-0x1.30e8280000000p+28, irt, -0x1.3ae5bc0000000p-2 * lt));
     const double q = kf * C24 * C24 - kb * C23 * C21;
     cd21 += q;
     cd23 += q;
     cd24 = fma(-0x1.0000000000000p+1, q, cd24);
     }
     {  // R107 (elementary)
-    const double kf = 0x1.4d3d25d880000p+45 * fexp(fma(-0x1.63d70a0000000p+0, lt, -0x1.0337600000000p+22 * irt));
-    const double kb = 0x1.1e1027309c000p+39 * fexp(fma(-0x1.a5a9440000000p-1, lt, -0x1.65ce040000000p+28 * irt));
+    const double kf = 0x1.d4040197c6493p+32 * fexp2(fma(-0x1.0337600000000p+22, irt, -0x1.63d70a0000000p+0 * lt));
+    const double kb = 0x1.adfebf10e16e4p+31 * fexp2(fma(-0x1.65ce040000000p+28, irt, -0x1.a5a9440000000p-1 * lt));
     const double q = kf * C24 * C2 - kb * C14 * C11;
     cd2 -= q;
     cd11 += q;
@@ -1066,8 +943,8 @@ struct LaneRhs<40> {
     cd24 -= q;
     }
     {  // R108 (elementary)
-    const double kf = 0x1.4e40000000000p+10 * fexp(fma(0x1.9c28f60000000p+0, lt, 0x1.8855800000000p+20 * irt));
-    const double kb = 0x1.0f0f1d4dd3c87p+13 * fexp(fma(0x1.6cda900000000p+0, lt, -0x1.ad523a0000000p+25 * irt));
+    const double kf = 0x1.d56f8cc313341p+24 * fexp2(fma(0x1.8855800000000p+20, irt, 0x1.9c28f60000000p+0 * lt));
+    const double kb = 0x1.e0d1f026960cbp+25 * fexp2(fma(-0x1.ad523a0000000p+25, irt, 0x1.6cda900000000p+0 * lt));
     const double q = kf * C24 * C2 - kb * C23 * C7;
     cd2 -= q;
     cd7 += q;
@@ -1075,8 +952,8 @@ struct LaneRhs<40> {
     cd24 -= q;
     }
     {  // R110 (elementary)
-    const double kf = 0x1.fe00000000000p+11 * fexp(fma(0x1.0000000000000p+1, lt, -0x1.e53ac00000000p+22 * irt));
-    const double kb = 0x1.5cdbdc0c6d652p-7 * fexp(fma(0x1.a877460000000p+1, lt, -0x1.7b5dd20000000p+27 * irt));
+    const double kf = 0x1.fe00000000000p+29 * fexp2(fma(-0x1.e53ac00000000p+22, irt, 0x1.0000000000000p+1 * lt));
+    const double kb = 0x1.3960b4660b263p+23 * fexp2(fma(-0x1.7b5dd20000000p+27, irt, 0x1.a877460000000p+1 * lt));
     const double q = kf * C23 * C3 - kb * C9 * C19;
     cd3 -= q;
     cd9 += q;
@@ -1084,8 +961,8 @@ struct LaneRhs<40> {
     cd23 -= q;
     }
     {  // R111 (elementary)
-    const double kf = 0x1.034f03b80a36dp-21 * fexp(fma(0x1.0000000000000p+2, lt, 0x1.febe000000000p+22 * irt));
-    const double kb = 0x1.e9dc03a70aa09p-31 * fexp(fma(0x1.35c45c0000000p+2, lt, -0x1.a2abd80000000p+27 * irt));
+    const double kf = 0x1.034f03b80a36dp+15 * fexp2(fma(0x1.febe000000000p+22, irt, 0x1.0000000000000p+2 * lt));
+    const double kb = 0x1.6956fe4daff67p+13 * fexp2(fma(-0x1.a2abd80000000p+27, irt, 0x1.35c45c0000000p+2 * lt));
     const double q = kf * C23 * C4 - kb * C9 * C12;
     cd4 -= q;
     cd9 += q;
@@ -1093,8 +970,8 @@ struct LaneRhs<40> {
     cd23 -= q;
     }
     {  // R113 (elementary)
-    const double kf = 0x1.2a05f20000000p+36 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.b994980f09000p+42 * fexp(fma(-0x1.624af00000000p-2, lt, -0x1.6c2d340000000p+28 * irt));
+    const double kf = 0x1.2a05f20000000p+36 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.980eee93d2c8fp+39 * fexp2(fma(-0x1.6c2d340000000p+28, irt, -0x1.624af00000000p-2 * lt));
     const double q = kf * C19 * C3 - kb * C1 * C11;
     cd1 += q;
     cd3 -= q;
@@ -1102,8 +979,8 @@ struct LaneRhs<40> {
     cd19 -= q;
     }
     {  // R114 (elementary)
-    const double kf = 0x1.2a05f20000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.01aeab1e1b880p+51 * fexp(fma(-0x1.8f85300000000p-1, lt, -0x1.3db4ca0000000p+28 * irt));
+    const double kf = 0x1.2a05f20000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.fb47243bc2213p+43 * fexp2(fma(-0x1.3db4ca0000000p+28, irt, -0x1.8f85300000000p-1 * lt));
     const double q = kf * C19 * C4 - kb * C1 * C14;
     cd1 += q;
     cd4 -= q;
@@ -1111,8 +988,8 @@ struct LaneRhs<40> {
     cd19 -= q;
     }
     {  // R115 (elementary)
-    const double kf = 0x1.f400000000000p+8 * fexp(fma(0x1.0000000000000p+1, lt, -0x1.cd94100000000p+24 * irt));
-    const double kb = 0x1.94f492398201dp+17 * fexp(fma(0x1.7d2a840000000p+0, lt, -0x1.d483520000000p+25 * irt));
+    const double kf = 0x1.f400000000000p+26 * fexp2(fma(-0x1.cd94100000000p+24, irt, 0x1.0000000000000p+1 * lt));
+    const double kb = 0x1.0b3d49a3949d5p+31 * fexp2(fma(-0x1.d483520000000p+25, irt, 0x1.7d2a840000000p+0 * lt));
     const double q = kf * C19 * C5 - kb * C12 * C1;
     cd1 += q;
     cd5 -= q;
@@ -1120,8 +997,8 @@ struct LaneRhs<40> {
     cd19 -= q;
     }
     {  // R116 (elementary)
-    const double kf = 0x1.8964020000000p+33 * fexp(fma(0.0, lt, -0x1.7f0e800000000p+22 * irt));
-    const double kb = 0x1.28b6b84d66666p+31 * fexp(fma(0x1.6c6a560000000p-4, lt, -0x1.2ede980000000p+28 * irt));
+    const double kf = 0x1.8964020000000p+33 * fexp2(fma(-0x1.7f0e800000000p+22, irt, 0.0 * lt));
+    const double kb = 0x1.026ecba798ddcp+32 * fexp2(fma(-0x1.2ede980000000p+28, irt, 0x1.6c6a560000000p-4 * lt));
     const double q = kf * C19 * C2 - kb * C4 * C11;
     cd2 -= q;
     cd4 += q;
@@ -1129,8 +1006,8 @@ struct LaneRhs<40> {
     cd19 -= q;
     }
     {  // R117 (elementary)
-    const double kf = 0x1.2a05f20000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.94f1411400000p+38 * fexp(fma(-0x1.3215fc0000000p-6, lt, -0x1.cebe600000000p+28 * irt));
+    const double kf = 0x1.2a05f20000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.68651a1a72c7dp+38 * fexp2(fma(-0x1.cebe600000000p+28, irt, -0x1.3215fc0000000p-6 * lt));
     const double q = kf * C19 * C7 - kb * C4 * C14;
     cd4 += q;
     cd7 -= q;
@@ -1138,37 +1015,37 @@ struct LaneRhs<40> {
     cd19 -= q;
     }
     {  // R118 (elementary)
-    const double kf = 0x1.dcd6500000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.828d1c44d9370p+55 * fexp(fma(-0x1.14b3e60000000p+0, lt, -0x1.0aee640000000p+29 * irt));
+    const double kf = 0x1.dcd6500000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.d2ced8d0b6626p+45 * fexp2(fma(-0x1.0aee640000000p+29, irt, -0x1.14b3e60000000p+0 * lt));
     const double q = kf * C19 * C19 - kb * C5 * C23;
     cd5 += q;
     cd19 = fma(-0x1.0000000000000p+1, q, cd19);
     cd23 += q;
     }
     {  // R120 (elementary)
-    const double kf = 0x1.bf08eb0000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.45ee2d5400000p+34 * fexp(fma(-0x1.fe3fd60000000p-5, lt, -0x1.1c99660000000p+25 * irt));
+    const double kf = 0x1.bf08eb0000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.b9fb5ac9f9a01p+33 * fexp2(fma(-0x1.1c99660000000p+25, irt, -0x1.fe3fd60000000p-5 * lt));
     const double q = kf * C20 * C6 - kb * C6 * C19;
     cd19 += q;
     cd20 -= q;
     }
     {  // R121 (elementary)
-    const double kf = 0x1.0c388d0000000p+33 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.871dcffe4cccdp+32 * fexp(fma(-0x1.fe3fd60000000p-5, lt, -0x1.1c99660000000p+25 * irt));
+    const double kf = 0x1.0c388d0000000p+33 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.093069ac5137bp+32 * fexp2(fma(-0x1.1c99660000000p+25, irt, -0x1.fe3fd60000000p-5 * lt));
     const double q = kf * C20 * C9 - kb * C9 * C19;
     cd19 += q;
     cd20 -= q;
     }
     {  // R122 (elementary)
-    const double kf = 0x1.a13b860000000p+32 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.3033a1c5ccccdp+32 * fexp(fma(-0x1.fe3fd60000000p-5, lt, -0x1.1c99660000000p+25 * irt));
+    const double kf = 0x1.a13b860000000p+32 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.9c84329a494e9p+31 * fexp2(fma(-0x1.1c99660000000p+25, irt, -0x1.fe3fd60000000p-5 * lt));
     const double q = kf * C20 * C10 - kb * C10 * C19;
     cd19 += q;
     cd20 -= q;
     }
     {  // R123 (elementary)
-    const double kf = 0x1.bf08eb0000000p+33 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.69781f0340000p+35 * fexp(fma(0x1.62467c0000000p-3, lt, -0x1.77c4f96800000p+29 * irt));
+    const double kf = 0x1.bf08eb0000000p+33 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.09dff03d0cdadp+37 * fexp2(fma(-0x1.77c4f96800000p+29, irt, 0x1.62467c0000000p-3 * lt));
     const double q = kf * C20 * C3 - kb * C5 * C9;
     cd3 -= q;
     cd5 += q;
@@ -1176,8 +1053,8 @@ struct LaneRhs<40> {
     cd20 -= q;
     }
     {  // R124 (elementary)
-    const double kf = 0x1.bf08eb0000000p+33 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.e2ee3048a0000p+39 * fexp(fma(-0x1.a212d80000000p-2, lt, -0x1.8fc0620000000p+28 * irt));
+    const double kf = 0x1.bf08eb0000000p+33 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.2e95bff44b0d0p+36 * fexp2(fma(-0x1.8fc0620000000p+28, irt, -0x1.a212d80000000p-2 * lt));
     const double q = kf * C20 * C3 - kb * C1 * C11;
     cd1 += q;
     cd3 -= q;
@@ -1185,8 +1062,8 @@ struct LaneRhs<40> {
     cd20 -= q;
     }
     {  // R125 (elementary)
-    const double kf = 0x1.bf08eb0000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.19cfd84dfce80p+51 * fexp(fma(-0x1.af69220000000p-1, lt, -0x1.6147f60000000p+28 * irt));
+    const double kf = 0x1.bf08eb0000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.7828a53cbe3afp+43 * fexp2(fma(-0x1.6147f60000000p+28, irt, -0x1.af69220000000p-1 * lt));
     const double q = kf * C20 * C4 - kb * C1 * C14;
     cd1 += q;
     cd4 -= q;
@@ -1194,8 +1071,8 @@ struct LaneRhs<40> {
     cd20 -= q;
     }
     {  // R126 (elementary)
-    const double kf = 0x1.04c533c000000p+36 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.33f862bae4800p+44 * fexp(fma(-0x1.258ea80000000p-1, lt, -0x1.0529580000000p+26 * irt));
+    const double kf = 0x1.04c533c000000p+36 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.139b05b4fbad8p+39 * fexp2(fma(-0x1.0529580000000p+26, irt, -0x1.258ea80000000p-1 * lt));
     const double q = kf * C20 * C5 - kb * C1 * C12;
     cd1 += q;
     cd5 -= q;
@@ -1203,8 +1080,8 @@ struct LaneRhs<40> {
     cd20 -= q;
     }
     {  // R127 (elementary)
-    const double kf = 0x1.a13b860000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.78e7377ef9db2p+19 * fexp(fma(0x1.095d0c0000000p-2, lt, -0x1.0f3c4e0000000p+28 * irt));
+    const double kf = 0x1.a13b860000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.da86e767220aep+21 * fexp2(fma(-0x1.0f3c4e0000000p+28, irt, 0x1.095d0c0000000p-2 * lt));
     const double q = kf * C20 * C2 - kb * C9 * C4 * C1;
     cd1 += q;
     cd2 -= q;
@@ -1213,8 +1090,8 @@ struct LaneRhs<40> {
     cd20 -= q;
     }
     {  // R128 (elementary)
-    const double kf = 0x1.65a0bc0000000p+33 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.79ef0a9347ae1p+29 * fexp(fma(0x1.0754f40000000p-1, lt, -0x1.7406600000000p+29 * irt));
+    const double kf = 0x1.65a0bc0000000p+33 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.24362c5d6af29p+34 * fexp2(fma(-0x1.7406600000000p+29, irt, 0x1.0754f40000000p-1 * lt));
     const double q = kf * C20 * C2 - kb * C6 * C9;
     cd2 -= q;
     cd6 += q;
@@ -1222,8 +1099,8 @@ struct LaneRhs<40> {
     cd20 -= q;
     }
     {  // R129 (elementary)
-    const double kf = 0x1.a13b860000000p+33 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.8aa2af0b851ecp+27 * fexp(fma(0x1.bf138c0000000p-2, lt, -0x1.f594762000000p+27 * irt));
+    const double kf = 0x1.a13b860000000p+33 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.77c8a44732fabp+31 * fexp2(fma(-0x1.f594762000000p+27, irt, 0x1.bf138c0000000p-2 * lt));
     const double q = kf * C20 * C10 - kb * C9 * C14;
     cd9 += q;
     cd10 -= q;
@@ -1231,24 +1108,24 @@ struct LaneRhs<40> {
     cd20 -= q;
     }
     {  // R130 (elementary)
-    const double kf = 0x1.8de76816d8000p+52 * fexp(fma(0.0, lt, -0x1.45e4b60000000p+28 * irt));
-    const double kb = 0x1.26f34953bd167p+15 * fexp(fma(0x1.8508700000000p+0, lt, 0x1.3c10320000000p+24 * irt));
+    const double kf = 0x1.8de76816d8000p+52 * fexp2(fma(-0x1.45e4b60000000p+28, irt, 0.0 * lt));
+    const double kb = 0x1.d78ce80d37de8p+28 * fexp2(fma(0x1.3c10320000000p+24, irt, 0x1.8508700000000p+0 * lt));
     const double q = kf * C22 - kb * C11 * C12;
     cd11 += q;
     cd12 += q;
     cd22 -= q;
     }
     {  // R131 (elementary)
-    const double kf = 0x1.380e9898d27fcp+140 * fexp(fma(-0x1.fd0e560000000p+2, lt, -0x1.6e530d8000000p+28 * irt));
-    const double kb = 0x1.15017ee7a3a97p+104 * fexp(fma(-0x1.9e62cc0000000p+2, lt, -0x1.f917440000000p+24 * irt));
+    const double kf = 0x1.9fc6e45b143b6p+68 * fexp2(fma(-0x1.6e530d8000000p+28, irt, -0x1.fd0e560000000p+2 * lt));
+    const double kb = 0x1.ca7de0fb7a400p+45 * fexp2(fma(-0x1.f917440000000p+24, irt, -0x1.9e62cc0000000p+2 * lt));
     const double q = kf * C25 - kb * C15 * C12;
     cd12 += q;
     cd15 += q;
     cd25 -= q;
     }
     {  // R132 (elementary)
-    const double kf = 0x1.a360000000000p+12 * fexp(fma(0x1.0000000000000p+1, lt, 0x1.41a7c00000000p+21 * irt));
-    const double kb = 0x1.013f316c89961p+8 * fexp(fma(0x1.0d4de80000000p+1, lt, -0x1.4addfa0000000p+26 * irt));
+    const double kf = 0x1.a360000000000p+30 * fexp2(fma(0x1.41a7c00000000p+21, irt, 0x1.0000000000000p+1 * lt));
+    const double kb = 0x1.ebfc162f6e990p+26 * fexp2(fma(-0x1.4addfa0000000p+26, irt, 0x1.0d4de80000000p+1 * lt));
     const double q = kf * C25 * C4 - kb * C6 * C26;
     cd4 -= q;
     cd6 += q;
@@ -1256,8 +1133,8 @@ struct LaneRhs<40> {
     cd26 += q;
     }
     {  // R133 (elementary)
-    const double kf = 0x1.d010000000000p+14 * fexp(fma(0x1.0000000000000p+1, lt, -0x1.0185c80000000p+24 * irt));
-    const double kb = 0x1.bb7d5c6459f1cp+6 * fexp(fma(0x1.1949fa0000000p+1, lt, -0x1.4c2c2c0000000p+25 * irt));
+    const double kf = 0x1.d010000000000p+32 * fexp2(fma(-0x1.0185c80000000p+24, irt, 0x1.0000000000000p+1 * lt));
+    const double kb = 0x1.7c459b4bf6844p+26 * fexp2(fma(-0x1.4c2c2c0000000p+25, irt, 0x1.1949fa0000000p+1 * lt));
     const double q = kf * C25 * C1 - kb * C5 * C26;
     cd1 -= q;
     cd5 += q;
@@ -1265,8 +1142,8 @@ struct LaneRhs<40> {
     cd26 += q;
     }
     {  // R134 (elementary)
-    const double kf = 0x1.b71758e219653p-6 * fexp(fma(0x1.e395820000000p+1, lt, -0x1.3371140000000p+25 * irt));
-    const double kb = 0x1.16a883590c366p-5 * fexp(fma(0x1.d7badc0000000p+1, lt, -0x1.1db4540000000p+26 * irt));
+    const double kf = 0x1.b7b35ddbc92e0p+28 * fexp2(fma(-0x1.3371140000000p+25, irt, 0x1.e395820000000p+1 * lt));
+    const double kb = 0x1.392ee68997766p+28 * fexp2(fma(-0x1.1db4540000000p+26, irt, 0x1.d7badc0000000p+1 * lt));
     const double q = kf * C25 * C12 - kb * C13 * C26;
     cd12 -= q;
     cd13 += q;
@@ -1274,8 +1151,8 @@ struct LaneRhs<40> {
     cd26 += q;
     }
     {  // R135 (elementary)
-    const double kf = 0x1.f1f2a11cc5b38p-20 * fexp(fma(0x1.528f5c0000000p+2, lt, 0x1.bd50000000000p+18 * irt));
-    const double kb = 0x1.171d6b90897ffp-28 * fexp(fma(0x1.5cf6400000000p+2, lt, -0x1.37e1860000000p+24 * irt));
+    const double kf = 0x1.7bffa3ec3f136p+28 * fexp2(fma(0x1.bd50000000000p+18, irt, 0x1.528f5c0000000p+2 * lt));
+    const double kb = 0x1.258df464ac294p+21 * fexp2(fma(-0x1.37e1860000000p+24, irt, 0x1.5cf6400000000p+2 * lt));
     const double q = kf * C25 * C3 - kb * C4 * C26;
     cd3 -= q;
     cd4 += q;
@@ -1283,8 +1160,8 @@ struct LaneRhs<40> {
     cd26 += q;
     }
     {  // R136 (elementary)
-    const double kf = 0x1.2a05f20000000p+34 * fexp(fma(0.0, lt, -0x1.0759f80000000p+26 * irt));
-    const double kb = 0x1.ffeda13cc0000p+35 * fexp(fma(-0x1.1b58d20000000p-1, lt, -0x1.c00bea0000000p+24 * irt));
+    const double kf = 0x1.2a05f20000000p+34 * fexp2(fma(-0x1.0759f80000000p+26, irt, 0.0 * lt));
+    const double kb = 0x1.0368edc134b70p+31 * fexp2(fma(-0x1.c00bea0000000p+24, irt, -0x1.1b58d20000000p-1 * lt));
     const double q = kf * C25 * C7 - kb * C8 * C26;
     cd7 -= q;
     cd8 += q;
@@ -1292,8 +1169,8 @@ struct LaneRhs<40> {
     cd26 += q;
     }
     {  // R137 (elementary)
-    const double kf = 0x1.31794b4000000p+35 * fexp(fma(0.0, lt, -0x1.6665830000000p+27 * irt));
-    const double kb = 0x1.bbb82de48f5c3p+29 * fexp(fma(-0x1.5028a20000000p-3, lt, 0x1.a687ec0000000p+23 * irt));
+    const double kf = 0x1.31794b4000000p+35 * fexp2(fma(-0x1.6665830000000p+27, irt, 0.0 * lt));
+    const double kb = 0x1.3ebde036ba18ep+28 * fexp2(fma(0x1.a687ec0000000p+23, irt, -0x1.5028a20000000p-3 * lt));
     const double q = kf * C25 * C2 - kb * C7 * C26;
     cd2 -= q;
     cd7 += q;
@@ -1301,16 +1178,16 @@ struct LaneRhs<40> {
     cd26 += q;
     }
     {  // R138 (elementary)
-    const double kf = 0x1.5d3ef79800000p+43 * fexp(fma(0.0, lt, -0x1.9afce40000000p+26 * irt));
-    const double kb = 0x1.fb8caea94b3d7p+6 * fexp(fma(0x1.ee703a0000000p+0, lt, -0x1.2342b00000000p+26 * irt));
+    const double kf = 0x1.5d3ef79800000p+43 * fexp2(fma(-0x1.9afce40000000p+26, irt, 0.0 * lt));
+    const double kb = 0x1.4ad7e3564b229p+24 * fexp2(fma(-0x1.2342b00000000p+26, irt, 0x1.ee703a0000000p+0 * lt));
     const double q = kf * C26 - kb * C12 * C14;
     cd12 += q;
     cd14 += q;
     cd26 -= q;
     }
     {  // R139 (elementary)
-    const double kf = 0x1.671e344000000p+34 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.25f7a9ca00000p+34 * fexp(fma(0x1.cf0a1c0000000p-2, lt, -0x1.30d30c0000000p+28 * irt));
+    const double kf = 0x1.671e344000000p+34 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.3483c52765fa8p+38 * fexp2(fma(-0x1.30d30c0000000p+28, irt, 0x1.cf0a1c0000000p-2 * lt));
     const double q = kf * C26 * C15 - kb * C14 * C25;
     cd14 += q;
     cd15 -= q;
@@ -1318,8 +1195,8 @@ struct LaneRhs<40> {
     cd26 -= q;
     }
     {  // R140 (elementary)
-    const double kf = 0x1.5f5c28f5c28f6p+2 * fexp(fma(0x1.6666660000000p+1, lt, -0x1.7640980000000p+24 * irt));
-    const double kb = 0x1.0c8bb75f018c3p+1 * fexp(fma(0x1.89306a0000000p+1, lt, -0x1.8f783c0000000p+25 * irt));
+    const double kf = 0x1.939b45cf211e8p+27 * fexp2(fma(-0x1.7640980000000p+24, irt, 0x1.6666660000000p+1 * lt));
+    const double kb = 0x1.a4423c53bda36p+28 * fexp2(fma(-0x1.8f783c0000000p+25, irt, 0x1.89306a0000000p+1 * lt));
     const double q = kf * C26 * C14 - kb * C11 * C25;
     cd11 += q;
     cd14 -= q;
@@ -1327,8 +1204,8 @@ struct LaneRhs<40> {
     cd26 -= q;
     }
     {  // R141 (elementary)
-    const double kf = 0x1.0c388d0000000p+33 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.cc4d8defd0000p+38 * fexp(fma(-0x1.24f26a0000000p-2, lt, -0x1.da919a0000000p+26 * irt));
+    const double kf = 0x1.0c388d0000000p+33 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.350d98e5b3c9bp+36 * fexp2(fma(-0x1.da919a0000000p+26, irt, -0x1.24f26a0000000p-2 * lt));
     const double q = kf * C26 * C7 - kb * C4 * C27;
     cd4 += q;
     cd7 -= q;
@@ -1336,16 +1213,16 @@ struct LaneRhs<40> {
     cd27 += q;
     }
     {  // R142 (elementary)
-    const double kf = 0x1.eff575daa5000p+53 * fexp(fma(-0x1.51eb860000000p-1, lt, -0x1.761d700000000p+25 * irt));
-    const double kb = 0x1.f44e3400e6000p+41 * fexp(fma(-0x1.7452c60000000p-1, lt, -0x1.3462fa8000000p+25 * irt));
+    const double kf = 0x1.02828fd1bbba1p+48 * fexp2(fma(-0x1.761d700000000p+25, irt, -0x1.51eb860000000p-1 * lt));
+    const double kb = 0x1.56f7264ee812dp+35 * fexp2(fma(-0x1.3462fa8000000p+25, irt, -0x1.7452c60000000p-1 * lt));
     const double q = kf * C27 - kb * C1 * C28;
     cd1 += q;
     cd27 -= q;
     cd28 += q;
     }
     {  // R143 (elementary)
-    const double kf = 0x1.2a05f20000000p+33 * fexp(fma(0.0, lt, -0x1.8c9fa50000000p+27 * irt));
-    const double kb = 0x1.955c9270a3d71p+24 * fexp(fma(-0x1.1fde940000000p+0, lt, -0x1.92f4380000000p+21 * irt));
+    const double kf = 0x1.2a05f20000000p+33 * fexp2(fma(-0x1.8c9fa50000000p+27, irt, 0.0 * lt));
+    const double kb = 0x1.74e7179b5a0e6p+14 * fexp2(fma(-0x1.92f4380000000p+21, irt, -0x1.1fde940000000p+0 * lt));
     const double q = kf * C28 * C2 - kb * C7 * C29;
     cd2 -= q;
     cd7 += q;
@@ -1353,8 +1230,8 @@ struct LaneRhs<40> {
     cd29 += q;
     }
     {  // R144 (elementary)
-    const double kf = 0x1.6da0000000000p+14 * fexp(fma(0x1.9c28f60000000p+0, lt, 0x1.1d28000000000p+17 * irt));
-    const double kb = 0x1.a4057a7b1b544p+6 * fexp(fma(0x1.81d7120000000p-1, lt, -0x1.4951000000000p+26 * irt));
+    const double kf = 0x1.00c006ab3837ap+29 * fexp2(fma(0x1.1d28000000000p+17, irt, 0x1.9c28f60000000p+0 * lt));
+    const double kb = 0x1.6933e3fa46b11p+13 * fexp2(fma(-0x1.4951000000000p+26, irt, 0x1.81d7120000000p-1 * lt));
     const double q = kf * C28 * C4 - kb * C6 * C29;
     cd4 -= q;
     cd6 += q;
@@ -1362,8 +1239,8 @@ struct LaneRhs<40> {
     cd29 += q;
     }
     {  // R145 (elementary)
-    const double kf = 0x1.22dee40000000p+30 * fexp(fma(0.0, lt, -0x1.0f54f00000000p+26 * irt));
-    const double kb = 0x1.d3dc6fe828f5cp+28 * fexp(fma(-0x1.8385c60000000p+0, lt, -0x1.b3c9380000000p+24 * irt));
+    const double kf = 0x1.22dee40000000p+30 * fexp2(fma(-0x1.0f54f00000000p+26, irt, 0.0 * lt));
+    const double kb = 0x1.2f9d4d1b437c5p+15 * fexp2(fma(-0x1.b3c9380000000p+24, irt, -0x1.8385c60000000p+0 * lt));
     const double q = kf * C28 * C7 - kb * C8 * C29;
     cd7 -= q;
     cd8 += q;
@@ -1371,8 +1248,8 @@ struct LaneRhs<40> {
     cd29 += q;
     }
     {  // R146 (elementary)
-    const double kf = 0x1.d600000000000p+7 * fexp(fma(0x1.4000000000000p+1, lt, -0x1.1cbaa00000000p+23 * irt));
-    const double kb = 0x1.ed625310d447fp-5 * fexp(fma(0x1.b3c2120000000p+0, lt, -0x1.a105840000000p+24 * irt));
+    const double kf = 0x1.4c5716816cbe5p+30 * fexp2(fma(-0x1.1cbaa00000000p+23, irt, 0x1.4000000000000p+1 * lt));
+    const double kb = 0x1.33df45e858c90p+11 * fexp2(fma(-0x1.a105840000000p+24, irt, 0x1.b3c2120000000p+0 * lt));
     const double q = kf * C28 * C3 - kb * C4 * C29;
     cd3 -= q;
     cd4 += q;
@@ -1380,8 +1257,8 @@ struct LaneRhs<40> {
     cd29 += q;
     }
     {  // R147 (elementary)
-    const double kf = 0x1.1c60000000000p+12 * fexp(fma(0x1.0000000000000p+1, lt, -0x1.3f36c00000000p+24 * irt));
-    const double kb = 0x1.fcf69ba3f11cap+0 * fexp(fma(0x1.3cba740000000p+0, lt, -0x1.54ed5e0000000p+25 * irt));
+    const double kf = 0x1.1c60000000000p+30 * fexp2(fma(-0x1.3f36c00000000p+24, irt, 0x1.0000000000000p+1 * lt));
+    const double kb = 0x1.1770d102ec0f2p+12 * fexp2(fma(-0x1.54ed5e0000000p+25, irt, 0x1.3cba740000000p+0 * lt));
     const double q = kf * C28 * C1 - kb * C5 * C29;
     cd1 -= q;
     cd5 += q;
@@ -1389,8 +1266,8 @@ struct LaneRhs<40> {
     cd29 += q;
     }
     {  // R148 (elementary)
-    const double kf = 0x1.8bd66277c45ccp-11 * fexp(fma(0x1.bae1480000000p+1, lt, -0x1.5dee080000000p+24 * irt));
-    const double kb = 0x1.d67594b427f63p-14 * fexp(fma(0x1.3419e40000000p+1, lt, -0x1.a0d7500000000p+25 * irt));
+    const double kf = 0x1.b42ce7469eaecp+20 * fexp2(fma(-0x1.5dee080000000p+24, irt, 0x1.bae1480000000p+1 * lt));
+    const double kb = 0x1.748c98d676003p+8 * fexp2(fma(-0x1.a0d7500000000p+25, irt, 0x1.3419e40000000p+1 * lt));
     const double q = kf * C28 * C12 - kb * C13 * C29;
     cd12 -= q;
     cd13 += q;
@@ -1398,40 +1275,40 @@ struct LaneRhs<40> {
     cd29 += q;
     }
     {  // R149 (elementary)
-    const double kf = 0x1.b1b48d5380000p+42 * fexp(fma(-0x1.c28f5c0000000p+0, lt, -0x1.11ba380000000p+26 * irt));
-    const double kb = 0x1.05b8dc0365540p+6 * fexp(fma(0x1.d4f80e0000000p+0, lt, 0x1.11696a0000000p+20 * irt));
+    const double kf = 0x1.e492c7d227120p+26 * fexp2(fma(-0x1.11ba380000000p+26, irt, -0x1.c28f5c0000000p+0 * lt));
+    const double kb = 0x1.6edbeb6b93dcep+22 * fexp2(fma(0x1.11696a0000000p+20, irt, 0x1.d4f80e0000000p+0 * lt));
     const double q = kf * C29 - kb * C9 * C15;
     cd9 += q;
     cd15 += q;
     cd29 -= q;
     }
     {  // R150 (elementary)
-    const double kf = 0x1.60816ea400000p+40 * fexp(fma(-0x1.c7ae140000000p+0, lt, -0x1.b9278c0000000p+25 * irt));
-    const double kb = 0x1.9f91bd6896417p+9 * fexp(fma(0x1.73a3ec0000000p+0, lt, -0x1.04ca940000000p+27 * irt));
+    const double kf = 0x1.5ba7114eed5bbp+24 * fexp2(fma(-0x1.b9278c0000000p+25, irt, -0x1.c7ae140000000p+0 * lt));
+    const double kb = 0x1.b2dd8d87c863dp+22 * fexp2(fma(-0x1.04ca940000000p+27, irt, 0x1.73a3ec0000000p+0 * lt));
     const double q = kf * C29 - kb * C10 * C12;
     cd10 += q;
     cd12 += q;
     cd29 -= q;
     }
     {  // R151 (elementary)
-    const double kf = 0x1.dcd6500000000p+30 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.0e466d6177d52p+66 * fexp(fma(-0x1.a9283a0000000p+0, lt, -0x1.22a2c60000000p+27 * irt));
+    const double kf = 0x1.dcd6500000000p+30 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.1866fc3a12029p+51 * fexp2(fma(-0x1.22a2c60000000p+27, irt, -0x1.a9283a0000000p+0 * lt));
     const double q = kf * C26 * C2 - kb * C30;
     cd2 -= q;
     cd26 -= q;
     cd30 += q;
     }
     {  // R152 (elementary)
-    const double kf = 0x1.15090bfbf0bc4p+67 * fexp(fma(-0x1.2000000000000p+2, lt, 0.0 * irt));
-    const double kb = 0x1.17ce407833333p+31 * fexp(fma(-0x1.43381e0000000p+1, lt, 0x1.9a759c0000000p+21 * irt));
+    const double kf = 0x1.87c9819a4d71cp+26 * fexp2(fma(0.0, irt, -0x1.2000000000000p+2 * lt));
+    const double kb = 0x1.523f15473e53cp+8 * fexp2(fma(0x1.9a759c0000000p+21, irt, -0x1.43381e0000000p+1 * lt));
     const double q = kf * C30 * C30 - kb * C27 * C27 * C2;
     cd2 += q;
     cd27 = fma(0x1.0000000000000p+1, q, cd27);
     cd30 = fma(-0x1.0000000000000p+1, q, cd30);
     }
     {  // R153 (elementary)
-    const double kf = 0x1.dae5dcb1d5de0p+65 * fexp(fma(-0x1.2000000000000p+2, lt, 0.0 * irt));
-    const double kb = 0x1.1fda73f200000p+30 * fexp(fma(-0x1.3af05a0000000p+1, lt, -0x1.92e8980000000p+28 * irt));
+    const double kf = 0x1.4fcdb3c9cacb3p+25 * fexp2(fma(0.0, irt, -0x1.2000000000000p+2 * lt));
+    const double kb = 0x1.047be2f73b300p+8 * fexp2(fma(-0x1.92e8980000000p+28, irt, -0x1.3af05a0000000p+1 * lt));
     const double q = kf * C30 * C30 - kb * C31 * C28 * C2;
     cd2 += q;
     cd28 += q;
@@ -1439,16 +1316,16 @@ struct LaneRhs<40> {
     cd31 += q;
     }
     {  // R154 (elementary)
-    const double kf = 0x1.1450dc240d000p+53 * fexp(fma(-0x1.19999a0000000p+0, lt, -0x1.496dfc0000000p+26 * irt));
-    const double kb = 0x1.f5cf25d8d79d1p+14 * fexp(fma(0x1.eb94740000000p-1, lt, -0x1.247c6a0000000p+25 * irt));
+    const double kf = 0x1.2825e0c59431fp+43 * fexp2(fma(-0x1.496dfc0000000p+26, irt, -0x1.19999a0000000p+0 * lt));
+    const double kb = 0x1.874701db84cdap+23 * fexp2(fma(-0x1.247c6a0000000p+25, irt, 0x1.eb94740000000p-1 * lt));
     const double q = kf * C27 - kb * C14 * C15;
     cd14 += q;
     cd15 += q;
     cd27 -= q;
     }
     {  // R155 (elementary)
-    const double kf = 0x1.7d78400000000p+25 * fexp(fma(0.0, lt, -0x1.febe000000000p+20 * irt));
-    const double kb = 0x1.0a81e7fc28f5cp+24 * fexp(fma(-0x1.4818ee0000000p-4, lt, -0x1.79ec260000000p+27 * irt));
+    const double kf = 0x1.7d78400000000p+25 * fexp2(fma(-0x1.febe000000000p+20, irt, 0.0 * lt));
+    const double kb = 0x1.4362e73a83e37p+23 * fexp2(fma(-0x1.79ec260000000p+27, irt, -0x1.4818ee0000000p-4 * lt));
     const double q = kf * C27 * C2 - kb * C7 * C28;
     cd2 -= q;
     cd7 += q;
@@ -1456,94 +1333,94 @@ struct LaneRhs<40> {
     cd28 += q;
     }
     {  // R156 (elementary)
-    const double kf = 0x1.bf08eb0000000p+35 * fexp(fma(0.0, lt, -0x1.5727a80000000p+26 * irt));
-    const double kb = 0x1.3def7c4aec000p+41 * fexp(fma(-0x1.c0f51a0000000p-1, lt, -0x1.60a8980000000p+25 * irt));
+    const double kf = 0x1.bf08eb0000000p+35 * fexp2(fma(-0x1.5727a80000000p+26, irt, 0.0 * lt));
+    const double kb = 0x1.56b0a6c312725p+33 * fexp2(fma(-0x1.60a8980000000p+25, irt, -0x1.c0f51a0000000p-1 * lt));
     const double q = kf * C30 - kb * C32;
     cd30 -= q;
     cd32 += q;
     }
     {  // R157 (elementary)
-    const double kf = 0x1.b48eb57e00000p+43 * fexp(fma(0.0, lt, -0x1.4731b80000000p+26 * irt));
-    const double kb = 0x1.f5a5a84484cd2p-36 * fexp(fma(0x1.2661fa0000000p+2, lt, -0x1.46e8c60000000p+27 * irt));
+    const double kf = 0x1.b48eb57e00000p+43 * fexp2(fma(-0x1.4731b80000000p+26, irt, 0.0 * lt));
+    const double kb = 0x1.4a681d7588904p+6 * fexp2(fma(-0x1.46e8c60000000p+27, irt, 0x1.2661fa0000000p+2 * lt));
     const double q = kf * C32 - kb * C14 * C14 * C4;
     cd4 += q;
     cd14 = fma(0x1.0000000000000p+1, q, cd14);
     cd32 -= q;
     }
     {  // R158 (elementary)
-    const double kf = 0x1.4dc9380000000p+29 * fexp(fma(0.0, lt, 0.0 * irt));
-    const double kb = 0x1.ab9df4286ccc5p+64 * fexp(fma(-0x1.ad5ef20000000p+0, lt, -0x1.22d2680000000p+27 * irt));
+    const double kf = 0x1.4dc9380000000p+29 * fexp2(fma(0.0, irt, 0.0 * lt));
+    const double kb = 0x1.9058b4d65853ap+49 * fexp2(fma(-0x1.22d2680000000p+27, irt, -0x1.ad5ef20000000p+0 * lt));
     const double q = kf * C32 * C2 - kb * C33;
     cd2 -= q;
     cd32 -= q;
     cd33 += q;
     }
     {  // R159 (elementary)
-    const double kf = 0x1.2a05f20000000p+35 * fexp(fma(0.0, lt, -0x1.2745d80000000p+26 * irt));
-    const double kb = 0x1.b4dcd83eef1edp+1 * fexp(fma(0x1.74a7720000000p+0, lt, -0x1.d9de240000000p+27 * irt));
+    const double kf = 0x1.2a05f20000000p+35 * fexp2(fma(-0x1.2745d80000000p+26, irt, 0.0 * lt));
+    const double kb = 0x1.d494dc740c1e3p+14 * fexp2(fma(-0x1.d9de240000000p+27, irt, 0x1.74a7720000000p+0 * lt));
     const double q = kf * C33 - kb * C4 * C34;
     cd4 += q;
     cd33 -= q;
     cd34 += q;
     }
     {  // R160 (elementary)
-    const double kf = 0x1.aa535d3d0c000p+54 * fexp(fma(0.0, lt, -0x1.3f36c00000000p+27 * irt));
-    const double kb = 0x1.324b2f021d10bp+16 * fexp(fma(0x1.04b19a0000000p+1, lt, 0x1.293b740000000p+24 * irt));
+    const double kf = 0x1.aa535d3d0c000p+54 * fexp2(fma(-0x1.3f36c00000000p+27, irt, 0.0 * lt));
+    const double kb = 0x1.8105effa3e629p+34 * fexp2(fma(0x1.293b740000000p+24, irt, 0x1.04b19a0000000p+1 * lt));
     const double q = kf * C34 - kb * C4 * C35;
     cd4 += q;
     cd34 -= q;
     cd35 += q;
     }
     {  // R161 (elementary)
-    const double kf = 0x1.74876e8000000p+36 * fexp(fma(0.0, lt, -0x1.bee6400000000p+25 * irt));
-    const double kb = 0x1.041739c6ccccdp+30 * fexp(fma(0x1.0f4d160000000p-1, lt, -0x1.47d74a0000000p+26 * irt));
+    const double kf = 0x1.74876e8000000p+36 * fexp2(fma(-0x1.bee6400000000p+25, irt, 0.0 * lt));
+    const double kb = 0x1.bb34ee854b826p+34 * fexp2(fma(-0x1.47d74a0000000p+26, irt, 0x1.0f4d160000000p-1 * lt));
     const double q = kf * C35 - kb * C36;
     cd35 -= q;
     cd36 += q;
     }
     {  // R162 (elementary)
-    const double kf = 0x1.355ecc730a800p+54 * fexp(fma(-0x1.5851ec0000000p+1, lt, -0x1.1286520000000p+26 * irt));
-    const double kb = 0x1.d00f25cf0307fp+16 * fexp(fma(-0x1.205fd00000000p-1, lt, -0x1.a7f07a0000000p+23 * irt));
+    const double kf = 0x1.0b76492056611p+30 * fexp2(fma(-0x1.1286520000000p+26, irt, -0x1.5851ec0000000p+1 * lt));
+    const double kb = 0x1.ba5cdc066ecd3p+11 * fexp2(fma(-0x1.a7f07a0000000p+23, irt, -0x1.205fd00000000p-1 * lt));
     const double q = kf * C36 - kb * C9 * C37;
     cd9 += q;
     cd36 -= q;
     cd37 += q;
     }
     {  // R163 (elementary)
-    const double kf = 0x1.2de538c66f000p+52 * fexp(fma(-0x1.4e147a0000000p+1, lt, -0x1.4c24520000000p+26 * irt));
-    const double kb = 0x1.0a21b2f06f694p+20 * fexp(fma(-0x1.b464dc0000000p-1, lt, -0x1.1ae59e0000000p+27 * irt));
+    const double kf = 0x1.adea1b726767cp+28 * fexp2(fma(-0x1.4c24520000000p+26, irt, -0x1.4e147a0000000p+1 * lt));
+    const double kb = 0x1.4e4d50f92b6dcp+12 * fexp2(fma(-0x1.1ae59e0000000p+27, irt, -0x1.b464dc0000000p-1 * lt));
     const double q = kf * C36 - kb * C10 * C17;
     cd10 += q;
     cd17 += q;
     cd36 -= q;
     }
     {  // R164 (elementary)
-    const double kf = 0x1.6bcc41e900000p+46 * fexp(fma(0.0, lt, -0x1.dba1b80000000p+25 * irt));
-    const double kb = 0x1.0958bb6d60000p+37 * fexp(fma(-0x1.a536500000000p-4, lt, -0x1.3b8d4c0000000p+25 * irt));
+    const double kf = 0x1.6bcc41e900000p+46 * fexp2(fma(-0x1.dba1b80000000p+25, irt, 0.0 * lt));
+    const double kb = 0x1.1767f120d29dfp+36 * fexp2(fma(-0x1.3b8d4c0000000p+25, irt, -0x1.a536500000000p-4 * lt));
     const double q = kf * C37 - kb * C1 * C38;
     cd1 += q;
     cd37 -= q;
     cd38 += q;
     }
     {  // R165 (elementary)
-    const double kf = 0x1.05ef39b200000p+42 * fexp(fma(-0x1.1c28f60000000p+0, lt, 0.0 * irt));
-    const double kb = 0x1.c18a9f13d513cp+71 * fexp(fma(-0x1.2b7b4a0000000p+1, lt, -0x1.95c9960000000p+26 * irt));
+    const double kf = 0x1.07c1a01530916p+32 * fexp2(fma(0.0, irt, -0x1.1c28f60000000p+0 * lt));
+    const double kb = 0x1.b0096fff6b3f8p+50 * fexp2(fma(-0x1.95c9960000000p+26, irt, -0x1.2b7b4a0000000p+1 * lt));
     const double q = kf * C14 * C4 - kb * C37;
     cd4 -= q;
     cd14 -= q;
     cd37 += q;
     }
     {  // R168 (elementary)
-    const double kf = 0x1.fdece9526af40p+61 * fexp(fma(-0x1.d70a3e0000000p-2, lt, -0x1.b022b58000000p+28 * irt));
-    const double kb = 0x1.4680bd799999ap+24 * fexp(fma(0x1.fc76080000000p-1, lt, 0x1.4af9180000000p+23 * irt));
+    const double kf = 0x1.cec45f1a33b42p+57 * fexp2(fma(-0x1.b022b58000000p+28, irt, -0x1.d70a3e0000000p-2 * lt));
+    const double kb = 0x1.38b93a09f2078p+33 * fexp2(fma(0x1.4af9180000000p+23, irt, 0x1.fc76080000000p-1 * lt));
     const double q = kf * C38 - kb * C4 * C11;
     cd4 += q;
     cd11 += q;
     cd38 -= q;
     }
     {  // R169 (elementary)
-    const double kf = 0x1.4780000000000p+11 * fexp(fma(0x1.07ae140000000p+1, lt, -0x1.d3e5400000000p+21 * irt));
-    const double kb = 0x1.0c954ca93de8bp-5 * fexp(fma(0x1.5c5b180000000p+1, lt, -0x1.2d08fa0000000p+26 * irt));
+    const double kf = 0x1.dc2d03289b6fbp+29 * fexp2(fma(-0x1.d3e5400000000p+21, irt, 0x1.07ae140000000p+1 * lt));
+    const double kb = 0x1.7a327c4dbf8f9p+19 * fexp2(fma(-0x1.2d08fa0000000p+26, irt, 0x1.5c5b180000000p+1 * lt));
     const double q = kf * C38 * C4 - kb * C1 * C10 * C6;
     cd1 += q;
     cd4 -= q;
@@ -1552,24 +1429,24 @@ struct LaneRhs<40> {
     cd38 -= q;
     }
     {  // R170 (elementary)
-    const double kf = 0x1.2110000000000p+14 * fexp(fma(0x1.828f5c0000000p+0, lt, 0x1.eb55400000000p+21 * irt));
-    const double kb = 0x1.63ae0e62a1774p-25 * fexp(fma(0x1.b9b1860000000p+1, lt, 0x1.15cf900000000p+25 * irt));
+    const double kf = 0x1.b31c40afbd2e0p+27 * fexp2(fma(0x1.eb55400000000p+21, irt, 0x1.828f5c0000000p+0 * lt));
+    const double kb = 0x1.71e7618277c26p+6 * fexp2(fma(0x1.15cf900000000p+25, irt, 0x1.b9b1860000000p+1 * lt));
     const double q = kf * C38 * C4 - kb * C4 * C9 * C6;
     cd6 += q;
     cd9 += q;
     cd38 -= q;
     }
     {  // R171 (elementary)
-    const double kf = 0x1.0900000000000p+12 * fexp(fma(0x1.0ccccc0000000p+1, lt, -0x1.36ca800000000p+24 * irt));
-    const double kb = 0x1.5296cdcbd2ea1p-8 * fexp(fma(0x1.6d758e0000000p+1, lt, -0x1.f397720000000p+24 * irt));
+    const double kf = 0x1.ee81d74a42119p+30 * fexp2(fma(-0x1.36ca800000000p+24, irt, 0x1.0ccccc0000000p+1 * lt));
+    const double kb = 0x1.1253291935339p+18 * fexp2(fma(-0x1.f397720000000p+24, irt, 0x1.6d758e0000000p+1 * lt));
     const double q = kf * C38 * C1 - kb * C1 * C10 * C5;
     cd5 += q;
     cd10 += q;
     cd38 -= q;
     }
     {  // R172 (elementary)
-    const double kf = 0x1.c1451f6000000p+35 * fexp(fma(-0x1.6666660000000p-2, lt, -0x1.7d87e00000000p+23 * irt));
-    const double kb = 0x1.aea15878a34cbp-7 * fexp(fma(0x1.af31900000000p+0, lt, 0x1.3b12b60000000p+26 * irt));
+    const double kf = 0x1.94e7a23e859b3p+32 * fexp2(fma(-0x1.7d87e00000000p+23, irt, -0x1.6666660000000p-2 * lt));
+    const double kb = 0x1.e0dab3338fbddp+8 * fexp2(fma(0x1.3b12b60000000p+26, irt, 0x1.af31900000000p+0 * lt));
     const double q = kf * C38 * C1 - kb * C4 * C9 * C5;
     cd1 -= q;
     cd4 += q;
@@ -1578,8 +1455,8 @@ struct LaneRhs<40> {
     cd38 -= q;
     }
     {  // R173 (elementary)
-    const double kf = 0x1.accf3dacbf296p-32 * fexp(fma(0x1.7333340000000p+2, lt, -0x1.18ea100000000p+23 * irt));
-    const double kb = 0x1.10f15c73ea2c3p-65 * fexp(fma(0x1.e2d3ae0000000p+2, lt, 0x1.295f4a0000000p+26 * irt));
+    const double kf = 0x1.ec92c9e8579e1p+20 * fexp2(fma(-0x1.18ea100000000p+23, irt, 0x1.7333340000000p+2 * lt));
+    const double kb = 0x1.fc752e17f1558p+2 * fexp2(fma(0x1.295f4a0000000p+26, irt, 0x1.e2d3ae0000000p+2 * lt));
     const double q = kf * C38 * C12 - kb * C4 * C9 * C13;
     cd4 += q;
     cd9 += q;
@@ -1588,8 +1465,8 @@ struct LaneRhs<40> {
     cd38 -= q;
     }
     {  // R174 (elementary)
-    const double kf = 0x1.dcd6500000000p+29 * fexp(fma(0.0, lt, -0x1.7c80340000000p+25 * irt));
-    const double kb = 0x1.9ac2cc99d248cp-3 * fexp(fma(0x1.488af00000000p+0, lt, 0x1.a98f3a0000000p+26 * irt));
+    const double kf = 0x1.dcd6500000000p+29 * fexp2(fma(-0x1.7c80340000000p+25, irt, 0.0 * lt));
+    const double kb = 0x1.2cc36fe9a7ba7p+9 * fexp2(fma(0x1.a98f3a0000000p+26, irt, 0x1.488af00000000p+0 * lt));
     const double q = kf * C38 * C7 - kb * C4 * C9 * C8;
     cd4 += q;
     cd7 -= q;
@@ -1598,8 +1475,8 @@ struct LaneRhs<40> {
     cd38 -= q;
     }
     {  // R175 (elementary)
-    const double kf = 0x1.92738f5028000p+50 * fexp(fma(-0x1.e666660000000p+0, lt, -0x1.7bda300000000p+23 * irt));
-    const double kb = 0x1.c483c85fd5a89p+7 * fexp(fma(0x1.96cbbe0000000p-4, lt, 0x1.51475e0000000p+26 * irt));
+    const double kf = 0x1.7780206bbf3b0p+33 * fexp2(fma(-0x1.7bda300000000p+23, irt, -0x1.e666660000000p+0 * lt));
+    const double kb = 0x1.a46971c2b1db0p+8 * fexp2(fma(0x1.51475e0000000p+26, irt, 0x1.96cbbe0000000p-4 * lt));
     const double q = kf * C38 * C3 - kb * C4 * C4 * C9;
     cd3 -= q;
     cd4 = fma(0x1.0000000000000p+1, q, cd4);
@@ -1607,81 +1484,81 @@ struct LaneRhs<40> {
     cd38 -= q;
     }
     {  // R5 (third_body)
-    const double kf = 0x1.4537251ebd400p+55 * fexp(fma(-0x1.6666660000000p+0, lt, -0x1.a07e8f0000000p+28 * irt));
-    const double kb = 0x1.64de7c2f90c00p+47 * fexp(fma(-0x1.bfb15c0000000p+0, lt, -0x1.bde0e40000000p+21 * irt));
+    const double kf = 0x1.ad1fd6ba434f6p+42 * fexp2(fma(-0x1.a07e8f0000000p+28, irt, -0x1.6666660000000p+0 * lt));
+    const double kb = 0x1.ab947e9a29ae7p+31 * fexp2(fma(-0x1.bde0e40000000p+21, irt, -0x1.bfb15c0000000p+0 * lt));
     const double q = (kf * C5 - kb * C1 * C1) * M0();
     cd1 = fma(0x1.0000000000000p+1, q, cd1);
     cd5 -= q;
     }
     {  // R6 (third_body)
-    const double kf = 0x1.6f766f4000000p+32 * fexp(fma(-0x1.0000000000000p-1, lt, 0.0 * irt));
-    const double kb = 0x1.81d880a2e9b00p+48 * fexp(fma(-0x1.3e0ce00000000p-1, lt, -0x1.dacde80000000p+28 * irt));
+    const double kf = 0x1.03d5d79a03db5p+28 * fexp2(fma(0.0, irt, -0x1.0000000000000p-1 * lt));
+    const double kb = 0x1.00345f663afa2p+43 * fexp2(fma(-0x1.dacde80000000p+28, irt, -0x1.3e0ce00000000p-1 * lt));
     const double q = (kf * C3 * C3 - kb * C2) * M1();
     cd2 += q;
     cd3 = fma(-0x1.0000000000000p+1, q, cd3);
     }
     {  // R7 (third_body)
-    const double kf = 0x1.126412e900000p+42 * fexp(fma(-0x1.0000000000000p+0, lt, 0.0 * irt));
-    const double kb = 0x1.2554127579c00p+49 * fexp(fma(-0x1.5f5a100000000p-1, lt, -0x1.9783100000000p+28 * irt));
+    const double kf = 0x1.126412e900000p+33 * fexp2(fma(0.0, irt, -0x1.0000000000000p+0 * lt));
+    const double kb = 0x1.039f25dff47d2p+43 * fexp2(fma(-0x1.9783100000000p+28, irt, -0x1.5f5a100000000p-1 * lt));
     const double q = (kf * C3 * C1 - kb * C4) * M2();
     cd1 -= q;
     cd3 -= q;
     cd4 += q;
     }
     {  // R8 (third_body)
-    const double kf = 0x1.0e0198eaee000p+55 * fexp(fma(-0x1.0000000000000p+1, lt, 0.0 * irt));
-    const double kb = 0x1.3bde5cba02571p+66 * fexp(fma(-0x1.beac860000000p+0, lt, -0x1.d8d0724000000p+28 * irt));
+    const double kf = 0x1.0e0198eaee000p+37 * fexp2(fma(0.0, irt, -0x1.0000000000000p+1 * lt));
+    const double kb = 0x1.83f8483e413c5p+50 * fexp2(fma(-0x1.d8d0724000000p+28, irt, -0x1.beac860000000p+0 * lt));
     const double q = (kf * C1 * C4 - kb * C6) * M3();
     cd1 -= q;
     cd4 -= q;
     cd6 += q;
     }
     {  // R9 (falloff)
-    const double kinf_f = 0x1.5faadb0000000p+30 * fexp(fma(0x1.3333340000000p-1, lt, 0.0 * irt));
-    const double k0_f = 0x1.217dfe6e98000p+49 * fexp(fma(-0x1.b851ec0000000p+0, lt, -0x1.0c11000000000p+21 * irt));
-    const double kinf_b = 0x1.e71aa37570000p+40 * fexp(fma(0x1.2c97740000000p-1, lt, -0x1.865d460000000p+27 * irt));
-    const double k0_b = 0x1.90fbc30ed0778p+59 * fexp(fma(-0x1.bb9ffe0000000p+0, lt, -0x1.8a8d8a0000000p+27 * irt));
+    const double kinf_f = 0x1.d0072a67767fcp+35 * fexp2(fma(0.0, irt, 0x1.3333340000000p-1 * lt));
+    const double k0_f = 0x1.9f1e654b4f45bp+33 * fexp2(fma(-0x1.0c11000000000p+21, irt, -0x1.b851ec0000000p+0 * lt));
+    const double kinf_b = 0x1.2881d573ae734p+46 * fexp2(fma(-0x1.865d460000000p+27, irt, 0x1.2c97740000000p-1 * lt));
+    const double k0_b = 0x1.093ffb1152f8fp+44 * fexp2(fma(-0x1.8a8d8a0000000p+27, irt, -0x1.bb9ffe0000000p+0 * lt));
     const double m_ = M4();
     const double conc = m_ > 0.0 ? m_ : p_rt;
     double fc = 0.0;
-    fc = fma(0x1.99999a0000000p-3, fexp(-(T / 0x1.4484c00000000p-100)), fc);
-    fc = fma(0x1.99999a0000000p-1, fexp(-(T / 0x1.93e5940000000p+99)), fc);
-    const double lnfc = flog(fc);
-    const double lfc = lnfc * kInvLn10;
+    fc = fma(0x1.99999a0000000p-3, fexp2(-(0x1.235995d2649cap+100 * T)), fc);
+    fc = fma(0x1.99999a0000000p-1, fexp2(-(0x1.d42e69bdf23bep-100 * T)), fc);
+    const double l2fc = flog2(fc);
+    const double lfc = l2fc * kLog10Of2;
     const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
     const double cco = fma(-kTroeC1, lfc, -kTroeC0);
-    const double kf = troe(kinf_f, k0_f, conc, lnfc, ntmp, cco);
-    const double kb = troe(kinf_b, k0_b, conc, lnfc, ntmp, cco);
+    const double kf = troe(kinf_f, k0_f, conc, l2fc, ntmp, cco);
+    const double kb = troe(kinf_b, k0_b, conc, l2fc, ntmp, cco);
     const double q = kf * C1 * C2 - kb * C7;
     cd1 -= q;
     cd2 -= q;
     cd7 += q;
     }
     {  // R16 (falloff)
-    const double kinf_f = 0x1.0c6452ac58000p+48 * fexp(fma(0.0, lt, -0x1.827ceb0000000p+27 * irt));
-    const double k0_f = 0x1.b548f93540000p+46 * fexp(fma(0.0, lt, -0x1.6b1b140000000p+27 * irt));
-    const double kinf_b = 0x1.017dfb13be22ep+18 * fexp(fma(0x1.29ef740000000p+0, lt, 0x1.6efb160000000p+23 * irt));
-    const double k0_b = 0x1.a386bad234ebap+16 * fexp(fma(0x1.29ef740000000p+0, lt, 0x1.728c440000000p+24 * irt));
+    const double kinf_f = 0x1.0c6452ac58000p+48 * fexp2(fma(-0x1.827ceb0000000p+27, irt, 0.0 * lt));
+    const double k0_f = 0x1.b548f93540000p+46 * fexp2(fma(-0x1.6b1b140000000p+27, irt, 0.0 * lt));
+    const double kinf_b = 0x1.65b78847004cbp+28 * fexp2(fma(0x1.6efb160000000p+23, irt, 0x1.29ef740000000p+0 * lt));
+    const double k0_b = 0x1.2369027e2aa3dp+27 * fexp2(fma(0x1.728c440000000p+24, irt, 0x1.29ef740000000p+0 * lt));
     const double m_ = M5();
     const double conc = m_ > 0.0 ? m_ : p_rt;
     double fc = 0.0;
-    fc = fma(0x1.0000000000000p-1, fexp(-(T / 0x1.4484c00000000p-100)), fc);
-    fc = fma(0x1.0000000000000p-1, fexp(-(T / 0x1.93e5940000000p+99)), fc);
-    const double lnfc = flog(fc);
-    const double lfc = lnfc * kInvLn10;
+    fc = fma(0x1.0000000000000p-1, fexp2(-(0x1.235995d2649cap+100 * T)), fc);
+    fc = fma(0x1.0000000000000p-1, fexp2(-(0x1.d42e69bdf23bep-100 * T)), fc);
+    const double l2fc = flog2(fc);
+    const double lfc = l2fc * kLog10Of2;
     const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
     const double cco = fma(-kTroeC1, lfc, -kTroeC0);
-    const double kf = troe(kinf_f, k0_f, conc, lnfc, ntmp, cco);
-    const double kb = troe(kinf_b, k0_b, conc, lnfc, ntmp, cco);
+    const double kf = troe(kinf_f, k0_f, conc, l2fc, ntmp, cco);
+    const double kb = troe(kinf_b, k0_b, conc, l2fc, ntmp, cco);
     const double q = kf * C8 - kb * C4 * C4;
     cd4 = fma(0x1.0000000000000p+1, q, cd4);
     cd8 -= q;
     }
     {  // R22 (falloff)
-    const double kinf_f = 0x1.12a8800000000p+24 * fexp(fma(0.0, lt, -0x1.3069b00000000p+23 * irt));
-    const double k0_f = 0x1.582b4c9a9db00p+60 * fexp(fma(-0x1.651eb80000000p+1, lt, -0x1.0b90180000000p+24 * irt));
-    const double kinf_b = 0x1.87633209b15e0p+53 * fexp(fma(-0x1.ee4cf80000000p-1, lt, -0x1.03c20c0000000p+29 * irt));
-    const double k0_b = 0x1.ea70c1371c568p+89 * fexp(fma(-0x1.e0b1ee0000000p+1, lt, -0x1.075ce60000000p+29 * irt));
+    const double kinf_f = 0x1.12a8800000000p+24 * fexp2(fma(-0x1.3069b00000000p+23, irt, 0.0 * lt));
+    const double k0_f = 0x1.3ee730e98e9c1p+35 * fexp2(fma(-0x1.0b90180000000p+24, irt, -0x1.651eb80000000p+1 * lt));
+    const double kinf_b = 0x1.e59553e956d76p+44 * fexp2(fma(-0x1.03c20c0000000p+29, irt, -0x1.ee4cf80000000p-1 * lt));
+    const double k0_b = 0x1.19e7a1f3fe30cp+56 * fexp2(fma(-0x1.075ce60000000p+29, irt, -0x1.e0b1ee0000000p+1 * lt));
     const double m_ = M6();
     const double conc = m_ > 0.0 ? m_ : p_rt;
     const double pr_f = k0_f * conc / fmax(kinf_f, 1.0e-60);
@@ -1694,281 +1571,489 @@ struct LaneRhs<40> {
     cd10 += q;
     }
     {  // R26 (third_body)
-    const double kf = 0x1.c4cdf80000000p+28 * fexp(fma(0x1.5168720000000p-1, lt, -0x1.daccd40000000p+25 * irt));
-    const double kb = 0x1.73e869ed06fefp+16 * fexp(fma(0x1.c86db60000000p-1, lt, 0x1.dfa10e0000000p+20 * irt));
+    const double kf = 0x1.afa86ab683a72p+34 * fexp2(fma(-0x1.daccd40000000p+25, irt, 0x1.5168720000000p-1 * lt));
+    const double kb = 0x1.79ed09e2f0ad0p+24 * fexp2(fma(0x1.dfa10e0000000p+20, irt, 0x1.c86db60000000p-1 * lt));
     const double q = (kf * C11 - kb * C9 * C1) * M7();
     cd1 += q;
     cd9 += q;
     cd11 -= q;
     }
     {  // R36 (third_body)
-    const double kf = 0x1.3dc747e5d87eep+121 * fexp(fma(-0x1.9333340000000p+2, lt, -0x1.8e9e630000000p+28 * irt));
-    const double kb = 0x1.fd684dac5b3acp+103 * fexp(fma(-0x1.8b7bf20000000p+2, lt, -0x1.2c9de60000000p+25 * irt));
+    const double kf = 0x1.873b0e46bd384p+64 * fexp2(fma(-0x1.8e9e630000000p+28, irt, -0x1.9333340000000p+2 * lt));
+    const double kb = 0x1.4c9dd43d1787bp+48 * fexp2(fma(-0x1.2c9de60000000p+25, irt, -0x1.8b7bf20000000p+2 * lt));
     const double q = (kf * C14 - kb * C1 * C11) * M8();
     cd1 += q;
     cd11 += q;
     cd14 -= q;
     }
     {  // R37 (third_body)
-    const double kf = 0x1.1cb0a65614918p+141 * fexp(fma(-0x1.0000000000000p+3, lt, -0x1.8514fb0000000p+28 * irt));
-    const double kb = 0x1.5595faa80c0d3p+119 * fexp(fma(-0x1.d315620000000p+2, lt, -0x1.7bd3e60000000p+28 * irt));
+    const double kf = 0x1.1cb0a65614918p+69 * fexp2(fma(-0x1.8514fb0000000p+28, irt, -0x1.0000000000000p+3 * lt));
+    const double kb = 0x1.a957da6425b01p+53 * fexp2(fma(-0x1.7bd3e60000000p+28, irt, -0x1.d315620000000p+2 * lt));
     const double q = (kf * C14 - kb * C5 * C9) * M9();
     cd5 += q;
     cd9 += q;
     cd14 -= q;
     }
     {  // R48 (falloff)
-    const double kinf_f = 0x1.0913e35900000p+41 * fexp(fma(-0x1.6147ae0000000p-1, lt, -0x1.656c000000000p+19 * irt));
-    const double k0_f = 0x1.0a7c08982a5e9p+86 * fexp(fma(-0x1.e000000000000p+1, lt, -0x1.f557c00000000p+21 * irt));
-    const double kinf_b = 0x1.2b68f9fa2c3f6p+78 * fexp(fma(-0x1.060d460000000p+1, lt, -0x1.6f20af2000000p+28 * irt));
-    const double k0_b = 0x1.2cffc47128800p+123 * fexp(fma(-0x1.46ddac0000000p+2, lt, -0x1.7258a8a000000p+28 * irt));
+    const double kinf_f = 0x1.ca56cd1f06e98p+34 * fexp2(fma(-0x1.656c000000000p+19, irt, -0x1.6147ae0000000p-1 * lt));
+    const double k0_f = 0x1.3ce7bfd2bd5a5p+52 * fexp2(fma(-0x1.f557c00000000p+21, irt, -0x1.e000000000000p+1 * lt));
+    const double kinf_b = 0x1.bddd0d7ce5f55p+59 * fexp2(fma(-0x1.6f20af2000000p+28, irt, -0x1.060d460000000p+1 * lt));
+    const double k0_b = 0x1.3447abcd6caf5p+77 * fexp2(fma(-0x1.7258a8a000000p+28, irt, -0x1.46ddac0000000p+2 * lt));
     const double m_ = M10();
     const double conc = m_ > 0.0 ? m_ : p_rt;
     double fc = 0.0;
-    fc = fma(0x1.0000000000000p+0, fexp(-(T / 0x1.1d00000000000p+9)), fc);
-    fc = fma(0x1.0000000000000p+0, fexp(-(0x1.93e5940000000p+99 / T)), fc);
-    const double lnfc = flog(fc);
-    const double lfc = lnfc * kInvLn10;
+    fc = fma(0x1.0000000000000p+0, fexp2(-(0x1.4bbfbdd1efffep-9 * T)), fc);
+    fc = fma(0x1.0000000000000p+0, fexp2(-(0x1.2359962b722d0p+100 * invT)), fc);
+    const double l2fc = flog2(fc);
+    const double lfc = l2fc * kLog10Of2;
     const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
     const double cco = fma(-kTroeC1, lfc, -kTroeC0);
-    const double kf = troe(kinf_f, k0_f, conc, lnfc, ntmp, cco);
-    const double kb = troe(kinf_b, k0_b, conc, lnfc, ntmp, cco);
+    const double kf = troe(kinf_f, k0_f, conc, l2fc, ntmp, cco);
+    const double kb = troe(kinf_b, k0_b, conc, l2fc, ntmp, cco);
     const double q = kf * C12 * C12 - kb * C16;
     cd12 = fma(-0x1.0000000000000p+1, q, cd12);
     cd16 += q;
     }
     {  // R49 (falloff)
-    const double kinf_f = 0x1.719e5fa300000p+43 * fexp(fma(-0x1.428f5c0000000p-1, lt, -0x1.871d000000000p+20 * irt));
-    const double k0_f = 0x1.001da4e1fe9aep+91 * fexp(fma(-0x1.30a3d80000000p+2, lt, -0x1.378dd00000000p+23 * irt));
-    const double kinf_b = 0x1.bf5be7da6fdb8p+59 * fexp(fma(-0x1.248bca0000000p-1, lt, -0x1.a61bb40000000p+28 * irt));
-    const double k0_b = 0x1.35fbcb677bb59p+107 * fexp(fma(-0x1.2ce3680000000p+2, lt, -0x1.ae51060000000p+28 * irt));
+    const double kinf_f = 0x1.d09d97b8751a6p+37 * fexp2(fma(-0x1.871d000000000p+20, irt, -0x1.428f5c0000000p-1 * lt));
+    const double k0_f = 0x1.1e278bd56dda1p+48 * fexp2(fma(-0x1.378dd00000000p+23, irt, -0x1.30a3d80000000p+2 * lt));
+    const double kinf_b = 0x1.954f16e614a41p+54 * fexp2(fma(-0x1.a61bb40000000p+28, irt, -0x1.248bca0000000p-1 * lt));
+    const double k0_b = 0x1.f341016a73215p+64 * fexp2(fma(-0x1.ae51060000000p+28, irt, -0x1.2ce3680000000p+2 * lt));
     const double m_ = M11();
     const double conc = m_ > 0.0 ? m_ : p_rt;
     double fc = 0.0;
-    fc = fma(0x1.bc6a7e0000000p-3, fexp(-(T / 0x1.2800000000000p+6)), fc);
-    fc = fma(0x1.90e5600000000p-1, fexp(-(T / 0x1.6fa0000000000p+11)), fc);
-    fc = fma(0x1.0000000000000p+0, fexp(-(0x1.b340000000000p+12 / T)), fc);
-    const double lnfc = flog(fc);
-    const double lfc = lnfc * kInvLn10;
+    fc = fma(0x1.bc6a7e0000000p-3, fexp2(-(0x1.3f6ba49a91758p-6 * T)), fc);
+    fc = fma(0x1.90e5600000000p-1, fexp2(-(0x1.012fef8327e8fp-11 * T)), fc);
+    fc = fma(0x1.0000000000000p+0, fexp2(-(0x1.39f76d1611d3bp+13 * invT)), fc);
+    const double l2fc = flog2(fc);
+    const double lfc = l2fc * kLog10Of2;
     const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
     const double cco = fma(-kTroeC1, lfc, -kTroeC0);
-    const double kf = troe(kinf_f, k0_f, conc, lnfc, ntmp, cco);
-    const double kb = troe(kinf_b, k0_b, conc, lnfc, ntmp, cco);
+    const double kf = troe(kinf_f, k0_f, conc, l2fc, ntmp, cco);
+    const double kb = troe(kinf_b, k0_b, conc, l2fc, ntmp, cco);
     const double q = kf * C12 * C1 - kb * C13;
     cd1 -= q;
     cd12 -= q;
     cd13 += q;
     }
     {  // R55 (third_body)
-    const double kf = 0x1.74876e8000000p+36 * fexp(fma(0.0, lt, -0x1.909ca40000000p+26 * irt));
-    const double kb = 0x1.ec57c8570a3d7p+23 * fexp(fma(0x1.4745380000000p-2, lt, 0x1.9329780000000p+23 * irt));
+    const double kf = 0x1.74876e8000000p+36 * fexp2(fma(-0x1.909ca40000000p+26, irt, 0.0 * lt));
+    const double kb = 0x1.c3eb3173826b7p+26 * fexp2(fma(0x1.9329780000000p+23, irt, 0x1.4745380000000p-2 * lt));
     const double q = (kf * C17 - kb * C1 * C14) * M12();
     cd1 += q;
     cd14 += q;
     cd17 -= q;
     }
     {  // R64 (third_body)
-    const double kf = 0x1.7970b794f0000p+49 * fexp(fma(-0x1.3333340000000p+0, lt, -0x1.eec8100000000p+25 * irt));
-    const double kb = 0x1.4401f22700000p+33 * fexp(fma(-0x1.cc4fa00000000p-1, lt, 0x1.4e995e0000000p+24 * irt));
+    const double kf = 0x1.b1909edeca7e6p+38 * fexp2(fma(-0x1.eec8100000000p+25, irt, -0x1.3333340000000p+0 * lt));
+    const double kb = 0x1.301dc050b0a08p+25 * fexp2(fma(0x1.4e995e0000000p+24, irt, -0x1.cc4fa00000000p-1 * lt));
     const double q = (kf * C15 - kb * C1 * C14) * M12();
     cd1 += q;
     cd14 += q;
     cd15 -= q;
     }
     {  // R166 (third_body)
-    const double kf = 0x1.56ba098000000p+34 * fexp(fma(0.0, lt, -0x1.8f04700000000p+27 * irt));
-    const double kb = 0x1.a5b62a1280320p-5 * fexp(fma(0x1.f0d3ae0000000p+0, lt, -0x1.513de0e000000p+27 * irt));
+    const double kf = 0x1.56ba098000000p+34 * fexp2(fma(-0x1.8f04700000000p+27, irt, 0.0 * lt));
+    const double kb = 0x1.235d612f09caap+13 * fexp2(fma(-0x1.513de0e000000p+27, irt, 0x1.f0d3ae0000000p+0 * lt));
     const double q = (kf * C38 - kb * C6 * C9) * M12();
     cd6 += q;
     cd9 += q;
     cd38 -= q;
     }
     {  // R167 (third_body)
-    const double kf = 0x1.b48eb57e00000p+43 * fexp(fma(0.0, lt, -0x1.c6e1380000000p+27 * irt));
-    const double kb = 0x1.16e4c05581062p+24 * fexp(fma(0x1.82a36a0000000p-1, lt, -0x1.de7ad60000000p+27 * irt));
+    const double kf = 0x1.b48eb57e00000p+43 * fexp2(fma(-0x1.c6e1380000000p+27, irt, 0.0 * lt));
+    const double kb = 0x1.e45d2eb20e8f3p+30 * fexp2(fma(-0x1.de7ad60000000p+27, irt, 0x1.82a36a0000000p-1 * lt));
     const double q = (kf * C38 - kb * C5 * C10) * M12();
     cd5 += q;
     cd10 += q;
     cd38 -= q;
     }
     {  // R86 (falloff)
-    const double kinf_f = 0x1.d9d8c3ed90000p+48 * fexp(fma(-0x1.fae1480000000p-1, lt, -0x1.9380e00000000p+22 * irt));
-    const double k0_f = 0x1.329ba8fa506b9p+117 * fexp(fma(-0x1.c51eb80000000p+2, lt, -0x1.aac9d00000000p+24 * irt));
-    const double kinf_b = 0x1.e7bf2db4245bdp+68 * fexp(fma(-0x1.2e3dc40000000p+0, lt, -0x1.9848f20000000p+28 * irt));
-    const double k0_b = 0x1.3b9a2c38152a0p+137 * fexp(fma(-0x1.d152000000000p+2, lt, -0x1.aca78c0000000p+28 * irt));
+    const double kinf_f = 0x1.f8592ae3e59d9p+39 * fexp2(fma(-0x1.9380e00000000p+22, irt, -0x1.fae1480000000p-1 * lt));
+    const double k0_f = 0x1.744837ad03a96p+53 * fexp2(fma(-0x1.aac9d00000000p+24, irt, -0x1.c51eb80000000p+2 * lt));
+    const double kinf_b = 0x1.3c1e2dc02ed72p+58 * fexp2(fma(-0x1.9848f20000000p+28, irt, -0x1.2e3dc40000000p+0 * lt));
+    const double k0_b = 0x1.d2ae7b3895482p+71 * fexp2(fma(-0x1.aca78c0000000p+28, irt, -0x1.d152000000000p+2 * lt));
     const double m_ = M13();
     const double conc = m_ > 0.0 ? m_ : p_rt;
     double fc = 0.0;
-    fc = fma(0x1.432ca60000000p-3, fexp(-(T / 0x1.f400000000000p+6)), fc);
-    fc = fma(0x1.af34d60000000p-1, fexp(-(T / 0x1.1560000000000p+11)), fc);
-    fc = fma(0x1.0000000000000p+0, fexp(-(0x1.ae20000000000p+12 / T)), fc);
-    const double lnfc = flog(fc);
-    const double lfc = lnfc * kInvLn10;
+    fc = fma(0x1.432ca60000000p-3, fexp2(-(0x1.7a31a0132b331p-7 * T)), fc);
+    fc = fma(0x1.af34d60000000p-1, fexp2(-(0x1.54de64aaf2369p-11 * T)), fc);
+    fc = fma(0x1.0000000000000p+0, fexp2(-(0x1.364504a6dddbcp+13 * invT)), fc);
+    const double l2fc = flog2(fc);
+    const double lfc = l2fc * kLog10Of2;
     const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
     const double cco = fma(-kTroeC1, lfc, -kTroeC0);
-    const double kf = troe(kinf_f, k0_f, conc, lnfc, ntmp, cco);
-    const double kb = troe(kinf_b, k0_b, conc, lnfc, ntmp, cco);
+    const double kf = troe(kinf_f, k0_f, conc, l2fc, ntmp, cco);
+    const double kb = troe(kinf_b, k0_b, conc, l2fc, ntmp, cco);
     const double q = kf * C18 * C1 - kb * C16;
     cd1 -= q;
     cd16 += q;
     cd18 -= q;
     }
     {  // R93 (falloff)
-    const double kinf_f = 0x1.d1a94a2000000p+42 * fexp(fma(0x1.c28f5c0000000p-2, lt, -0x1.62353f0000000p+28 * irt));
-    const double k0_f = 0x1.ea7457a7c18a1p+158 * fexp(fma(-0x1.29eb860000000p+3, lt, -0x1.8e755f0000000p+28 * irt));
-    const double kinf_b = 0x1.db0c3690e5604p+23 * fexp(fma(0x1.814e3c0000000p-1, lt, -0x1.6cafae0000000p+27 * irt));
-    const double k0_b = 0x1.f45734685fcd6p+139 * fexp(fma(-0x1.1feb1c0000000p+3, lt, -0x1.c52fee0000000p+27 * irt));
+    const double kinf_f = 0x1.c4ed80e7a3586p+46 * fexp2(fma(-0x1.62353f0000000p+28, irt, 0x1.c28f5c0000000p-2 * lt));
+    const double k0_f = 0x1.1ba694291eb78p+75 * fexp2(fma(-0x1.8e755f0000000p+28, irt, -0x1.29eb860000000p+3 * lt));
+    const double kinf_b = 0x1.95df0ff2384f5p+30 * fexp2(fma(-0x1.6cafae0000000p+27, irt, 0x1.814e3c0000000p-1 * lt));
+    const double k0_b = 0x1.fc5d2cf237a09p+58 * fexp2(fma(-0x1.c52fee0000000p+27, irt, -0x1.1feb1c0000000p+3 * lt));
     const double m_ = M14();
     const double conc = m_ > 0.0 ? m_ : p_rt;
     double fc = 0.0;
-    fc = fma(0x1.0fdf3c0000000p-2, fexp(-(T / 0x1.6800000000000p+7)), fc);
-    fc = fma(0x1.7810620000000p-1, fexp(-(T / 0x1.02c0000000000p+10)), fc);
-    fc = fma(0x1.0000000000000p+0, fexp(-(0x1.5290000000000p+12 / T)), fc);
-    const double lnfc = flog(fc);
-    const double lfc = lnfc * kInvLn10;
+    fc = fma(0x1.0fdf3c0000000p-2, fexp2(-(0x1.06a2764633554p-7 * T)), fc);
+    fc = fma(0x1.7810620000000p-1, fexp2(-(0x1.6d67996cccfc3p-10 * T)), fc);
+    fc = fma(0x1.0000000000000p+0, fexp2(-(0x1.e87143bbc5b6dp+12 * invT)), fc);
+    const double l2fc = flog2(fc);
+    const double lfc = l2fc * kLog10Of2;
     const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
     const double cco = fma(-kTroeC1, lfc, -kTroeC0);
-    const double kf = troe(kinf_f, k0_f, conc, lnfc, ntmp, cco);
-    const double kb = troe(kinf_b, k0_b, conc, lnfc, ntmp, cco);
+    const double kf = troe(kinf_f, k0_f, conc, l2fc, ntmp, cco);
+    const double kb = troe(kinf_b, k0_b, conc, l2fc, ntmp, cco);
     const double q = kf * C21 - kb * C23 * C5;
     cd5 += q;
     cd21 -= q;
     cd23 += q;
     }
     {  // R94 (falloff)
-    const double kinf_f = 0x1.017df80000000p+30 * fexp(fma(0x1.d0e5600000000p-2, lt, -0x1.d0c8600000000p+22 * irt));
-    const double k0_f = 0x1.ce3922c2af443p+119 * fexp(fma(-0x1.e7ae140000000p+2, lt, -0x1.bcfa100000000p+24 * irt));
-    const double kinf_b = 0x1.83665740c8000p+40 * fexp(fma(0x1.6cc78e0000000p-2, lt, -0x1.2edfd20000000p+27 * irt));
-    const double k0_b = 0x1.5bb5c58e44559p+130 * fexp(fma(-0x1.edeff20000000p+2, lt, -0x1.57f8d00000000p+27 * irt));
+    const double kinf_f = 0x1.114edc398b4b1p+34 * fexp2(fma(-0x1.d0c8600000000p+22, irt, 0x1.d0e5600000000p-2 * lt));
+    const double k0_f = 0x1.3535f6503834dp+51 * fexp2(fma(-0x1.bcfa100000000p+24, irt, -0x1.e7ae140000000p+2 * lt));
+    const double kinf_b = 0x1.bee1b7f58da4ep+43 * fexp2(fma(-0x1.2edfd20000000p+27, irt, 0x1.6cc78e0000000p-2 * lt));
+    const double k0_b = 0x1.f995c6ef57c32p+60 * fexp2(fma(-0x1.57f8d00000000p+27, irt, -0x1.edeff20000000p+2 * lt));
     const double m_ = M15();
     const double conc = m_ > 0.0 ? m_ : p_rt;
     double fc = 0.0;
-    fc = fma(0x1.94af500000000p-6, fexp(-(T / 0x1.a400000000000p+7)), fc);
-    fc = fma(0x1.f35a860000000p-1, fexp(-(T / 0x1.ec00000000000p+9)), fc);
-    fc = fma(0x1.0000000000000p+0, fexp(-(0x1.1160000000000p+12 / T)), fc);
-    const double lnfc = flog(fc);
-    const double lfc = lnfc * kInvLn10;
+    fc = fma(0x1.94af500000000p-6, fexp2(-(0x1.c23b13e60edb5p-8 * T)), fc);
+    fc = fma(0x1.f35a860000000p-1, fexp2(-(0x1.8057e54783511p-10 * T)), fc);
+    fc = fma(0x1.0000000000000p+0, fexp2(-(0x1.8a6591da95702p+12 * invT)), fc);
+    const double l2fc = flog2(fc);
+    const double lfc = l2fc * kLog10Of2;
     const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
     const double cco = fma(-kTroeC1, lfc, -kTroeC0);
-    const double kf = troe(kinf_f, k0_f, conc, lnfc, ntmp, cco);
-    const double kb = troe(kinf_b, k0_b, conc, lnfc, ntmp, cco);
+    const double kf = troe(kinf_f, k0_f, conc, l2fc, ntmp, cco);
+    const double kb = troe(kinf_b, k0_b, conc, l2fc, ntmp, cco);
     const double q = kf * C21 * C1 - kb * C18;
     cd1 -= q;
     cd18 += q;
     cd21 -= q;
     }
     {  // R95 (falloff)
-    const double kinf_f = 0x1.6a65700000000p+32 * fexp(fma(0x1.147ae20000000p-2, lt, -0x1.1e22000000000p+20 * irt));
-    const double k0_f = 0x1.287626ee52198p+80 * fexp(fma(-0x1.ee147a0000000p+1, lt, -0x1.a7eb700000000p+23 * irt));
-    const double kinf_b = 0x1.7b102e2734080p+51 * fexp(fma(0x1.132f020000000p-3, lt, -0x1.be02500000000p+28 * irt));
-    const double k0_b = 0x1.36189986c6210p+99 * fexp(fma(-0x1.ff70ce0000000p+1, lt, -0x1.ca238a0000000p+28 * irt));
+    const double kinf_f = 0x1.e83b7f97942bcp+34 * fexp2(fma(-0x1.1e22000000000p+20, irt, 0x1.147ae20000000p-2 * lt));
+    const double k0_f = 0x1.6301b0bd56537p+45 * fexp2(fma(-0x1.a7eb700000000p+23, irt, -0x1.ee147a0000000p+1 * lt));
+    const double kinf_b = 0x1.b63f047b3bc53p+52 * fexp2(fma(-0x1.be02500000000p+28, irt, 0x1.132f020000000p-3 * lt));
+    const double k0_b = 0x1.3eaa7f3287252p+63 * fexp2(fma(-0x1.ca238a0000000p+28, irt, -0x1.ff70ce0000000p+1 * lt));
     const double m_ = M16();
     const double conc = m_ > 0.0 ? m_ : p_rt;
     double fc = 0.0;
-    fc = fma(0x1.be76c80000000p-3, fexp(-(T / 0x1.9f00000000000p+7)), fc);
-    fc = fma(0x1.90624e0000000p-1, fexp(-(T / 0x1.4ce0000000000p+11)), fc);
-    fc = fma(0x1.0000000000000p+0, fexp(-(0x1.7cf0000000000p+12 / T)), fc);
-    const double lnfc = flog(fc);
-    const double lfc = lnfc * kInvLn10;
+    fc = fma(0x1.be76c80000000p-3, fexp2(-(0x1.c7a7bdc6e6f07p-8 * T)), fc);
+    fc = fma(0x1.90624e0000000p-1, fexp2(-(0x1.1c09331a387a3p-11 * T)), fc);
+    fc = fma(0x1.0000000000000p+0, fexp2(-(0x1.12c9cf68db79ep+13 * invT)), fc);
+    const double l2fc = flog2(fc);
+    const double lfc = l2fc * kLog10Of2;
     const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
     const double cco = fma(-kTroeC1, lfc, -kTroeC0);
-    const double kf = troe(kinf_f, k0_f, conc, lnfc, ntmp, cco);
-    const double kb = troe(kinf_b, k0_b, conc, lnfc, ntmp, cco);
+    const double kf = troe(kinf_f, k0_f, conc, l2fc, ntmp, cco);
+    const double kb = troe(kinf_b, k0_b, conc, l2fc, ntmp, cco);
     const double q = kf * C24 * C1 - kb * C21;
     cd1 -= q;
     cd21 += q;
     cd24 -= q;
     }
     {  // R109 (falloff)
-    const double kinf_f = 0x1.4dc9380000000p+32 * fexp(fma(0.0, lt, -0x1.3275200000000p+23 * irt));
-    const double k0_f = 0x1.d462db8b40f6ap+114 * fexp(fma(-0x1.d147ae0000000p+2, lt, -0x1.ccf0000000000p+24 * irt));
-    const double kinf_b = 0x1.1d0f31509c000p+40 * fexp(fma(0x1.6004320000000p-3, lt, -0x1.2b1f600000000p+27 * irt));
-    const double k0_b = 0x1.9002a52cd108ap+122 * fexp(fma(-0x1.c6479a0000000p+2, lt, -0x1.51960e0000000p+27 * irt));
+    const double kinf_f = 0x1.4dc9380000000p+32 * fexp2(fma(-0x1.3275200000000p+23, irt, 0.0 * lt));
+    const double k0_f = 0x1.5baa49ed6ae52p+49 * fexp2(fma(-0x1.ccf0000000000p+24, irt, -0x1.d147ae0000000p+2 * lt));
+    const double kinf_b = 0x1.a0781456b96d8p+41 * fexp2(fma(-0x1.2b1f600000000p+27, irt, 0x1.6004320000000p-3 * lt));
+    const double k0_b = 0x1.b1c70cd7437adp+58 * fexp2(fma(-0x1.51960e0000000p+27, irt, -0x1.c6479a0000000p+2 * lt));
     const double m_ = M17();
     const double conc = m_ > 0.0 ? m_ : p_rt;
     double fc = 0.0;
-    fc = fma(0x1.fe91000000000p-3, fexp(-(T / 0x1.8a00000000000p+6)), fc);
-    fc = fma(0x1.805bc00000000p-1, fexp(-(T / 0x1.4580000000000p+10)), fc);
-    fc = fma(0x1.0000000000000p+0, fexp(-(0x1.0470000000000p+12 / T)), fc);
-    const double lnfc = flog(fc);
-    const double lfc = lnfc * kInvLn10;
+    fc = fma(0x1.fe91000000000p-3, fexp2(-(0x1.dff101b829d3bp-7 * T)), fc);
+    fc = fma(0x1.805bc00000000p-1, fexp2(-(0x1.2278b1ffc7853p-10 * T)), fc);
+    fc = fma(0x1.0000000000000p+0, fexp2(-(0x1.77bb5d1fc7413p+12 * invT)), fc);
+    const double l2fc = flog2(fc);
+    const double lfc = l2fc * kLog10Of2;
     const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
     const double cco = fma(-kTroeC1, lfc, -kTroeC0);
-    const double kf = troe(kinf_f, k0_f, conc, lnfc, ntmp, cco);
-    const double kb = troe(kinf_b, k0_b, conc, lnfc, ntmp, cco);
+    const double kf = troe(kinf_f, k0_f, conc, l2fc, ntmp, cco);
+    const double kb = troe(kinf_b, k0_b, conc, l2fc, ntmp, cco);
     const double q = kf * C23 * C1 - kb * C24;
     cd1 -= q;
     cd23 -= q;
     cd24 += q;
     }
     {  // R112 (falloff)
-    const double kinf_f = 0x1.6bcc41e900000p+44 * fexp(fma(-0x1.99999a0000000p-1, lt, 0.0 * irt));
-    const double k0_f = 0x1.5af1d78b58c40p+71 * fexp(fma(-0x1.91eb860000000p+1, lt, -0x1.3a16400000000p+22 * irt));
-    const double kinf_b = 0x1.0c826847b96d8p+61 * fexp(fma(-0x1.ecae640000000p-1, lt, -0x1.bab9f60000000p+28 * irt));
-    const double k0_b = 0x1.00120dbafe4bap+88 * fexp(fma(-0x1.a6b0c80000000p+1, lt, -0x1.bfa2500000000p+28 * irt));
+    const double kinf_f = 0x1.3cb4554a4a17dp+37 * fexp2(fma(0.0, irt, -0x1.99999a0000000p-1 * lt));
+    const double k0_f = 0x1.21baa887a24cap+43 * fexp2(fma(-0x1.3a16400000000p+22, irt, -0x1.91eb860000000p+1 * lt));
+    const double kinf_b = 0x1.53c54074353b8p+52 * fexp2(fma(-0x1.bab9f60000000p+28, irt, -0x1.ecae640000000p-1 * lt));
+    const double k0_b = 0x1.36d3b559f2ae2p+58 * fexp2(fma(-0x1.bfa2500000000p+28, irt, -0x1.a6b0c80000000p+1 * lt));
     const double m_ = M18();
     const double conc = m_ > 0.0 ? m_ : p_rt;
     double fc = 0.0;
-    fc = fma(0x1.47ae140000000p-2, fexp(-(T / 0x1.3800000000000p+6)), fc);
-    fc = fma(0x1.5c28f60000000p-1, fexp(-(T / 0x1.f2c0000000000p+10)), fc);
-    fc = fma(0x1.0000000000000p+0, fexp(-(0x1.5d60000000000p+12 / T)), fc);
-    const double lnfc = flog(fc);
-    const double lfc = lnfc * kInvLn10;
+    fc = fma(0x1.47ae140000000p-2, fexp2(-(0x1.2f0a39b3764ebp-6 * T)), fc);
+    fc = fma(0x1.5c28f60000000p-1, fexp2(-(0x1.7b2446a6c9247p-11 * T)), fc);
+    fc = fma(0x1.0000000000000p+0, fexp2(-(0x1.f80aa4fb241e6p+12 * invT)), fc);
+    const double l2fc = flog2(fc);
+    const double lfc = l2fc * kLog10Of2;
     const double ntmp = fma(-kTroeN1, lfc, kTroeN0);
     const double cco = fma(-kTroeC1, lfc, -kTroeC0);
-    const double kf = troe(kinf_f, k0_f, conc, lnfc, ntmp, cco);
-    const double kb = troe(kinf_b, k0_b, conc, lnfc, ntmp, cco);
+    const double kf = troe(kinf_f, k0_f, conc, l2fc, ntmp, cco);
+    const double kb = troe(kinf_b, k0_b, conc, l2fc, ntmp, cco);
     const double q = kf * C19 * C1 - kb * C12;
     cd1 -= q;
     cd12 += q;
     cd19 -= q;
     }
     {  // R119 (third_body)
-    const double kf = 0x1.0c388d0000000p+33 * fexp(fma(0.0, lt, -0x1.3265800000000p+21 * irt));
-    const double kb = 0x1.871dcffe4cccdp+32 * fexp(fma(-0x1.fe3fd60000000p-5, lt, -0x1.2fbfbe0000000p+25 * irt));
+    const double kf = 0x1.0c388d0000000p+33 * fexp2(fma(-0x1.3265800000000p+21, irt, 0.0 * lt));
+    const double kb = 0x1.093069ac5137bp+32 * fexp2(fma(-0x1.2fbfbe0000000p+25, irt, -0x1.fe3fd60000000p-5 * lt));
     const double q = (kf * C20 - kb * C19) * M19();
     cd19 += q;
     cd20 -= q;
     }
-    f[0] = cd0 * 0x1.c051ec0000000p+4;
-    f[1] = cd1 * 0x1.020c4a0000000p+0;
-    f[2] = cd2 * 0x1.0000000000000p+5;
-    f[3] = cd3 * 0x1.0000000000000p+4;
-    f[4] = cd4 * 0x1.1020c40000000p+4;
-    f[5] = cd5 * 0x1.020c4a0000000p+1;
-    f[6] = cd6 * 0x1.20418a0000000p+4;
-    f[7] = cd7 * 0x1.0810620000000p+5;
-    f[8] = cd8 * 0x1.1020c40000000p+5;
-    f[9] = cd9 * 0x1.c028f60000000p+4;
-    f[10] = cd10 * 0x1.60147a0000000p+5;
-    f[11] = cd11 * 0x1.d049ba0000000p+4;
-    f[12] = cd12 * 0x1.e116880000000p+3;
-    f[13] = cd13 * 0x1.00ac080000000p+4;
-    f[14] = cd14 * 0x1.e06a7e0000000p+4;
-    f[15] = cd15 * 0x1.f08b440000000p+4;
-    f[16] = cd16 * 0x1.e116880000000p+4;
-    f[17] = cd17 * 0x1.f08b440000000p+4;
-    f[18] = cd18 * 0x1.d0f5c20000000p+4;
-    f[19] = cd19 * 0x1.c0d4fe0000000p+3;
-    f[20] = cd20 * 0x1.c0d4fe0000000p+3;
-    f[21] = cd21 * 0x1.c0d4fe0000000p+4;
-    f[22] = cd22 * 0x1.606a7e0000000p+5;
-    f[23] = cd23 * 0x1.a093740000000p+4;
-    f[24] = cd24 * 0x1.b0b43a0000000p+4;
-    f[25] = cd25 * 0x1.708b440000000p+5;
-    f[26] = cd26 * 0x1.687ae20000000p+5;
-    f[27] = cd27 * 0x1.e87ae20000000p+5;
-    f[28] = cd28 * 0x1.e06a7e0000000p+5;
-    f[29] = cd29 * 0x1.d85a1c0000000p+5;
-    f[30] = cd30 * 0x1.343d700000000p+6;
-    f[31] = cd31 * 0x1.f08b440000000p+5;
-    f[32] = cd32 * 0x1.343d700000000p+6;
-    f[33] = cd33 * 0x1.b43d700000000p+6;
-    f[34] = cd34 * 0x1.7035400000000p+6;
-    f[35] = cd35 * 0x1.2c2d0e0000000p+6;
-    f[36] = cd36 * 0x1.2c2d0e0000000p+6;
-    f[37] = cd37 * 0x1.7845a20000000p+5;
-    f[38] = cd38 * 0x1.7035400000000p+5;
+    cd[0] = cd0;
+    cd[1] = cd1;
+    cd[2] = cd2;
+    cd[3] = cd3;
+    cd[4] = cd4;
+    cd[5] = cd5;
+    cd[6] = cd6;
+    cd[7] = cd7;
+    cd[8] = cd8;
+    cd[9] = cd9;
+    cd[10] = cd10;
+    cd[11] = cd11;
+    cd[12] = cd12;
+    cd[13] = cd13;
+    cd[14] = cd14;
+    cd[15] = cd15;
+    cd[16] = cd16;
+    cd[17] = cd17;
+    cd[18] = cd18;
+    cd[19] = cd19;
+    cd[20] = cd20;
+    cd[21] = cd21;
+    cd[22] = cd22;
+    cd[23] = cd23;
+    cd[24] = cd24;
+    cd[25] = cd25;
+    cd[26] = cd26;
+    cd[27] = cd27;
+    cd[28] = cd28;
+    cd[29] = cd29;
+    cd[30] = cd30;
+    cd[31] = cd31;
+    cd[32] = cd32;
+    cd[33] = cd33;
+    cd[34] = cd34;
+    cd[35] = cd35;
+    cd[36] = cd36;
+    cd[37] = cd37;
+    cd[38] = cd38;
+  }
+
+  // s: [rho*Y (39), rho*T] of this lane's state; f: the right-hand side
+  static __device__ __forceinline__ void eval(const double (&s)[40], double P, double (&f)[40]) {
+    double rho = s[0];
+    rho += s[1];
+    rho += s[2];
+    rho += s[3];
+    rho += s[4];
+    rho += s[5];
+    rho += s[6];
+    rho += s[7];
+    rho += s[8];
+    rho += s[9];
+    rho += s[10];
+    rho += s[11];
+    rho += s[12];
+    rho += s[13];
+    rho += s[14];
+    rho += s[15];
+    rho += s[16];
+    rho += s[17];
+    rho += s[18];
+    rho += s[19];
+    rho += s[20];
+    rho += s[21];
+    rho += s[22];
+    rho += s[23];
+    rho += s[24];
+    rho += s[25];
+    rho += s[26];
+    rho += s[27];
+    rho += s[28];
+    rho += s[29];
+    rho += s[30];
+    rho += s[31];
+    rho += s[32];
+    rho += s[33];
+    rho += s[34];
+    rho += s[35];
+    rho += s[36];
+    rho += s[37];
+    rho += s[38];
+    const double T = s[39] / rho;
+    const double irho = 1.0 / rho;
+    double C[39], cd[39];
+    C[0] = s[0] * 0x1.245cd2eb40a46p-5;
+    C[1] = s[1] * 0x1.fbefbe72dfd0bp-1;
+    C[2] = s[2] * 0x1.0000000000000p-5;
+    C[3] = s[3] * 0x1.0000000000000p-4;
+    C[4] = s[4] * 0x1.e1a7dc7865ca7p-5;
+    C[5] = s[5] * 0x1.fbefbe72dfd0bp-2;
+    C[6] = s[6] * 0x1.c6b4f7f1539dfp-5;
+    C[7] = s[7] * 0x1.f05d519a5a4afp-6;
+    C[8] = s[8] * 0x1.e1a7dc7865ca7p-6;
+    C[9] = s[9] * 0x1.24778b96770f5p-5;
+    C[10] = s[10] * 0x1.74476f46bcafbp-6;
+    C[11] = s[11] * 0x1.1a4ebab921f45p-5;
+    C[12] = s[12] * 0x1.1072f8c06c358p-4;
+    C[13] = s[13] * 0x1.fea8d69a8976dp-5;
+    C[14] = s[14] * 0x1.10d4897263b9dp-5;
+    C[15] = s[15] * 0x1.07f7f2b66042cp-5;
+    C[16] = s[16] * 0x1.1072f8c06c358p-5;
+    C[17] = s[17] * 0x1.07f7f2b66042cp-5;
+    C[18] = s[18] * 0x1.19e6472ab1c54p-5;
+    C[19] = s[19] * 0x1.24077255ac595p-4;
+    C[20] = s[20] * 0x1.24077255ac595p-4;
+    C[21] = s[21] * 0x1.24077255ac595p-5;
+    C[22] = s[22] * 0x1.73ec922c64208p-6;
+    C[23] = s[23] * 0x1.3aa42a8f7dbc3p-5;
+    C[24] = s[24] * 0x1.2ee9ec61a82a7p-5;
+    C[25] = s[25] * 0x1.63a5ee375c49ep-6;
+    C[26] = s[26] * 0x1.6b9aa47c82749p-6;
+    C[27] = s[27] * 0x1.0c5383d6ca193p-6;
+    C[28] = s[28] * 0x1.10d4897263b9dp-6;
+    C[29] = s[29] * 0x1.157cec54345d8p-6;
+    C[30] = s[30] * 0x1.a93a23d4ccfb1p-7;
+    C[31] = s[31] * 0x1.07f7f2b66042cp-6;
+    C[32] = s[32] * 0x1.a93a23d4ccfb1p-7;
+    C[33] = s[33] * 0x1.2c755e4980b9ap-7;
+    C[34] = s[34] * 0x1.63f903191dee4p-7;
+    C[35] = s[35] * 0x1.b4a6878cdb28cp-7;
+    C[36] = s[36] * 0x1.b4a6878cdb28cp-7;
+    C[37] = s[37] * 0x1.5c57ffe4ff8dcp-6;
+    C[38] = s[38] * 0x1.63f903191dee4p-6;
+    const bool hi = T > 0x1.f400000000000p+9;
+    double cpm = 0.0;
+    if (hi) {
+      cpm = fma(s[0] * irho, 0x1.28ba9057d1783p+8 * (0x1.769c23b7952d2p+1 + T * (0x1.8610723573f79p-10 + T * (-0x1.3132c2a042109p-21 + T * (0x1.bc12905f47c3dp-34 + T * -0x1.e6a15668d1fd9p-48)))), cpm);
+      cpm = fma(s[1] * irho, 0x1.01c2d34acaff7p+13 * (0x1.4000000000000p+1 + T * (0.0 + T * (0.0 + T * (0.0 + T * 0.0)))), cpm);
+      cpm = fma(s[2] * irho, 0x1.03d2b851eb852p+8 * (0x1.d94a3c64345d0p+1 + T * (0x1.41a93860283abp-11 + T * (-0x1.0e559221b1d58p-23 + T * (0x1.384f8c6a8c0c9p-36 + T * -0x1.478e1a3741480p-50)))), cpm);
+      cpm = fma(s[3] * irho, 0x1.03d2b851eb852p+9 * (0x1.456238da3c212p+1 + T * (-0x1.ce39030add37ep-16 + T * (-0x1.aa722cde846c4p-29 + T * (0x1.4040bc0d8605ep-38 + T * -0x1.f79a23c6c03bdp-52)))), cpm);
+      cpm = fma(s[4] * irho, 0x1.e8d949731098dp+8 * (0x1.6eaf6f6ecdbe1p+1 + T * (0x1.14f4d0c23ad0ap-10 + T * (-0x1.163020518c34ep-22 + T * (0x1.0c7922a4a2d04p-35 + T * -0x1.7fe9359e80e81p-50)))), cpm);
+      cpm = fma(s[5] * irho, 0x1.01c2d350092cdp+12 * (0x1.7ee6f2e8c0486p+1 + T * (0x1.6f090d9fefacdp-11 + T * (-0x1.e3f135bb38dc3p-25 + T * (-0x1.44cea998664c2p-37 + T * 0x1.c8327bfb6303ap-50)))), cpm);
+      cpm = fma(s[6] * irho, 0x1.cd7f5ff609dd0p+8 * (0x1.5608e15011905p+1 + T * (0x1.90982cf6c7e1cp-9 + T * (-0x1.d4b3c7a091cb6p-21 + T * (0x1.081a10711c1a4p-33 + T * -0x1.cc908a9d50493p-48)))), cpm);
+      cpm = fma(s[7] * irho, 0x1.f7c6fae7924afp+7 * (0x1.0119fbbf289f6p+2 + T * (0x1.2593e46a1f9dfp-9 + T * (-0x1.5431502070c84p-21 + T * (0x1.f675fa32f618cp-34 + T * -0x1.84c80e71ea191p-47)))), cpm);
+      cpm = fma(s[8] * irho, 0x1.e8d94983d7907p+7 * (0x1.24aec4a4095f2p+2 + T * (0x1.1c2c4a4f9e3cbp-8 + T * (-0x1.8bdbdb3ee32aap-20 + T * (0x1.0243c5162bd81p-32 + T * -0x1.01e7632962eb8p-46)))), cpm);
+      cpm = fma(s[9] * irho, 0x1.28d5af07bfe7ep+8 * (0x1.8335c182ecaefp+1 + T * (0x1.7a31384b0ee0ep-10 + T * (-0x1.2e4d82c084790p-21 + T * (0x1.bffa067a23237p-34 + T * -0x1.f1fc9016ead82p-48)))), cpm);
+      cpm = fma(s[10] * irho, 0x1.79d6b356da017p+7 * (0x1.1d0828c36da88p+2 + T * (0x1.9b9696515d0c4p-9 + T * (-0x1.572bbc2739f1ap-20 + T * (0x1.07390665390c5p-32 + T * -0x1.2caa8fbeb8df6p-46)))), cpm);
+      cpm = fma(s[11] * irho, 0x1.1e860685553efp+8 * (0x1.c754a7f8012e0p+1 + T * (0x1.b682cd3e25996p-9 + T * (-0x1.665ce9ec232b2p-20 + T * (0x1.0fa472a0a4455p-32 + T * -0x1.34bd6d4c2e4e2p-46)))), cpm);
+      cpm = fma(s[12] * irho, 0x1.148494a2b9d3dp+9 * (0x1.7d330e4a459e7p+1 + T * (0x1.7bf7d0ba1fd49p-8 + T * (-0x1.09286973eb98fp-19 + T * (0x1.51e0ab53b03a6p-32 + T * -0x1.42c57f31cb480p-46)))), cpm);
+      cpm = fma(s[13] * irho, 0x1.03249374bc6a8p+9 * (0x1.aef87ad080b67p+0 + T * (0x1.4f7431802ab2bp-7 + T * (-0x1.040e35941a681p-18 + T * (0x1.750a9e764526bp-31 + T * -0x1.95a1dd4aaed6dp-45)))), cpm);
+      cpm = fma(s[14] * irho, 0x1.14e7994e1a3f4p+8 * (-0x1.29b956f9360c5p-1 + T * (0x1.d4fb29078981ep-7 + T * (-0x1.02da607522242p-17 + T * (0x1.98ffbf1c3e520p-30 + T * 0.0)))), cpm);
+      cpm = fma(s[15] * irho, 0x1.0be922424a277p+8 * (0x1.e2a9930be0dedp+1 + T * (0x1.01eee717c07fdp-7 + T * (-0x1.6488a8c446c70p-19 + T * (0x1.b1b1dcc557332p-32 + T * -0x1.7c93377953d3bp-46)))), cpm);
+      cpm = fma(s[16] * irho, 0x1.148494a2b9d3dp+8 * (0x1.34dc2b0ea1837p+2 + T * (0x1.c585f11b35bb8p-7 + T * (-0x1.31d51d0b8ec61p-18 + T * (0x1.71b57f19a838bp-31 + T * -0x1.4417f1a209b9ep-45)))), cpm);
+      cpm = fma(s[17] * irho, 0x1.0be922424a277p+8 * (0x1.df9ac1b7c5d49p+1 + T * (0x1.2279c187d63ffp-7 + T * (-0x1.1dc11f954f259p-18 + T * (0x1.154c454622351p-30 + T * -0x1.a998e1c3ec971p-44)))), cpm);
+      cpm = fma(s[18] * irho, 0x1.1e1c0389f83bep+8 * (0x1.126ca61b881bcp+2 + T * (0x1.976f0de602e4fp-7 + T * (-0x1.28366dd505844p-18 + T * (0x1.846ccefec2441p-31 + T * -0x1.7a9e6cab2d327p-45)))), cpm);
+      cpm = fma(s[19] * irho, 0x1.2863e90ff9724p+9 * (0x1.6fe28bbb5f921p+1 + T * (0x1.df4030068403dp-9 + T * (-0x1.7a3607a17a275p-20 + T * (0x1.1e1208519dbd9p-32 + T * -0x1.522e0f41fe4e3p-46)))), cpm);
+      cpm = fma(s[20] * irho, 0x1.2863e90ff9724p+9 * (0x1.256183d389aa6p+1 + T * (0x1.3120cfb16b35fp-8 + T * (-0x1.0e0906cfb21aep-19 + T * (0x1.cb7e14e4de1f4p-32 + T * -0x1.31fd42b26d354p-45)))), cpm);
+      cpm = fma(s[21] * irho, 0x1.2863e90ff9724p+8 * (0x1.049f4a5d9c3d6p+1 + T * (0x1.dfe6a5720731ep-7 + T * (-0x1.c25a4ed3d3908p-18 + T * (0x1.94aeec0be93f2p-30 + T * -0x1.1b109c49479cdp-43)))), cpm);
+      cpm = fma(s[22] * irho, 0x1.797a7aa68f4b6p+7 * (0x1.59dcf38b7d772p+2 + T * (0x1.80242581cd52bp-7 + T * (-0x1.1b9f84391e21fp-18 + T * (0x1.77e1ab96723c6p-31 + T * -0x1.7128a8eac22f7p-45)))), cpm);
+      cpm = fma(s[23] * irho, 0x1.3f5713ad5bee4p+8 * (0x1.0971c7ee6bae0p+2 + T * (0x1.86b42b3f9ab1ep-8 + T * (-0x1.3e7de3eb387edp-19 + T * (0x1.00f66a3bafde2p-31 + T * -0x1.455f2b475f023p-45)))), cpm);
+      cpm = fma(s[24] * irho, 0x1.33700096feb4ap+8 * (0x1.8224031487768p+1 + T * (0x1.52803e497ede9p-7 + T * (-0x1.3a1fef6b5677dp-18 + T * (0x1.17b98c3c9686ep-30 + T * -0x1.847bd21d4a0a4p-44)))), cpm);
+      cpm = fma(s[25] * irho, 0x1.68f59ea57214fp+7 * (0x1.a960a7be2821ep-1 + T * (0x1.b9037309df683p-6 + T * (-0x1.d1fc866c5ac12p-17 + T * (0x1.dd9eff9b15bf0p-29 + T * -0x1.80ba465eec50fp-42)))), cpm);
+      cpm = fma(s[26] * irho, 0x1.7108bfc2224eep+7 * (0x1.715ca8219cb2dp+1 + T * (0x1.4945d1eddf464p-6 + T * (-0x1.29706021400c0p-17 + T * (0x1.8b2885f927e26p-30 + T * 0.0)))), cpm);
+      cpm = fma(s[27] * irho, 0x1.10555c74751cep+7 * (0x1.f4d63f1162d3ep+0 + T * (0x1.afeec33e440d9p-6 + T * (-0x1.a7afef5c5cbc2p-17 + T * (0x1.2f294619f38b8p-29 + T * 0.0)))), cpm);
+      cpm = fma(s[28] * irho, 0x1.14e7993d5347ap+7 * (0x1.9fa9e5ed044fcp+0 + T * (0x1.9c2271983e67dp-6 + T * (-0x1.a5e2869b51b8cp-17 + T * (0x1.3498f77908422p-29 + T * 0.0)))), cpm);
+      cpm = fma(s[29] * irho, 0x1.19a1cb039ef0fp+7 * (0x1.a416232243f7ap+2 + T * (0x1.15c8f688c5d25p-6 + T * (-0x1.3894f4cfc2708p-17 + T * (0x1.e85dafb029bb6p-30 + T * 0.0)))), cpm);
+      cpm = fma(s[30] * irho, 0x1.af93d5347a5b1p+6 * (0x1.b1d47e7cb2ae1p+2 + T * (0x1.6357a14abfa13p-6 + T * (-0x1.41d2138ffbd5ap-17 + T * (0x1.aeeaddfd9036dp-30 + T * 0.0)))), cpm);
+      cpm = fma(s[31] * irho, 0x1.0be92231832fdp+7 * (0x1.e79f2823e084ep+0 + T * (0x1.d1c4ec8c3865bp-6 + T * (-0x1.bf7f44eeb209bp-17 + T * (0x1.3c57cc99adf86p-29 + T * 0.0)))), cpm);
+      cpm = fma(s[32] * irho, 0x1.af93d5347a5b1p+6 * (0x1.35bfd1e23569cp+3 + T * (0x1.34bf03e4d09f7p-6 + T * (-0x1.23a2b6ebe421cp-17 + T * (0x1.938755aa34d79p-30 + T * 0.0)))), cpm);
+      cpm = fma(s[33] * irho, 0x1.30f20e8add3e3p+6 * (0x1.ae80987683eaep+3 + T * (0x1.506bfc3c20f99p-6 + T * (-0x1.39a086249982bp-17 + T * (0x1.ad90fcb7dc7bap-30 + T * 0.0)))), cpm);
+      cpm = fma(s[34] * irho, 0x1.6949f13561e1ap+6 * (0x1.29e2cc07d5e25p+3 + T * (0x1.5f9bc8034a9e7p-6 + T * (-0x1.6528655d0532cp-17 + T * (0x1.0389665afce1bp-29 + T * 0.0)))), cpm);
+      cpm = fma(s[35] * irho, 0x1.bb2be596c82e0p+6 * (0x1.52aaa9a1cf732p+1 + T * (0x1.a5d278d079bf3p-6 + T * (-0x1.ca7bbf737701dp-17 + T * (0x1.5e4443e746d41p-29 + T * 0.0)))), cpm);
+      cpm = fma(s[36] * irho, 0x1.bb2be596c82e0p+6 * (0x1.9afc1ac324d85p+1 + T * (0x1.7e2b97bbfc789p-6 + T * (-0x1.93f65f3c91806p-17 + T * (0x1.2e9f6c132879dp-29 + T * 0.0)))), cpm);
+      cpm = fma(s[37] * irho, 0x1.618bc31df761dp+7 * (0x1.bad19f9a649abp+0 + T * (0x1.0894798c4274fp-6 + T * (-0x1.044771a062409p-17 + T * (0x1.78d3d656b5c5dp-30 + T * 0.0)))), cpm);
+      cpm = fma(s[38] * irho, 0x1.6949f127f5e85p+7 * (0x1.5be9b13415057p+1 + T * (0x1.938e119a140f7p-7 + T * (-0x1.94a69161b7cb6p-18 + T * (0x1.23bf509827fa9p-30 + T * 0.0)))), cpm);
+    } else {
+      cpm = fma(s[0] * irho, 0x1.28ba9057d1783p+8 * (0x1.a63b0c4588a05p+1 + T * (0x1.712962facc0e9p-10 + T * (-0x1.09f7a2b098bd4p-18 + T * (0x1.83ae94da0fe59p-28 + T * -0x1.58152f3dbcf65p-39)))), cpm);
+      cpm = fma(s[1] * irho, 0x1.01c2d34acaff7p+13 * (0x1.4000000000000p+1 + T * (0.0 + T * (0.0 + T * (0.0 + T * 0.0)))), cpm);
+      cpm = fma(s[2] * irho, 0x1.03d2b851eb852p+8 * (0x1.9b417ca2120e2p+1 + T * (0x1.27904dfc9e5cep-10 + T * (-0x1.3507ec57048a6p-21 + T * (0x1.6927dfded5549p-30 + T * -0x1.eda02e4e9106fp-41)))), cpm);
+      cpm = fma(s[3] * irho, 0x1.03d2b851eb852p+9 * (0x1.792495e17e34cp+1 + T * (-0x1.ad6f7594e8c10p-10 + T * (0x1.44f206ae86a97p-19 + T * (-0x1.b8960c8cd58ecp-30 + T * 0x1.b60dad5a2c8b3p-42)))), cpm);
+      cpm = fma(s[4] * irho, 0x1.e8d949731098dp+8 * (0x1.080501d23d242p+2 + T * (-0x1.a6c41f4a374cap-9 + T * (0x1.b6101eb7dedbep-18 + T * (-0x1.8e78ee8164a9cp-28 + T * 0x1.2240d8be85bd5p-39)))), cpm);
+      cpm = fma(s[5] * irho, 0x1.01c2d350092cdp+12 * (0x1.a628ed5f138bdp+1 + T * (0x1.b08222e154b9ep-11 + T * (-0x1.b52cbef7ef399p-21 + T * (-0x1.a0bbe70f69bcfp-34 + T * 0x1.d18b923980a1ep-42)))), cpm);
+      cpm = fma(s[6] * irho, 0x1.cd7f5ff609dd0p+8 * (0x1.b18409e55c0fdp+1 + T * (0x1.c7790c169fe5dp-9 + T * (-0x1.aa74d89269c73p-18 + T * (0x1.dee092cb7ea3cp-28 + T * -0x1.60c559aac818ep-39)))), cpm);
+      cpm = fma(s[7] * irho, 0x1.f7c6fae7924afp+7 * (0x1.1350a899bcaa1p+2 + T * (-0x1.373d054674594p-8 + T * (0x1.62fa28e3a8ea6p-16 + T * (-0x1.a110b0905e0fcp-26 + T * 0x1.46f1288fc5c1cp-37)))), cpm);
+      cpm = fma(s[8] * irho, 0x1.e8d94983d7907p+7 * (0x1.b1c2b0ea18373p+1 + T * (0x1.ae8552d47d093p-8 + T * (-0x1.3ee773fac0950p-23 + T * (-0x1.3de20a2d8a14dp-28 + T * 0x1.5bd5b656f46cdp-39)))), cpm);
+      cpm = fma(s[9] * irho, 0x1.28d5af07bfe7ep+8 * (0x1.a19806f262889p+1 + T * (0x1.8c58a4980b8b3p-10 + T * (-0x1.04800b08e2c9bp-18 + T * (0x1.7f9698eb1c752p-28 + T * -0x1.5c5181d89285ep-39)))), cpm);
+      cpm = fma(s[10] * irho, 0x1.79d6b356da017p+7 * (0x1.234af4f0d844dp+1 + T * (0x1.45205f5fd0b9ep-7 + T * (-0x1.5d4592f5a845bp-17 + T * (0x1.d7e00903b44b7p-28 + T * -0x1.29fb0d256cd4cp-39)))), cpm);
+      cpm = fma(s[11] * irho, 0x1.1e860685553efp+8 * (0x1.72fc7a398201dp+1 + T * (0x1.96446da0caeeep-8 + T * (-0x1.42e5a98191c27p-17 + T * (0x1.76760551ca70ep-27 + T * -0x1.41edcd30beeb1p-38)))), cpm);
+      cpm = fma(s[12] * irho, 0x1.148494a2b9d3dp+9 * (0x1.d41e76e38c2bfp+1 + T * (0x1.16bcc8dd4edc2p-9 + T * (0x1.6e4e659e7b1a3p-18 + T * (-0x1.c6cada0b83d8bp-28 + T * 0x1.5b0478af296dap-39)))), cpm);
+      cpm = fma(s[13] * irho, 0x1.03249374bc6a8p+9 * (0x1.8eb734b51372ap-1 + T * (0x1.1e568242bae5ap-6 + T * (-0x1.d2fa819a83265p-16 + T * (0x1.05f7c9c3f6e46p-25 + T * -0x1.aea1e766ae70ep-37)))), cpm);
+      cpm = fma(s[14] * irho, 0x1.14e7994e1a3f4p+8 * (0x1.591f1645bca2bp+1 + T * (0x1.42d6f412ede0ap-8 + T * (0x1.bcabddd64bccbp-21 + T * (-0x1.2e935feb740d0p-31 + T * -0x1.bdf8fddb1e1b3p-42)))), cpm);
+      cpm = fma(s[15] * irho, 0x1.0be922424a277p+8 * (0x1.0d9817b95a294p+1 + T * (0x1.d8f25f83733c9p-8 + T * (0x1.664240277b618p-18 + T * (-0x1.fafcbebd8fc7ap-28 + T * 0x1.241dc474f011fp-39)))), cpm);
+      cpm = fma(s[16] * irho, 0x1.148494a2b9d3dp+8 * (0x1.7668f4b61fe22p+0 + T * (0x1.fbbab674c6a67p-7 + T * (0x1.83ec5aa4cd9a5p-18 + T * (-0x1.b03012a1e9c75p-27 + T * 0x1.42bad76692a1bp-38)))), cpm);
+      cpm = fma(s[17] * irho, 0x1.0be922424a277p+8 * (0x1.61e03e841f33fp+1 + T * (0x1.876a6f2bff2ecp-7 + T * (-0x1.ef1c02ca6da7ap-18 + T * (0x1.0a0bd49f52b27p-29 + T * 0.0)))), cpm);
+      cpm = fma(s[18] * irho, 0x1.1e1c0389f83bep+8 * (0x1.13932d6ece13fp+2 + T * (-0x1.122932b551339p-8 + T * (0x1.a0f98cacccd65p-15 + T * (-0x1.014b347d2de42p-24 + T * 0x1.95791def45bc0p-36)))), cpm);
+      cpm = fma(s[19] * irho, 0x1.2863e90ff9724p+9 * (0x1.e19f746480de1p+1 + T * (0x1.fbf7d158743a2p-11 + T * (0x1.771ffa66e83e0p-19 + T * (-0x1.08a1f3bb46844p-28 + T * 0x1.daf7390cac908p-40)))), cpm);
+      cpm = fma(s[20] * irho, 0x1.2863e90ff9724p+9 * (0x1.0cb5ee035346ap+2 + T * (-0x1.36326518bab75p-9 + T * (0x1.14409b5702698p-17 + T * (-0x1.cb9b5a07323d1p-28 + T * 0x1.1179431daea17p-39)))), cpm);
+      cpm = fma(s[21] * irho, 0x1.2863e90ff9724p+8 * (0x1.fac71d356ff96p+1 + T * (-0x1.f0244a6c1abf8p-8 + T * (0x1.defb3b4522b25p-15 + T * (-0x1.2908fcd07cb16p-24 + T * 0x1.dac91dbd28c88p-36)))), cpm);
+      cpm = fma(s[22] * irho, 0x1.797a7aa68f4b6p+7 * (0x1.2eaf76e6106abp+2 + T * (-0x1.a28ce427d2efep-9 + T * (0x1.8ec0772eb57cep-15 + T * (-0x1.ed90d262d7aa3p-25 + T * 0x1.81d0f2a50dc3bp-36)))), cpm);
+      cpm = fma(s[23] * irho, 0x1.3f5713ad5bee4p+8 * (0x1.9e0b72c73f3bap-1 + T * (0x1.7ec17f28e481ap-6 + T * (-0x1.29f09105c533cp-15 + T * (0x1.e14c5845a203fp-26 + T * -0x1.2b17c43e837e8p-37)))), cpm);
+      cpm = fma(s[24] * irho, 0x1.33700096feb4ap+8 * (0x1.9b3219c31fa4ep+1 + T * (0x1.8d17f1df63fcdp-10 + T * (0x1.b2e198409699cp-16 + T * (-0x1.3339cad4b897fp-25 + T * 0x1.02dedc9720552p-36)))), cpm);
+      cpm = fma(s[25] * irho, 0x1.68f59ea57214fp+7 * (0x1.15498ca66c0ffp+1 + T * (0x1.5d97e24e2d237p-6 + T * (-0x1.acff45bbb4ce8p-18 + T * (-0x1.018f4704e51a1p-33 + T * 0.0)))), cpm);
+      cpm = fma(s[26] * irho, 0x1.7108bfc2224eep+7 * (0x1.74e62ad7441f1p+1 + T * (0x1.4d3151fd3ae33p-6 + T * (-0x1.4206a99644805p-17 + T * (0x1.1d280428550a3p-29 + T * -0x1.81d4b92e2b024p-43)))), cpm);
+      cpm = fma(s[27] * irho, 0x1.10555c74751cep+7 * (0x1.a1236b2999ac6p+1 + T * (0x1.6bf6efabb70d0p-6 + T * (-0x1.053d7af963800p-17 + T * (-0x1.0983bf6c7b32ap-32 + T * 0x1.fccf7c342220dp-42)))), cpm);
+      cpm = fma(s[28] * irho, 0x1.14e7993d5347ap+7 * (0x1.8b509ebe71954p+1 + T * (0x1.4dd7288f4e0dcp-6 + T * (-0x1.cb8bccb7708ecp-18 + T * (-0x1.905318e65fa7ep-31 + T * 0x1.3c73807617e5ap-41)))), cpm);
+      cpm = fma(s[29] * irho, 0x1.19a1cb039ef0fp+7 * (0x1.f8932e301419fp+1 + T * (0x1.8ed7fda31b87fp-6 + T * (-0x1.15d2c05f70557p-16 + T * (0x1.3b1ac1221623bp-28 + T * -0x1.75919a0a7a109p-42)))), cpm);
+      cpm = fma(s[30] * irho, 0x1.af93d5347a5b1p+6 * (0x1.1aeafbb6f016bp+1 + T * (0x1.2e2f3583b7b37p-5 + T * (-0x1.da0f43874b909p-16 + T * (0x1.8da5a743c3ff8p-27 + T * -0x1.156fbca566d5ep-39)))), cpm);
+      cpm = fma(s[31] * irho, 0x1.0be92231832fdp+7 * (0x1.944a57bd00511p+1 + T * (0x1.904da5c0bd76ap-6 + T * (-0x1.22e96d05b2a72p-17 + T * (-0x1.04f1d14f0a606p-34 + T * 0x1.eb57bcad2a681p-42)))), cpm);
+      cpm = fma(s[32] * irho, 0x1.af93d5347a5b1p+6 * (0x1.43b4ccbb5a08bp+1 + T * (0x1.5b72262f8c012p-5 + T * (-0x1.393c692a25e41p-15 + T * (0x1.1e48c0f339dd7p-26 + T * -0x1.a134f58b4c605p-39)))), cpm);
+      cpm = fma(s[33] * irho, 0x1.30f20e8add3e3p+6 * (0x1.ff146e7701135p+0 + T * (0x1.ddc767e8598bbp-5 + T * (-0x1.d01ba1f45fe82p-15 + T * (0x1.be59e2473ce95p-26 + T * -0x1.4fc21504096eap-38)))), cpm);
+      cpm = fma(s[34] * irho, 0x1.6949f13561e1ap+6 * (0x1.bd5b92377a95ap+1 + T * (0x1.4a193dd18d4a0p-5 + T * (-0x1.14ea6e782db5ap-15 + T * (0x1.cda868a48a234p-27 + T * -0x1.33a7850078c3cp-39)))), cpm);
+      cpm = fma(s[35] * irho, 0x1.bb2be596c82e0p+6 * (0x1.4c9a25905d5adp+2 + T * (0x1.043e3563c7cd2p-6 + T * (0x1.7b9c7c4eeb122p-22 + T * (-0x1.a380b7b5a0d5cp-28 + T * 0x1.11f64e1eafecap-39)))), cpm);
+      cpm = fma(s[36] * irho, 0x1.bb2be596c82e0p+6 * (0x1.853c57a9e00dcp+2 + T * (0x1.a5f2ba8881b83p-7 + T * (0x1.125dfa29a9147p-19 + T * (-0x1.a34b96bfa03c3p-28 + T * 0x1.fa265e4f865bap-40)))), cpm);
+      cpm = fma(s[37] * irho, 0x1.618bc31df761dp+7 * (0x1.07283f191a834p+2 + T * (0x1.ee0b28e595de3p-8 + T * (0x1.fa7422129ff3ep-19 + T * (-0x1.72393312daf39p-28 + T * 0x1.99df4e016bdccp-40)))), cpm);
+      cpm = fma(s[38] * irho, 0x1.6949f127f5e85p+7 * (0x1.6f7bbd0fc0676p+0 + T * (0x1.0ba76a4703902p-6 + T * (-0x1.648a6dfc430a3p-17 + T * (0x1.c87ae70772a4cp-29 + T * -0x1.c4cf5e9412c52p-42)))), cpm);
+    }
+    rates(C, T, P, cd);
+    f[0] = cd[0] * 0x1.c051ec0000000p+4;
+    f[1] = cd[1] * 0x1.020c4a0000000p+0;
+    f[2] = cd[2] * 0x1.0000000000000p+5;
+    f[3] = cd[3] * 0x1.0000000000000p+4;
+    f[4] = cd[4] * 0x1.1020c40000000p+4;
+    f[5] = cd[5] * 0x1.020c4a0000000p+1;
+    f[6] = cd[6] * 0x1.20418a0000000p+4;
+    f[7] = cd[7] * 0x1.0810620000000p+5;
+    f[8] = cd[8] * 0x1.1020c40000000p+5;
+    f[9] = cd[9] * 0x1.c028f60000000p+4;
+    f[10] = cd[10] * 0x1.60147a0000000p+5;
+    f[11] = cd[11] * 0x1.d049ba0000000p+4;
+    f[12] = cd[12] * 0x1.e116880000000p+3;
+    f[13] = cd[13] * 0x1.00ac080000000p+4;
+    f[14] = cd[14] * 0x1.e06a7e0000000p+4;
+    f[15] = cd[15] * 0x1.f08b440000000p+4;
+    f[16] = cd[16] * 0x1.e116880000000p+4;
+    f[17] = cd[17] * 0x1.f08b440000000p+4;
+    f[18] = cd[18] * 0x1.d0f5c20000000p+4;
+    f[19] = cd[19] * 0x1.c0d4fe0000000p+3;
+    f[20] = cd[20] * 0x1.c0d4fe0000000p+3;
+    f[21] = cd[21] * 0x1.c0d4fe0000000p+4;
+    f[22] = cd[22] * 0x1.606a7e0000000p+5;
+    f[23] = cd[23] * 0x1.a093740000000p+4;
+    f[24] = cd[24] * 0x1.b0b43a0000000p+4;
+    f[25] = cd[25] * 0x1.708b440000000p+5;
+    f[26] = cd[26] * 0x1.687ae20000000p+5;
+    f[27] = cd[27] * 0x1.e87ae20000000p+5;
+    f[28] = cd[28] * 0x1.e06a7e0000000p+5;
+    f[29] = cd[29] * 0x1.d85a1c0000000p+5;
+    f[30] = cd[30] * 0x1.343d700000000p+6;
+    f[31] = cd[31] * 0x1.f08b440000000p+5;
+    f[32] = cd[32] * 0x1.343d700000000p+6;
+    f[33] = cd[33] * 0x1.b43d700000000p+6;
+    f[34] = cd[34] * 0x1.7035400000000p+6;
+    f[35] = cd[35] * 0x1.2c2d0e0000000p+6;
+    f[36] = cd[36] * 0x1.2c2d0e0000000p+6;
+    f[37] = cd[37] * 0x1.7845a20000000p+5;
+    f[38] = cd[38] * 0x1.7035400000000p+5;
     double tmp = 0.0;
     if (hi) {
       tmp = fma(-(0x1.28ba9057d1783p+8 * (T * (0x1.769c23b7952d2p+1 + T * (0x1.8610723573f79p-11 + T * (-0x1.96ee58c9aaf66p-23 + T * (0x1.bc12905f47c3dp-36 + T * -0x1.854ddeba4197bp-50)))) + -0x1.cd661b089a027p+9)), f[0], tmp);

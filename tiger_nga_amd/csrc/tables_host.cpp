@@ -3,6 +3,7 @@
 #include "tables_host.h"
 
 #include <algorithm>
+#include <cmath>
 #include <utility>
 #include <vector>
 
@@ -14,6 +15,9 @@ static int seterr(std::string* err, const char* msg) {
   if (err) *err = msg;
   return -1;
 }
+
+// A of A T^b exp(e / (R T)) for the temperature in units of kTUnit
+static double scaled_A(const double* k) { return (double)(k[0] * powl((long double)kTUnit, k[1])); }
 
 static int seterr(std::string* err, const std::string& msg) { return seterr(err, msg.c_str()); }
 
@@ -79,8 +83,8 @@ int build_table_blob(const tgr_mech_tables* t, std::vector<char>& blob, tgr_mech
       const tgr_rxn& x = t->rxn[order[g]];
       if (x.nr > 3 || x.np > 3) return seterr(err, "more than three concentration factors");
       for (int q = 0; q < 3; ++q) {
-        D(rx + q * kRow + dl) = x.f[q];
-        D(rx + (3 + q) * kRow + dl) = x.rev ? x.b[q] : 0.0;
+        D(rx + q * kRow + dl) = q ? x.f[q] : scaled_A(x.f);
+        D(rx + (3 + q) * kRow + dl) = x.rev ? (q ? x.b[q] : scaled_A(x.b)) : 0.0;
       }
       auto put = [](int& w, int q, int v) { w = (w & ~(255 << (8 * q))) | (v << (8 * q)); };
       for (int q = 0; q < x.nr; ++q) put(i0, q, x.reac[q]);
@@ -90,22 +94,25 @@ int build_table_blob(const tgr_mech_tables* t, std::vector<char>& blob, tgr_mech
         put(i0, 3, x.m);
       }
       if (x.kind == 2) {
-        if (g >= 64) return seterr(err, "more than 64 fall-off reactions");
+        if (g >= 32) return seterr(err, "more than 32 fall-off reactions");
         i1 |= 1 << 24;
-        const size_t f = L.fo + dl;
-        int kinds = 0;
-        for (int q = 0; q < 3; ++q) {
-          D(f + q * kRow) = x.f0[q];
-          D(f + (3 + q) * kRow) = x.rev ? x.b0[q] : 0.0;
-          if (q < x.nfc) {
-            D(f + (6 + q) * kRow) = x.fc_c[q];
-            // exp(-T / d) as exp(-(1/d) T); exp(-d / T) as exp(-d (1/T))
-            D(f + (9 + q) * kRow) = x.fc_kind[q] ? x.fc_d[q] : 1.0 / x.fc_d[q];
-            kinds |= (x.fc_kind[q] & 1) << q;
-          }
-        }
         if (x.m >= t->n_third) return seterr(err, "third-body index out of range");
-        I(L.fo + 12 * kRow + il) = kinds | (x.m >= 0 ? x.m : kZero) << 8;
+        for (int dir = 0; dir < (x.rev ? 2 : 1); ++dir) {
+          const size_t f = L.fo + dl + dir * 32 * 8;
+          int kinds = 0;
+          for (int q = 0; q < 3; ++q) {
+            const double* k0 = dir ? x.b0 : x.f0;
+            D(f + q * kRow) = q ? k0[q] : scaled_A(k0);
+            if (q < x.nfc) {
+              D(f + (3 + q) * kRow) = x.fc_c[q];
+              // exp(-T / d) as 2^(-(log2(e) / d) T); exp(-d / T) as 2^(-(log2(e) d) (1/T))
+              const long double l2e = 1.442695040888963407359924681001892137L;
+              D(f + (6 + q) * kRow) = (double)(x.fc_kind[q] ? l2e * x.fc_d[q] : l2e / x.fc_d[q]);
+              kinds |= (x.fc_kind[q] & 1) << q;
+            }
+          }
+          I(L.fo + 9 * kRow + il + dir * 32 * 4) = kinds | (x.m >= 0 ? x.m : kZero) << 8 | 1 << 16;
+        }
       }
       if (x.rev) i1 |= 1 << 25;
     }

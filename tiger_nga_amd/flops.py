@@ -2,7 +2,7 @@
 
 Convention: add, sub, mul, div = 1 flop; fma = 2; compares, selects and
 data movement = 0; exp and log count the operations of the project's own FP64
-implementations (tiger_nga_amd/csrc/fp64_math.h): exp 33, log 32.  Per cell
+implementations (tiger_nga_amd/csrc/fp64_math.h, 2^x and log2): exp 25, log 23.  Per cell
 step:
 
   F = (nfe + nfe_dq) * F_rhs + nlu * F_lu + nni * F_solve + nfe_dq * 3 neq + nst * F_step
@@ -19,10 +19,10 @@ step:
 """
 from __future__ import annotations
 
-EXP = 33.0
-LOG = 32.0
+EXP = 25.0
+LOG = 23.0
 ARRH = 1 + 2 + EXP + 1            # e*irt, fma(b, lt, .), exp, A*
-TROE = 2 + (LOG + 2) + 3 + (2 + 1 + EXP) + 4  # one direction of GETLINDRATECOEFF
+TROE = 2 + (LOG + 2) + 2 + (1 + 2 + 1 + 1 + EXP) + 4  # one direction of GETLINDRATECOEFF
 
 
 def rhs_flops(info: dict) -> float:

@@ -337,3 +337,26 @@ def test_four_waves_per_simd_step_matches_two(oracle, torch_dev):
     rho = RHO_[..., None]
     ew = (np.abs(rho * (S4[..., sp] - SC_o[..., sp])) / (1e-6 * np.abs(rho * SC_o[..., sp]) + 1e-12)).max(axis=3)
     assert np.sort(ew.ravel())[-3] <= 1.0 and ew.max() <= 10.0
+
+
+@pytest.mark.parametrize("mech,n", [("h2", 1), ("h2", 65), ("gri30", 64 * 256 - 1), ("gri30", 64 * 256),
+                                    ("ethyred", 64 * 256 + 63)])
+def test_batched_rate_mappings_agree(mech, n, torch_dev):
+    """Batched rates one state per lane and one per wavefront, on both sides of
+    the state count where the default changes.  Bound: the exponents of the rate
+    constants, up to 60, carry a few roundings each (60 x 4 x 1.1e-16)."""
+    torch = torch_dev
+    from tiger_nga_amd.finitechem import FiniteChem
+    _, Y, T, rho, P, _ = inputs.states(mech, n=n, seed=41)
+    fc = FiniteChem(mech)
+    sol = torch.from_numpy(np.ascontiguousarray(inputs.packed_state(Y, T, rho).T)).cuda()
+    C = (sol[:-1] / torch.from_numpy(fc.molar_mass).cuda()[:, None]).contiguous()
+    Td = torch.from_numpy(T).cuda()
+    got = []
+    for mapping in (1, 0):
+        fc.set_option("rhs_mapping", mapping)
+        got.append((fc.compute_rhs(sol, P), fc.prodrates(C, Td, torch.full_like(Td, P))))
+    fc.close()
+    for a, b in zip(*got):
+        assert torch.isfinite(b).all()
+        assert float((a - b).norm() / b.norm()) <= 3e-14

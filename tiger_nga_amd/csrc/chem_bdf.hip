@@ -9,10 +9,6 @@
 
 #include "bdf_wave.h"
 #include "chem_kernels.h"
-#include "lane_rhs_dme39.h"
-#include "lane_rhs_ethyred.h"
-#include "lane_rhs_gri30.h"
-#include "lane_rhs_h2.h"
 
 namespace tgr {
 
@@ -113,21 +109,6 @@ __global__ __launch_bounds__(kBlock) void rhs_kernel(DevMech m, int64_t n, doubl
     const double v = rhs_wave<NEQ>((tchar*)tab_s, *(TGR_LDS RhsLds<NEQ>*)&rl[w], m.tmid, yv, p_gp);
     if (lane < NEQ) f[lane * n + c] = v;
   }
-}
-
-// Lane per state: each lane evaluates a whole right-hand side with the
-// generated code of the mechanism (lane_rhs_<mech>.h); component-major
-// arrays, so lane c's loads and stores of component k are coalesced.
-template <int NEQ>
-__global__ __launch_bounds__(64) void rhs_lanes_kernel(int64_t n, double p_gp, const double* y, double* f) {
-  const int64_t c = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (c >= n) return;
-  double s[NEQ], o[NEQ];
-#pragma unroll
-  for (int k = 0; k < NEQ; ++k) s[k] = y[k * n + c];
-  LaneRhs<NEQ>::eval(s, p_gp, o);
-#pragma unroll
-  for (int k = 0; k < NEQ; ++k) f[k * n + c] = o[k];
 }
 
 // Temperature from mixture enthalpy, lane per state (no routine in the
@@ -274,19 +255,6 @@ extern "C" int tgr_launch_prodrates(const DevMech* m, int64_t n, const double* C
     case 37: hipLaunchKernelGGL(prodrates_kernel<37>, g, b, 0, s, *m, n, C, T, P, cdot); break;
     case 40: hipLaunchKernelGGL(prodrates_kernel<40>, g, b, 0, s, *m, n, C, T, P, cdot); break;
     case 46: hipLaunchKernelGGL(prodrates_kernel<46>, g, b, 0, s, *m, n, C, T, P, cdot); break;
-    default: return -1;
-  }
-  return hipGetLastError() == hipSuccess ? 0 : -2;
-}
-
-extern "C" int tgr_launch_rhs_lanes(int neq, int64_t n, double p_gp, const double* y, double* f, hipStream_t s) {
-  if (n <= 0) return 0;
-  const dim3 grid((unsigned)((n + 63) / 64));
-  switch (neq) {
-    case 10: hipLaunchKernelGGL(rhs_lanes_kernel<10>, grid, dim3(64), 0, s, n, p_gp, y, f); break;
-    case 37: hipLaunchKernelGGL(rhs_lanes_kernel<37>, grid, dim3(64), 0, s, n, p_gp, y, f); break;
-    case 40: hipLaunchKernelGGL(rhs_lanes_kernel<40>, grid, dim3(64), 0, s, n, p_gp, y, f); break;
-    case 46: hipLaunchKernelGGL(rhs_lanes_kernel<46>, grid, dim3(64), 0, s, n, p_gp, y, f); break;
     default: return -1;
   }
   return hipGetLastError() == hipSuccess ? 0 : -2;

@@ -271,6 +271,17 @@ size_t step_shape(const tgr_chem* c, int64_t ncell, int* grid, bool* lanes) {
   return (size_t)*grid * tgr_step_block_waves() * c->neq * 64 * sizeof(double);
 }
 
+// Mapping of the batched rates of n states (option "rhs_mapping").  One state
+// per lane costs the time of one wave's 10,000 to 20,000 instructions however
+// few states there are, and pays once every CU has a wave (16,384 states on 256
+// CUs): rates of GRI-3.0 by wave / by lane 7 / 36 us at 256 states, 18 / 37 at
+// 8,192, 33 / 37 at 16,384, 54 / 38 at 32,768, 362 / 138 at 262,144; EthyRedF
+// 18 / 23, 31 / 23, 54 / 25, 352 / 92.  H2's rates are short: by lane always
+// (7 / 7 us at one state, 213 / 19 at 262,144).
+bool rates_by_lane(const tgr_chem* c, int64_t n) {
+  return c->rhs_lanes && (c->neq <= 10 || n >= (int64_t)64 * c->n_cu);
+}
+
 // Layout of an external scratch block (tgr_chem_source_chemistry_device_noalloc):
 // the work counter at byte 0, the counter totals at byte 64, the per-wave
 // Jacobian workspace from byte 256.
@@ -912,7 +923,9 @@ int tgr_chem_prodrates_device(tgr_chem* c, int64_t n, const double* C, const dou
                               double* cdot, void* stream) {
   if (!c || (n > 0 && (!C || !T || !P || !cdot))) return fail(TGR_E_ARG, "NULL argument");
   if (n < 0 || n > 0x7fffffff) return fail(TGR_E_ARG, "bad n");
-  if (tgr_launch_prodrates(&c->dm, n, C, T, P, cdot, (hipStream_t)stream)) return fail(TGR_E_HIP, "launch");
+  const int rc = rates_by_lane(c, n) ? tgr_launch_prodrates_lanes(c->neq, n, C, T, P, cdot, (hipStream_t)stream)
+                                     : tgr_launch_prodrates(&c->dm, n, C, T, P, cdot, (hipStream_t)stream);
+  if (rc) return fail(TGR_E_HIP, "launch");
   return 0;
 }
 
@@ -1014,8 +1027,8 @@ int tgr_chem_temperature_device(tgr_chem* c, int64_t n, const double* Y, const d
 int tgr_chem_rhs_device(tgr_chem* c, int64_t n, double p_gp, const double* sol, double* rhs, void* stream) {
   if (!c || (n > 0 && (!sol || !rhs))) return fail(TGR_E_ARG, "NULL argument");
   if (n < 0 || n > 0x7fffffff) return fail(TGR_E_ARG, "bad n");
-  const int rc = c->rhs_lanes ? tgr_launch_rhs_lanes(c->neq, n, p_gp, sol, rhs, (hipStream_t)stream)
-                              : tgr_launch_rhs(&c->dm, n, p_gp, sol, rhs, (hipStream_t)stream);
+  const int rc = rates_by_lane(c, n) ? tgr_launch_rhs_lanes(c->neq, n, p_gp, sol, rhs, (hipStream_t)stream)
+                                     : tgr_launch_rhs(&c->dm, n, p_gp, sol, rhs, (hipStream_t)stream);
   if (rc) return fail(TGR_E_HIP, "launch");
   return 0;
 }

@@ -20,6 +20,8 @@ int tgr_launch_temperature(const tgr::DevMech* m, int64_t n, const double* Y, co
                            double* T, int* iters, hipStream_t s);
 int tgr_launch_props(const tgr::PropsParams* p, int neq, int lane_map, hipStream_t s);
 int tgr_launch_rhs_lanes(int neq, int64_t n, double p_gp, const double* y, double* f, hipStream_t s);
+int tgr_launch_prodrates_lanes(int neq, int64_t n, const double* C, const double* T, const double* P, double* cdot,
+                               hipStream_t s);
 int tgr_surr_occupancy(int neq, int adaptive);
 // waves per workgroup of the guided-solve kernel (its workspace share per block)
 int tgr_surr_block_waves(void);

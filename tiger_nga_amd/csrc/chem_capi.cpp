@@ -136,26 +136,26 @@ int build_tables(tgr_chem* c) {
   // transport table: mucoeff, kOverEps, W (64 lanes each), then the Wilke
   // pair factors A(k,j) = (1/sqrt 8) (1 + W_k/W_j)^-1/2 and
   // B(k,j) = (W_j/W_k)^1/4 at [j][k] (finitechem.f90:376-380); then, for the
-  // thread-per-cell kernel, (sqrt A(k,j), sqrt A(k,j) B(k,j)) at [k][j], zero
-  // for j = k (the reference's sum skips it)
+  // thread-per-cell kernel, A at [k / part][j][k % part] with 1/4 on the diagonal
+  // (0 past the species), W_k^1/4 and W_k^1/2
   const int n = c->t->nsp;
   const size_t pair = 192 + 2 * (size_t)n * 64;
-  std::vector<double> pt(pair + 2 * (size_t)n * n, 0.0);
+  const int part = tgr::kPropsPart(n);
+  const size_t w14 = pair + (size_t)tgr::kPropsParts(n) * n * part;
+  std::vector<double> pt(w14 + 2 * (size_t)n, 0.0);
   for (int k = 0; k < n; ++k) {
     pt[k] = c->t->mucoeff[k];
     pt[64 + k] = c->t->koveps[k];
     pt[128 + k] = c->t->W[k];
+    pt[w14 + k] = std::pow(c->t->W[k], 0.25);
+    pt[w14 + n + k] = std::sqrt(c->t->W[k]);
   }
   for (int k = n; k < 64; ++k) pt[128 + k] = 1.0;
   for (int j = 0; j < n; ++j)
     for (int k = 0; k < n; ++k) {
       pt[192 + (size_t)j * 64 + k] = (1.0 / std::sqrt(8.0)) * std::pow(1.0 + (c->t->W[k] / c->t->W[j]), -0.5);
       pt[192 + (size_t)n * 64 + (size_t)j * 64 + k] = std::pow(c->t->W[j] / c->t->W[k], 0.25);
-      if (j != k) {
-        const double sa = std::sqrt(pt[192 + (size_t)j * 64 + k]);
-        pt[pair + 2 * ((size_t)k * n + j)] = sa;
-        pt[pair + 2 * ((size_t)k * n + j) + 1] = sa * pt[192 + (size_t)n * 64 + (size_t)j * 64 + k];
-      }
+      pt[pair + ((size_t)(k / part) * n + j) * part + k % part] = j == k ? 0.25 : pt[192 + (size_t)j * 64 + k];
     }
   HIP_TRY(hipMalloc(&c->d_props, pt.size() * sizeof(double)));
   HIP_TRY(hipMemcpy(c->d_props, pt.data(), pt.size() * sizeof(double), hipMemcpyHostToDevice));

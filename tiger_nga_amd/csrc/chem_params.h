@@ -125,9 +125,19 @@ struct DiffParams {
   double w_h2o, w_co, w_co2, w_ch4;
 };
 
+// Species whose Wilke sums the thread-per-cell properties kernel accumulates in
+// one pass (three sums each in registers, two waves per SIMD; the scalar
+// registers hold two columns of 18), an even number; the pair matrix of that
+// kernel is stored part by part.
+__host__ __device__ constexpr int kPropsParts(int nsp) { return (nsp + 17) / 18; }
+__host__ __device__ constexpr int kPropsPart(int nsp) {
+  return ((nsp + kPropsParts(nsp) - 1) / kPropsParts(nsp) + 1) / 2 * 2;
+}
+
 // Transport / equation-of-state properties of a whole Fortran-layout block.
 // ptab: mucoeff[64], kOverEps[64], W[64], then A[nsp][64] and B[nsp][64]
-// (pair factors, row j, lane k).
+// (pair factors, row j, lane k), then for the thread-per-cell kernel A by parts
+// of the species k, [part][j][kPropsPart], W^1/4[nsp] and W^1/2[nsp].
 struct PropsParams {
   const double* ptab;
   const char* mtab;  // mechanism table block (thermo rows)

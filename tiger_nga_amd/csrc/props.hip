@@ -14,12 +14,14 @@
 //    masses only, (1/sqrt 8)(1 + W_k/W_j)^-1/2 and (W_j/W_k)^1/4, precomputed
 //    on the host;
 //  * props_lane_kernel: one thread per cell, every lane busy in the double
-//    sum.  With a = (1/sqrt 8)(1 + W_k/W_j)^-1/2 and b = (W_j/W_k)^1/4 the
-//    reference's pair term a (1 + sqrt(eta_k/eta_j) b)^2 is written
-//    (sqrt(a) + u sqrt(a) b)^2, u = sqrt(eta_k) / sqrt(eta_j), so each pair
-//    costs a product, two fused multiply-adds and a weight product; the
-//    factor pairs (sqrt a, sqrt a b) sit in LDS as one 16-byte broadcast read
-//    per pair, with zeros on the diagonal (the reference skips j = k).
+//    sum.  With g_k = W_k^1/4 / sqrt(eta_k) and a_kj = (1/sqrt 8)(1 + W_k/W_j)^-1/2
+//    the reference's pair term a_kj (1 + sqrt(eta_k/eta_j) (W_j/W_k)^1/4)^2 is
+//    a_kj (g_k + g_j)^2 / g_k^2, so that species k's sum over j is
+//      (g_k^2 sum_j a_kj y_j + 2 g_k sum_j a_kj y_j g_j + sum_j a_kj y_j g_j^2) / g_k^2:
+//    three products of one constant matrix with a lane's vectors, three fused
+//    multiply-adds a pair whose matrix element comes from a scalar register.
+//    The diagonal a_kk = 1/4 makes j = k the reference's own term (its phi is
+//    1), and with y_j = Y_j / W_j the factor W_mix cancels.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -107,115 +109,171 @@ __global__ __launch_bounds__(256) void props_kernel(PropsParams p) {
   }
 }
 
-// One thread per cell (the block's cells in their storage order, so every
-// field access is coalesced).  ise / yw: 1/sqrt(eta_j) and Y_j W_mix / W_j of
-// all species in registers; the loop over k keeps one species' eta, cp and
-// pair sums at a time.  Sums run in species order (the wave kernel's are
-// tree reductions) and eta = mucoeff sqrt(T) den / num takes omegamu's
-// numerator and denominator with one division: rounding-level differences.
+// N doubles (even) at a wave-uniform address into scalar registers
+typedef double d8 __attribute__((ext_vector_type(8), aligned(8)));
+typedef double d4 __attribute__((ext_vector_type(4), aligned(8)));
+typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
+
+template <int N>
+__device__ __forceinline__ void load_row(double (&m)[N], const TGR_CONST double* r) {
+  constexpr int n8 = N / 8 * 8, n4 = n8 + (N - n8) / 4 * 4;
+#pragma unroll
+  for (int i = 0; i < n8; i += 8) {
+    const d8 v = *(const TGR_CONST d8*)(r + i);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) m[i + e] = v[e];
+  }
+#pragma unroll
+  for (int i = n8; i < n4; i += 4) {
+    const d4 v = *(const TGR_CONST d4*)(r + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m[i + e] = v[e];
+  }
+#pragma unroll
+  for (int i = n4; i < N; i += 2) {
+    const d2 v = *(const TGR_CONST d2*)(r + i);
+    m[i] = v[0];
+    m[i + 1] = v[1];
+  }
+}
+
+
+// Threads of its workgroup: its g_k take 8 nsp bytes of LDS a thread, and eight
+// waves on a CU need the LDS of two workgroups of four waves.
 template <int NEQ>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void props_lane_kernel(PropsParams p) {
-  constexpr int nsp = NEQ - 1;
+constexpr int props_block() {
+  return 2 * (256 * 8 + 96) * (NEQ - 1) <= 160 * 1024 ? 256 : 128;
+}
+
+// One thread per cell (the block's cells in their storage order, so every
+// field access is coalesced).  A first loop over the species forms W_mix, the
+// conductivity sums and g (to LDS); then, for a part of the species k at a
+// time, a loop over j adds column j of the pair matrix times y_j, y_j g_j and
+// y_j g_j^2 to the part's sums: 3 x 18 independent chains (GRI-3.0), the next
+// column's scalar loads under way.  Sums run in species order (the wave
+// kernel's are tree reductions) and eta = mucoeff sqrt(T) den / num takes
+// omegamu's numerator and denominator with one division: rounding-level
+// differences.
+template <int NEQ>
+__global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per_eu(2))) void props_lane_kernel(
+    PropsParams p) {
+  constexpr int nsp = NEQ - 1, kBlock = props_block<NEQ>(), kPart = kPropsPart(nsp);
   constexpr TabLayout L = tab_layout<NEQ>();
-  constexpr int kPair = 192 + 2 * nsp * 64;  // [k][j] (sqrt a, sqrt a b), host table
-  __shared__ double2 pair[nsp * nsp];
-  const TGR_GLOBAL double* src = (const TGR_GLOBAL double*)(p.ptab + kPair);
-  for (int i = threadIdx.x; i < nsp * nsp; i += blockDim.x) {
-    const double a = src[2 * i], b = src[2 * i + 1];
-    pair[i].x = a;
-    pair[i].y = b;
+  constexpr int kPair = 192 + 2 * nsp * 64;
+  __shared__ double gs[nsp][kBlock];
+  __shared__ __attribute__((aligned(16))) double cps[nsp * 12];  // cp rows, [species][T > tmid][6]
+  for (int t = threadIdx.x; t < nsp * 12; t += kBlock) {
+    const int k = t / 12, hi = (t / 6) % 2, c = t % 6;
+    cps[t] = *(const double*)(p.mtab + L.th + (hi ? 0 : 13 * kRow) + (7 + c) * kRow + k * 8);
   }
   __syncthreads();
   const int64_t ncell = (int64_t)p.nx * p.ny * p.nz;
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (c >= ncell) return;
   if (p.mask && p.mask[p.mask_base + (int64_t)((c / p.nx) % p.ny) * p.mask_ld + (int)(c % p.nx)] == 1) return;
   const TGR_CONST double* pt = (const TGR_CONST double*)p.ptab;
+  const TGR_CONST double* w14 = pt + kPair + nsp * kPropsParts(nsp) * kPart;
+  const TGR_CONST double* w12 = w14 + nsp;
   const TGR_GLOBAL double* ys = (const TGR_GLOBAL double*)p.sc + (int64_t)p.isc_sc0 * p.plane + c;
   const double T = p.sc[(int64_t)p.isc_T0 * p.plane + c];
   const TGR_CONST double* iw = (const TGR_CONST double*)(p.mtab + L.iw);  // 1 / W_k
-  // finitechem_W: mass fractions clipped to [0, 1]; yw first holds Y_j / W_j
-  // (each Y read once), scaled by W_mix below
-  double ise[nsp], yw[nsp];
-  double sy = 0.0, syw = 0.0;
-#pragma unroll
-  for (int q = 0; q < nsp; ++q) {
-    const double Y = ys[q * p.plane];
-    const double yt = fmin(fmax(Y, 0.0), 1.0);
-    sy += yt;
-    syw = fma(yt, iw[q], syw);
-    yw[q] = Y * iw[q];
-  }
-  const double Wmix = sy / syw;
   const double temp = fmin(fmax(T, 50.0), 5000.0);  // Tmin, Tmax (finitechem.f90:7-8)
   const double st = sqrt(temp);
-  if (p.visc) {
+  const double* cr = cps + (temp > p.tmid ? 6 : 0);
+  // Both loops take kCh species at a time: the next chunk's Y are loaded while
+  // one computes (a load takes longer than one species), and the chains of a
+  // chunk's species overlap.
+  constexpr int kCh = 4;
+  double Yn[kCh];
 #pragma unroll
-    for (int q = 0; q < nsp; ++q) {
+  for (int u = 0; u < kCh; ++u) Yn[u] = ys[(u < nsp ? u : 0) * p.plane];
+  // finitechem_W: mass fractions clipped to [0, 1]
+  double sy = 0.0, syw = 0.0, s1 = 0.0, s2 = 0.0, cpm = 0.0;
+#pragma unroll 1
+  for (int k0 = 0; k0 < nsp; k0 += kCh) {
+    double Yc[kCh];
+#pragma unroll
+    for (int u = 0; u < kCh; ++u) {
+      const int kn = k0 + kCh + u;
+      Yc[u] = Yn[u];
+      Yn[u] = ys[(kn < nsp ? kn : 0) * p.plane];
+    }
+#pragma unroll
+    for (int u = 0; u < kCh; ++u) {
+      const int k = k0 + u;
+      if (nsp % kCh && k >= nsp) break;
+      const double Y = Yc[u];
+      const double yt = fmin(fmax(Y, 0.0), 1.0);
+      sy += yt;
+      syw = fma(yt, iw[k], syw);
       double num, den;
-      omegamu_nd(temp * pt[64 + q], num, den);
-      ise[q] = sqrt(num / (pt[q] * st * den));  // 1 / sqrt(eta_j)
-      yw[q] *= Wmix;
+      omegamu_nd(temp * pt[64 + k], num, den);
+      const double ms = pt[k] * st * den;
+      if (p.visc) gs[k][threadIdx.x] = w14[k] * sqrt(num / ms);
+      if (p.diff) {
+        const double eta = ms / num;
+        const double* d = cr + k * 12;
+        const double cpk = d[0] * (d[1] + temp * (d[2] + temp * (d[3] + temp * (d[4] + temp * d[5]))));
+        const double cond = eta * fma(1.25 * kRcst, iw[k], cpk);
+        const double yk = Y * iw[k];
+        s1 += yk / cond;
+        s2 += yk * cond;
+        cpm += Y * cpk;
+      }
     }
   }
-  // COMPTHERMODATA cp rows (both temperature ranges; each lane picks its own)
-  const TGR_CONST double* thi = (const TGR_CONST double*)(p.mtab + L.th);
-  const TGR_CONST double* tlo = thi + 13 * 64;
-  const bool hi = temp > p.tmid;
-  double visc = 0.0, s1 = 0.0, s2 = 0.0, cpm = 0.0;
+  const double Wmix = sy / syw;
+  if (p.rho) p.rho[c] = p.p_thermo * Wmix / (kRcst * T);
+  if (p.visc) {
+    double visc = 0.0;
+#pragma unroll
+    for (int k0 = 0; k0 < nsp; k0 += kPart) {
+      const TGR_CONST double* col = pt + kPair + (k0 / kPart) * nsp * kPart;  // [part][j][kPart]
+      double a[kPart], b[kPart], d[kPart], m[kPart];
+#pragma unroll
+      for (int k = 0; k < kPart; ++k) a[k] = b[k] = d[k] = 0.0;
+      load_row(m, col);
+#pragma unroll
+      for (int u = 0; u < kCh; ++u) Yn[u] = ys[(u < nsp ? u : 0) * p.plane];
 #pragma unroll 1
-  for (int k = 0; k < nsp; ++k) {
-    const double Y = ys[k * p.plane];
-    double num, den;
-    omegamu_nd(temp * pt[64 + k], num, den);
-    const double eta = pt[k] * st * den / num;
-    const double ywk = Y * iw[k] * Wmix;
-    if (p.visc) {
-      const double se = sqrt(eta);
-      // the factor pairs in chunks of kCh, each chunk's LDS reads issued
-      // while the previous chunk computes.  The row offset passes through an
-      // empty asm statement that takes the running sum as an input, so the
-      // compiler cannot hoist every read of the row into registers at once.
-      constexpr int kCh = 4, nch = (nsp + kCh - 1) / kCh;
-      double2 buf[2][kCh];
-      int row = k * nsp;
+      for (int q0 = 0; q0 < nsp; q0 += kCh) {
+        double Yc[kCh];
 #pragma unroll
-      for (int i = 0; i < kCh; ++i)
-        if (i < nsp) buf[0][i] = pair[row + i];
-      double s = 0.0;
+        for (int u = 0; u < kCh; ++u) {
+          const int qn = q0 + kCh + u;
+          Yc[u] = Yn[u];
+          Yn[u] = ys[(qn < nsp ? qn : 0) * p.plane];
+        }
 #pragma unroll
-      for (int ch = 0; ch < nch; ++ch) {
-        asm volatile("" : "+v"(row) : "v"(s));
+        for (int u = 0; u < kCh; ++u) {
+          const int q = q0 + u;
+          if (nsp % kCh && q >= nsp) break;
+          double mn[kPart];
+          load_row(mn, col + (q + 1 < nsp ? q + 1 : 0) * kPart);
+          const double g = gs[q][threadIdx.x];
+          const double y = Yc[u] * iw[q], yg = y * g, ygg = yg * g;
 #pragma unroll
-        for (int i = 0; i < kCh; ++i)
-          if ((ch + 1) * kCh + i < nsp) buf[(ch + 1) & 1][i] = pair[row + (ch + 1) * kCh + i];
-#pragma unroll
-        for (int i = 0; i < kCh; ++i) {
-          const int q = ch * kCh + i;
-          if (q < nsp) {
-            const double f = fma(se * ise[q], buf[ch & 1][i].y, buf[ch & 1][i].x);
-            s = fma(yw[q] * f, f, s);
+          for (int k = 0; k < kPart; ++k) {
+            a[k] = fma(m[k], y, a[k]);
+            b[k] = fma(m[k], yg, b[k]);
+            d[k] = fma(m[k], ygg, d[k]);
           }
+#pragma unroll
+          for (int k = 0; k < kPart; ++k) m[k] = mn[k];
         }
       }
-      s += ywk;
-      visc += Y > 0.0 ? ywk * eta / s : 0.0;
+#pragma unroll
+      for (int k = 0; k < kPart; ++k)
+        if (k0 + k < nsp) {
+          const double Y = ys[(k0 + k) * p.plane], g = gs[k0 + k][threadIdx.x];
+          const double s = fma(g, fma(g, a[k], 2.0 * b[k]), d[k]);
+          visc += Y > 0.0 ? Y * iw[k0 + k] * w12[k0 + k] / s : 0.0;
+        }
     }
-    if (p.diff) {
-      const double ac = hi ? thi[7 * 64 + k] : tlo[7 * 64 + k], d1 = hi ? thi[8 * 64 + k] : tlo[8 * 64 + k],
-                   d2 = hi ? thi[9 * 64 + k] : tlo[9 * 64 + k], d3 = hi ? thi[10 * 64 + k] : tlo[10 * 64 + k],
-                   d4 = hi ? thi[11 * 64 + k] : tlo[11 * 64 + k], d5 = hi ? thi[12 * 64 + k] : tlo[12 * 64 + k];
-      const double cpk = ac * (d1 + temp * (d2 + temp * (d3 + temp * (d4 + temp * d5))));
-      const double cond = eta * fma(1.25 * kRcst, iw[k], cpk);
-      s1 += ywk / cond;
-      s2 += ywk * cond;
-      cpm += Y * cpk;
-    }
+    p.visc[c] = visc;
   }
-  if (p.rho) p.rho[c] = p.p_thermo * Wmix / (kRcst * T);
-  if (p.visc) p.visc[c] = visc;
   if (p.diff) {
-    const double D = 0.5 * (s2 + (1.0 / s1)) / cpm;
+    const double D = 0.5 * (s2 * Wmix + (1.0 / (s1 * Wmix))) / cpm;
 #pragma unroll 1
     for (int k = 0; k < nsp; ++k) p.diff[(int64_t)(p.isc_sc0 + k) * p.plane + c] = p.lewis ? D / p.lewis[k] : D;
     p.diff[(int64_t)p.isc_T0 * p.plane + c] = D;
@@ -231,16 +289,21 @@ extern "C" int tgr_launch_props(const PropsParams* p, int neq, int lane_map, hip
   const int64_t ncell = (int64_t)p->nx * p->ny * p->nz;
   if (ncell <= 0) return 0;
   if (lane_map) {
-    const int64_t nb = (ncell + 255) / 256;
-    if (nb > 0x7fffffff) return -1;
-    const dim3 grid((unsigned)nb), block(256);
+#define TGR_PROPS_LAUNCH(NEQ_)                                                                                   \
+  case NEQ_: {                                                                                                  \
+    const int64_t nb = (ncell + props_block<NEQ_>() - 1) / props_block<NEQ_>();                                 \
+    if (nb > 0x7fffffff) return -1;                                                                             \
+    hipLaunchKernelGGL(props_lane_kernel<NEQ_>, dim3((unsigned)nb), dim3(props_block<NEQ_>()), 0, s, *p);       \
+    break;                                                                                                      \
+  }
     switch (neq) {
-      case 10: hipLaunchKernelGGL(props_lane_kernel<10>, grid, block, 0, s, *p); break;
-      case 37: hipLaunchKernelGGL(props_lane_kernel<37>, grid, block, 0, s, *p); break;
-      case 40: hipLaunchKernelGGL(props_lane_kernel<40>, grid, block, 0, s, *p); break;
-      case 46: hipLaunchKernelGGL(props_lane_kernel<46>, grid, block, 0, s, *p); break;
+      TGR_PROPS_LAUNCH(10)
+      TGR_PROPS_LAUNCH(37)
+      TGR_PROPS_LAUNCH(40)
+      TGR_PROPS_LAUNCH(46)
       default: return -1;
     }
+#undef TGR_PROPS_LAUNCH
     return hipGetLastError() == hipSuccess ? 0 : -2;
   }
   const int64_t need = (ncell + 3) / 4;

@@ -127,9 +127,9 @@ struct DiffParams {
 
 // Species whose Wilke sums the thread-per-cell properties kernel accumulates in
 // one pass (three sums each in registers, two waves per SIMD; the scalar
-// registers hold two columns of 18), an even number; the pair matrix of that
-// kernel is stored part by part.
-__host__ __device__ constexpr int kPropsParts(int nsp) { return (nsp + 17) / 18; }
+// registers hold two columns of at most 20), an even number; the pair matrix of
+// that kernel is stored part by part.
+__host__ __device__ constexpr int kPropsParts(int nsp) { return (nsp + 19) / 20; }
 __host__ __device__ constexpr int kPropsPart(int nsp) {
   return ((nsp + kPropsParts(nsp) - 1) / kPropsParts(nsp) + 1) / 2 * 2;
 }

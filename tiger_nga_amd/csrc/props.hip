@@ -138,19 +138,30 @@ __device__ __forceinline__ void load_row(double (&m)[N], const TGR_CONST double*
 }
 
 
-// Threads of its workgroup: its g_k take 8 nsp bytes of LDS a thread, and eight
-// waves on a CU need the LDS of two workgroups of four waves.
+// Threads of a workgroup (its g_k take 8 nsp bytes of LDS a thread, the cp rows
+// 96 nsp bytes): four waves where two such workgroups fit a CU, else two waves;
+// the cp rows are in LDS where they do not cost a resident workgroup.  DME39,
+// 1,200 and 332,000 cells: 50.8 and 213 us so, 51.8 and 209 with four waves, 52.7
+// and 249 with two and the cp rows in LDS (a third of the pair loop padding
+// then: 3 parts of 14).
+constexpr int kLdsBytes = 160 * 1024;
 template <int NEQ>
 constexpr int props_block() {
-  return 2 * (256 * 8 + 96) * (NEQ - 1) <= 160 * 1024 ? 256 : 128;
+  return 2 * (256 * 8 + 96) * (NEQ - 1) <= kLdsBytes ? 256 : 128;
+}
+template <int NEQ>
+constexpr bool props_cp_lds() {
+  return kLdsBytes / ((props_block<NEQ>() * 8 + 96) * (NEQ - 1)) == kLdsBytes / (props_block<NEQ>() * 8 * (NEQ - 1));
 }
 
 // One thread per cell (the block's cells in their storage order, so every
 // field access is coalesced).  A first loop over the species forms W_mix, the
-// conductivity sums and g (to LDS); then, for a part of the species k at a
-// time, a loop over j adds column j of the pair matrix times y_j, y_j g_j and
-// y_j g_j^2 to the part's sums: 3 x 18 independent chains (GRI-3.0), the next
-// column's scalar loads under way.  Sums run in species order (the wave
+// conductivity sums and g (to LDS; in registers for up to 20 species); then, for
+// a part of the species k at a time, a loop over j adds column j of the pair
+// matrix times y_j, y_j g_j and y_j g_j^2 to the part's sums: 3 x 18 independent
+// chains (GRI-3.0), the next column's scalar loads under way.  Bound by VALU
+// issue (64 % busy, 8,400 instructions a wave of which 3,900 are the pairs');
+// 130^3 GRI-3.0 cells in 0.83 ms, 1.03 ms with a 16-byte LDS read per pair.  Sums run in species order (the wave
 // kernel's are tree reductions) and eta = mucoeff sqrt(T) den / num takes
 // omegamu's numerator and denominator with one division: rounding-level
 // differences.
@@ -160,13 +171,17 @@ __global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per
   constexpr int nsp = NEQ - 1, kBlock = props_block<NEQ>(), kPart = kPropsPart(nsp);
   constexpr TabLayout L = tab_layout<NEQ>();
   constexpr int kPair = 192 + 2 * nsp * 64;
-  __shared__ double gs[nsp][kBlock];
-  __shared__ __attribute__((aligned(16))) double cps[nsp * 12];  // cp rows, [species][T > tmid][6]
-  for (int t = threadIdx.x; t < nsp * 12; t += kBlock) {
-    const int k = t / 12, hi = (t / 6) % 2, c = t % 6;
-    cps[t] = *(const double*)(p.mtab + L.th + (hi ? 0 : 13 * kRow) + (7 + c) * kRow + k * 8);
+  constexpr bool kOne = kPropsParts(nsp) == 1;  // few species: one part, everything in registers
+  __shared__ double gs[kOne ? 1 : nsp][kBlock];
+  constexpr bool kCpLds = props_cp_lds<NEQ>();
+  __shared__ __attribute__((aligned(16))) double cps[kCpLds ? nsp * 12 : 2];  // cp rows, [species][T > tmid][6]
+  if constexpr (kCpLds) {
+    for (int t = threadIdx.x; t < nsp * 12; t += kBlock) {
+      const int k = t / 12, hi = (t / 6) % 2, c = t % 6;
+      cps[t] = *(const double*)(p.mtab + L.th + (hi ? 0 : 13 * kRow) + (7 + c) * kRow + k * 8);
+    }
+    __syncthreads();
   }
-  __syncthreads();
   const int64_t ncell = (int64_t)p.nx * p.ny * p.nz;
   const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (c >= ncell) return;
@@ -179,16 +194,20 @@ __global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per
   const TGR_CONST double* iw = (const TGR_CONST double*)(p.mtab + L.iw);  // 1 / W_k
   const double temp = fmin(fmax(T, 50.0), 5000.0);  // Tmin, Tmax (finitechem.f90:7-8)
   const double st = sqrt(temp);
-  const double* cr = cps + (temp > p.tmid ? 6 : 0);
+  const bool hi = temp > p.tmid;
+  const double* cr = cps + (hi ? 6 : 0);
+  const TGR_CONST double* thi = (const TGR_CONST double*)(p.mtab + L.th);
+  const TGR_CONST double* tlo = thi + 13 * 64;
   // Both loops take kCh species at a time: the next chunk's Y are loaded while
   // one computes (a load takes longer than one species), and the chains of a
   // chunk's species overlap.
-  constexpr int kCh = 4;
+  constexpr int kCh = kOne ? nsp : 4;
   double Yn[kCh];
 #pragma unroll
   for (int u = 0; u < kCh; ++u) Yn[u] = ys[(u < nsp ? u : 0) * p.plane];
   // finitechem_W: mass fractions clipped to [0, 1]
   double sy = 0.0, syw = 0.0, s1 = 0.0, s2 = 0.0, cpm = 0.0;
+  double g1[kOne ? nsp : 1];
 #pragma unroll 1
   for (int k0 = 0; k0 < nsp; k0 += kCh) {
     double Yc[kCh];
@@ -196,7 +215,7 @@ __global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per
     for (int u = 0; u < kCh; ++u) {
       const int kn = k0 + kCh + u;
       Yc[u] = Yn[u];
-      Yn[u] = ys[(kn < nsp ? kn : 0) * p.plane];
+      if constexpr (kCh < nsp) Yn[u] = ys[(kn < nsp ? kn : 0) * p.plane];
     }
 #pragma unroll
     for (int u = 0; u < kCh; ++u) {
@@ -209,10 +228,19 @@ __global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per
       double num, den;
       omegamu_nd(temp * pt[64 + k], num, den);
       const double ms = pt[k] * st * den;
-      if (p.visc) gs[k][threadIdx.x] = w14[k] * sqrt(num / ms);
+      if (p.visc) {
+        const double g = w14[k] * sqrt(num / ms);
+        if constexpr (kOne) g1[u] = g;
+        else gs[k][threadIdx.x] = g;
+      }
       if (p.diff) {
         const double eta = ms / num;
-        const double* d = cr + k * 12;
+        double d[6];
+#pragma unroll
+        for (int e = 0; e < 6; ++e) {
+          if constexpr (kCpLds) d[e] = cr[k * 12 + e];
+          else d[e] = hi ? thi[(7 + e) * 64 + k] : tlo[(7 + e) * 64 + k];
+        }
         const double cpk = d[0] * (d[1] + temp * (d[2] + temp * (d[3] + temp * (d[4] + temp * d[5]))));
         const double cond = eta * fma(1.25 * kRcst, iw[k], cpk);
         const double yk = Y * iw[k];
@@ -226,8 +254,24 @@ __global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per
   if (p.rho) p.rho[c] = p.p_thermo * Wmix / (kRcst * T);
   if (p.visc) {
     double visc = 0.0;
+    if constexpr (kOne) {
+      const TGR_CONST double* col = pt + kPair;
 #pragma unroll
-    for (int k0 = 0; k0 < nsp; k0 += kPart) {
+      for (int k = 0; k < nsp; ++k) {
+        double a = 0.0, b = 0.0, d = 0.0;
+#pragma unroll
+        for (int q = 0; q < nsp; ++q) {
+          const double y = Yn[q] * iw[q], yg = y * g1[q];
+          a = fma(col[q * kPart + k], y, a);
+          b = fma(col[q * kPart + k], yg, b);
+          d = fma(col[q * kPart + k], yg * g1[q], d);
+        }
+        const double s = fma(g1[k], fma(g1[k], a, 2.0 * b), d);
+        visc += Yn[k] > 0.0 ? Yn[k] * iw[k] * w12[k] / s : 0.0;
+      }
+    }
+#pragma unroll
+    for (int k0 = 0; k0 < (kOne ? 0 : nsp); k0 += kPart) {
       const TGR_CONST double* col = pt + kPair + (k0 / kPart) * nsp * kPart;  // [part][j][kPart]
       double a[kPart], b[kPart], d[kPart], m[kPart];
 #pragma unroll
@@ -242,7 +286,7 @@ __global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per
         for (int u = 0; u < kCh; ++u) {
           const int qn = q0 + kCh + u;
           Yc[u] = Yn[u];
-          Yn[u] = ys[(qn < nsp ? qn : 0) * p.plane];
+          if constexpr (kCh < nsp) Yn[u] = ys[(qn < nsp ? qn : 0) * p.plane];
         }
 #pragma unroll
         for (int u = 0; u < kCh; ++u) {

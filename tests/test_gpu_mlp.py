@@ -127,3 +127,23 @@ def test_training_reduces_loss(torch_dev):
     # the trained parameters round-trip through the host
     p = net.get_params()
     assert np.all(np.isfinite(p)) and p.size == net.nparam
+
+
+@pytest.mark.parametrize("nin,nout,hidden,layers,B", [(8, 8, 64, 1, 64), (130, 200, 128, 2, 320), (38, 37, 256, 4, 8256),
+                                                      (64, 256, 192, 3, 192), (38, 37, 320, 2, 128)])
+def test_widths_and_batches(torch_dev, nin, nout, hidden, layers, B):
+    """Forward and gradients at other widths (the last beyond the fused kernels),
+    at batches of one 64-row tile, an odd number of 32-row slices and more
+    than one row tile per CU; bounds as above."""
+    torch = torch_dev
+    from tiger_nga_amd import mlp
+    net, flat, params, x, tgt = _net_case(torch, nin, nout, hidden, layers, B)
+    got = net.forward(_bf(torch, x)).cpu().numpy()
+    ref, _, _ = mlp_ref.forward(params, x, quantize=True)
+    assert np.abs(got - ref).max() / np.abs(ref).max() < 5e-3 and np.all(got[:, nout:] == 0.0)
+    g, loss = net.gradients(_bf(torch, x), torch.from_numpy(tgt).cuda())
+    lq, gq = mlp_ref.loss_and_grad(params, x, tgt, nout, quantize=True)
+    assert abs(loss - lq) <= 1e-3 * lq
+    for (dW, db), (rW, rb) in zip(mlp.unflatten(g, nin, nout, hidden, layers), gq):
+        for a, r in ((dW, rW), (db, rb)):
+            assert np.linalg.norm(a - r) < 1e-2 * np.linalg.norm(r)

@@ -102,7 +102,7 @@ struct tgr_chem {
   double* d_out_scale = nullptr;
   std::vector<float> h_in_shift, h_in_scale;
   DevBuf b_x, b_guess, b_rej;
-  DevBuf b_diff;  // diffusion workspace: W_gp, cp_mix, corr_vel x / y / z (5 planes)
+  DevBuf b_diff;  // diffusion workspace: W_gp, cp_mix, corr_vel x / y / z (5 planes), fluxes
   unsigned int* d_rej_count = nullptr;
   unsigned long long* d_stotals = nullptr;
   int surr_nsub = 8, surr_guess = 0, surr_newton_max = 8;
@@ -1008,10 +1008,23 @@ int tgr_chem_diffusion_device(tgr_chem* c, double dt, const tgr_grid* g, const t
     *idx[q] = species_index(c->t, names[q]);
     *wk[q] = *idx[q] >= 0 ? c->t->W[*idx[q]] : 1.0;
   }
+  // fourth order: all species' fluxes at once where 1 GiB holds them (one pass
+  // is two launches), at least two species a pass; where the memory for that is
+  // not to be had, the general kernels, which need five planes
+  if (m->st1 == 1 && m->st2 == 2 && tgr::diff_small_plane(gm.plane)) {
+    p.nchunk = (int)std::min<int64_t>(c->nsp, std::max<int64_t>(2, ((int64_t)1 << 30) / (48 * gm.plane)));
+    p.nslice = (int)std::min<int64_t>((p.nchunk + 3) / 4, std::max<int64_t>(1, 6 * 256 * (int64_t)c->n_cu / gm.plane));
+    if (c->b_diff.ensure((size_t)gm.plane * (2 + 4 * p.nslice + 6 * p.nchunk) * sizeof(double))) {
+      (void)hipGetLastError();
+      p.nchunk = p.nslice = 0;
+    }
+  }
   if ((rc = c->b_diff.ensure((size_t)gm.plane * 5 * sizeof(double)))) return rc;
   p.wg = (double*)c->b_diff.p;
   p.cpm = p.wg + gm.plane;
   p.cvel = p.cpm + gm.plane;
+  p.eT = p.cvel + 3 * p.nslice * gm.plane;
+  p.flux = p.eT + p.nslice * gm.plane;
   if (tgr_launch_diffusion(&p, c->neq, (hipStream_t)stream)) return fail(TGR_E_HIP, "diffusion kernel launch failed");
   return 0;
 }

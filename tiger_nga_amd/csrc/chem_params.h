@@ -104,7 +104,10 @@ struct tgr_metric_dev {
   const double *grad_xm, *grad_ym, *grad_zm;
 };
 
-// One launch of the three kernels (filled by the C-ABI layer).
+// planes that 32-bit byte offsets address
+__host__ __device__ constexpr bool diff_small_plane(int64_t plane) { return plane < ((int64_t)1 << 29); }
+
+// One launch of the diffusion kernels (filled by the C-ABI layer).
 struct DiffParams {
   DiffGeom gm;
   tgr_metric_dev m;
@@ -117,7 +120,11 @@ struct DiffParams {
   const int* mask;
   double* wg;     // [plane] W_gp
   double* cpm;    // [plane] cp_mix (cv)
-  double* cvel;   // [3][plane] corr_vel_x, _y, _z
+  double* cvel;   // [3][plane] corr_vel_x, _y, _z (fourth order: [nslice][3][plane])
+  int nchunk;     // fourth order: species per pass through the flux workspace (0: other kernels)
+  int nslice;     // fourth order: parts that the species of a pass are split into
+  double* eT;     // [nslice][plane] temperature term by part
+  double* flux;   // [nchunk][x, y, z][corrected, Fickian][plane]
   double* corr;   // diff_corr(..., nsp + 1) or null
   double* dgp;    // diff_gp(..., 3) or null
   double* src;    // the transport source (..., nscalar) or null

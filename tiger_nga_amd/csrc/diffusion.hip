@@ -18,6 +18,8 @@
 //                     grad_m(T), the H2O / CO / CO2 dump, gas radiation, the
 //                     cp-gradient term, / cp, * dt, and the optional update of
 //                     the transport source.
+// Second order has a pair of its own (diff_sums2_kernel, diff_main2_kernel), and
+// fourth order stores the face fluxes (diff_vel_kernel and the three after it).
 // Readings where the reference text does not conform (the CPU oracle's too):
 // SC(i-st2:j+st1) at 652 read as i+st1; the z sections k-st2:k-st1 at
 // 634-635 and 706 read as k-st2:k+st1 (identical at second order); Cp_sp(isc)
@@ -33,7 +35,6 @@
 #include "chem_kernels.h"
 
 namespace tgr {
-
 
 namespace {
 
@@ -62,27 +63,72 @@ __device__ __forceinline__ void cp_species(const char* tab, const TabLayout& L, 
 
 }  // namespace
 
+// Order of the workgroups: 256 consecutive cells of a plane each, kStrip of
+// them side by side, then the next plane.  The hardware deals workgroups to
+// the 8 XCDs in turn, so XCD e (blockIdx % 8) takes the e-th contiguous piece
+// of that order: its resident workgroups cover a brick of kStrip chunks by
+// some 16 planes, whose halo is a third of its volume (GRI-3.0 128^3: 1394 us in
+// the order of the planes, 1415 / 1376 / 1376 / 1436 us with strips of 2 / 4 / 8 /
+// 16).
+constexpr int kXcd = 8, kStrip = 4;
+struct Brick {
+  int plane, nz, per_xcd;  // cells of a plane, planes, workgroups per XCD
+};
+
+__device__ __forceinline__ bool brick_cell(const Brick& b, int& q, int& z) {
+  const unsigned seq = (blockIdx.x % kXcd) * (unsigned)b.per_xcd + blockIdx.x / kXcd;
+  const unsigned per_strip = (unsigned)b.nz * kStrip;
+  const unsigned strip = seq / per_strip, r = seq - strip * per_strip;
+  z = (int)(r / kStrip);
+  q = (int)((strip * kStrip + r % kStrip) * 256 + threadIdx.x);
+  return q < b.plane;
+}
+
+// a[byte offset]: a wave-uniform base and a 32-bit lane offset (the launcher
+// checks that a plane has less than 2^32 bytes)
+__device__ __forceinline__ double ldo(const double* a, unsigned off) {
+  return *(const double*)((const char*)a + off);
+}
+
+// cp rows of the species in LDS, [species][T > tmid][6]
+template <int NEQ>
+__device__ __forceinline__ void stage_cp(double* cps, const char* tab) {
+  constexpr TabLayout L = tab_layout<NEQ>();
+  for (int t = threadIdx.x; t < (NEQ - 1) * 12; t += 256) {
+    const int k = t / 12, hi = (t / 6) % 2, c = t % 6;
+    cps[t] = *(const double*)(tab + L.th + (hi ? 0 : 13 * kRow) + (7 + c) * kRow + k * 8);
+  }
+  __syncthreads();
+}
+
+__device__ __forceinline__ double cp_lds(const double* c, double T) {
+  return c[0] * (c[1] + T * (c[2] + T * (c[3] + T * (c[4] + T * c[5]))));
+}
+
 template <int NEQ>
 __global__ __launch_bounds__(256) void diff_cell_kernel(DiffParams p) {
   constexpr TabLayout L = tab_layout<NEQ>();
   constexpr int N = NEQ - 1;
+  __shared__ __attribute__((aligned(16))) double cps[N * 12];
+  stage_cp<NEQ>(cps, p.mech.tab);
   const DiffGeom& g = p.gm;
   const int64_t n = (int64_t)g.nxo * g.nyo * g.nzo;
-  const double* W = (const double*)(p.mech.tab + L.w);
+  const TGR_CONST double* iw = (const TGR_CONST double*)(p.mech.tab + L.iw);  // 1 / W_k
   for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
     const int i = g.imino_ + (int)(c % g.nxo), j = g.jmino_ + (int)((c / g.nxo) % g.nyo);
     double w = 1.0, cp = 0.0;
     if (!wall(g, p.mask, i, j)) {
       const double T = p.sc[(int64_t)g.isc_T0 * g.plane + c];
+      const double* Y = p.sc + (int64_t)g.isc_sc0 * g.plane + c;
+      const double* cr = cps + (T > p.mech.tmid ? 6 : 0);
       double s1 = 0.0, s2 = 0.0;
+#pragma unroll 4
       for (int k = 0; k < N; ++k) {
-        const double yk = p.sc[(int64_t)(g.isc_sc0 + k) * g.plane + c];
+        const double yk = Y[k * g.plane];
         const double y = fmin(fmax(yk, 0.0), 1.0);
         s1 += y;
-        s2 += y / W[k];
-        double cpk;
-        cp_species(p.mech.tab, L, p.mech.tmid, T, k, cpk);
-        cp += yk * cpk;
+        s2 = fma(y, iw[k], s2);
+        cp += yk * cp_lds(cr + k * 12, T);
       }
       w = s1 / s2;
       if (p.cv) cp = cp - 8314.34 / w;
@@ -302,48 +348,6 @@ __global__ __launch_bounds__(256) void diff_main_kernel(DiffParams p) {
 //     time (Brick below), so that the y and z neighbours are L2 hits.
 // GRI-3.0 128^3, molar term on: 2.37 -> 1.36 ms a call (separate W_gp / cp pass
 // 0.25 ms and face sums 0.44 ms -> 0.53 ms; main 1.79 -> 0.83 ms).
-
-// Order of the workgroups: 256 consecutive cells of a plane each, kStrip of
-// them side by side, then the next plane.  The hardware deals workgroups to
-// the 8 XCDs in turn, so XCD e (blockIdx % 8) takes the e-th contiguous piece
-// of that order: its resident workgroups cover a brick of kStrip chunks by
-// some 16 planes, whose halo is a third of its volume (GRI-3.0 128^3: 1394 us in
-// the order of the planes, 1415 / 1376 / 1376 / 1436 us with strips of 2 / 4 / 8 /
-// 16).
-constexpr int kXcd = 8, kStrip = 4;
-struct Brick {
-  int plane, nz, per_xcd;  // cells of a plane, planes, workgroups per XCD
-};
-
-__device__ __forceinline__ bool brick_cell(const Brick& b, int& q, int& z) {
-  const unsigned seq = (blockIdx.x % kXcd) * (unsigned)b.per_xcd + blockIdx.x / kXcd;
-  const unsigned per_strip = (unsigned)b.nz * kStrip;
-  const unsigned strip = seq / per_strip, r = seq - strip * per_strip;
-  z = (int)(r / kStrip);
-  q = (int)((strip * kStrip + r % kStrip) * 256 + threadIdx.x);
-  return q < b.plane;
-}
-
-// a[byte offset]: a wave-uniform base and a 32-bit lane offset (the launcher
-// checks that a plane has less than 2^32 bytes)
-__device__ __forceinline__ double ldo(const double* a, unsigned off) {
-  return *(const double*)((const char*)a + off);
-}
-
-// cp rows of the species in LDS, [species][T > tmid][6]
-template <int NEQ>
-__device__ __forceinline__ void stage_cp(double* cps, const char* tab) {
-  constexpr TabLayout L = tab_layout<NEQ>();
-  for (int t = threadIdx.x; t < (NEQ - 1) * 12; t += 256) {
-    const int k = t / 12, hi = (t / 6) % 2, c = t % 6;
-    cps[t] = *(const double*)(tab + L.th + (hi ? 0 : 13 * kRow) + (7 + c) * kRow + k * 8);
-  }
-  __syncthreads();
-}
-
-__device__ __forceinline__ double cp_lds(const double* c, double T) {
-  return c[0] * (c[1] + T * (c[2] + T * (c[3] + T * (c[4] + T * c[5]))));
-}
 
 // W_gp and cp_mix of the interior and one cell around it, correction
 // velocities at the face cells (diff_cell_kernel and diff_face_kernel; a face
@@ -591,6 +595,300 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
   if (src) src[(int64_t)g.isc_T0 * g.plane + o] += eT;
 }
 
+// ---- wider stencils with widths known at compile time (fourth order) ----------
+// After diff_cell_kernel: the correction velocities (diff_vel_kernel), every
+// face's fluxes once per species into a workspace (diff_flux_kernel), the
+// cells' sums of them (diff_div_kernel) and the temperature term
+// (diff_temp_kernel), where diff_main_kernel has every cell recompute the fluxes
+// of its 12 faces from 4 points each.  A species costs a face 38 loads and six
+// stores and a cell 24 loads, all along x; weights and points that do not depend
+// on the species stay in registers.  The species of a pass are split into
+// nslice parts (blockIdx.y) until there are six workgroups per CU: at 16 x 17 x
+// 18 cells one part leaves three quarters of the chip without work.  The
+// workspace holds nchunk species, one pass of them at a time.
+// Bound by the fluxes' way through memory (128 bytes per cell and species at
+// half the copy rate; two or three wavefronts per SIMD give the same time, four
+// spill).  DME39, 61 x 47 x 35 cells: 1262 -> 345 us a call; GRI-3.0, 126 x 124
+// x 120: 20.2 -> 4.35 ms; 16 x 17 x 18: 824 -> 61 us.  Twelve and 24 workgroups
+// per CU: 364 and 446 us at the first of these.
+
+// Weights of the P = ST1 + ST2 + 1 stencil points of the faces of a cell.
+template <int P>
+struct Weights {
+  double w[3][P], g[3][P], u[3][P], gw[3];  // interpolation, gradient, w / W_gp, sum grad * W_gp
+};
+
+template <int ST1, int ST2, bool MOLAR>
+__device__ __forceinline__ void face_weights(const DiffParams& p, int i, int j, int k,
+                                             Weights<ST1 + ST2 + 1>& F) {
+  constexpr int P = ST1 + ST2 + 1;
+  const DiffGeom& g = p.gm;
+  const tgr_metric_dev& m = p.m;
+  const int fi0 = g.imin_ - ST1, fni = g.imax_ + ST2 - fi0 + 1, fj0 = g.jmin_ - ST1, fnj = g.jmax_ + ST2 - fj0 + 1;
+  const int64_t o = c3(g, i, j, k), step[3] = {1, g.nxo, (int64_t)g.nxo * g.nyo};
+#pragma unroll
+  for (int d = 0; d < 3; ++d) F.gw[d] = 0.0;
+#pragma unroll
+  for (int t = 0; t < P; ++t) {
+    const int s = t - ST2;
+    F.w[0][t] = op(m.interp_sc_x, i, fi0, fni, j, g.jmino_, g.nyo, s, -ST2);
+    F.w[1][t] = op(m.interp_sc_y, i, g.imino_, g.nxo, j, fj0, fnj, s, -ST2);
+    F.w[2][t] = op(m.interp_sc_z, i, g.imino_, g.nxo, j, fj0, fnj, s, -ST2);
+    F.g[0][t] = op(m.grad_x, i, fi0, fni, j, fj0, fnj, s, -ST2);
+    F.g[1][t] = op(m.grad_y, i, fi0, fni, j, fj0, fnj, s, -ST2);
+    F.g[2][t] = op(m.grad_z, i, fi0, fni, j, fj0, fnj, s, -ST2);
+    if constexpr (MOLAR) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const double wg = p.wg[o + s * step[d]];
+        F.u[d][t] = F.w[d][t] / wg;
+        F.gw[d] += F.g[d][t] * wg;
+      }
+    }
+  }
+}
+
+// Y and D of one species at the stencil points of a cell's faces
+template <int ST1, int ST2>
+struct FacePoints {
+  double y[3][ST1 + ST2 + 1], d[3][ST1 + ST2 + 1];
+  __device__ __forceinline__ void load(const double* Y, const double* D, unsigned oc, int64_t sy, int64_t sz) {
+    const int64_t step[3] = {1, sy, sz};
+    const double yc = ldo(Y, oc), dc = ldo(D, oc);
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int t = 0; t < ST1 + ST2 + 1; ++t) {
+        y[q][t] = t == ST2 ? yc : ldo(Y + (t - ST2) * step[q], oc);
+        d[q][t] = t == ST2 ? dc : ldo(D + (t - ST2) * step[q], oc);
+      }
+  }
+};
+
+// species [s0, s1) of n that a workgroup of slice blockIdx.y has
+__device__ __forceinline__ void slice(int n, int& s0, int& s1) {
+  s0 = n * (int)blockIdx.y / (int)gridDim.y;
+  s1 = n * ((int)blockIdx.y + 1) / (int)gridDim.y;
+}
+
+template <int STP>
+__device__ __forceinline__ void cell_gradient(const DiffParams& p, const double* f, int i, int j, int64_t o,
+                                              double (&out)[3]) {
+  const DiffGeom& g = p.gm;
+  const int nx = g.imax_ - g.imin_ + 1, ny = g.jmax_ - g.jmin_ + 1;
+  const int64_t step[3] = {1, g.nxo, (int64_t)g.nxo * g.nyo};
+#pragma unroll
+  for (int d = 0; d < 3; ++d) out[d] = 0.0;
+#pragma unroll
+  for (int s = -STP; s <= STP; ++s)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const double* gm = d == 0 ? p.m.grad_xm : (d == 1 ? p.m.grad_ym : p.m.grad_zm);
+      out[d] += op(gm, i, g.imin_, nx, j, g.jmin_, ny, s, -STP) * f[o + s * step[d]];
+    }
+}
+
+// cell of the face range that this thread has
+template <int ST1, int ST2>
+__device__ __forceinline__ bool face_cell(const DiffParams& p, const Brick& bk, int& i, int& j, int& k) {
+  int q, z;
+  if (!brick_cell(bk, q, z)) return false;
+  const int fni = p.gm.imax_ - p.gm.imin_ + 1 + ST1 + ST2;
+  i = p.gm.imin_ - ST1 + q % fni;
+  j = p.gm.jmin_ - ST1 + q / fni;
+  k = p.gm.kmin_ - ST1 + z;
+  return true;
+}
+
+template <int NEQ, bool MOLAR, int ST1, int ST2>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void diff_vel_kernel(DiffParams p, Brick bk) {
+  constexpr int N = NEQ - 1, P = ST1 + ST2 + 1;
+  const DiffGeom& g = p.gm;
+  int i, j, k;
+  if (!face_cell<ST1, ST2>(p, bk, i, j, k)) return;
+  const int64_t o = c3(g, i, j, k), sy = g.nxo, sz = (int64_t)g.nxo * g.nyo;
+  double v[3] = {0.0, 0.0, 0.0};
+  if (!wall(g, p.mask, i, j)) {
+    Weights<P> F;
+    face_weights<ST1, ST2, MOLAR>(p, i, j, k, F);
+    const unsigned oc = (unsigned)o * 8u;
+    int s0, s1;
+    slice(N, s0, s1);
+    const double* __restrict__ Y = p.sc + (int64_t)(g.isc_sc0 + s0) * g.plane;
+    const double* __restrict__ D = p.diff + (int64_t)(g.isc_sc0 + s0) * g.plane;
+#pragma unroll 1
+    for (int sp = s0; sp < s1; ++sp, Y += g.plane, D += g.plane) {
+      FacePoints<ST1, ST2> s;
+      s.load(Y, D, oc, sy, sz);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        double a = 0, b = 0, ii = 0;
+#pragma unroll
+        for (int t = 0; t < P; ++t) {
+          a += F.w[d][t] * s.d[d][t];
+          b += F.g[d][t] * s.y[d][t];
+          if constexpr (MOLAR) ii += F.u[d][t] * s.y[d][t];
+        }
+        v[d] += a * b;
+        if constexpr (MOLAR) v[d] += a * ii * F.gw[d];
+      }
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < 3; ++d) p.cvel[(3 * blockIdx.y + d) * g.plane + o] = v[d];
+}
+
+template <int NEQ, bool MOLAR, int ST1, int ST2>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void diff_flux_kernel(DiffParams p, Brick bk,
+                                                                                                int sp0, int nsp) {
+  constexpr int P = ST1 + ST2 + 1;
+  const DiffGeom& g = p.gm;
+  int i, j, k;
+  if (!face_cell<ST1, ST2>(p, bk, i, j, k)) return;
+  const int64_t o = c3(g, i, j, k), sy = g.nxo, sz = (int64_t)g.nxo * g.nyo;
+  int s0, s1;
+  slice(nsp, s0, s1);
+  double* __restrict__ to = p.flux + 6 * s0 * g.plane + o;
+  if (wall(g, p.mask, i, j)) {  // no flux through a wall face
+    for (int q = 6 * s0; q < 6 * s1; ++q, to += g.plane) *to = 0.0;
+    return;
+  }
+  Weights<P> F;
+  face_weights<ST1, ST2, MOLAR>(p, i, j, k, F);
+  double v[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    double c = p.cvel[d * g.plane + o];
+    for (int q = 1; q < (int)gridDim.y; ++q) c += p.cvel[(3 * q + d) * g.plane + o];
+    v[d] = -c;
+  }
+  const unsigned oc = (unsigned)o * 8u;
+  const double* __restrict__ Y = p.sc + (int64_t)(g.isc_sc0 + sp0 + s0) * g.plane;
+  const double* __restrict__ D = p.diff + (int64_t)(g.isc_sc0 + sp0 + s0) * g.plane;
+#pragma unroll 1
+  for (int sp = s0; sp < s1; ++sp, Y += g.plane, D += g.plane, to += 6 * g.plane) {
+    FacePoints<ST1, ST2> s;
+    s.load(Y, D, oc, sy, sz);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      double yi = 0, a = 0, b = 0, ii = 0;
+#pragma unroll
+      for (int t = 0; t < P; ++t) {
+        yi += F.w[d][t] * s.y[d][t];
+        a += F.w[d][t] * s.d[d][t];
+        b += F.g[d][t] * s.y[d][t];
+        if constexpr (MOLAR) ii += F.u[d][t] * s.y[d][t];
+      }
+      double c = v[d] * yi;
+      if constexpr (MOLAR) c += a * ii * F.gw[d];
+      to[2 * d * g.plane] = c;
+      to[(2 * d + 1) * g.plane] = a * b;
+    }
+  }
+}
+
+template <int NEQ, int ST1, int ST2>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void diff_div_kernel(DiffParams p, Brick bk,
+                                                                                               int sp0, int nsp) {
+  constexpr int N = NEQ - 1, P = ST1 + ST2 + 1;
+  __shared__ __attribute__((aligned(16))) double cps[N * 12];
+  stage_cp<NEQ>(cps, p.mech.tab);
+  const DiffGeom& g = p.gm;
+  int q, z;
+  if (!brick_cell(bk, q, z)) return;
+  const int nx = g.imax_ - g.imin_ + 1, ny = g.jmax_ - g.jmin_ + 1;
+  const int i = g.imin_ + q % nx, j = g.jmin_ + q / nx, k = g.kmin_ + z;
+  if (wall(g, p.mask, i, j)) return;
+  const int64_t o = c3(g, i, j, k), step[3] = {1, g.nxo, (int64_t)g.nxo * g.nyo};
+  const double* Tf = p.sc + (int64_t)g.isc_T0 * g.plane;
+  const double T = Tf[o];
+  double tg[3];
+  cell_gradient<ST1 + ST2>(p, Tf, i, j, o, tg);
+  double dv[3][P], im[3][P];
+#pragma unroll
+  for (int t = 0; t < P; ++t)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const double* a = d == 0 ? p.m.div_u : (d == 1 ? p.m.div_v : p.m.div_w);
+      const double* b = d == 0 ? p.m.interp_u_xm : (d == 1 ? p.m.interp_v_ym : p.m.interp_w_zm);
+      dv[d][t] = op(a, i, g.imin_, nx, j, g.jmin_, ny, t - ST1, -ST1);
+      im[d][t] = op(b, i, g.imin_, nx, j, g.jmin_, ny, t - ST1, -ST1);
+    }
+  const double* cr = cps + (T > p.mech.tmid ? 6 : 0);
+  const unsigned oc = (unsigned)o * 8u;
+  int s0, s1;
+  slice(nsp, s0, s1);
+  const double* __restrict__ fl = p.flux + 6 * s0 * g.plane;
+  double eT = sp0 ? p.eT[blockIdx.y * g.plane + o] : 0.0;  // this slice's part of the temperature term
+#pragma unroll 1
+  for (int sq = s0; sq < s1; ++sq, fl += 6 * g.plane) {
+    const int sp = sp0 + sq;
+    double fc[3][P], ff[3][P];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+      for (int t = 0; t < P; ++t) {
+        fc[d][t] = ldo(fl + 2 * d * g.plane + (t - ST1) * step[d], oc);
+        ff[d][t] = ldo(fl + (2 * d + 1) * g.plane + (t - ST1) * step[d], oc);
+      }
+    double dcor = 0.0, dfick = 0.0, fm[3] = {};
+#pragma unroll
+    for (int t = 0; t < P; ++t) {
+      dcor += dv[0][t] * fc[0][t] + dv[1][t] * fc[1][t] + dv[2][t] * fc[2][t];
+      dfick += dv[0][t] * ff[0][t] + dv[1][t] * ff[1][t] + dv[2][t] * ff[2][t];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) fm[d] += im[d][t] * (fc[d][t] + ff[d][t]);
+    }
+    const double cpk = cp_lds(cr + sp * 12, T);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) eT = eT + cpk * fm[d] * tg[d];
+    if (p.corr) p.corr[(int64_t)sp * g.plane + o] = dcor * p.dt;
+    if (p.src) p.src[(int64_t)(g.isc_sc0 + sp) * g.plane + o] += dcor * p.dt;
+    if (p.dgp) {
+      const int slot = sp == p.i_h2o ? 0 : (sp == p.i_co ? 1 : (sp == p.i_co2 ? 2 : -1));
+      if (slot >= 0) p.dgp[(int64_t)slot * g.plane + o] = dfick + dcor;
+    }
+  }
+  p.eT[blockIdx.y * g.plane + o] = eT;
+}
+
+// The temperature term: the slices' sums, radiation, the cp-gradient part, / cp
+template <int ST1, int ST2>
+__global__ __launch_bounds__(256) void diff_temp_kernel(DiffParams p, Brick bk, int sc_T) {
+  const DiffGeom& g = p.gm;
+  int q, z;
+  if (!brick_cell(bk, q, z)) return;
+  const int nx = g.imax_ - g.imin_ + 1;
+  const int i = g.imin_ + q % nx, j = g.jmin_ + q / nx, k = g.kmin_ + z;
+  if (wall(g, p.mask, i, j)) return;
+  const int64_t o = c3(g, i, j, k);
+  const double* Tf = p.sc + (int64_t)g.isc_T0 * g.plane;
+  double tg[3], cg[3];
+  cell_gradient<ST1 + ST2>(p, Tf, i, j, o, tg);
+  cell_gradient<ST1 + ST2>(p, p.cpm, i, j, o, cg);
+  double eT = p.eT[o];
+  for (int q = 1; q < p.nslice; ++q) eT += p.eT[q * g.plane + o];
+  if (p.gasrad) eT += gas_radiation(p, Tf[o], o);
+  const double dT = p.diff[(int64_t)g.isc_T0 * g.plane + o];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) eT = eT + dT * cg[d] * tg[d];
+  eT = eT / p.cpm[o] * p.dt;
+  if (p.corr) p.corr[(int64_t)sc_T * g.plane + o] = eT;
+  if (p.src) p.src[(int64_t)g.isc_T0 * g.plane + o] += eT;
+}
+
+template <int NEQ, bool MOLAR, int ST1, int ST2>
+void launch_wide(const DiffParams& p, const Brick& bf, const Brick& bm, hipStream_t s) {
+  const dim3 gf(bf.per_xcd * kXcd, p.nslice), gc(bm.per_xcd * kXcd, p.nslice), b(256);
+  hipLaunchKernelGGL((diff_vel_kernel<NEQ, MOLAR, ST1, ST2>), gf, b, 0, s, p, bf);
+  for (int sp0 = 0; sp0 < NEQ - 1; sp0 += p.nchunk) {
+    const int nsp = NEQ - 1 - sp0 < p.nchunk ? NEQ - 1 - sp0 : p.nchunk;
+    hipLaunchKernelGGL((diff_flux_kernel<NEQ, MOLAR, ST1, ST2>), gf, b, 0, s, p, bf, sp0, nsp);
+    hipLaunchKernelGGL((diff_div_kernel<NEQ, ST1, ST2>), gc, b, 0, s, p, bm, sp0, nsp);
+  }
+  hipLaunchKernelGGL((diff_temp_kernel<ST1, ST2>), dim3(bm.per_xcd * kXcd), b, 0, s, p, bm, NEQ - 1);
+}
+
 }  // namespace tgr
 
 using namespace tgr;
@@ -603,16 +901,18 @@ extern "C" int tgr_launch_diffusion(const DiffParams* p, int neq, hipStream_t s)
                         (g.kmax_ - g.kmin_ + 1 + st1 + st2);
   const int64_t nint = (int64_t)(g.imax_ - g.imin_ + 1) * (g.jmax_ - g.jmin_ + 1) * (g.kmax_ - g.kmin_ + 1);
   auto blocks = [](int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 256, 65535); };
-  // second order (the reference's default stencil) has its own pair of
-  // kernels, which address a plane by 32-bit byte offsets; other orders and
+  // second order (the reference's default stencil) and fourth order have their
+  // own kernels, which address a plane by 32-bit byte offsets; other widths and
   // larger planes take the general ones
-  const bool o2 = st1 == 0 && st2 == 1 && g.plane < ((int64_t)1 << 29);
+  const bool small = diff_small_plane(g.plane);
+  const bool o2 = small && st1 == 0 && st2 == 1, o4 = p->nchunk > 0;
   auto brick = [](int64_t ni, int64_t nj, int64_t nk) {
     const int64_t pl = ni * nj, chunks = (pl + 255) / 256, strips = (chunks + kStrip - 1) / kStrip;
     return Brick{(int)pl, (int)nk, (int)((strips * kStrip * nk + kXcd - 1) / kXcd)};
   };
   const int nx = g.imax_ - g.imin_ + 1, ny = g.jmax_ - g.jmin_ + 1, nz = g.kmax_ - g.kmin_ + 1;
   const Brick bs = brick(nx + 2, ny + 2, nz + 2), bm = brick(nx, ny, nz);
+  const Brick bf = brick(nx + st1 + st2, ny + st1 + st2, nz + st1 + st2);
 #define TGR_DIFF_LAUNCH2(NEQ_, MOLAR_)                                                                        \
   hipLaunchKernelGGL((diff_sums2_kernel<NEQ_, MOLAR_>), dim3(bs.per_xcd * kXcd), dim3(256), 0, s, *p, bs);   \
   hipLaunchKernelGGL((diff_main2_kernel<NEQ_, MOLAR_>), dim3(bm.per_xcd * kXcd), dim3(256), 0, s, *p, bm);
@@ -621,6 +921,10 @@ extern "C" int tgr_launch_diffusion(const DiffParams* p, int neq, hipStream_t s)
     TGR_DIFF_LAUNCH2(NEQ_, true)                                                                \
   } else if (o2) {                                                                              \
     TGR_DIFF_LAUNCH2(NEQ_, false)                                                               \
+  } else if (o4) {                                                                              \
+    hipLaunchKernelGGL(diff_cell_kernel<NEQ_>, dim3(blocks(ncell)), dim3(256), 0, s, *p);     \
+    if (p->molar) launch_wide<NEQ_, true, 1, 2>(*p, bf, bm, s);                                 \
+    else launch_wide<NEQ_, false, 1, 2>(*p, bf, bm, s);                                         \
   } else {                                                                                      \
     hipLaunchKernelGGL(diff_cell_kernel<NEQ_>, dim3(blocks(ncell)), dim3(256), 0, s, *p);     \
     hipLaunchKernelGGL(diff_face_kernel<NEQ_>, dim3(blocks(nface)), dim3(256), 0, s, *p);     \

@@ -293,3 +293,37 @@ def test_dense_solves_match_numpy(emu, oracle, workload):
             worst[w] = max(worst[w], e / kappa)
             assert e <= 2e-14 * kappa, (c, w, e, kappa)
     print("\n%s: worst error / condition number: LU %.1e, Gauss-Jordan %.1e" % (workload, *worst))
+
+
+def test_pivot_choice_by_words(emu):
+    """The pivot search takes the largest high words first and the low words
+    among equal ones: first columns whose entries share their high word, tie
+    exactly, are subnormal (high word zero), or are all NaN, and a later column
+    of zeros; the last two are reported as that column by both solves."""
+    neq = 10
+    rng = np.random.default_rng(8)
+    base = rng.uniform(-1.0, 1.0, (neq, neq)) + 4.0 * np.eye(neq)[::-1]
+    near = base.copy()
+    near[:, 0] = 1.5 + rng.permutation(neq) * 2.0 ** -48  # one high word, ten low words
+    tie = base.copy()
+    tie[:, 0] = np.where(np.arange(neq) % 2, 1.5, -1.5)
+    tiny = base.copy()
+    tiny[:, 0] = rng.permutation(neq) * 5e-324 * 3.0e6  # high word zero, one entry zero
+    nan, zero = base.copy(), base.copy()
+    nan[:, 0] = np.nan
+    zero[:, 3] = 0.0
+    a = np.ascontiguousarray(np.array([near, tie, tiny, nan, zero]))
+    n = len(a)
+    x = rng.uniform(0.5, 1.5, (n, neq))
+    b = np.ascontiguousarray(np.einsum("nij,nj->ni", a, x))
+    xlu, xinv = np.zeros((n, neq)), np.zeros((n, neq))
+    info = np.zeros((n, 2), dtype=np.int32)
+    assert emu.emu_linsolve(neq, n, a.ctypes.data, b.ctypes.data, xlu.ctypes.data, xinv.ctypes.data,
+                            info.ctypes.data) == 0
+    assert info[:2].tolist() == [[0, 0]] * 2 and info[3].tolist() == [1, 1] and info[4].tolist() == [4, 4], info
+    # the subnormal column is found (its reciprocal pivot overflows, so only the choice is compared)
+    assert info[2].tolist() != [1, 1]
+    for c in range(2):
+        kappa = np.linalg.cond(a[c], np.inf)
+        for got in (xlu[c], xinv[c]):
+            assert np.abs(got - x[c]).max() <= 2e-14 * kappa * np.abs(x[c]).max(), c

@@ -380,7 +380,10 @@ __device__ __forceinline__ void load_rows(uint16_t* As, const uint16_t* x, int64
   }
 }
 
-// Inference: 16 MT rows through all layers.
+// Inference: 16 MT rows through all layers.  262,144 rows of the 64-256-256-256-256-64
+// network: 603 -> 355 us, 339 TFLOP/s on the padded widths.  A wave's weight loads,
+// LDS fragments, products and GELU follow one another, and the other waves of its
+// SIMD overlap them in part only; held to six waves a SIMD (80 registers) 422 us.
 template <int MT>
 __global__ __launch_bounds__(64 * kFusedWaves) void mlp_infer_kernel(FusedArgs g) {
   __shared__ __attribute__((aligned(16))) uint16_t As[16 * MT * kActRow];
@@ -428,7 +431,9 @@ __global__ __launch_bounds__(64 * kFusedWaves) void mlp_infer_kernel(FusedArgs g
 // next product's weights (16 columns, at most 256 deep) before it finishes the
 // present one, and GELU' is formed with GELU (one erf).  Leaves the layers'
 // inputs and output gradients transposed in HBM (rows in the fast index, four a
-// lane), which is what the weight gradients' products contract over.
+// lane), which is what the weight gradients' products contract over.  4,096 rows:
+// 48 us; a training step 323 -> 89 us (33 launches before), of it the weight
+// gradients 22 and the sums with Adam 9 us.
 template <int MT>
 __global__ __launch_bounds__(64 * kTrainWaves) void mlp_train_kernel(FusedArgs g) {
   __shared__ __attribute__((aligned(16))) uint16_t As[16 * MT * kActRow];

@@ -444,7 +444,7 @@ def bench_diffusion(a, torch, fc, mech, Y, T, rho, P, dt, nx, sp):
            "roofline": {"bound": "hbm", "achieved": B / ks / 1e9, "peak": PEAK_HBM / 1e9, "unit": "GB/s",
                         "frac": B / ks / PEAK_HBM, "traffic": None, "kernel_ms": ks * 1e3,
                         "algorithmic_bytes_per_call": B,
-                        "kernel": "tgr::diff_sums2_kernel + diff_main2_kernel (one call)"}}
+                        "kernel": "tgr::diff_cell_kernel + diff_face2_kernel + diff_main2_kernel (one call)"}}
     tr = traffic_record(a.workload, "tgr::diff_")
     if tr:
         out["roofline"]["traffic"] = tr["hbm_bytes_per_launch"]

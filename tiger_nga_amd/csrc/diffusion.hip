@@ -18,7 +18,7 @@
 //                     grad_m(T), the H2O / CO / CO2 dump, gas radiation, the
 //                     cp-gradient term, / cp, * dt, and the optional update of
 //                     the transport source.
-// Second order has a pair of its own (diff_sums2_kernel, diff_main2_kernel), and
+// Second order has a pair of its own (diff_face2_kernel, diff_main2_kernel), and
 // fourth order stores the face fluxes (diff_vel_kernel and the three after it).
 // Readings where the reference text does not conform (the CPU oracle's too):
 // SC(i-st2:j+st1) at 652 read as i+st1; the z sections k-st2:k-st1 at
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256) void diff_cell_kernel(DiffParams p) {
   stage_cp<NEQ>(cps, p.mech.tab);
   const DiffGeom& g = p.gm;
   const int64_t n = (int64_t)g.nxo * g.nyo * g.nzo;
-  const TGR_CONST double* iw = (const TGR_CONST double*)(p.mech.tab + L.iw);  // 1 / W_k
+  const TGR_CONST double* W = (const TGR_CONST double*)(p.mech.tab + L.w);
   for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
     const int i = g.imino_ + (int)(c % g.nxo), j = g.jmino_ + (int)((c / g.nxo) % g.nyo);
     double w = 1.0, cp = 0.0;
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(256) void diff_cell_kernel(DiffParams p) {
         const double yk = Y[k * g.plane];
         const double y = fmin(fmax(yk, 0.0), 1.0);
         s1 += y;
-        s2 = fma(y, iw[k], s2);
+        s2 += y / W[k];
         cp += yk * cp_lds(cr + k * 12, T);
       }
       w = s1 / s2;
@@ -332,103 +332,97 @@ __global__ __launch_bounds__(256) void diff_main_kernel(DiffParams p) {
 }
 
 // ---- second order (st1 = 0, st2 = 1) ----------------------------------------
-// Two passes over the species fields: diff_sums2_kernel (W_gp, cp_mix and the
-// correction velocities, whose species sums the second pass needs complete)
-// and diff_main2_kernel (the per-cell terms).  Both are bound by the rate at
-// which the L1 serves the loads of Y and D (0.6 accesses per clock and CU,
-// VALU busy a quarter of the time): each species costs a cell 8 (14) of them
-// and about 35 (105) FP64 instructions, so
+// After diff_cell_kernel: diff_face2_kernel (the correction velocities, whose
+// species sums the next pass needs complete) and diff_main2_kernel (the
+// per-cell terms).  Both are bound by the rate at which the L1 serves the loads
+// of Y and D (0.6 accesses per clock and CU, VALU busy a quarter of the time):
+// each species costs a cell 8 (14) of them and about 35 (105) FP64 instructions,
+// so
 //   * everything that does not depend on the species is formed before the
 //     species loop (operator coefficients, w / W_gp, sum grad * W_gp, the
-//     correction velocity, and the products of the divergence and enthalpy
-//     weights), and the loop loads the next species while it computes one;
+//     correction velocity), and the loop loads the next species while it
+//     computes one;
 //   * the cp coefficients are read from LDS, where the lanes of a wave differ
 //     only in the temperature range;
 //   * workgroups that share stencil planes run on the same XCD at the same
-//     time (Brick below), so that the y and z neighbours are L2 hits.
-// GRI-3.0 128^3, molar term on: 2.37 -> 1.36 ms a call (separate W_gp / cp pass
-// 0.25 ms and face sums 0.44 ms -> 0.53 ms; main 1.79 -> 0.83 ms).
+//     time (Brick above), so that the y and z neighbours are L2 hits.
+// Every product and sum is rounded as the reference's text orders them (the
+// molar factor apart: w (Y / W_gp) is (w / W_gp) Y).  Beside a wall, where W_gp
+// jumps to 1, the molar fluxes of the species nearly cancel in the temperature
+// term, and another order of the sums (the velocities' molar part summed apart,
+// the divergence and enthalpy weights folded into the fluxes') moves single
+// cells by up to 2.3e-12 of the field (2,000 random blocks).  GRI-3.0 128^3,
+// molar term on: 2.37 -> 1.52 ms a call; in that other order 1.36.
 
-// W_gp and cp_mix of the interior and one cell around it, correction
-// velocities at the face cells (diff_cell_kernel and diff_face_kernel; a face
-// interpolates its cell and the one before it).  The molar term
-// sum_k a_k (w0 Y0_k / W0 + w1 Y1_k / W1) is summed as (w0 / W0) sum a_k Y0_k +
-// (w1 / W1) sum a_k Y1_k, so that W_gp of the four cells can be summed in the
-// same pass instead of being read back.
+// correction velocities at the face cells (diff_face_kernel; a face
+// interpolates its cell and the one before it in each direction)
 template <int NEQ, bool MOLAR>
-__global__ __launch_bounds__(256) void diff_sums2_kernel(DiffParams p, Brick bk) {
+__global__ __launch_bounds__(256) void diff_face2_kernel(DiffParams p, Brick bk) {
   constexpr int N = NEQ - 1;
-  constexpr TabLayout L = tab_layout<NEQ>();
-  __shared__ __attribute__((aligned(16))) double cps[N * 12];
-  stage_cp<NEQ>(cps, p.mech.tab);
   const DiffGeom& g = p.gm;
   const tgr_metric_dev& m = p.m;
   int q, z;
   if (!brick_cell(bk, q, z)) return;
   const int fni = g.imax_ + 1 - g.imin_ + 1, fnj = g.jmax_ + 1 - g.jmin_ + 1;  // face range
-  const int i = g.imin_ - 1 + q % (fni + 1), j = g.jmin_ - 1 + q / (fni + 1), k = g.kmin_ - 1 + z;
+  const int i = g.imin_ + q % fni, j = g.jmin_ + q / fni, k = g.kmin_ + z;
   const int64_t o = c3(g, i, j, k);
-  const bool face = i >= g.imin_ && j >= g.jmin_ && k >= g.kmin_;
   if (wall(g, p.mask, i, j)) {
-    p.wg[o] = 1.0;
-    p.cpm[o] = 0.0;
-    if (face) p.cvel[o] = p.cvel[g.plane + o] = p.cvel[2 * g.plane + o] = 0.0;
+    p.cvel[o] = p.cvel[g.plane + o] = p.cvel[2 * g.plane + o] = 0.0;
     return;
   }
-  const double T = p.sc[(int64_t)g.isc_T0 * g.plane + o];
-  // offsets of the cell and of the ones before it (the cell itself outside the face range)
-  const unsigned oc = (unsigned)o * 8u;
-  unsigned on[3] = {oc, oc, oc};
-  double w[3][2] = {}, gg[3][2] = {};
-  bool wn[3] = {false, false, false};
-  if (face) {
-    on[0] = oc - 8u;
-    on[1] = oc - (unsigned)g.nxo * 8u;
-    on[2] = oc - (unsigned)g.nxo * (unsigned)g.nyo * 8u;
-    wn[0] = wall(g, p.mask, i - 1, j);
-    wn[1] = wall(g, p.mask, i, j - 1);
+  // coefficients of the two stencil points (s = -1, 0) per direction
+  const int64_t step[3] = {1, g.nxo, (int64_t)g.nxo * g.nyo};
+  double w[3][2], gg[3][2], wi[3][2], gw[3];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      w[0][t] = op(m.interp_sc_x, i, g.imin_, fni, j, g.jmino_, g.nyo, t - 1, -1);
-      w[1][t] = op(m.interp_sc_y, i, g.imino_, g.nxo, j, g.jmin_, fnj, t - 1, -1);
-      w[2][t] = op(m.interp_sc_z, i, g.imino_, g.nxo, j, g.jmin_, fnj, t - 1, -1);
-      gg[0][t] = op(m.grad_x, i, g.imin_, fni, j, g.jmin_, fnj, t - 1, -1);
-      gg[1][t] = op(m.grad_y, i, g.imin_, fni, j, g.jmin_, fnj, t - 1, -1);
-      gg[2][t] = op(m.grad_z, i, g.imin_, fni, j, g.jmin_, fnj, t - 1, -1);
+  for (int t = 0; t < 2; ++t) {
+    w[0][t] = op(m.interp_sc_x, i, g.imin_, fni, j, g.jmino_, g.nyo, t - 1, -1);
+    w[1][t] = op(m.interp_sc_y, i, g.imino_, g.nxo, j, g.jmin_, fnj, t - 1, -1);
+    w[2][t] = op(m.interp_sc_z, i, g.imino_, g.nxo, j, g.jmin_, fnj, t - 1, -1);
+    gg[0][t] = op(m.grad_x, i, g.imin_, fni, j, g.jmin_, fnj, t - 1, -1);
+    gg[1][t] = op(m.grad_y, i, g.imin_, fni, j, g.jmin_, fnj, t - 1, -1);
+    gg[2][t] = op(m.grad_z, i, g.imin_, fni, j, g.jmin_, fnj, t - 1, -1);
+  }
+  if constexpr (MOLAR) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const double w0 = p.wg[o - step[d]], w1 = p.wg[o];
+      gw[d] = 0.0;
+      gw[d] += gg[d][0] * w0;
+      gw[d] += gg[d][1] * w1;
+      wi[d][0] = 1.0 / w0;
+      wi[d][1] = 1.0 / w1;
     }
   }
+  const unsigned oc = (unsigned)o * 8u;
+  const unsigned on[3] = {oc - 8u, oc - (unsigned)g.nxo * 8u, oc - (unsigned)g.nxo * (unsigned)g.nyo * 8u};
   const double* __restrict__ Y = p.sc + (int64_t)g.isc_sc0 * g.plane;
   const double* __restrict__ D = p.diff + (int64_t)g.isc_sc0 * g.plane;
-  const TGR_CONST double* iw = (const TGR_CONST double*)(p.mech.tab + L.iw);  // 1 / W_k
-  const double* cr = cps + (T > p.mech.tmid ? 6 : 0);
   double yc = ldo(Y, oc), dc = ldo(D, oc), yn[3], dn[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) yn[d] = ldo(Y, on[d]), dn[d] = ldo(D, on[d]);
-  double fick[3] = {}, m0[3] = {}, m1[3] = {}, s1 = 0.0, s2 = 0.0, t1[3] = {}, t2[3] = {}, cp = 0.0;
+  double acc[3] = {0.0, 0.0, 0.0};
 #pragma unroll 1
   for (int sp = 0; sp < N; ++sp) {
-    const int64_t step = sp + 1 < N ? g.plane : 0;
-    Y += step;
-    D += step;
+    const int64_t next = sp + 1 < N ? g.plane : 0;
+    Y += next;
+    D += next;
     const double yc2 = ldo(Y, oc), dc2 = ldo(D, oc);
     double yn2[3], dn2[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) yn2[d] = ldo(Y, on[d]), dn2[d] = ldo(D, on[d]);
-    const double r = iw[sp];
-    const double y = fmin(fmax(yc, 0.0), 1.0);
-    s1 += y;
-    s2 = fma(y, r, s2);
-    cp += yc * cp_lds(cr + sp * 12, T);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      const double a = w[d][0] * dn[d] + w[d][1] * dc;
-      fick[d] += a * (gg[d][0] * yn[d] + gg[d][1] * yc);
+      double a = 0, b = 0;
+      a += w[d][0] * dn[d];
+      b += gg[d][0] * yn[d];
+      a += w[d][1] * dc;
+      b += gg[d][1] * yc;
+      acc[d] += a * b;
       if constexpr (MOLAR) {
-        m0[d] = fma(a, yn[d], m0[d]);
-        m1[d] = fma(a, yc, m1[d]);
-        const double yt = fmin(fmax(yn[d], 0.0), 1.0);
-        t1[d] += yt;
-        t2[d] = fma(yt, r, t2[d]);
+        double ii = 0;
+        ii += w[d][0] * (yn[d] * wi[d][0]);
+        ii += w[d][1] * (yc * wi[d][1]);
+        acc[d] += a * ii * gw[d];
       }
     }
     yc = yc2;
@@ -436,30 +430,16 @@ __global__ __launch_bounds__(256) void diff_sums2_kernel(DiffParams p, Brick bk)
 #pragma unroll
     for (int d = 0; d < 3; ++d) yn[d] = yn2[d], dn[d] = dn2[d];
   }
-  const double wc = s1 / s2;
-  p.wg[o] = wc;
-  p.cpm[o] = p.cv ? cp - 8314.34 / wc : cp;
-  if (!face) return;
 #pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    double v = fick[d];
-    if constexpr (MOLAR) {
-      const double wb = wn[d] ? 1.0 : t1[d] / t2[d];
-      v += (w[d][0] / wb * m0[d] + w[d][1] / wc * m1[d]) * (gg[d][0] * wb + gg[d][1] * wc);
-    }
-    p.cvel[d * g.plane + o] = v;
-  }
+  for (int d = 0; d < 3; ++d) p.cvel[d * g.plane + o] = acc[d];
 }
 
-// The per-cell terms (diff_main_kernel: faces at the cell and the next one in
-// each direction, each interpolating two cells).  Per face and species, with
-// the weights below, a = w0 D0 + w1 D1, the Fickian flux f = a (g0 Y0 + g1 Y1) and
-// the correction c = v (w0 Y0 + w1 Y1) + a (u0 Y0 + u1 Y1); the species term sums
-// dv c, the enthalpy flux cp_k sum e (c + f), the dump dv c and dv f.
+// What a face of a cell (diff_main_kernel: at the cell and the next one in each
+// direction, each interpolating two cells) has that does not depend on the
+// species: interpolation and gradient weights, -correction velocity, the molar
+// term's w / W_gp and sum grad * W_gp.
 struct FaceW {
-  double w0, w1, g0, g1;  // interpolation and gradient weights
-  double v, u0, u1;       // -correction velocity; molar term: w / W_gp times sum grad * W_gp
-  double dv, e;           // divergence weight; interp_m weight times the cell's T gradient
+  double w0, w1, g0, g1, v, u0, u1, gw;
 };
 
 // Y and D at a cell and its neighbours: the cell, then -, + in x, y, z
@@ -467,13 +447,13 @@ struct Stencil {
   double y[7], d[7];
 };
 
-__device__ __forceinline__ void load_stencil(Stencil& s, const double* Y, const double* D, unsigned oc, unsigned oxp,
-                                             unsigned oyp, int64_t sy, int64_t sz) {
+__device__ __forceinline__ void load_stencil(Stencil& s, const double* Y, const double* D, unsigned oc, int64_t sy,
+                                             int64_t sz) {
   s.y[0] = ldo(Y, oc), s.d[0] = ldo(D, oc);
   s.y[1] = ldo(Y - 1, oc), s.d[1] = ldo(D - 1, oc);
-  s.y[2] = ldo(Y, oxp), s.d[2] = ldo(D, oxp);
+  s.y[2] = ldo(Y + 1, oc), s.d[2] = ldo(D + 1, oc);
   s.y[3] = ldo(Y - sy, oc), s.d[3] = ldo(D - sy, oc);
-  s.y[4] = ldo(Y, oyp), s.d[4] = ldo(D, oyp);
+  s.y[4] = ldo(Y + sy, oc), s.d[4] = ldo(D + sy, oc);
   s.y[5] = ldo(Y - sz, oc), s.d[5] = ldo(D - sz, oc);
   s.y[6] = ldo(Y + sz, oc), s.d[6] = ldo(D + sz, oc);
 }
@@ -506,18 +486,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
       tg[d] += c * Tf[o + s * step[d]];
       cg[d] += c * p.cpm[o + s * step[d]];
     }
-  // wall faces carry no flux (the z faces of a non-wall cell are never walls):
-  // weights 0 and the cell itself as the neighbour, whose values are finite
-  const bool live[3] = {!wall(g, p.mask, i + 1, j), !wall(g, p.mask, i, j + 1), true};
+  // wall faces carry no flux (the z faces of a non-wall cell are never walls)
+  const bool live[3][2] = {{true, !wall(g, p.mask, i + 1, j)}, {true, !wall(g, p.mask, i, j + 1)}, {true, true}};
   FaceW fw[3][2];
+  double dv[3][2], im[3][2];
 #pragma unroll
   for (int d = 0; d < 3; ++d)
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
       // the face cell is (i, j, k) + f along d; its two points are (-1, 0) for f = 0 and (0, +1) for f = 1
       FaceW& F = fw[d][f];
-      F = FaceW{};
-      if (f && !live[d]) continue;
       const int fi = d == 0 ? i + f : i, fj = d == 1 ? j + f : j;
       const int64_t fo = o + f * step[d];
       if (d == 0) {
@@ -534,17 +512,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
       F.v = -p.cvel[d * g.plane + fo];
       if constexpr (MOLAR) {
         const double wa = p.wg[fo - step[d]], wb = p.wg[fo];
-        const double gw = F.g0 * wa + F.g1 * wb;
-        F.u0 = F.w0 / wa * gw;
-        F.u1 = F.w1 / wb * gw;
+        F.u0 = F.w0 / wa;
+        F.u1 = F.w1 / wb;
+        F.gw = F.g0 * wa + F.g1 * wb;
       }
-      const double* dv = d == 0 ? p.m.div_u : (d == 1 ? p.m.div_v : p.m.div_w);
-      const double* im = d == 0 ? p.m.interp_u_xm : (d == 1 ? p.m.interp_v_ym : p.m.interp_w_zm);
-      F.dv = op(dv, i, g.imin_, nx, j, g.jmin_, ny, f, 0);
-      F.e = op(im, i, g.imin_, nx, j, g.jmin_, ny, f, 0) * tg[d];
+      const double* du = d == 0 ? p.m.div_u : (d == 1 ? p.m.div_v : p.m.div_w);
+      const double* iu = d == 0 ? p.m.interp_u_xm : (d == 1 ? p.m.interp_v_ym : p.m.interp_w_zm);
+      dv[d][f] = op(du, i, g.imin_, nx, j, g.jmin_, ny, f, 0);
+      im[d][f] = op(iu, i, g.imin_, nx, j, g.jmin_, ny, f, 0);
     }
   const unsigned oc = (unsigned)o * 8u;
-  const unsigned oxp = live[0] ? oc + 8u : oc, oyp = live[1] ? oc + (unsigned)sy * 8u : oc;
   const double* __restrict__ Y = p.sc + (int64_t)g.isc_sc0 * g.plane;
   const double* __restrict__ D = p.diff + (int64_t)g.isc_sc0 * g.plane;
   const double* cr = cps + (T > p.mech.tmid ? 6 : 0);
@@ -553,31 +530,45 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
   double* __restrict__ dgp = p.dgp;
   double eT = 0.0;  // temperature term before the cp-gradient part and / cp
   Stencil s;
-  load_stencil(s, Y, D, oc, oxp, oyp, sy, sz);
+  load_stencil(s, Y, D, oc, sy, sz);
 #pragma unroll 1
   for (int sp = 0; sp < N; ++sp) {
     const int64_t next = sp + 1 < N ? g.plane : 0;
     Y += next;
     D += next;
     Stencil s2;
-    load_stencil(s2, Y, D, oc, oxp, oyp, sy, sz);
-    double dcor = 0.0, dfick = 0.0, en = 0.0;
+    load_stencil(s2, Y, D, oc, sy, sz);
+    double dcor = 0.0, dfick = 0.0, fm[3] = {0.0, 0.0, 0.0};
+    double fc[3][2], ff[3][2];
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
+    for (int d = 0; d < 3; ++d)
 #pragma unroll
-      for (int d = 0; d < 3; ++d) {
+      for (int f = 0; f < 2; ++f) {
         const FaceW& F = fw[d][f];
         const double y0 = f ? s.y[0] : s.y[2 * d + 1], y1 = f ? s.y[2 * d + 2] : s.y[0];
         const double d0 = f ? s.d[0] : s.d[2 * d + 1], d1 = f ? s.d[2 * d + 2] : s.d[0];
-        const double a = F.w0 * d0 + F.w1 * d1;
-        double c = F.v * (F.w0 * y0 + F.w1 * y1);
-        if constexpr (MOLAR) c += a * (F.u0 * y0 + F.u1 * y1);
-        const double fick = a * (F.g0 * y0 + F.g1 * y1);
-        dcor += F.dv * c;
-        dfick += F.dv * fick;
-        en += F.e * (c + fick);
+        double syf = 0, a = 0, b = 0;
+        syf += F.w0 * y0;
+        a += F.w0 * d0;
+        b += F.g0 * y0;
+        syf += F.w1 * y1;
+        a += F.w1 * d1;
+        b += F.g1 * y1;
+        double c = F.v * syf;
+        if constexpr (MOLAR) c += a * (F.u0 * y0 + F.u1 * y1) * F.gw;
+        fc[d][f] = live[d][f] ? c : 0.0;
+        ff[d][f] = live[d][f] ? a * b : 0.0;
       }
-    eT += cp_lds(cr + sp * 12, T) * en;
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      dcor += dv[0][f] * fc[0][f] + dv[1][f] * fc[1][f] + dv[2][f] * fc[2][f];
+      dfick += dv[0][f] * ff[0][f] + dv[1][f] * ff[1][f] + dv[2][f] * ff[2][f];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) fm[d] += im[d][f] * (fc[d][f] + ff[d][f]);
+    }
+    const double cpk = cp_lds(cr + sp * 12, T);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) eT = eT + cpk * fm[d] * tg[d];
     if (corr) corr[(int64_t)sp * g.plane + o] = dcor * p.dt;
     if (src) src[(int64_t)(g.isc_sc0 + sp) * g.plane + o] += dcor * p.dt;
     if (dgp) {
@@ -911,10 +902,11 @@ extern "C" int tgr_launch_diffusion(const DiffParams* p, int neq, hipStream_t s)
     return Brick{(int)pl, (int)nk, (int)((strips * kStrip * nk + kXcd - 1) / kXcd)};
   };
   const int nx = g.imax_ - g.imin_ + 1, ny = g.jmax_ - g.jmin_ + 1, nz = g.kmax_ - g.kmin_ + 1;
-  const Brick bs = brick(nx + 2, ny + 2, nz + 2), bm = brick(nx, ny, nz);
+  const Brick bm = brick(nx, ny, nz);
   const Brick bf = brick(nx + st1 + st2, ny + st1 + st2, nz + st1 + st2);
 #define TGR_DIFF_LAUNCH2(NEQ_, MOLAR_)                                                                        \
-  hipLaunchKernelGGL((diff_sums2_kernel<NEQ_, MOLAR_>), dim3(bs.per_xcd * kXcd), dim3(256), 0, s, *p, bs);   \
+  hipLaunchKernelGGL(diff_cell_kernel<NEQ_>, dim3(blocks(ncell)), dim3(256), 0, s, *p);                     \
+  hipLaunchKernelGGL((diff_face2_kernel<NEQ_, MOLAR_>), dim3(bf.per_xcd * kXcd), dim3(256), 0, s, *p, bf);   \
   hipLaunchKernelGGL((diff_main2_kernel<NEQ_, MOLAR_>), dim3(bm.per_xcd * kXcd), dim3(256), 0, s, *p, bm);
 #define TGR_DIFF_LAUNCH(NEQ_)                                                                  \
   if (o2 && p->molar) {                                                                         \

@@ -164,7 +164,7 @@ def test_fourth_order_workgroup_edges(torch_dev, oracle, mech, nx, ny, nz, molar
             assert np.abs(got[..., k] - want[..., k]).max() <= 1e-12 * scale + 1e-300, k
 
 
-@pytest.mark.parametrize("case", make_diffusion.CASES[:3], ids=make_diffusion.name)
+@pytest.mark.parametrize("case", make_diffusion.CASES, ids=make_diffusion.name)
 def test_walls_round_as_recorded(torch_dev, case):
     """Cells beside walls, where the molar fluxes nearly cancel and another
     order of the sums shows at 1e-12 of the field: the recorded outputs (sums in

@@ -1013,8 +1013,8 @@ int tgr_chem_diffusion_device(tgr_chem* c, double dt, const tgr_grid* g, const t
   // not to be had, the general kernels, which need five planes
   if (m->st1 == 1 && m->st2 == 2 && tgr::diff_small_plane(gm.plane)) {
     p.nchunk = (int)std::min<int64_t>(c->nsp, std::max<int64_t>(2, ((int64_t)1 << 30) / (48 * gm.plane)));
-    p.nslice = (int)std::min<int64_t>((p.nchunk + 3) / 4, std::max<int64_t>(1, 6 * 256 * (int64_t)c->n_cu / gm.plane));
-    if (c->b_diff.ensure((size_t)gm.plane * (2 + 4 * p.nslice + 6 * p.nchunk) * sizeof(double))) {
+    p.nslice = (int)std::min<int64_t>((p.nchunk + 3) / 4, std::max<int64_t>(1, 2 * 256 * (int64_t)c->n_cu / gm.plane));
+    if (c->b_diff.ensure((size_t)gm.plane * (6 + 6 * p.nchunk) * sizeof(double))) {
       (void)hipGetLastError();
       p.nchunk = p.nslice = 0;
     }
@@ -1023,8 +1023,8 @@ int tgr_chem_diffusion_device(tgr_chem* c, double dt, const tgr_grid* g, const t
   p.wg = (double*)c->b_diff.p;
   p.cpm = p.wg + gm.plane;
   p.cvel = p.cpm + gm.plane;
-  p.eT = p.cvel + 3 * p.nslice * gm.plane;
-  p.flux = p.eT + p.nslice * gm.plane;
+  p.eT = p.cvel + 3 * gm.plane;
+  p.flux = p.eT + gm.plane;
   if (tgr_launch_diffusion(&p, c->neq, (hipStream_t)stream)) return fail(TGR_E_HIP, "diffusion kernel launch failed");
   return 0;
 }

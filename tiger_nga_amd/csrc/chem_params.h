@@ -120,10 +120,10 @@ struct DiffParams {
   const int* mask;
   double* wg;     // [plane] W_gp
   double* cpm;    // [plane] cp_mix (cv)
-  double* cvel;   // [3][plane] corr_vel_x, _y, _z (fourth order: [nslice][3][plane])
+  double* cvel;   // [3][plane] corr_vel_x, _y, _z
   int nchunk;     // fourth order: species per pass through the flux workspace (0: other kernels)
-  int nslice;     // fourth order: parts that the species of a pass are split into
-  double* eT;     // [nslice][plane] temperature term by part
+  int nslice;     // fourth order: parts that the species of a pass are split into for the fluxes
+  double* eT;     // [plane] temperature term of the passes so far
   double* flux;   // [nchunk][x, y, z][corrected, Fickian][plane]
   double* corr;   // diff_corr(..., nsp + 1) or null
   double* dgp;    // diff_gp(..., 3) or null

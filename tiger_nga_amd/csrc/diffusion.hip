@@ -19,7 +19,7 @@
 //                     cp-gradient term, / cp, * dt, and the optional update of
 //                     the transport source.
 // Second order has a pair of its own (diff_face2_kernel, diff_main2_kernel), and
-// fourth order stores the face fluxes (diff_vel_kernel and the three after it).
+// fourth order stores the face fluxes (diff_vel_kernel and the two after it).
 // Readings where the reference text does not conform (the CPU oracle's too):
 // SC(i-st2:j+st1) at 652 read as i+st1; the z sections k-st2:k-st1 at
 // 634-635 and 706 read as k-st2:k+st1 (identical at second order); Cp_sp(isc)
@@ -588,79 +588,61 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
 
 // ---- wider stencils with widths known at compile time (fourth order) ----------
 // After diff_cell_kernel: the correction velocities (diff_vel_kernel), every
-// face's fluxes once per species into a workspace (diff_flux_kernel), the
-// cells' sums of them (diff_div_kernel) and the temperature term
-// (diff_temp_kernel), where diff_main_kernel has every cell recompute the fluxes
-// of its 12 faces from 4 points each.  A species costs a face 38 loads and six
-// stores and a cell 24 loads, all along x; weights and points that do not depend
-// on the species stay in registers.  The species of a pass are split into
-// nslice parts (blockIdx.y) until there are six workgroups per CU: at 16 x 17 x
-// 18 cells one part leaves three quarters of the chip without work.  The
-// workspace holds nchunk species, one pass of them at a time.
-// Bound by the fluxes' way through memory (128 bytes per cell and species at
-// half the copy rate; two or three wavefronts per SIMD give the same time, four
-// spill).  DME39, 61 x 47 x 35 cells: 1262 -> 345 us a call; GRI-3.0, 126 x 124
-// x 120: 20.2 -> 4.35 ms; 16 x 17 x 18: 824 -> 61 us.  Twelve and 24 workgroups
-// per CU: 364 and 446 us at the first of these.
+// face's fluxes once per species into a workspace (diff_flux_kernel) and the
+// cells' sums of them (diff_div_kernel), where diff_main_kernel has every cell
+// recompute the fluxes of its 12 faces from 4 points each.  Every product and
+// sum has the rounding that it has in the general kernels, so the outputs are
+// theirs to the last bit (the molar quotients are divided, and the sums over the
+// species run in their order: beside walls another order moves single cells by
+// up to 2e-12 of the field).  A thread has a face of one direction (blockIdx.y):
+// a species costs it eight loads and two stores, and a cell 24 loads, all along
+// x; weights that do not depend on the species stay in registers.  The fluxes
+// have no sum over the species, so those of a pass are split over blockIdx.z
+// until there are six workgroups per CU.  The workspace holds nchunk species, one
+// pass of them at a time.
+// DME39, 61 x 47 x 35 cells: 1144 (the general kernels) -> 354 us a call; GRI-3.0,
+// 126 x 124 x 120: 18.4 -> 5.34 ms; DME39, 16 x 17 x 18: 830 -> 87 us (294 us, 4.30
+// ms and 64 us with products for the quotients and the species' sums split over
+// workgroups).
 
-// Weights of the P = ST1 + ST2 + 1 stencil points of the faces of a cell.
+// Weights of the P = ST1 + ST2 + 1 stencil points of the faces in direction d.
 template <int P>
 struct Weights {
-  double w[3][P], g[3][P], u[3][P], gw[3];  // interpolation, gradient, w / W_gp, sum grad * W_gp
+  double w[P], g[P], wg[P], gw;  // interpolation, gradient, W_gp, sum grad * W_gp
 };
 
 template <int ST1, int ST2, bool MOLAR>
-__device__ __forceinline__ void face_weights(const DiffParams& p, int i, int j, int k,
+__device__ __forceinline__ void face_weights(const DiffParams& p, int d, int i, int j, int64_t o, int64_t step,
                                              Weights<ST1 + ST2 + 1>& F) {
-  constexpr int P = ST1 + ST2 + 1;
   const DiffGeom& g = p.gm;
   const tgr_metric_dev& m = p.m;
   const int fi0 = g.imin_ - ST1, fni = g.imax_ + ST2 - fi0 + 1, fj0 = g.jmin_ - ST1, fnj = g.jmax_ + ST2 - fj0 + 1;
-  const int64_t o = c3(g, i, j, k), step[3] = {1, g.nxo, (int64_t)g.nxo * g.nyo};
+  F.gw = 0.0;
 #pragma unroll
-  for (int d = 0; d < 3; ++d) F.gw[d] = 0.0;
-#pragma unroll
-  for (int t = 0; t < P; ++t) {
+  for (int t = 0; t < ST1 + ST2 + 1; ++t) {
     const int s = t - ST2;
-    F.w[0][t] = op(m.interp_sc_x, i, fi0, fni, j, g.jmino_, g.nyo, s, -ST2);
-    F.w[1][t] = op(m.interp_sc_y, i, g.imino_, g.nxo, j, fj0, fnj, s, -ST2);
-    F.w[2][t] = op(m.interp_sc_z, i, g.imino_, g.nxo, j, fj0, fnj, s, -ST2);
-    F.g[0][t] = op(m.grad_x, i, fi0, fni, j, fj0, fnj, s, -ST2);
-    F.g[1][t] = op(m.grad_y, i, fi0, fni, j, fj0, fnj, s, -ST2);
-    F.g[2][t] = op(m.grad_z, i, fi0, fni, j, fj0, fnj, s, -ST2);
+    F.w[t] = d == 0 ? op(m.interp_sc_x, i, fi0, fni, j, g.jmino_, g.nyo, s, -ST2)
+                    : op(d == 1 ? m.interp_sc_y : m.interp_sc_z, i, g.imino_, g.nxo, j, fj0, fnj, s, -ST2);
+    F.g[t] = op(d == 0 ? m.grad_x : (d == 1 ? m.grad_y : m.grad_z), i, fi0, fni, j, fj0, fnj, s, -ST2);
     if constexpr (MOLAR) {
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const double wg = p.wg[o + s * step[d]];
-        F.u[d][t] = F.w[d][t] / wg;
-        F.gw[d] += F.g[d][t] * wg;
-      }
+      F.wg[t] = p.wg[o + s * step];
+      F.gw += F.g[t] * F.wg[t];
     }
   }
 }
 
-// Y and D of one species at the stencil points of a cell's faces
+// Y and D of one species at the stencil points of a face
 template <int ST1, int ST2>
 struct FacePoints {
-  double y[3][ST1 + ST2 + 1], d[3][ST1 + ST2 + 1];
-  __device__ __forceinline__ void load(const double* Y, const double* D, unsigned oc, int64_t sy, int64_t sz) {
-    const int64_t step[3] = {1, sy, sz};
-    const double yc = ldo(Y, oc), dc = ldo(D, oc);
+  double y[ST1 + ST2 + 1], d[ST1 + ST2 + 1];
+  __device__ __forceinline__ void load(const double* Y, const double* D, unsigned oc, int64_t step) {
 #pragma unroll
-    for (int q = 0; q < 3; ++q)
-#pragma unroll
-      for (int t = 0; t < ST1 + ST2 + 1; ++t) {
-        y[q][t] = t == ST2 ? yc : ldo(Y + (t - ST2) * step[q], oc);
-        d[q][t] = t == ST2 ? dc : ldo(D + (t - ST2) * step[q], oc);
-      }
+    for (int t = 0; t < ST1 + ST2 + 1; ++t) {
+      y[t] = ldo(Y + (t - ST2) * step, oc);
+      d[t] = ldo(D + (t - ST2) * step, oc);
+    }
   }
 };
-
-// species [s0, s1) of n that a workgroup of slice blockIdx.y has
-__device__ __forceinline__ void slice(int n, int& s0, int& s1) {
-  s0 = n * (int)blockIdx.y / (int)gridDim.y;
-  s1 = n * ((int)blockIdx.y + 1) / (int)gridDim.y;
-}
 
 template <int STP>
 __device__ __forceinline__ void cell_gradient(const DiffParams& p, const double* f, int i, int j, int64_t o,
@@ -692,89 +674,88 @@ __device__ __forceinline__ bool face_cell(const DiffParams& p, const Brick& bk, 
 }
 
 template <int NEQ, bool MOLAR, int ST1, int ST2>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void diff_vel_kernel(DiffParams p, Brick bk) {
+__global__ __launch_bounds__(256) void diff_vel_kernel(DiffParams p, Brick bk) {
   constexpr int N = NEQ - 1, P = ST1 + ST2 + 1;
   const DiffGeom& g = p.gm;
   int i, j, k;
   if (!face_cell<ST1, ST2>(p, bk, i, j, k)) return;
-  const int64_t o = c3(g, i, j, k), sy = g.nxo, sz = (int64_t)g.nxo * g.nyo;
-  double v[3] = {0.0, 0.0, 0.0};
+  const int d = blockIdx.y;
+  const int64_t o = c3(g, i, j, k), step = d == 0 ? 1 : (d == 1 ? g.nxo : (int64_t)g.nxo * g.nyo);
+  double v = 0.0;
   if (!wall(g, p.mask, i, j)) {
     Weights<P> F;
-    face_weights<ST1, ST2, MOLAR>(p, i, j, k, F);
+    face_weights<ST1, ST2, MOLAR>(p, d, i, j, o, step, F);
     const unsigned oc = (unsigned)o * 8u;
-    int s0, s1;
-    slice(N, s0, s1);
-    const double* __restrict__ Y = p.sc + (int64_t)(g.isc_sc0 + s0) * g.plane;
-    const double* __restrict__ D = p.diff + (int64_t)(g.isc_sc0 + s0) * g.plane;
+    const double* __restrict__ Y = p.sc + (int64_t)g.isc_sc0 * g.plane;
+    const double* __restrict__ D = p.diff + (int64_t)g.isc_sc0 * g.plane;
+    FacePoints<ST1, ST2> s;
+    s.load(Y, D, oc, step);
 #pragma unroll 1
-    for (int sp = s0; sp < s1; ++sp, Y += g.plane, D += g.plane) {
-      FacePoints<ST1, ST2> s;
-      s.load(Y, D, oc, sy, sz);
+    for (int sp = 0; sp < N; ++sp) {
+      const int64_t next = sp + 1 < N ? g.plane : 0;
+      Y += next;
+      D += next;
+      FacePoints<ST1, ST2> s2;
+      s2.load(Y, D, oc, step);
+      double a = 0, b = 0, ii = 0;
 #pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        double a = 0, b = 0, ii = 0;
-#pragma unroll
-        for (int t = 0; t < P; ++t) {
-          a += F.w[d][t] * s.d[d][t];
-          b += F.g[d][t] * s.y[d][t];
-          if constexpr (MOLAR) ii += F.u[d][t] * s.y[d][t];
-        }
-        v[d] += a * b;
-        if constexpr (MOLAR) v[d] += a * ii * F.gw[d];
+      for (int t = 0; t < P; ++t) {
+        a += F.w[t] * s.d[t];
+        b += F.g[t] * s.y[t];
+        if constexpr (MOLAR) ii += F.w[t] * (s.y[t] / F.wg[t]);
       }
+      v += a * b;
+      if constexpr (MOLAR) v += a * ii * F.gw;
+      s = s2;
     }
   }
-#pragma unroll
-  for (int d = 0; d < 3; ++d) p.cvel[(3 * blockIdx.y + d) * g.plane + o] = v[d];
+  p.cvel[d * g.plane + o] = v;
 }
 
 template <int NEQ, bool MOLAR, int ST1, int ST2>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void diff_flux_kernel(DiffParams p, Brick bk,
-                                                                                                int sp0, int nsp) {
+__global__ __launch_bounds__(256) void diff_flux_kernel(DiffParams p, Brick bk, int sp0, int nsp) {
   constexpr int P = ST1 + ST2 + 1;
   const DiffGeom& g = p.gm;
   int i, j, k;
   if (!face_cell<ST1, ST2>(p, bk, i, j, k)) return;
-  const int64_t o = c3(g, i, j, k), sy = g.nxo, sz = (int64_t)g.nxo * g.nyo;
-  int s0, s1;
-  slice(nsp, s0, s1);
-  double* __restrict__ to = p.flux + 6 * s0 * g.plane + o;
+  const int d = blockIdx.y;
+  const int64_t o = c3(g, i, j, k), step = d == 0 ? 1 : (d == 1 ? g.nxo : (int64_t)g.nxo * g.nyo);
+  // this workgroup's part of the species
+  const int s0 = nsp * (int)blockIdx.z / (int)gridDim.z, s1 = nsp * ((int)blockIdx.z + 1) / (int)gridDim.z;
+  if (s0 == s1) return;
+  double* __restrict__ to = p.flux + (6 * s0 + 2 * d) * g.plane + o;
   if (wall(g, p.mask, i, j)) {  // no flux through a wall face
-    for (int q = 6 * s0; q < 6 * s1; ++q, to += g.plane) *to = 0.0;
+    for (int sp = s0; sp < s1; ++sp, to += 6 * g.plane) to[0] = to[g.plane] = 0.0;
     return;
   }
   Weights<P> F;
-  face_weights<ST1, ST2, MOLAR>(p, i, j, k, F);
-  double v[3];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    double c = p.cvel[d * g.plane + o];
-    for (int q = 1; q < (int)gridDim.y; ++q) c += p.cvel[(3 * q + d) * g.plane + o];
-    v[d] = -c;
-  }
+  face_weights<ST1, ST2, MOLAR>(p, d, i, j, o, step, F);
+  const double v = -p.cvel[d * g.plane + o];
   const unsigned oc = (unsigned)o * 8u;
   const double* __restrict__ Y = p.sc + (int64_t)(g.isc_sc0 + sp0 + s0) * g.plane;
   const double* __restrict__ D = p.diff + (int64_t)(g.isc_sc0 + sp0 + s0) * g.plane;
+  FacePoints<ST1, ST2> s;
+  s.load(Y, D, oc, step);
 #pragma unroll 1
-  for (int sp = s0; sp < s1; ++sp, Y += g.plane, D += g.plane, to += 6 * g.plane) {
-    FacePoints<ST1, ST2> s;
-    s.load(Y, D, oc, sy, sz);
+  for (int sp = s0; sp < s1; ++sp, to += 6 * g.plane) {
+    const int64_t next = sp + 1 < s1 ? g.plane : 0;
+    Y += next;
+    D += next;
+    FacePoints<ST1, ST2> s2;
+    s2.load(Y, D, oc, step);
+    double yi = 0, a = 0, b = 0, ii = 0;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      double yi = 0, a = 0, b = 0, ii = 0;
-#pragma unroll
-      for (int t = 0; t < P; ++t) {
-        yi += F.w[d][t] * s.y[d][t];
-        a += F.w[d][t] * s.d[d][t];
-        b += F.g[d][t] * s.y[d][t];
-        if constexpr (MOLAR) ii += F.u[d][t] * s.y[d][t];
-      }
-      double c = v[d] * yi;
-      if constexpr (MOLAR) c += a * ii * F.gw[d];
-      to[2 * d * g.plane] = c;
-      to[(2 * d + 1) * g.plane] = a * b;
+    for (int t = 0; t < P; ++t) {
+      yi += F.w[t] * s.y[t];
+      a += F.w[t] * s.d[t];
+      b += F.g[t] * s.y[t];
+      if constexpr (MOLAR) ii += F.w[t] * (s.y[t] / F.wg[t]);
     }
+    double c = v * yi;
+    if constexpr (MOLAR) c += a * ii * F.gw;
+    to[0] = c;
+    to[g.plane] = a * b;
+    s = s2;
   }
 }
 
@@ -807,13 +788,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
     }
   const double* cr = cps + (T > p.mech.tmid ? 6 : 0);
   const unsigned oc = (unsigned)o * 8u;
-  int s0, s1;
-  slice(nsp, s0, s1);
-  const double* __restrict__ fl = p.flux + 6 * s0 * g.plane;
-  double eT = sp0 ? p.eT[blockIdx.y * g.plane + o] : 0.0;  // this slice's part of the temperature term
+  const double* __restrict__ fl = p.flux;
+  double eT = sp0 ? p.eT[o] : 0.0;  // temperature term of the species so far
 #pragma unroll 1
-  for (int sq = s0; sq < s1; ++sq, fl += 6 * g.plane) {
-    const int sp = sp0 + sq;
+  for (int sp = sp0; sp < sp0 + nsp; ++sp, fl += 6 * g.plane) {
     double fc[3][P], ff[3][P];
 #pragma unroll
     for (int d = 0; d < 3; ++d)
@@ -840,44 +818,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
       if (slot >= 0) p.dgp[(int64_t)slot * g.plane + o] = dfick + dcor;
     }
   }
-  p.eT[blockIdx.y * g.plane + o] = eT;
-}
-
-// The temperature term: the slices' sums, radiation, the cp-gradient part, / cp
-template <int ST1, int ST2>
-__global__ __launch_bounds__(256) void diff_temp_kernel(DiffParams p, Brick bk, int sc_T) {
-  const DiffGeom& g = p.gm;
-  int q, z;
-  if (!brick_cell(bk, q, z)) return;
-  const int nx = g.imax_ - g.imin_ + 1;
-  const int i = g.imin_ + q % nx, j = g.jmin_ + q / nx, k = g.kmin_ + z;
-  if (wall(g, p.mask, i, j)) return;
-  const int64_t o = c3(g, i, j, k);
-  const double* Tf = p.sc + (int64_t)g.isc_T0 * g.plane;
-  double tg[3], cg[3];
-  cell_gradient<ST1 + ST2>(p, Tf, i, j, o, tg);
+  if (sp0 + nsp < N) {
+    p.eT[o] = eT;
+    return;
+  }
+  double cg[3];
   cell_gradient<ST1 + ST2>(p, p.cpm, i, j, o, cg);
-  double eT = p.eT[o];
-  for (int q = 1; q < p.nslice; ++q) eT += p.eT[q * g.plane + o];
-  if (p.gasrad) eT += gas_radiation(p, Tf[o], o);
+  if (p.gasrad) eT += gas_radiation(p, T, o);
   const double dT = p.diff[(int64_t)g.isc_T0 * g.plane + o];
 #pragma unroll
   for (int d = 0; d < 3; ++d) eT = eT + dT * cg[d] * tg[d];
   eT = eT / p.cpm[o] * p.dt;
-  if (p.corr) p.corr[(int64_t)sc_T * g.plane + o] = eT;
+  if (p.corr) p.corr[(int64_t)N * g.plane + o] = eT;
   if (p.src) p.src[(int64_t)g.isc_T0 * g.plane + o] += eT;
 }
 
 template <int NEQ, bool MOLAR, int ST1, int ST2>
 void launch_wide(const DiffParams& p, const Brick& bf, const Brick& bm, hipStream_t s) {
-  const dim3 gf(bf.per_xcd * kXcd, p.nslice), gc(bm.per_xcd * kXcd, p.nslice), b(256);
-  hipLaunchKernelGGL((diff_vel_kernel<NEQ, MOLAR, ST1, ST2>), gf, b, 0, s, p, bf);
+  const dim3 gv(bf.per_xcd * kXcd, 3), gf(bf.per_xcd * kXcd, 3, p.nslice), gc(bm.per_xcd * kXcd), b(256);
+  hipLaunchKernelGGL((diff_vel_kernel<NEQ, MOLAR, ST1, ST2>), gv, b, 0, s, p, bf);
   for (int sp0 = 0; sp0 < NEQ - 1; sp0 += p.nchunk) {
     const int nsp = NEQ - 1 - sp0 < p.nchunk ? NEQ - 1 - sp0 : p.nchunk;
     hipLaunchKernelGGL((diff_flux_kernel<NEQ, MOLAR, ST1, ST2>), gf, b, 0, s, p, bf, sp0, nsp);
     hipLaunchKernelGGL((diff_div_kernel<NEQ, ST1, ST2>), gc, b, 0, s, p, bm, sp0, nsp);
   }
-  hipLaunchKernelGGL((diff_temp_kernel<ST1, ST2>), dim3(bm.per_xcd * kXcd), b, 0, s, p, bm, NEQ - 1);
 }
 
 }  // namespace tgr

@@ -147,3 +147,21 @@ def test_widths_and_batches(torch_dev, nin, nout, hidden, layers, B):
     for (dW, db), (rW, rb) in zip(mlp.unflatten(g, nin, nout, hidden, layers), gq):
         for a, r in ((dW, rW), (db, rb)):
             assert np.linalg.norm(a - r) < 1e-2 * np.linalg.norm(r)
+
+
+@pytest.mark.parametrize("B", [64, 320, 16448])
+def test_fused_forward_equals_the_layered_one(torch_dev, B):
+    """A network of 256 hidden units and the same one with 64 more of weight
+    zero, which is too wide for the fused pass and goes layer by layer: the same
+    products, sums, GELU and roundings, so the same outputs to the last bit."""
+    torch = torch_dev
+    from tiger_nga_amd import mlp
+    net, flat, _, x, _ = _net_case(torch, B=B)
+    wide = mlp.MLP(38, 37, 320, 4)
+    wflat = np.zeros(wide.nparam, dtype=np.float32)
+    for (W, b), (Wn, bn) in zip(mlp.unflatten(wflat, 38, 37, 320, 4), mlp.unflatten(flat, 38, 37, 256, 4)):
+        W[:Wn.shape[0], :Wn.shape[1]] = Wn
+        b[:bn.shape[0]] = bn
+    wide.set_params(wflat)
+    x = _bf(torch, 2.0 * x)
+    assert torch.equal(net.forward(x), wide.forward(x))

@@ -72,26 +72,6 @@ __device__ __forceinline__ float gelu_both(float x, float& d) {
   return 0.5f * x * c;
 }
 
-// GELU for inference, where the activations take longer than the products:
-// Phi(-|x|) e^(x^2/2) as a polynomial in t = 1 / (1 + 0.35 |x|), interpolated at the
-// Chebyshev points of 0 <= |x| <= 14 (4e-8 relative, so the tail keeps its digits
-// where 1 + erf cancels): 17 instructions.  Training keeps the erf form, whose
-// rounding its trajectories carry on from.
-__device__ __forceinline__ float gelu_infer(float x) {
-  const float t = __builtin_amdgcn_rcpf(fmaf(0.35f, fabsf(x), 1.0f));
-  float q = -0.029679522004471565f;
-  q = fmaf(q, t, 0.14654583029291723f);
-  q = fmaf(q, t, -0.26096122829493434f);
-  q = fmaf(q, t, 0.16505099585712943f);
-  q = fmaf(q, t, -0.02704660826705285f);
-  q = fmaf(q, t, 0.10711458759705554f);
-  q = fmaf(q, t, 0.11944491684589224f);
-  q = fmaf(q, t, 0.1399122981253345f);
-  q = fmaf(q, t, 0.13961871256104424f);
-  q *= t * __builtin_amdgcn_exp2f(-0.72134752044448170f * (x * x));
-  return x * (x < 0.0f ? q : 1.0f - q);
-}
-
 enum Act { kNone = 0, kGelu = 1, kGeluGrad = 2 };
 
 struct GemmArgs {
@@ -381,9 +361,12 @@ __device__ __forceinline__ void load_rows(uint16_t* As, const uint16_t* x, int64
 }
 
 // Inference: 16 MT rows through all layers.  262,144 rows of the 64-256-256-256-256-64
-// network: 603 -> 355 us, 339 TFLOP/s on the padded widths.  A wave's weight loads,
+// network: 603 -> 397 us, 303 TFLOP/s on the padded widths.  A wave's weight loads,
 // LDS fragments, products and GELU follow one another, and the other waves of its
-// SIMD overlap them in part only; held to six waves a SIMD (80 registers) 422 us.
+// SIMD overlap them in part only.  GELU is the layered pass's, by erf: a polynomial
+// with the hardware's reciprocal and exponential took 355 us (six waves a SIMD
+// 422), but was three times as far from GELU for positive arguments, and the
+// outputs are those of the layered pass to the last bit this way.
 template <int MT>
 __global__ __launch_bounds__(64 * kFusedWaves) void mlp_infer_kernel(FusedArgs g) {
   __shared__ __attribute__((aligned(16))) uint16_t As[16 * MT * kActRow];
@@ -413,10 +396,10 @@ __global__ __launch_bounds__(64 * kFusedWaves) void mlp_infer_kernel(FusedArgs g
           *reinterpret_cast<float4*>(g.out + (row0 + row) * N + col) = float4{v[0], v[1], v[2], v[3]};
         } else {
           ushort4 h;
-          h.x = f2bf(gelu_infer(v[0]));
-          h.y = f2bf(gelu_infer(v[1]));
-          h.z = f2bf(gelu_infer(v[2]));
-          h.w = f2bf(gelu_infer(v[3]));
+          h.x = f2bf(gelu(v[0]));
+          h.y = f2bf(gelu(v[1]));
+          h.z = f2bf(gelu(v[2]));
+          h.w = f2bf(gelu(v[3]));
           *reinterpret_cast<ushort4*>(As + row * kActRow + col) = h;
         }
       }

@@ -175,3 +175,68 @@ def test_walls_round_as_recorded(torch_dev, case):
         assert np.abs(w).max() > 0.0
         print("%s: largest difference over the rms %.1e" % (k, np.abs(a - w).max() / np.sqrt(np.mean(w * w))))
         assert np.array_equal(a, w), k
+
+
+@pytest.mark.parametrize("order", [2, 4])
+@pytest.mark.parametrize("nx,ny,nz", [(1, 1, 300), (1, 300, 2), (35, 35, 3)])
+def test_thin_blocks(torch_dev, oracle, order, nx, ny, nz):
+    """Blocks one cell wide, and a plane of several workgroups and a remainder;
+    bound as above."""
+    torch = torch_dev
+    from tiger_nga_amd.finitechem import FiniteChem
+    nover = order - 1
+    sh = (nx + 2 * nover, ny + 2 * nover, nz + 2 * nover)
+    _, Y, T, rho, P, dt = inputs.states("h2", n=499, seed=31)
+    nsp = Y.shape[1]
+    g = Grid.block(nx, ny, nz, nsp + 1, 1, nsp + 1, nover=nover)
+    pick = np.arange(np.prod(sh)) * 7919 % 499
+    SC_ = np.asfortranarray(np.concatenate([Y, T[:, None]], axis=1)[pick].reshape(sh + (nsp + 1,), order="F"))
+    RHO_ = np.asfortranarray(rho[pick].reshape(sh, order="F"))
+    rng = np.random.default_rng(8)
+    DIFF_ = np.asfortranarray(10.0 ** rng.uniform(-5.0, -4.0, SC_.shape))
+    x, y = (np.cumsum(np.concatenate([[0.0], 1e-4 * (1.0 + 0.3 * rng.random(n))])) for n in sh[:2])
+    m = metric.cartesian(g, x, y, 1.1e-4, order)
+    dc_o, gp_o = oracle.diffusion("h2", g, m, dt, RHO_, SC_, DIFF_, molar=True)
+    fc = FiniteChem("h2")
+    md = {k: (v if k in ("st1", "st2") else _dev(torch, np.asfortranarray(v))) for k, v in m.items()}
+    dc, gp = (_dev(torch, np.zeros(sh + (n,), order="F")) for n in (nsp + 1, 3))
+    fc.diffusion(dt, g, md, _dev(torch, RHO_), _dev(torch, SC_), _dev(torch, DIFF_), diff_corr=dc, diff_gp=gp, molar=True)
+    torch.cuda.synchronize()
+    fc.close()
+    for got, want in ((dc.cpu().numpy(), dc_o), (gp.cpu().numpy(), gp_o)):
+        for k in range(want.shape[-1]):
+            scale = max(np.abs(want[..., k]).max(), 1e-300)
+            assert np.abs(got[..., k] - want[..., k]).max() <= 1e-12 * scale + 1e-300, k
+
+
+def test_column_of_four_million_cells(torch_dev):
+    """1 x 1 x (2^22 + 3) cells: no more workgroups than cells / 256, which a
+    launch of whole workgroups per plane exceeds.  Its first and last 500 planes
+    equal the same planes as a block of their own."""
+    torch = torch_dev
+    from tiger_nga_amd.finitechem import FiniteChem
+    nz, part = (1 << 22) + 3, 500
+    fc = FiniteChem("h2")
+    nsp = fc.nsp
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    face = np.arange(4) * 1e-4
+
+    def run(RHO_, SC_, DIFF_, n):
+        g = Grid.block(1, 1, n, nsp + 1, 1, nsp + 1, nover=1)
+        md = {k: (v if k in ("st1", "st2") else _dev(torch, np.asfortranarray(v)))
+              for k, v in metric.cartesian(g, face, face, 1.1e-4, 2).items()}
+        fortran = lambda a: a.permute(*reversed(range(a.ndim)))
+        corr = torch.zeros(nsp + 1, n + 2, 3, 3, dtype=torch.float64, device="cuda")
+        fc.diffusion(1e-6, g, md, fortran(RHO_.contiguous()), fortran(SC_.contiguous()), fortran(DIFF_.contiguous()),
+                     diff_corr=fortran(corr), molar=True)
+        return corr
+    SC_ = torch.rand(nsp + 1, nz + 2, 3, 3, generator=gen, dtype=torch.float64, device="cuda")
+    SC_[:nsp] /= SC_[:nsp].sum(0)
+    SC_[nsp] = 400.0 + 1600.0 * SC_[nsp]
+    DIFF_ = 1e-5 + 1e-4 * torch.rand(SC_.shape, generator=gen, dtype=torch.float64, device="cuda")
+    RHO_ = torch.ones(nz + 2, 3, 3, dtype=torch.float64, device="cuda")
+    whole = run(RHO_, SC_, DIFF_, nz)
+    assert float(whole[:, 1:-1, 1, 1].abs().min()) > 0.0
+    for z in (slice(0, part + 2), slice(nz - part, nz + 2)):
+        assert torch.equal(whole[:, z][:, 1:-1], run(RHO_[z], SC_[:, z], DIFF_[:, z], part)[:, 1:-1])
+    fc.close()

@@ -995,6 +995,7 @@ int tgr_chem_diffusion_device(tgr_chem* c, double dt, const tgr_grid* g, const t
   gm.isc_sc0 = g->isc_sc - 1, gm.isc_T0 = g->isc_T - 1;
   p.m = *md;
   p.mech = c->dm;
+  p.n_cu = c->n_cu;
   p.dt = dt;
   p.molar = (flags & TGR_DIFF_MOLAR) != 0;
   p.gasrad = (flags & TGR_DIFF_GASRAD) != 0;

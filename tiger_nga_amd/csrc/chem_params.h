@@ -121,6 +121,7 @@ struct DiffParams {
   double* wg;     // [plane] W_gp
   double* cpm;    // [plane] cp_mix (cv)
   double* cvel;   // [3][plane] corr_vel_x, _y, _z
+  int n_cu;
   int nchunk;     // fourth order: species per pass through the flux workspace (0: other kernels)
   int nslice;     // fourth order: parts that the species of a pass are split into for the fluxes
   double* eT;     // [plane] temperature term of the passes so far

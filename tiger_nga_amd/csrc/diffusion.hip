@@ -63,25 +63,57 @@ __device__ __forceinline__ void cp_species(const char* tab, const TabLayout& L, 
 
 }  // namespace
 
-// Order of the workgroups: 256 consecutive cells of a plane each, kStrip of
-// them side by side, then the next plane.  The hardware deals workgroups to
-// the 8 XCDs in turn, so XCD e (blockIdx % 8) takes the e-th contiguous piece
-// of that order: its resident workgroups cover a brick of kStrip chunks by
-// some 16 planes, whose halo is a third of its volume (GRI-3.0 128^3: 1394 us in
-// the order of the planes, 1415 / 1376 / 1376 / 1436 us with strips of 2 / 4 / 8 /
-// 16).
+// Order of the workgroups: each takes consecutive cells of the range in storage
+// order, whatever its extents, so that a block one cell wide fills its waves like
+// a cube (GRI-3.0, second order, 1 x 1 x 4096 cells: 565 us with every plane
+// rounded up to whole workgroups, 55 this way; 35 x 35 x 200: 224 and 154).  The
+// workgroups of a plane, `row`, are taken kStrip at a time through all planes, then the next
+// kStrip; the hardware deals workgroups to the 8 XCDs in turn, so XCD e (blockIdx
+// % 8) takes the e-th eighth of that order: its resident workgroups cover a brick
+// of kStrip workgroups by some 16 planes, whose halo is a third of its volume
+// (GRI-3.0 128^3: 1610 us in plain order, 1504 in this one).
 constexpr int kXcd = 8, kStrip = 4;
-struct Brick {
-  int plane, nz, per_xcd;  // cells of a plane, planes, workgroups per XCD
+struct Cells {
+  int ni, nj;         // extents of the range
+  unsigned n, wg;     // its cells and workgroups
+  unsigned row;       // workgroups of a plane (rounded: the bricks lean a little)
+  unsigned threads;   // of a workgroup
 };
 
-__device__ __forceinline__ bool brick_cell(const Brick& b, int& q, int& z) {
-  const unsigned seq = (blockIdx.x % kXcd) * (unsigned)b.per_xcd + blockIdx.x / kXcd;
-  const unsigned per_strip = (unsigned)b.nz * kStrip;
-  const unsigned strip = seq / per_strip, r = seq - strip * per_strip;
-  z = (int)(r / kStrip);
-  q = (int)((strip * kStrip + r % kStrip) * 256 + threadIdx.x);
-  return q < b.plane;
+__device__ __forceinline__ bool range_cell(const Cells& c, int& i, int& j, int& k) {
+  const unsigned e = blockIdx.x % kXcd, first = (unsigned)((uint64_t)e * c.wg / kXcd),
+                 last = (unsigned)((uint64_t)(e + 1) * c.wg / kXcd), seq = first + blockIdx.x / kXcd;
+  unsigned w = seq;
+  const unsigned rows = c.row ? c.wg / c.row : 0;  // whole rows; the cells past them follow in plain order
+  if (seq < rows * c.row) {
+    const unsigned whole = c.row / kStrip * kStrip, strip = seq / (rows * kStrip) * kStrip;
+    const unsigned s0 = strip < whole ? strip : whole, width = strip < whole ? kStrip : c.row - whole;
+    const unsigned r = seq - s0 * rows;
+    w = r / width * c.row + s0 + r % width;
+  }
+  const unsigned q = w * blockDim.x + threadIdx.x, r = q / (unsigned)c.ni;
+  i = (int)(q - r * (unsigned)c.ni);
+  j = (int)(r % (unsigned)c.nj);
+  k = (int)(r / (unsigned)c.nj);
+  return seq < last && q < c.n;
+}
+
+// the cell of the face range / of the interior that this thread has
+template <int ST1, int ST2>
+__device__ __forceinline__ bool face_cell(const DiffParams& p, const Cells& cl, int& i, int& j, int& k) {
+  const bool in = range_cell(cl, i, j, k);
+  i += p.gm.imin_ - ST1;
+  j += p.gm.jmin_ - ST1;
+  k += p.gm.kmin_ - ST1;
+  return in;
+}
+
+__device__ __forceinline__ bool interior_cell(const DiffParams& p, const Cells& cl, int& i, int& j, int& k) {
+  const bool in = range_cell(cl, i, j, k);
+  i += p.gm.imin_;
+  j += p.gm.jmin_;
+  k += p.gm.kmin_;
+  return in;
 }
 
 // a[byte offset]: a wave-uniform base and a 32-bit lane offset (the launcher
@@ -94,7 +126,7 @@ __device__ __forceinline__ double ldo(const double* a, unsigned off) {
 template <int NEQ>
 __device__ __forceinline__ void stage_cp(double* cps, const char* tab) {
   constexpr TabLayout L = tab_layout<NEQ>();
-  for (int t = threadIdx.x; t < (NEQ - 1) * 12; t += 256) {
+  for (int t = threadIdx.x; t < (NEQ - 1) * 12; t += blockDim.x) {
     const int k = t / 12, hi = (t / 6) % 2, c = t % 6;
     cps[t] = *(const double*)(tab + L.th + (hi ? 0 : 13 * kRow) + (7 + c) * kRow + k * 8);
   }
@@ -345,26 +377,25 @@ __global__ __launch_bounds__(256) void diff_main_kernel(DiffParams p) {
 //   * the cp coefficients are read from LDS, where the lanes of a wave differ
 //     only in the temperature range;
 //   * workgroups that share stencil planes run on the same XCD at the same
-//     time (Brick above), so that the y and z neighbours are L2 hits.
+//     time (Cells above), so that the y and z neighbours are L2 hits.
 // Every product and sum is rounded as the reference's text orders them (the
 // molar factor apart: w (Y / W_gp) is (w / W_gp) Y).  Beside a wall, where W_gp
 // jumps to 1, the molar fluxes of the species nearly cancel in the temperature
 // term, and another order of the sums (the velocities' molar part summed apart,
 // the divergence and enthalpy weights folded into the fluxes') moves single
 // cells by up to 2.3e-12 of the field (2,000 random blocks).  GRI-3.0 128^3,
-// molar term on: 2.37 -> 1.52 ms a call; in that other order 1.36.
+// molar term on: 2.37 -> 1.50 ms a call; in that other order 1.36.
 
 // correction velocities at the face cells (diff_face_kernel; a face
 // interpolates its cell and the one before it in each direction)
 template <int NEQ, bool MOLAR>
-__global__ __launch_bounds__(256) void diff_face2_kernel(DiffParams p, Brick bk) {
+__global__ __launch_bounds__(256) void diff_face2_kernel(DiffParams p, Cells cl) {
   constexpr int N = NEQ - 1;
   const DiffGeom& g = p.gm;
   const tgr_metric_dev& m = p.m;
-  int q, z;
-  if (!brick_cell(bk, q, z)) return;
+  int i, j, k;
+  if (!face_cell<0, 1>(p, cl, i, j, k)) return;
   const int fni = g.imax_ + 1 - g.imin_ + 1, fnj = g.jmax_ + 1 - g.jmin_ + 1;  // face range
-  const int i = g.imin_ + q % fni, j = g.jmin_ + q / fni, k = g.kmin_ + z;
   const int64_t o = c3(g, i, j, k);
   if (wall(g, p.mask, i, j)) {
     p.cvel[o] = p.cvel[g.plane + o] = p.cvel[2 * g.plane + o] = 0.0;
@@ -459,16 +490,15 @@ __device__ __forceinline__ void load_stencil(Stencil& s, const double* Y, const 
 }
 
 template <int NEQ, bool MOLAR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void diff_main2_kernel(DiffParams p, Brick bk) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void diff_main2_kernel(DiffParams p, Cells cl) {
   constexpr int N = NEQ - 1;
   __shared__ __attribute__((aligned(16))) double cps[N * 12];
   stage_cp<NEQ>(cps, p.mech.tab);
   const DiffGeom& g = p.gm;
-  int q, z;
-  if (!brick_cell(bk, q, z)) return;
+  int i, j, k;
+  if (!interior_cell(p, cl, i, j, k)) return;
   const int nx = g.imax_ - g.imin_ + 1, ny = g.jmax_ - g.jmin_ + 1;
   const int fni = nx + 1, fnj = ny + 1;
-  const int i = g.imin_ + q % nx, j = g.jmin_ + q / nx, k = g.kmin_ + z;
   if (wall(g, p.mask, i, j)) return;
   const int64_t o = c3(g, i, j, k);
   const int64_t sy = g.nxo, sz = (int64_t)g.nxo * g.nyo;
@@ -600,8 +630,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
 // have no sum over the species, so those of a pass are split over blockIdx.z
 // until there are six workgroups per CU.  The workspace holds nchunk species, one
 // pass of them at a time.
-// DME39, 61 x 47 x 35 cells: 1144 (the general kernels) -> 354 us a call; GRI-3.0,
-// 126 x 124 x 120: 18.4 -> 5.34 ms; DME39, 16 x 17 x 18: 830 -> 87 us (294 us, 4.30
+// DME39, 61 x 47 x 35 cells: 1144 (the general kernels) -> 309 us a call; GRI-3.0,
+// 126 x 124 x 120: 18.4 -> 5.31 ms; DME39, 16 x 17 x 18: 830 -> 80 us (294 us, 4.30
 // ms and 64 us with products for the quotients and the species' sums split over
 // workgroups).
 
@@ -661,24 +691,12 @@ __device__ __forceinline__ void cell_gradient(const DiffParams& p, const double*
     }
 }
 
-// cell of the face range that this thread has
-template <int ST1, int ST2>
-__device__ __forceinline__ bool face_cell(const DiffParams& p, const Brick& bk, int& i, int& j, int& k) {
-  int q, z;
-  if (!brick_cell(bk, q, z)) return false;
-  const int fni = p.gm.imax_ - p.gm.imin_ + 1 + ST1 + ST2;
-  i = p.gm.imin_ - ST1 + q % fni;
-  j = p.gm.jmin_ - ST1 + q / fni;
-  k = p.gm.kmin_ - ST1 + z;
-  return true;
-}
-
 template <int NEQ, bool MOLAR, int ST1, int ST2>
-__global__ __launch_bounds__(256) void diff_vel_kernel(DiffParams p, Brick bk) {
+__global__ __launch_bounds__(256) void diff_vel_kernel(DiffParams p, Cells cl) {
   constexpr int N = NEQ - 1, P = ST1 + ST2 + 1;
   const DiffGeom& g = p.gm;
   int i, j, k;
-  if (!face_cell<ST1, ST2>(p, bk, i, j, k)) return;
+  if (!face_cell<ST1, ST2>(p, cl, i, j, k)) return;
   const int d = blockIdx.y;
   const int64_t o = c3(g, i, j, k), step = d == 0 ? 1 : (d == 1 ? g.nxo : (int64_t)g.nxo * g.nyo);
   double v = 0.0;
@@ -713,11 +731,11 @@ __global__ __launch_bounds__(256) void diff_vel_kernel(DiffParams p, Brick bk) {
 }
 
 template <int NEQ, bool MOLAR, int ST1, int ST2>
-__global__ __launch_bounds__(256) void diff_flux_kernel(DiffParams p, Brick bk, int sp0, int nsp) {
+__global__ __launch_bounds__(256) void diff_flux_kernel(DiffParams p, Cells cl, int sp0, int nsp) {
   constexpr int P = ST1 + ST2 + 1;
   const DiffGeom& g = p.gm;
   int i, j, k;
-  if (!face_cell<ST1, ST2>(p, bk, i, j, k)) return;
+  if (!face_cell<ST1, ST2>(p, cl, i, j, k)) return;
   const int d = blockIdx.y;
   const int64_t o = c3(g, i, j, k), step = d == 0 ? 1 : (d == 1 ? g.nxo : (int64_t)g.nxo * g.nyo);
   // this workgroup's part of the species
@@ -760,16 +778,15 @@ __global__ __launch_bounds__(256) void diff_flux_kernel(DiffParams p, Brick bk, 
 }
 
 template <int NEQ, int ST1, int ST2>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void diff_div_kernel(DiffParams p, Brick bk,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void diff_div_kernel(DiffParams p, Cells cl,
                                                                                                int sp0, int nsp) {
   constexpr int N = NEQ - 1, P = ST1 + ST2 + 1;
   __shared__ __attribute__((aligned(16))) double cps[N * 12];
   stage_cp<NEQ>(cps, p.mech.tab);
   const DiffGeom& g = p.gm;
-  int q, z;
-  if (!brick_cell(bk, q, z)) return;
+  int i, j, k;
+  if (!interior_cell(p, cl, i, j, k)) return;
   const int nx = g.imax_ - g.imin_ + 1, ny = g.jmax_ - g.jmin_ + 1;
-  const int i = g.imin_ + q % nx, j = g.jmin_ + q / nx, k = g.kmin_ + z;
   if (wall(g, p.mask, i, j)) return;
   const int64_t o = c3(g, i, j, k), step[3] = {1, g.nxo, (int64_t)g.nxo * g.nyo};
   const double* Tf = p.sc + (int64_t)g.isc_T0 * g.plane;
@@ -833,14 +850,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
   if (p.src) p.src[(int64_t)g.isc_T0 * g.plane + o] += eT;
 }
 
+// workgroups to launch: the same number for every XCD
+unsigned launch_groups(const Cells& c) { return (c.wg + kXcd - 1) / kXcd * kXcd; }
+
 template <int NEQ, bool MOLAR, int ST1, int ST2>
-void launch_wide(const DiffParams& p, const Brick& bf, const Brick& bm, hipStream_t s) {
-  const dim3 gv(bf.per_xcd * kXcd, 3), gf(bf.per_xcd * kXcd, 3, p.nslice), gc(bm.per_xcd * kXcd), b(256);
-  hipLaunchKernelGGL((diff_vel_kernel<NEQ, MOLAR, ST1, ST2>), gv, b, 0, s, p, bf);
+void launch_wide(const DiffParams& p, const Cells& cf, const Cells& cm, hipStream_t s) {
+  const unsigned nf = launch_groups(cf);
+  const dim3 gv(nf, 3), gf(nf, 3, p.nslice), gc(launch_groups(cm)), b(cf.threads), bc(cm.threads);
+  hipLaunchKernelGGL((diff_vel_kernel<NEQ, MOLAR, ST1, ST2>), gv, b, 0, s, p, cf);
   for (int sp0 = 0; sp0 < NEQ - 1; sp0 += p.nchunk) {
     const int nsp = NEQ - 1 - sp0 < p.nchunk ? NEQ - 1 - sp0 : p.nchunk;
-    hipLaunchKernelGGL((diff_flux_kernel<NEQ, MOLAR, ST1, ST2>), gf, b, 0, s, p, bf, sp0, nsp);
-    hipLaunchKernelGGL((diff_div_kernel<NEQ, ST1, ST2>), gc, b, 0, s, p, bm, sp0, nsp);
+    hipLaunchKernelGGL((diff_flux_kernel<NEQ, MOLAR, ST1, ST2>), gf, b, 0, s, p, cf, sp0, nsp);
+    hipLaunchKernelGGL((diff_div_kernel<NEQ, ST1, ST2>), gc, bc, 0, s, p, cm, sp0, nsp);
   }
 }
 
@@ -861,17 +882,18 @@ extern "C" int tgr_launch_diffusion(const DiffParams* p, int neq, hipStream_t s)
   // larger planes take the general ones
   const bool small = diff_small_plane(g.plane);
   const bool o2 = small && st1 == 0 && st2 == 1, o4 = p->nchunk > 0;
-  auto brick = [](int64_t ni, int64_t nj, int64_t nk) {
-    const int64_t pl = ni * nj, chunks = (pl + 255) / 256, strips = (chunks + kStrip - 1) / kStrip;
-    return Brick{(int)pl, (int)nk, (int)((strips * kStrip * nk + kXcd - 1) / kXcd)};
+  auto range = [&](int halo) {
+    const int ni = g.imax_ - g.imin_ + 1 + halo, nj = g.jmax_ - g.jmin_ + 1 + halo, nk = g.kmax_ - g.kmin_ + 1 + halo;
+    const int64_t n = (int64_t)ni * nj * nk;
+    // a wave per workgroup until every CU has four workgroups of four
+    const int64_t t = n < (int64_t)4 * 256 * p->n_cu ? 64 : 256, row = ((int64_t)ni * nj + t / 2) / t;
+    return Cells{ni, nj, (unsigned)n, (unsigned)((n + t - 1) / t), (unsigned)(row > kStrip ? row : 0), (unsigned)t};
   };
-  const int nx = g.imax_ - g.imin_ + 1, ny = g.jmax_ - g.jmin_ + 1, nz = g.kmax_ - g.kmin_ + 1;
-  const Brick bm = brick(nx, ny, nz);
-  const Brick bf = brick(nx + st1 + st2, ny + st1 + st2, nz + st1 + st2);
+  const Cells cm = range(0), cf = range(st1 + st2);
 #define TGR_DIFF_LAUNCH2(NEQ_, MOLAR_)                                                                        \
   hipLaunchKernelGGL(diff_cell_kernel<NEQ_>, dim3(blocks(ncell)), dim3(256), 0, s, *p);                     \
-  hipLaunchKernelGGL((diff_face2_kernel<NEQ_, MOLAR_>), dim3(bf.per_xcd * kXcd), dim3(256), 0, s, *p, bf);   \
-  hipLaunchKernelGGL((diff_main2_kernel<NEQ_, MOLAR_>), dim3(bm.per_xcd * kXcd), dim3(256), 0, s, *p, bm);
+  hipLaunchKernelGGL((diff_face2_kernel<NEQ_, MOLAR_>), dim3(launch_groups(cf)), dim3(cf.threads), 0, s, *p, cf); \
+  hipLaunchKernelGGL((diff_main2_kernel<NEQ_, MOLAR_>), dim3(launch_groups(cm)), dim3(cm.threads), 0, s, *p, cm);
 #define TGR_DIFF_LAUNCH(NEQ_)                                                                  \
   if (o2 && p->molar) {                                                                         \
     TGR_DIFF_LAUNCH2(NEQ_, true)                                                                \
@@ -879,8 +901,8 @@ extern "C" int tgr_launch_diffusion(const DiffParams* p, int neq, hipStream_t s)
     TGR_DIFF_LAUNCH2(NEQ_, false)                                                               \
   } else if (o4) {                                                                              \
     hipLaunchKernelGGL(diff_cell_kernel<NEQ_>, dim3(blocks(ncell)), dim3(256), 0, s, *p);     \
-    if (p->molar) launch_wide<NEQ_, true, 1, 2>(*p, bf, bm, s);                                 \
-    else launch_wide<NEQ_, false, 1, 2>(*p, bf, bm, s);                                         \
+    if (p->molar) launch_wide<NEQ_, true, 1, 2>(*p, cf, cm, s);                                 \
+    else launch_wide<NEQ_, false, 1, 2>(*p, cf, cm, s);                                         \
   } else {                                                                                      \
     hipLaunchKernelGGL(diff_cell_kernel<NEQ_>, dim3(blocks(ncell)), dim3(256), 0, s, *p);     \
     hipLaunchKernelGGL(diff_face_kernel<NEQ_>, dim3(blocks(nface)), dim3(256), 0, s, *p);     \

@@ -177,7 +177,10 @@ typedef struct {
  * SC(i-st2:j+st1) at 652 as i+st1; z sections k-st2:k-st1 at 634-635 and 706
  * as k-st2:k+st1 (identical at second order); Cp_sp(isc) at 720-730 as the
  * species' own cp.  The burner heat loss (796-802) and the external ignition
- * source (842-859), fixed to single cases' meshes, stay with the caller. */
+ * source (842-859), fixed to single cases' meshes, stay with the caller.  The
+ * context keeps five planes of workspace for the largest block it has had, and
+ * at fourth order the fluxes of a pass ("diff_flux_mb" below): the first call of
+ * a size allocates, later ones only enqueue. */
 int tgr_chem_diffusion_device(tgr_chem *ctx, double dt, const tgr_grid *g, const tgr_metric *m, int flags,
                               const double *RHO_, const double *SC_, const double *DIFF_, const int *mask,
                               double *diff_corr, double *diff_gp, double *src, void *stream);
@@ -322,6 +325,12 @@ int tgr_chem_set_option_real(tgr_chem *ctx, const char *key, double value);
  *   "props_mapping"  tgr_chem_properties_device: 1 (default) a thread per
  *                 cell (the Wilke double sum in every lane), 0 a wavefront per
  *                 cell (species in lanes); the same results to rounding
+ *   "diff_flux_mb"  tgr_chem_diffusion_device at fourth order: most MiB of
+ *                 workspace for the face fluxes (two species' at least; default
+ *                 1024; 0: none, every cell recomputes the fluxes of its faces),
+ *                 the same results to the last bit; setting it gives the present
+ *                 workspace back.  Less is taken where that would leave less than
+ *                 three quarters of the free memory
  *   "jacobian"    0 (default): the Jacobian by difference quotients, one
  *                 right-hand side per column, as CVODE's FCVDENSE builds it for
  *                 the reference (finitechem.f90:1028); 1: the analytic Jacobian

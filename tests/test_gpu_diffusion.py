@@ -240,3 +240,91 @@ def test_column_of_four_million_cells(torch_dev):
     for z in (slice(0, part + 2), slice(nz - part, nz + 2)):
         assert torch.equal(whole[:, z][:, 1:-1], run(RHO_[z], SC_[:, z], DIFF_[:, z], part)[:, 1:-1])
     fc.close()
+
+
+@pytest.mark.parametrize("case", make_diffusion.CASES[3:], ids=make_diffusion.name)
+def test_fourth_order_workspace_sizes(torch_dev, case):
+    """Fourth order without a flux workspace (the general kernels), with one
+    that holds a part of the species at a time, and with the default: the same
+    outputs to the last bit."""
+    ref = make_diffusion.outputs(case, lambda fc: fc.set_option("diff_flux_mb", 0))
+    for mb in (1, 1024):
+        got = make_diffusion.outputs(case, lambda fc: fc.set_option("diff_flux_mb", mb))
+        for k in ref:
+            assert np.array_equal(got[k], ref[k]), (mb, k)
+
+
+def _block(torch, mech, nx, ny, nz, order):
+    """Fields of a block on the GPU and a call of the correction on them."""
+    from tiger_nga_amd.finitechem import FiniteChem
+    fc = FiniteChem(mech)
+    nsp, nover = fc.nsp, order - 1
+    g = Grid.block(nx, ny, nz, nsp + 1, 1, nsp + 1, nover=nover)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    fortran = lambda a: a.permute(*reversed(range(a.ndim)))
+    shp = tuple(reversed(g.shape))
+    SC_ = torch.rand((nsp + 1,) + shp, generator=gen, dtype=torch.float64, device="cuda")
+    SC_[:nsp] /= SC_[:nsp].sum(0)
+    SC_[nsp] = 400.0 + 1600.0 * SC_[nsp]
+    DIFF_ = 1e-5 + 1e-4 * torch.rand(SC_.shape, generator=gen, dtype=torch.float64, device="cuda")
+    RHO_ = torch.ones(shp, dtype=torch.float64, device="cuda")
+    corr = torch.zeros_like(SC_)
+
+    ops = {o: {k: (v if k in ("st1", "st2") else _dev(torch, np.asfortranarray(v))) for k, v in
+               metric.cartesian(g, np.arange(g.shape[0] + 1) * 1e-4, np.arange(g.shape[1] + 1) * 1e-4, 1.1e-4, o).items()}
+           for o in {2, order}}
+
+    def call(order=order, stream=None):
+        fc.diffusion(1e-6, g, ops[order], fortran(RHO_), fortran(SC_), fortran(DIFF_), diff_corr=fortran(corr),
+                     stream=stream)
+        return corr
+    return fc, call
+
+
+def test_fourth_order_takes_a_quarter_of_the_memory(torch_dev):
+    """With 3 GiB free a block whose fluxes would fill 1 GiB gets a smaller
+    workspace, once, and the outputs are those of the general kernels."""
+    torch = torch_dev
+    fc, call = _block(torch, "gri30", 120, 120, 120, 4)
+    fc.set_option("diff_flux_mb", 0)
+    want = call().clone()
+    fc.set_option("diff_flux_mb", 1024)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    hog = torch.empty(torch.cuda.mem_get_info()[0] - (3 << 30), dtype=torch.uint8, device="cuda")
+    free0 = torch.cuda.mem_get_info()[0]
+    left = []
+    for _ in range(2):
+        assert torch.equal(call(), want)
+        left.append(torch.cuda.mem_get_info()[0])
+    del hog
+    torch.cuda.empty_cache()
+    fc.close()
+    assert free0 - left[0] <= free0 // 4 and left[0] == left[1] and free0 > left[0]
+
+
+def test_orders_under_capture(torch_dev):
+    """Second order captured in a graph, then fourth order captured on a context
+    that has had this block at second order only (nothing may be allocated:
+    it runs without a flux workspace), then fourth order called, whose
+    workspace leaves the second-order graph's alone: every replay equals the
+    eager call."""
+    torch = torch_dev
+    fc, call = _block(torch, "h2", 13, 11, 9, 4)
+    side = torch.cuda.Stream()
+    graphs = {}
+    with torch.cuda.stream(side):
+        call(2, side.cuda_stream)
+    torch.cuda.synchronize()
+    for order in (2, 4):
+        graphs[order] = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graphs[order], stream=side):
+            call(order, torch.cuda.current_stream().cuda_stream)
+    want = {order: call(order).clone() for order in (4, 2)}
+    for _ in range(3):
+        for order in (2, 4):
+            out = call(6 - order)
+            graphs[order].replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want[order])
+    fc.close()

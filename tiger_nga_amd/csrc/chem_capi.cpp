@@ -102,7 +102,10 @@ struct tgr_chem {
   double* d_out_scale = nullptr;
   std::vector<float> h_in_shift, h_in_scale;
   DevBuf b_x, b_guess, b_rej;
-  DevBuf b_diff;  // diffusion workspace: W_gp, cp_mix, corr_vel x / y / z (5 planes), fluxes
+  DevBuf b_diff;  // diffusion workspace: W_gp, cp_mix, corr_vel x / y / z (5 planes)
+  DevBuf b_flux;  // fourth order: temperature term (1 plane), fluxes (6 planes a species)
+  int64_t flux_mb = 1024;          // its largest size, MiB ("diff_flux_mb")
+  size_t flux_refused = SIZE_MAX;  // the smallest size that there was no memory for
   unsigned int* d_rej_count = nullptr;
   unsigned long long* d_stotals = nullptr;
   int surr_nsub = 8, surr_guess = 0, surr_newton_max = 8;
@@ -282,6 +285,44 @@ bool rates_by_lane(const tgr_chem* c, int64_t n) {
   return c->rhs_lanes && (c->neq <= 10 || n >= (int64_t)64 * c->n_cu);
 }
 
+// Species whose fluxes the fourth-order diffusion of a block of `plane` cells
+// keeps at once in b_flux, 0 for the general kernels, which need none.  All of
+// them where "diff_flux_mb" allows it (one pass is two launches), at least two.  The
+// workspace grows only outside of a capture, leaves the caller three quarters of
+// the free memory and halves its wish where that or the allocation fails; the
+// size that failed is remembered, so that later calls do not ask for it again
+// and take the same passes.  The outputs are the same to the last bit in any
+// number of passes.
+int flux_species(tgr_chem* c, int64_t plane, hipStream_t s) {
+  if (!c->flux_mb) return 0;
+  auto bytes = [&](int64_t n) { return (size_t)plane * (1 + 6 * n) * sizeof(double); };
+  int64_t n = std::min<int64_t>(c->nsp, std::max<int64_t>(2, (c->flux_mb << 20) / (48 * plane)));
+  if (bytes(n) <= c->b_flux.cap) return (int)n;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+    for (; bytes(n) > c->b_flux.cap; n = std::max<int64_t>(2, n / 2)) {
+      if (bytes(n) < c->flux_refused) {
+        size_t free_b = 0, total = 0;
+        void* q = nullptr;
+        if (hipMemGetInfo(&free_b, &total) == hipSuccess && bytes(n) <= free_b / 4 &&
+            hipMalloc(&q, bytes(n)) == hipSuccess) {
+          c->b_flux.release();
+          c->b_flux.p = q;
+          c->b_flux.cap = bytes(n);
+          break;
+        }
+        (void)hipGetLastError();
+        c->flux_refused = bytes(n);
+      }
+      if (n == 2) return 0;
+    }
+  } else {
+    (void)hipGetLastError();
+    n = ((int64_t)(c->b_flux.cap / sizeof(double)) / plane - 1) / 6;  // what is there
+  }
+  return n >= 2 ? (int)n : 0;
+}
+
 // Layout of an external scratch block (tgr_chem_source_chemistry_device_noalloc):
 // the work counter at byte 0, the counter totals at byte 64, the per-wave
 // Jacobian workspace from byte 256.
@@ -415,6 +456,7 @@ int tgr_chem_destroy(tgr_chem* c) {
   c->b_guess.release();
   c->b_rej.release();
   c->b_diff.release();
+  c->b_flux.release();
   c->b_ws.release();
   c->b_rho.release();
   c->b_sc.release();
@@ -462,6 +504,11 @@ int tgr_chem_set_option(tgr_chem* c, const char* key, int64_t v) {
   } else if (!strcmp(key, "jacobian")) {
     if (v != 0 && v != 1) return fail(TGR_E_ARG, "jacobian must be 0 (difference quotients) or 1 (analytic)");
     c->jac = (int)v;
+  } else if (!strcmp(key, "diff_flux_mb")) {
+    if (v < 0 || v > (1 << 20)) return fail(TGR_E_ARG, "diff_flux_mb must be 0..1048576");
+    c->flux_mb = v;
+    c->b_flux.release();
+    c->flux_refused = SIZE_MAX;
   } else if (!strcmp(key, "max_order")) {
     if (v < 1 || v > 5) return fail(TGR_E_ARG, "max_order must be 1..5");
     c->qmax = (int)v;
@@ -1009,23 +1056,16 @@ int tgr_chem_diffusion_device(tgr_chem* c, double dt, const tgr_grid* g, const t
     *idx[q] = species_index(c->t, names[q]);
     *wk[q] = *idx[q] >= 0 ? c->t->W[*idx[q]] : 1.0;
   }
-  // fourth order: all species' fluxes at once where 1 GiB holds them (one pass
-  // is two launches), at least two species a pass; where the memory for that is
-  // not to be had, the general kernels, which need five planes
-  if (m->st1 == 1 && m->st2 == 2 && tgr::diff_small_plane(gm.plane)) {
-    p.nchunk = (int)std::min<int64_t>(c->nsp, std::max<int64_t>(2, ((int64_t)1 << 30) / (48 * gm.plane)));
-    p.nslice = (int)std::min<int64_t>((p.nchunk + 3) / 4, std::max<int64_t>(1, 2 * 256 * (int64_t)c->n_cu / gm.plane));
-    if (c->b_diff.ensure((size_t)gm.plane * (6 + 6 * p.nchunk) * sizeof(double))) {
-      (void)hipGetLastError();
-      p.nchunk = p.nslice = 0;
-    }
-  }
   if ((rc = c->b_diff.ensure((size_t)gm.plane * 5 * sizeof(double)))) return rc;
+  if (m->st1 == 1 && m->st2 == 2 && tgr::diff_small_plane(gm.plane)) {
+    p.nchunk = flux_species(c, gm.plane, (hipStream_t)stream);
+    p.nslice = (int)std::min<int64_t>((p.nchunk + 3) / 4, std::max<int64_t>(1, 2 * 256 * (int64_t)c->n_cu / gm.plane));
+  }
   p.wg = (double*)c->b_diff.p;
   p.cpm = p.wg + gm.plane;
   p.cvel = p.cpm + gm.plane;
-  p.eT = p.cvel + 3 * gm.plane;
-  p.flux = p.eT + gm.plane;
+  p.eT = (double*)c->b_flux.p;
+  p.flux = p.eT ? p.eT + gm.plane : nullptr;
   if (tgr_launch_diffusion(&p, c->neq, (hipStream_t)stream)) return fail(TGR_E_HIP, "diffusion kernel launch failed");
   return 0;
 }

@@ -122,7 +122,7 @@ struct DiffParams {
   double* cpm;    // [plane] cp_mix (cv)
   double* cvel;   // [3][plane] corr_vel_x, _y, _z
   int n_cu;
-  int nchunk;     // fourth order: species per pass through the flux workspace (0: other kernels)
+  int nchunk;     // fourth order: species per pass through the flux workspace (0: the general kernels)
   int nslice;     // fourth order: parts that the species of a pass are split into for the fluxes
   double* eT;     // [plane] temperature term of the passes so far
   double* flux;   // [nchunk][x, y, z][corrected, Fickian][plane]

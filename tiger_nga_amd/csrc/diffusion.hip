@@ -78,6 +78,8 @@ struct Cells {
   unsigned n, wg;     // its cells and workgroups
   unsigned row;       // workgroups of a plane (rounded: the bricks lean a little)
   unsigned threads;   // of a workgroup
+  int k0;             // first plane of the range
+  int64_t base;       // cells of the block before the ones that 32-bit offsets reach
 };
 
 __device__ __forceinline__ bool range_cell(const Cells& c, int& i, int& j, int& k) {
@@ -94,7 +96,7 @@ __device__ __forceinline__ bool range_cell(const Cells& c, int& i, int& j, int& 
   const unsigned q = w * blockDim.x + threadIdx.x, r = q / (unsigned)c.ni;
   i = (int)(q - r * (unsigned)c.ni);
   j = (int)(r % (unsigned)c.nj);
-  k = (int)(r / (unsigned)c.nj);
+  k = c.k0 + (int)(r / (unsigned)c.nj);
   return seq < last && q < c.n;
 }
 
@@ -117,7 +119,7 @@ __device__ __forceinline__ bool interior_cell(const DiffParams& p, const Cells& 
 }
 
 // a[byte offset]: a wave-uniform base and a 32-bit lane offset (the launcher
-// checks that a plane has less than 2^32 bytes)
+// keeps the cells that a launch reaches below 2^32 bytes)
 __device__ __forceinline__ double ldo(const double* a, unsigned off) {
   return *(const double*)((const char*)a + off);
 }
@@ -424,10 +426,10 @@ __global__ __launch_bounds__(256) void diff_face2_kernel(DiffParams p, Cells cl)
       wi[d][1] = 1.0 / w1;
     }
   }
-  const unsigned oc = (unsigned)o * 8u;
+  const unsigned oc = (unsigned)(o - cl.base) * 8u;
   const unsigned on[3] = {oc - 8u, oc - (unsigned)g.nxo * 8u, oc - (unsigned)g.nxo * (unsigned)g.nyo * 8u};
-  const double* __restrict__ Y = p.sc + (int64_t)g.isc_sc0 * g.plane;
-  const double* __restrict__ D = p.diff + (int64_t)g.isc_sc0 * g.plane;
+  const double* __restrict__ Y = p.sc + (int64_t)g.isc_sc0 * g.plane + cl.base;
+  const double* __restrict__ D = p.diff + (int64_t)g.isc_sc0 * g.plane + cl.base;
   double yc = ldo(Y, oc), dc = ldo(D, oc), yn[3], dn[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) yn[d] = ldo(Y, on[d]), dn[d] = ldo(D, on[d]);
@@ -551,9 +553,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
       dv[d][f] = op(du, i, g.imin_, nx, j, g.jmin_, ny, f, 0);
       im[d][f] = op(iu, i, g.imin_, nx, j, g.jmin_, ny, f, 0);
     }
-  const unsigned oc = (unsigned)o * 8u;
-  const double* __restrict__ Y = p.sc + (int64_t)g.isc_sc0 * g.plane;
-  const double* __restrict__ D = p.diff + (int64_t)g.isc_sc0 * g.plane;
+  const unsigned oc = (unsigned)(o - cl.base) * 8u;
+  const double* __restrict__ Y = p.sc + (int64_t)g.isc_sc0 * g.plane + cl.base;
+  const double* __restrict__ D = p.diff + (int64_t)g.isc_sc0 * g.plane + cl.base;
   const double* cr = cps + (T > p.mech.tmid ? 6 : 0);
   double* __restrict__ corr = p.corr;
   double* __restrict__ src = p.src;
@@ -878,22 +880,35 @@ extern "C" int tgr_launch_diffusion(const DiffParams* p, int neq, hipStream_t s)
   const int64_t nint = (int64_t)(g.imax_ - g.imin_ + 1) * (g.jmax_ - g.jmin_ + 1) * (g.kmax_ - g.kmin_ + 1);
   auto blocks = [](int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 256, 65535); };
   // second order (the reference's default stencil) and fourth order have their
-  // own kernels, which address a plane by 32-bit byte offsets; other widths and
-  // larger planes take the general ones
-  const bool small = diff_small_plane(g.plane);
-  const bool o2 = small && st1 == 0 && st2 == 1, o4 = p->nchunk > 0;
-  auto range = [&](int halo) {
-    const int ni = g.imax_ - g.imin_ + 1 + halo, nj = g.jmax_ - g.jmin_ + 1 + halo, nk = g.kmax_ - g.kmin_ + 1 + halo;
+  // own kernels, which reach 2^29 cells by 32-bit byte offsets: second order
+  // takes larger blocks by as many planes at a time (with the ones beside them)
+  // as that allows; fourth order of larger blocks, and other widths, take the
+  // general kernels
+  const int64_t sz = (int64_t)g.nxo * g.nyo;
+  const int slab = diff_small_plane(g.plane) ? g.nzo : (int)(((int64_t)1 << 29) / sz) - 2;
+  const bool o2 = slab > 0 && st1 == 0 && st2 == 1, o4 = p->nchunk > 0;
+  // planes [k0, k0 + slab) of the range that reaches `halo` cells past the interior
+  auto range = [&](int halo, int k0, int slab) {
+    const int ni = g.imax_ - g.imin_ + 1 + halo, nj = g.jmax_ - g.jmin_ + 1 + halo;
+    const int nk = std::min(g.kmax_ - g.kmin_ + 1 + halo - k0, slab);
     const int64_t n = (int64_t)ni * nj * nk;
     // a wave per workgroup until every CU has four workgroups of four
     const int64_t t = n < (int64_t)4 * 256 * p->n_cu ? 64 : 256, row = ((int64_t)ni * nj + t / 2) / t;
-    return Cells{ni, nj, (unsigned)n, (unsigned)((n + t - 1) / t), (unsigned)(row > kStrip ? row : 0), (unsigned)t};
+    return Cells{ni, nj, (unsigned)n, (unsigned)((n + t - 1) / t), (unsigned)(row > kStrip ? row : 0), (unsigned)t,
+                 k0, diff_small_plane(g.plane) ? 0 : (g.kmin_ + k0 - 1 - g.kmino_) * sz};
   };
-  const Cells cm = range(0), cf = range(st1 + st2);
-#define TGR_DIFF_LAUNCH2(NEQ_, MOLAR_)                                                                        \
-  hipLaunchKernelGGL(diff_cell_kernel<NEQ_>, dim3(blocks(ncell)), dim3(256), 0, s, *p);                     \
-  hipLaunchKernelGGL((diff_face2_kernel<NEQ_, MOLAR_>), dim3(launch_groups(cf)), dim3(cf.threads), 0, s, *p, cf); \
-  hipLaunchKernelGGL((diff_main2_kernel<NEQ_, MOLAR_>), dim3(launch_groups(cm)), dim3(cm.threads), 0, s, *p, cm);
+  const int nz = g.kmax_ - g.kmin_ + 1;
+  const Cells cm = range(0, 0, nz), cf = range(st1 + st2, 0, nz + st1 + st2);
+#define TGR_DIFF_LAUNCH2(NEQ_, MOLAR_)                                                                              \
+  hipLaunchKernelGGL(diff_cell_kernel<NEQ_>, dim3(blocks(ncell)), dim3(256), 0, s, *p);                           \
+  for (int k0 = 0; k0 <= nz; k0 += slab) {                                                                          \
+    const Cells c = range(1, k0, slab);                                                                             \
+    hipLaunchKernelGGL((diff_face2_kernel<NEQ_, MOLAR_>), dim3(launch_groups(c)), dim3(c.threads), 0, s, *p, c);    \
+  }                                                                                                                 \
+  for (int k0 = 0; k0 < nz; k0 += slab) {                                                                           \
+    const Cells c = range(0, k0, slab);                                                                             \
+    hipLaunchKernelGGL((diff_main2_kernel<NEQ_, MOLAR_>), dim3(launch_groups(c)), dim3(c.threads), 0, s, *p, c);    \
+  }
 #define TGR_DIFF_LAUNCH(NEQ_)                                                                  \
   if (o2 && p->molar) {                                                                         \
     TGR_DIFF_LAUNCH2(NEQ_, true)                                                                \

@@ -365,3 +365,39 @@ def test_second_order_beyond_32_bit_offsets(torch_dev):
         assert float(own[:, 1:-1, 1:-1, 1:-1].abs().max()) > 0.0
         assert torch.equal(whole[:, z][:, 1:-1], own[:, 1:-1])
     fc.close()
+
+
+@pytest.mark.parametrize("mech,molar,wall", [("h2", True, True), ("gri30", False, False), ("ethyred", True, False)])
+def test_general_stencil_vs_oracle(torch_dev, oracle, mech, molar, wall):
+    """Sixth order, the stencil that only the general kernels take; bound as above."""
+    torch = torch_dev
+    from tiger_nga_amd.finitechem import FiniteChem
+    order, nover = 6, 5
+    sh = (5 + 2 * nover, 4 + 2 * nover, 3 + 2 * nover)
+    _, Y, T, rho, P, dt = inputs.states(mech, n=499, seed=37)
+    nsp = Y.shape[1]
+    g = Grid.block(5, 4, 3, nsp + 1, 1, nsp + 1, nover=nover)
+    pick = np.arange(np.prod(sh)) * 7919 % 499
+    SC_ = np.asfortranarray(np.concatenate([Y, T[:, None]], axis=1)[pick].reshape(sh + (nsp + 1,), order="F"))
+    RHO_ = np.asfortranarray(rho[pick].reshape(sh, order="F"))
+    rng = np.random.default_rng(9)
+    DIFF_ = np.asfortranarray(10.0 ** rng.uniform(-5.0, -4.0, SC_.shape))
+    x, y = (np.cumsum(np.concatenate([[0.0], 1e-4 * (1.0 + 0.3 * rng.random(n))])) for n in sh[:2])
+    m = metric.cartesian(g, x, y, 1.1e-4, order)
+    assert (m["st1"], m["st2"]) == (2, 3)
+    mask = None
+    if wall:
+        mask = np.zeros(g.mask_shape, dtype=np.int32, order="F")
+        mask[:, nover + 1] = 1
+    dc_o, gp_o = oracle.diffusion(mech, g, m, dt, RHO_, SC_, DIFF_, mask=mask, molar=molar, gasrad=True)
+    fc = FiniteChem(mech)
+    md = {k: (v if k in ("st1", "st2") else _dev(torch, np.asfortranarray(v))) for k, v in m.items()}
+    dc, gp = (_dev(torch, np.zeros(sh + (n,), order="F")) for n in (nsp + 1, 3))
+    fc.diffusion(dt, g, md, _dev(torch, RHO_), _dev(torch, SC_), _dev(torch, DIFF_),
+                 mask=None if mask is None else _dev(torch, mask), diff_corr=dc, diff_gp=gp, molar=molar, gasrad=True)
+    torch.cuda.synchronize()
+    fc.close()
+    for got, want in ((dc.cpu().numpy(), dc_o), (gp.cpu().numpy(), gp_o)):
+        for k in range(want.shape[-1]):
+            scale = max(np.abs(want[..., k]).max(), 1e-300)
+            assert np.abs(got[..., k] - want[..., k]).max() <= 1e-12 * scale + 1e-300, k

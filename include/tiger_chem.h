@@ -306,11 +306,12 @@ int tgr_chem_set_option_real(tgr_chem *ctx, const char *key, double value);
  *   "grid"        size of the persistent grid in workgroups of 8 waves (0: occupancy x CUs);
  *                 every wave pulls cells
  *                 from a device work counter
- *   "rhs_mapping" tgr_chem_rhs_device, tgr_chem_prodrates_device: 1 (default) one
- *                 state per lane (generated straight-line code of the mechanism)
- *                 from 64 states per CU on (H2: always) and one state per
- *                 wavefront below, 0 one state per wavefront; the same results
- *                 to rounding
+ *   "rhs_mapping" tgr_chem_rhs_device, tgr_chem_prodrates_device: 0 one state
+ *                 per wavefront, 1 one state per lane (generated straight-line
+ *                 code of the mechanism), 2 (default) per lane from 64 states per
+ *                 CU on (H2: always) and per wavefront below.  The two give the
+ *                 same results to rounding; 0 and 1 give a state the same bits in
+ *                 a batch of any size
  *   "step_mapping"  0 (default): a wavefront per cell (the species in lanes);
  *                 1: a thread per cell -- the same CVODE-semantics BDF with the
  *                 cell's vectors and Nordsieck history in the thread's registers

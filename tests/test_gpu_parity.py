@@ -360,3 +360,49 @@ def test_batched_rate_mappings_agree(mech, n, torch_dev):
     for a, b in zip(*got):
         assert torch.isfinite(b).all()
         assert float((a - b).norm() / b.norm()) <= 3e-14
+
+
+@pytest.mark.parametrize("mech", MECHS)
+def test_prodrates_by_lane_vs_reference_golden(mech, torch_dev):
+    """As test_prodrates_vs_reference_golden, one state per lane."""
+    torch = torch_dev
+    from tiger_nga_amd.finitechem import FiniteChem
+    d = np.load(os.path.join(GOLD, "%s_mech.npz" % mech))
+    fc = FiniteChem(mech)
+    fc.set_option("rhs_mapping", 1)
+    C, T, P = (torch.tensor(np.ascontiguousarray(d[k].T), device="cuda") for k in ("C", "T", "P"))
+    cd = fc.prodrates(C, T, P).cpu().numpy().T
+    fc.close()
+    scale = np.abs(d["W"]).sum(axis=1, keepdims=True)
+    assert (np.abs(cd - d["CDOT"]) / np.maximum(scale, 1e-300)).max() < 1e-12
+
+
+@pytest.mark.parametrize("mech", MECHS)
+def test_batched_rates_pinned_mappings(mech, torch_dev):
+    """rhs_mapping 0 and 1 give a state the same bits in a batch of any size, and
+    the default is the one of them that the number of states asks for (64 per CU
+    and more by lane; H2 always)."""
+    torch = torch_dev
+    from tiger_nga_amd.finitechem import FiniteChem
+    edge = 64 * torch.cuda.get_device_properties(0).multi_processor_count
+    _, Y, T, rho, P, _ = inputs.states(mech, n=edge, seed=43)
+    fc = FiniteChem(mech)
+    sol = torch.from_numpy(np.ascontiguousarray(inputs.packed_state(Y, T, rho).T)).cuda()
+    C = (sol[:-1] / torch.from_numpy(fc.molar_mass).cuda()[:, None]).contiguous()
+    Td = torch.from_numpy(T).cuda()
+
+    def rates(n, mapping=None):
+        if mapping is not None:
+            fc.set_option("rhs_mapping", mapping)
+        Tn = Td[:n].contiguous()
+        return fc.compute_rhs(sol[:, :n].contiguous(), P), fc.prodrates(C[:, :n].contiguous(), Tn, torch.full_like(Tn, P))
+    default = {n: rates(n) for n in (edge - 1, edge)}
+    whole = {m: rates(edge, m) for m in (0, 1)}
+    for m in (0, 1):
+        for n in (1, 300, edge - 1):
+            for a, b in zip(rates(n, m), whole[m]):
+                assert torch.equal(a, b[:, :n]), (m, n)
+    for n, m in ((edge - 1, int(mech == "h2")), (edge, 1)):
+        for a, b, o in zip(default[n], whole[m], whole[1 - m]):
+            assert torch.equal(a, b[:, :n]) and not torch.equal(a, o[:, :n]), n
+    fc.close()

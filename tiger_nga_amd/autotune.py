@@ -126,7 +126,7 @@ def tune(mech: str, cells: int = 32 ** 3, seed: int = 7, reps: int = 2, log=prin
     rec["rhs_mapping"] = best_map
     rec["measured"]["rhs_ms"] = {("lane" if k else "wave"): v * 1e3 for k, v in times.items()}
     log("  rhs: lane %.3f ms, wave %.3f ms -> %s" % (times[1] * 1e3, times[0] * 1e3, "lane" if best_map else "wave"))
-    fc.set_option("rhs_mapping", best_map)
+    fc.set_option("rhs_mapping", 2 if best_map else 0)
     # persistent grid of the step kernel
     R_d, S0, g, Pg = surrogate.block_states(fc, WORKLOAD[mech], cells, seed, 0)
     S = S0.clone()
@@ -354,7 +354,8 @@ def apply(fc, cells: int, path=CACHE) -> dict:
               "surr_guess", "surr_h0_fac", "surr_jac_theta", "surr_max_jac", "surr_keep", "surr_tol_y",
               "surr_newton_tol"):
         if k in rec:
-            fc.set_option(k, rec[k])
+            # "lane" was timed on a whole block: smaller batches go by their size
+            fc.set_option(k, 2 if k == "rhs_mapping" and rec[k] else rec[k])
             done[k] = rec[k]
     return done
 

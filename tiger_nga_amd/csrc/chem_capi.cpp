@@ -77,7 +77,7 @@ struct tgr_chem {
   int jac = 0;  // 0: difference-quotient Jacobian (the reference's CVODE FCVDENSE); 1: analytic
   int step_mapping = 0;  // 0: a wave per cell; 1: a thread per cell (small mechanisms, bdf_lane.h)
   int step_waves = 2;    // wave per cell: resident waves per SIMD (2, or 4 where the kernel supports it)
-  int rhs_lanes = 1;  // batched right-hand side: one state per lane (1) or per wave (0)
+  int rhs_mapping = 2;  // batched rates: one state per lane (1), per wave (0), or by the number of states (2)
   int64_t grid_override = 0;
   int device = 0;
   int n_cu = 0;
@@ -274,7 +274,7 @@ size_t step_shape(const tgr_chem* c, int64_t ncell, int* grid, bool* lanes) {
   return (size_t)*grid * tgr_step_block_waves() * c->neq * 64 * sizeof(double);
 }
 
-// Mapping of the batched rates of n states (option "rhs_mapping").  One state
+// Mapping of the batched rates of n states (option "rhs_mapping" 2).  One state
 // per lane costs the time of one wave's 10,000 to 20,000 instructions however
 // few states there are, and pays once every CU has a wave (16,384 states on 256
 // CUs): rates of GRI-3.0 by wave / by lane 7 / 36 us at 256 states, 18 / 37 at
@@ -282,7 +282,7 @@ size_t step_shape(const tgr_chem* c, int64_t ncell, int* grid, bool* lanes) {
 // 18 / 23, 31 / 23, 54 / 25, 352 / 92.  H2's rates are short: by lane always
 // (7 / 7 us at one state, 213 / 19 at 262,144).
 bool rates_by_lane(const tgr_chem* c, int64_t n) {
-  return c->rhs_lanes && (c->neq <= 10 || n >= (int64_t)64 * c->n_cu);
+  return c->rhs_mapping == 2 ? c->neq <= 10 || n >= (int64_t)64 * c->n_cu : c->rhs_mapping == 1;
 }
 
 // Species whose fluxes the fourth-order diffusion of a block of `plane` cells
@@ -489,8 +489,9 @@ int tgr_chem_set_option(tgr_chem* c, const char* key, int64_t v) {
   if (!c || !key) return fail(TGR_E_ARG, "NULL argument");
   if (!strcmp(key, "grid")) c->grid_override = v;
   else if (!strcmp(key, "rhs_mapping")) {
-    if (v != 0 && v != 1) return fail(TGR_E_ARG, "rhs_mapping must be 0 (wave per state) or 1 (lane per state)");
-    c->rhs_lanes = (int)v;
+    if (v < 0 || v > 2)
+      return fail(TGR_E_ARG, "rhs_mapping must be 0 (wave per state), 1 (lane per state) or 2 (by the number of states)");
+    c->rhs_mapping = (int)v;
   } else if (!strcmp(key, "step_waves")) {
     if (!tgr_step_waves_supported(c->neq, (int)v))
       return fail(TGR_E_ARG, "step_waves must be 2, or 4 for a 10-equation mechanism (H2)");

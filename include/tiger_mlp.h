@@ -15,7 +15,8 @@
  * rounded up, out_pad_last = nout rounded up, hidden layers `hidden`), padded
  * entries zero.  Inputs x: BF16 bit patterns [B][in_pad] row-major, padded
  * columns zero; outputs and targets FP32, outputs [B][out_pad], targets
- * [B][nout].  B must be a positive multiple of 64.  All arrays are device
+ * [B][nout].  B must be a positive multiple of 64; x must be 16-byte aligned,
+ * outputs and targets only as floats are.  All arrays are device
  * memory; every call is enqueued on `stream` (a hipStream_t, NULL = default).
  * Return 0 or a negative code; tgr_mlp_last_error() gives the message. */
 #ifndef TIGER_MLP_H

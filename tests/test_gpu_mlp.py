@@ -165,3 +165,26 @@ def test_fused_forward_equals_the_layered_one(torch_dev, B):
     wide.set_params(wflat)
     x = _bf(torch, 2.0 * x)
     assert torch.equal(net.forward(x), wide.forward(x))
+
+
+@pytest.mark.parametrize("hidden", [256, 320])
+def test_output_and_targets_at_any_offset(torch_dev, hidden):
+    """Outputs and targets that are views one element past the start of a larger
+    tensor, in the fused pass and layer by layer: the results of aligned ones,
+    and nothing written outside.  Input rows must be 16-byte aligned."""
+    torch = torch_dev
+    from tiger_nga_amd import mlp
+    net, _, _, x, tgt = _net_case(torch, hidden=hidden, B=192)
+    x, tgt = _bf(torch, x), torch.from_numpy(tgt).cuda()
+    want = net.forward(x)
+    big = torch.full((want.numel() + 2,), 7.0, device="cuda")
+    out = big[1:-1].view(want.shape)
+    assert out.data_ptr() % 16 == 4
+    assert torch.equal(net.forward(x, out=out), want) and float(big[0]) == float(big[-1]) == 7.0
+    ts = torch.empty(tgt.numel() + 1, device="cuda")[1:].view(tgt.shape).copy_(tgt)
+    for a, b in zip(net.gradients(x, tgt), net.gradients(x, ts)):
+        assert np.array_equal(a, b)
+    xs = torch.empty(x.numel() + 1, dtype=x.dtype, device="cuda")[1:].view(x.shape).copy_(x)
+    for call in (lambda: net.forward(xs), lambda: net.gradients(xs, tgt), lambda: net.train_step(xs, tgt, 1e-3)):
+        with pytest.raises(mlp.MLPError, match="16-byte aligned"):
+            call()

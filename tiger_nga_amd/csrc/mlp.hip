@@ -72,6 +72,11 @@ __device__ __forceinline__ float gelu_both(float x, float& d) {
   return 0.5f * x * c;
 }
 
+// four outputs of a row, aligned as floats are: the caller's array may be a view
+// that starts anywhere in a larger one (the hardware takes the store as one
+// instruction either way)
+typedef float row4 __attribute__((ext_vector_type(4), aligned(4)));
+
 enum Act { kNone = 0, kGelu = 1, kGeluGrad = 2 };
 
 struct GemmArgs {
@@ -393,7 +398,7 @@ __global__ __launch_bounds__(64 * kFusedWaves) void mlp_infer_kernel(FusedArgs g
 #pragma unroll
           for (int q = 0; q < 4; ++q)
             if (col + q >= g.nout) v[q] = 0.0f;
-          *reinterpret_cast<float4*>(g.out + (row0 + row) * N + col) = float4{v[0], v[1], v[2], v[3]};
+          *reinterpret_cast<row4*>(g.out + (row0 + row) * N + col) = row4{v[0], v[1], v[2], v[3]};
         } else {
           ushort4 h;
           h.x = f2bf(gelu(v[0]));
@@ -1024,7 +1029,8 @@ int loss_and_grad(tgr_mlp* h, const uint16_t* x, const float* tgt, int64_t B, hi
   return 0;
 }
 
-// the fused passes load x in 16-byte pieces, as the product kernel does
+// the fused passes load x in 16-byte pieces, as the product kernel does (which
+// checks its operands itself)
 int check_input(const uint16_t* x) {
   return (uintptr_t)x & 15 ? fail(TGR_MLP_E_ARG, "the input rows must be 16-byte aligned") : 0;
 }

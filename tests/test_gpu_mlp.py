@@ -188,3 +188,35 @@ def test_output_and_targets_at_any_offset(torch_dev, hidden):
     for call in (lambda: net.forward(xs), lambda: net.gradients(xs, tgt), lambda: net.train_step(xs, tgt, 1e-3)):
         with pytest.raises(mlp.MLPError, match="16-byte aligned"):
             call()
+
+
+def test_training_where_the_fused_workspace_does_not_fit(torch_dev):
+    """A batch whose fused workspace (3.4 GB) is more than the free memory but
+    whose layered one (2.5 GB) is not: the gradients, losses and trained
+    parameters of the fused pass, then a small batch by the fused pass again."""
+    torch = torch_dev
+    from tiger_nga_amd import mlp
+    B = 1 << 18
+    nets = [_net_case(torch, B=64) for _ in range(2)]
+    rng = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.zeros(B, 64, device="cuda", dtype=torch.bfloat16)
+    x[:, :38] = torch.randn(B, 38, generator=rng, device="cuda").to(torch.bfloat16)
+    tgt = torch.tanh(x[:, :37].float()).contiguous()
+
+    def train(net):
+        g, _ = net.gradients(x, tgt)
+        losses = [net.train_step(x, tgt, 1e-3, want_loss=True) for _ in range(2)]
+        small = [net.train_step(x[:256], tgt[:256], 1e-3, want_loss=True) for _ in range(2)]
+        return g, np.array(losses + small), net.get_params()
+    want = train(nets[0][0])
+    nets[0][0].close()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    hog = torch.empty(torch.cuda.mem_get_info()[0] - int(2.95e9), dtype=torch.uint8, device="cuda")
+    got = train(nets[1][0])
+    free = torch.cuda.mem_get_info()[0]
+    del hog
+    torch.cuda.empty_cache()
+    assert free < 1.0e9  # the layered workspace is there
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[2], want[2])
+    assert np.abs(got[1] - want[1]).max() <= 1e-5 * want[1].max()  # sums of the squared errors in another order

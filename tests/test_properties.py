@@ -175,7 +175,7 @@ def test_properties_mappings_agree_on_full_block(oracle):
 @pytest.mark.gpu
 @pytest.mark.parametrize("wl,n", [("h2", 1), ("h2", 257), ("gri30", 256), ("dme39", 129), ("ethyred", 385)])
 def test_thread_per_cell_workgroup_edges(wl, n, oracle):
-    """One cell, exactly one workgroup and one cell over (workgroups of 128 or
+    """One cell, exactly one workgroup and one cell over (workgroups of 64 or
     256 by mechanism), a species of mass fraction 0 and one slightly negative,
     against the oracle; bound as above."""
     import torch

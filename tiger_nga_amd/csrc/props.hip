@@ -139,15 +139,22 @@ __device__ __forceinline__ void load_row(double (&m)[N], const TGR_CONST double*
 
 
 // Threads of a workgroup (its g_k take 8 nsp bytes of LDS a thread, the cp rows
-// 96 nsp bytes): four waves where two such workgroups fit a CU, else two waves;
-// the cp rows are in LDS where they do not cost a resident workgroup.  DME39,
-// 1,200 and 332,000 cells: 50.8 and 213 us so, 51.8 and 209 with four waves, 52.7
-// and 249 with two and the cp rows in LDS (a third of the pair loop padding
-// then: 3 parts of 14).
+// 96 nsp bytes): four waves where two such workgroups fit a CU, else one, of which
+// eight fit if the g_k of no more than 40 species are in LDS; EthyRedF's other
+// five are in registers.  Workgroups of two waves with all g_k in LDS leave EthyRedF
+// six waves a CU and a second, nearly empty round from 98,305 cells: 100,000 /
+// 131,072 / 1,000,000 cells 130 / 140 / 695 us, this way 80 / 83 / 638; DME39, 50,000
+// / 262,144 cells: 59 / 180 us with two waves, 54 / 147 with four, 51 / 133 with one.
+// The cp rows are in LDS where they do not cost a resident workgroup.
 constexpr int kLdsBytes = 160 * 1024;
 template <int NEQ>
 constexpr int props_block() {
-  return 2 * (256 * 8 + 96) * (NEQ - 1) <= kLdsBytes ? 256 : 128;
+  return 2 * (256 * 8 + 96) * (NEQ - 1) <= kLdsBytes ? 256 : 64;
+}
+template <int NEQ>
+constexpr int props_lds_species() {
+  const int fit = kLdsBytes / 8 / (props_block<NEQ>() * 8);
+  return props_block<NEQ>() == 64 && NEQ - 1 > fit ? fit : NEQ - 1;
 }
 template <int NEQ>
 constexpr bool props_cp_lds() {
@@ -161,8 +168,8 @@ constexpr bool props_cp_lds() {
 // matrix times y_j, y_j g_j and y_j g_j^2 to the part's sums: 3 x 18 independent
 // chains (GRI-3.0), the next column's scalar loads under way.  Bound by VALU
 // issue (64 % busy, 8,400 instructions a wave of which 3,900 are the pairs');
-// 130^3 GRI-3.0 cells in 0.83 ms, 1.03 ms with a 16-byte LDS read per pair.  Sums run in species order (the wave
-// kernel's are tree reductions) and eta = mucoeff sqrt(T) den / num takes
+// 130^3 GRI-3.0 cells in 0.83 ms, 1.03 ms with a 16-byte LDS read per pair.  Sums
+// run in species order (the wave kernel's are tree reductions) and eta = mucoeff sqrt(T) den / num takes
 // omegamu's numerator and denominator with one division: rounding-level
 // differences.
 template <int NEQ>
@@ -172,7 +179,10 @@ __global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per
   constexpr TabLayout L = tab_layout<NEQ>();
   constexpr int kPair = 192 + 2 * nsp * 64;
   constexpr bool kOne = kPropsParts(nsp) == 1;  // few species: one part, everything in registers
-  __shared__ double gs[kOne ? 1 : nsp][kBlock];
+  // g_k of kLds species in LDS, of the kReg past them in registers
+  constexpr int kLds = kOne ? 1 : props_lds_species<NEQ>(), kReg = kOne ? 0 : nsp - kLds;
+  __shared__ double gs[kLds][kBlock];
+  double gr[kReg ? kReg : 1];
   constexpr bool kCpLds = props_cp_lds<NEQ>();
   __shared__ __attribute__((aligned(16))) double cps[kCpLds ? nsp * 12 : 2];  // cp rows, [species][T > tmid][6]
   if constexpr (kCpLds) {
@@ -201,15 +211,19 @@ __global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per
   // Both loops take kCh species at a time: the next chunk's Y are loaded while
   // one computes (a load takes longer than one species), and the chains of a
   // chunk's species overlap.
-  constexpr int kCh = kOne ? nsp : 4;
+  constexpr int kCh = kOne ? nsp : (kReg ? kReg : 4);
+  constexpr int kLoop = kReg ? kLds : nsp;  // species of the loops; the ones in registers are one chunk more
+  static_assert(!kReg || kLds % kCh == 0, "whole chunks");
   double Yn[kCh];
 #pragma unroll
   for (int u = 0; u < kCh; ++u) Yn[u] = ys[(u < nsp ? u : 0) * p.plane];
   // finitechem_W: mass fractions clipped to [0, 1]
   double sy = 0.0, syw = 0.0, s1 = 0.0, s2 = 0.0, cpm = 0.0;
   double g1[kOne ? nsp : 1];
-#pragma unroll 1
-  for (int k0 = 0; k0 < nsp; k0 += kCh) {
+#pragma unroll
+  for (int tail = 0; tail < (kReg ? 2 : 1); ++tail)
+#pragma unroll 1  // (one turn of the tail: its register indices are constants)
+  for (int k0 = tail ? kLds : 0; k0 < (tail ? nsp : kLoop); k0 += kCh) {
     double Yc[kCh];
 #pragma unroll
     for (int u = 0; u < kCh; ++u) {
@@ -231,6 +245,7 @@ __global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per
       if (p.visc) {
         const double g = w14[k] * sqrt(num / ms);
         if constexpr (kOne) g1[u] = g;
+        else if (tail) gr[k - kLds] = g;
         else gs[k][threadIdx.x] = g;
       }
       if (p.diff) {
@@ -279,8 +294,10 @@ __global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per
       load_row(m, col);
 #pragma unroll
       for (int u = 0; u < kCh; ++u) Yn[u] = ys[(u < nsp ? u : 0) * p.plane];
+#pragma unroll
+      for (int tail = 0; tail < (kReg ? 2 : 1); ++tail)
 #pragma unroll 1
-      for (int q0 = 0; q0 < nsp; q0 += kCh) {
+      for (int q0 = tail ? kLds : 0; q0 < (tail ? nsp : kLoop); q0 += kCh) {
         double Yc[kCh];
 #pragma unroll
         for (int u = 0; u < kCh; ++u) {
@@ -294,7 +311,9 @@ __global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per
           if (nsp % kCh && q >= nsp) break;
           double mn[kPart];
           load_row(mn, col + (q + 1 < nsp ? q + 1 : 0) * kPart);
-          const double g = gs[q][threadIdx.x];
+          double g;
+          if (tail) g = gr[q - kLds];
+          else g = gs[q][threadIdx.x];
           const double y = Yc[u] * iw[q], yg = y * g, ygg = yg * g;
 #pragma unroll
           for (int k = 0; k < kPart; ++k) {
@@ -309,7 +328,8 @@ __global__ __launch_bounds__(props_block<NEQ>()) __attribute__((amdgpu_waves_per
 #pragma unroll
       for (int k = 0; k < kPart; ++k)
         if (k0 + k < nsp) {
-          const double Y = ys[(k0 + k) * p.plane], g = gs[k0 + k][threadIdx.x];
+          const double Y = ys[(k0 + k) * p.plane], g = k0 + k < kLds ? gs[k0 + k < kLds ? k0 + k : 0][threadIdx.x]
+                                                                          : gr[k0 + k < kLds ? 0 : k0 + k - kLds];
           const double s = fma(g, fma(g, a[k], 2.0 * b[k]), d[k]);
           visc += Y > 0.0 ? Y * iw[k0 + k] * w12[k0 + k] / s : 0.0;
         }

@@ -1,6 +1,8 @@
 """The BF16-MFMA perceptron kernels against the FP64 CPU reference
 (tests/mlp_ref.py): the product kernel in its four operand layouts, the
 forward pass, the loss gradient of every parameter, and Adam training."""
+import gc
+
 import numpy as np
 import pytest
 
@@ -191,12 +193,12 @@ def test_output_and_targets_at_any_offset(torch_dev, hidden):
 
 
 def test_training_where_the_fused_workspace_does_not_fit(torch_dev):
-    """A batch whose fused workspace (3.4 GB) is more than the free memory but
-    whose layered one (2.5 GB) is not: the gradients, losses and trained
+    """A batch whose fused workspace (13.4 GB) is more than the free memory but
+    whose layered one (10.0 GB) is not: the gradients, losses and trained
     parameters of the fused pass, then a small batch by the fused pass again."""
     torch = torch_dev
     from tiger_nga_amd import mlp
-    B = 1 << 18
+    B = 1 << 20
     nets = [_net_case(torch, B=64) for _ in range(2)]
     rng = torch.Generator(device="cuda").manual_seed(2)
     x = torch.zeros(B, 64, device="cuda", dtype=torch.bfloat16)
@@ -210,13 +212,18 @@ def test_training_where_the_fused_workspace_does_not_fit(torch_dev):
         return g, np.array(losses + small), net.get_params()
     want = train(nets[0][0])
     nets[0][0].close()
+    gc.collect()  # what earlier tests left
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
-    hog = torch.empty(torch.cuda.mem_get_info()[0] - int(2.95e9), dtype=torch.uint8, device="cuda")
+    hog, free0 = [], torch.cuda.mem_get_info()[0]
+    while free0 > 11.8e9 and len(hog) < 8:  # memory freed before may come back late
+        hog.append(torch.empty(free0 - int(11.7e9), dtype=torch.uint8, device="cuda"))
+        torch.cuda.synchronize()
+        free0 = torch.cuda.mem_get_info()[0]
     got = train(nets[1][0])
-    free = torch.cuda.mem_get_info()[0]
+    taken = free0 - torch.cuda.mem_get_info()[0]
     del hog
     torch.cuda.empty_cache()
-    assert free < 1.0e9  # the layered workspace is there
+    assert free0 < 12.0e9 and 8.5e9 < taken < 10.6e9  # the layered workspace
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[2], want[2])
     assert np.abs(got[1] - want[1]).max() <= 1e-5 * want[1].max()  # sums of the squared errors in another order

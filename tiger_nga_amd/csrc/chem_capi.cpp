@@ -279,8 +279,8 @@ size_t step_shape(const tgr_chem* c, int64_t ncell, int* grid, bool* lanes) {
 // few states there are, and pays once every CU has a wave (16,384 states on 256
 // CUs): rates of GRI-3.0 by wave / by lane 7 / 36 us at 256 states, 18 / 37 at
 // 8,192, 33 / 37 at 16,384, 54 / 38 at 32,768, 362 / 138 at 262,144; EthyRedF
-// 18 / 23, 31 / 23, 54 / 25, 352 / 92.  H2's rates are short: by lane always
-// (7 / 7 us at one state, 213 / 19 at 262,144).
+// 18 / 23 at 8,192, 31 / 23 at 16,384, 54 / 25 at 32,768, 352 / 92 at 262,144.
+// H2's rates are short: by lane always (7 / 7 us at one state, 213 / 19 at 262,144).
 bool rates_by_lane(const tgr_chem* c, int64_t n) {
   return c->rhs_mapping == 2 ? c->neq <= 10 || n >= (int64_t)64 * c->n_cu : c->rhs_mapping == 1;
 }

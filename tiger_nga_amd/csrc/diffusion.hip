@@ -369,9 +369,8 @@ __global__ __launch_bounds__(256) void diff_main_kernel(DiffParams p) {
 // After diff_cell_kernel: diff_face2_kernel (the correction velocities, whose
 // species sums the next pass needs complete) and diff_main2_kernel (the
 // per-cell terms).  Both are bound by the rate at which the L1 serves the loads
-// of Y and D (0.6 accesses per clock and CU, VALU busy a quarter of the time):
-// each species costs a cell 8 (14) of them and about 35 (105) FP64 instructions,
-// so
+// of Y and D (0.7 accesses per clock and CU, VALU busy 23 and 39 %): each species
+// costs a cell 8 (14) of them and 50 (155) VALU instructions, so
 //   * everything that does not depend on the species is formed before the
 //     species loop (operator coefficients, w / W_gp, sum grad * W_gp, the
 //     correction velocity), and the loop loads the next species while it
@@ -631,7 +630,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
 // x; weights that do not depend on the species stay in registers.  The fluxes
 // have no sum over the species, so those of a pass are split over blockIdx.z
 // until there are six workgroups per CU.  The workspace holds nchunk species, one
-// pass of them at a time.
+// pass of them at a time.  The velocities are bound by FP64 (divisions; VALU 54 %
+// busy) and L1 accesses (0.85 a clock and CU), the fluxes and their sums by the
+// fluxes' way through memory (128 bytes per cell and species).
 // DME39, 61 x 47 x 35 cells: 1144 (the general kernels) -> 309 us a call; GRI-3.0,
 // 126 x 124 x 120: 18.4 -> 5.31 ms; DME39, 16 x 17 x 18: 830 -> 80 us (294 us, 4.30
 // ms and 64 us with products for the quotients and the species' sums split over

@@ -355,8 +355,8 @@ def apply(fc, cells: int, path=CACHE) -> dict:
               "surr_newton_tol"):
         if k in rec:
             # "lane" was timed on a whole block: smaller batches go by their size
-            fc.set_option(k, 2 if k == "rhs_mapping" and rec[k] else rec[k])
-            done[k] = rec[k]
+            done[k] = 2 if k == "rhs_mapping" and rec[k] else rec[k]
+            fc.set_option(k, done[k])
     return done
 
 
